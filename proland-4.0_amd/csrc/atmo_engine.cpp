@@ -302,25 +302,30 @@ int jg_for_set(const atmo_params &p) {
 struct JSeg {   // a run of P_J tiles whose sets share one G
     int G, off, cnt;
 };
+struct NSeg {   // a run of P_SN tiles whose sets share one row class (texels per thread)
+    int cls, off, cnt;
+    int rows;   // largest rows-per-workgroup x RNU*RMU_S of its sets (k_inscatterN staging)
+};
 
 // Kernel variants chosen by the autotuner, with the times measured for each.
 struct Tuning {
-    int jG = 4, snCap = 4, snXcd = 1, snSb = 1;   // jG = 0: per-set choice
+    int jG = 4, snCap = 4, snXcd = 1, snSb = 2;   // jG = 0: per-set choice
     float msJ[5] = {0, 0, 0, 0, 0};  // G = 2, 3, 4, 8, per set (order-2 + order->=3 launches)
     float msN[27] = {};   // [direct, staged 1, staged 2][caps 1, 2, 4][plain, XCD, XCD + line order]
 };
 
-// staged samples per LDS round of a k_inscatterN form (1 direct: 0; 0, the
-// default before tuning: the one-sample rounds of form 3)
-int form_sb(int form) { return form == 1 ? 0 : (form == 2 ? 2 : 1); }
-// largest rows-per-workgroup x RNU*RMU_S of a batch (k_inscatterN staging)
-int sn_max_row_texels(const std::vector<atmo_params> &ps, int snCap) {
+// staged samples per LDS round of a k_inscatterN form (1 direct: 0; 3: 1; 0, the
+// default before tuning, as form 2: rounds of two samples, the faster ones at
+// every class but 16x64x16x4 (32 against 30 us); 32x128x32x8: 149 against 167 us)
+int form_sb(int form) { return form == 1 ? 0 : (form == 3 ? 1 : 2); }
+// mu rows a k_inscatterN workgroup covers with the cap snCap
+int sn_rows(const atmo_params &p, int snCap) {
+    return std::max(1, std::min(std::min(snCap, 4), 256 / (p.RES_MU_S * p.RES_NU)));
+}
+// largest LDS row staging of a tile table's segments
+int sn_max_row_texels(const std::vector<NSeg> &segs) {
     int m = 0;
-    for (const atmo_params &p : ps) {
-        const int W4 = p.RES_MU_S * p.RES_NU;
-        const int rpw = std::max(1, std::min(std::min(snCap, 4), 256 / W4));
-        m = std::max(m, rpw * W4);
-    }
+    for (const NSeg &g : segs) m = std::max(m, g.rows);
     return m;
 }
 
@@ -341,9 +346,10 @@ struct Plan {
     // kernel variants (picked by the autotuner)
     int jG = 4;        // k_inscatterS texels per thread (0: per set, see jg_for_set)
     std::vector<JSeg> jseg;   // P_J tiles grouped by the per-set G
+    std::vector<NSeg> nseg;   // P_SN tiles grouped by row class
     int snCap = 4;     // k_inscatterN max mu rows per workgroup
     int snXcd = 1;     // k_inscatterN XCD-banded tile order
-    int snSb = 1;      // k_inscatterN: 0 direct gathers, > 0 LDS-staged rows (samples per round)
+    int snSb = 2;      // k_inscatterN: 0 direct gathers, > 0 LDS-staged rows (samples per round)
     bool tuned = false;
     void drop_graph() {
         if (gexec) (void)hipGraphExecDestroy(gexec);
@@ -453,15 +459,88 @@ atmo_status upload_dirs(DevBuf &buf, hipStream_t xs, const atmo_options &o, size
     return ATMO_OK;
 }
 
+// The k_inscatterN tiles (workgroups of up to snCap mu rows) of a batch, grouped
+// by row class, most texels per thread first; appended to `tiles`.
+void build_sn_tiles(const std::vector<atmo_params> &ps, int snCap, int snXcd, std::vector<uint2> &tiles,
+                    std::vector<NSeg> &segs) {
+    struct Key {
+        uint32_t key, tile;
+    };
+    std::vector<Key> k, tmp;
+    std::vector<uint2> v;
+    const int base = (int)tiles.size();
+    for (int cls = 4; cls >= 1; --cls) {
+        NSeg seg{cls, (int)tiles.size() - base, 0, 0};
+        v.clear();
+        for (int i = 0; i < (int)ps.size(); ++i) {
+            const atmo_params &p = ps[i];
+            const int W4 = p.RES_MU_S * p.RES_NU;
+            if (row_class(W4) != cls) continue;
+            const int rpw = sn_rows(p, snCap), ngy = (p.RES_MU + rpw - 1) / rpw, nt = p.RES_R * ngy;
+            seg.rows = std::max(seg.rows, rpw * W4);
+            if (snXcd == 2) {
+                // "line order": a view ray is a straight line, fixed by its impact
+                // parameter r sqrt(1 - mu^2) and its half (up / down); rays of different
+                // layers on nearby lines gather the same dJ rows.  Sort a set's tiles by
+                // (half, impact parameter): as FP32 bit patterns, three radix passes.
+                k.resize(nt);
+                tmp.resize(nt);
+                for (int l = 0, t = 0; l < p.RES_R; ++l) {
+                    const LayerGeom g = layer_geom(p, l);
+                    for (int y = 0; y < ngy; ++y, ++t) {
+                        const double mu = row_mu(p, g, y * rpw);
+                        const float b = (float)(g.r * std::sqrt(std::max(0.0, 1.0 - mu * mu)));
+                        uint32_t u;
+                        memcpy(&u, &b, 4);
+                        k[t] = {u | (y * rpw < p.RES_MU / 2 ? 0u : 0x80000000u), (uint32_t)t};
+                    }
+                }
+                for (int sh = 0; sh < 33; sh += 11) {
+                    unsigned at[2049] = {0};
+                    for (const Key &e : k) at[((e.key >> sh) & 2047u) + 1] += 1;
+                    for (int q = 0; q < 2048; ++q) at[q + 1] += at[q];
+                    for (const Key &e : k) tmp[at[(e.key >> sh) & 2047u]++] = e;
+                    k.swap(tmp);
+                }
+                for (const Key &e : k) v.push_back(make_uint2((unsigned)i, e.tile));
+            } else {
+                for (int t = 0; t < nt; ++t) v.push_back(make_uint2((unsigned)i, (unsigned)t));
+            }
+        }
+        seg.cnt = (int)v.size();
+        if (!seg.cnt) continue;
+        segs.push_back(seg);
+        if (snXcd) {
+            // Workgroups are dealt round-robin to the 8 XCDs (each with its own L2);
+            // deal them so that XCD x runs a contiguous band of the launch's tiles (mu
+            // rows, or lines in line order), whose rays gather from overlapping parts
+            // of the dJ table.
+            const size_t nt = v.size(), chunk = (nt + kXcds - 1) / kXcds;
+            for (size_t q = 0; q < chunk; ++q)
+                for (size_t x = 0; x < kXcds; ++x)
+                    if (x * chunk + q < nt) tiles.push_back(v[x * chunk + q]);
+        } else {
+            tiles.insert(tiles.end(), v.begin(), v.end());
+        }
+    }
+}
+
 // Tile tables of every pass for a batch.  The spherical-integral passes list
 // the most expensive tiles first so mixed-resolution batches drain evenly.
 void build_tiles(const std::vector<atmo_params> &ps, const atmo_options &o,
                  std::vector<uint2> &tiles, int off[P_COUNT], int cnt[P_COUNT], int snCap = 4,
-                 int snXcd = 1, std::vector<JSeg> *jseg = nullptr) {
+                 int snXcd = 1, std::vector<JSeg> *jseg = nullptr, std::vector<NSeg> *nseg = nullptr) {
     tiles.clear();
     const int n = (int)ps.size();
     for (int pass = 0; pass < P_COUNT; ++pass) {
         off[pass] = (int)tiles.size();
+        if (pass == P_SN) {
+            std::vector<NSeg> segs;
+            if (o.orders >= 2) build_sn_tiles(ps, snCap, snXcd, tiles, segs);
+            cnt[pass] = (int)tiles.size() - off[pass];
+            if (nseg) nseg->swap(segs);
+            continue;
+        }
         std::vector<std::pair<double, uint2>> v;
         for (int i = 0; i < n; ++i) {
             const atmo_params &p = ps[i];
@@ -478,13 +557,6 @@ void build_tiles(const std::vector<atmo_params> &ps, const atmo_options &o,
                 nt = (long long)p.RES_R * ((p.RES_MU + rpw - 1) / rpw);
                 break;
             }
-            case P_SN: {
-                // workgroups of up to snCap mu rows (k_inscatterN)
-                const int W4 = p.RES_MU_S * p.RES_NU;
-                const int rpw = std::max(1, std::min(snCap, 256 / W4));
-                nt = (long long)p.RES_R * ((p.RES_MU + rpw - 1) / rpw);
-                break;
-            }
             case P_J:
                 // grouped by the per-set G (descending), most expensive first inside a group
                 nt = (long long)p.RES_R * p.RES_MU_S;
@@ -495,7 +567,6 @@ void build_tiles(const std::vector<atmo_params> &ps, const atmo_options &o,
             }
             if (pass == P_J && o.orders < 2) nt = 0;
             if (pass == P_EN && o.orders < 2) nt = 0;
-            if (pass == P_SN && o.orders < 2) nt = 0;
             for (long long t = 0; t < nt; ++t) v.push_back({cost, make_uint2((unsigned)i, (unsigned)t)});
         }
         if (pass == P_J || pass == P_EN)
@@ -503,41 +574,6 @@ void build_tiles(const std::vector<atmo_params> &ps, const atmo_options &o,
                              [](const std::pair<double, uint2> &a, const std::pair<double, uint2> &b) {
                                  return a.first > b.first;
                              });
-        if (pass == P_SN && snXcd == 2) {
-            // "line order": a view ray is a straight line, fixed by its impact
-            // parameter r sqrt(1 - mu^2) and its half (up / down); rays of different
-            // layers on nearby lines gather the same dJ rows.  Sort the tiles by
-            // (set, half, impact parameter) before dealing them to the XCDs.
-            std::vector<std::pair<std::pair<double, double>, uint2>> k;
-            k.reserve(v.size());
-            for (auto &e : v) {
-                const atmo_params &p = ps[e.second.x];
-                const int W4 = p.RES_MU_S * p.RES_NU;
-                const int rpw = std::max(1, std::min(std::min(snCap, 4), 256 / W4));
-                const int ngy = (p.RES_MU + rpw - 1) / rpw;
-                const int l = (int)e.second.y / ngy, yb = ((int)e.second.y % ngy) * rpw;
-                const LayerGeom g = layer_geom(p, l);
-                const double mu = row_mu(p, g, yb);
-                const double half = yb < p.RES_MU / 2 ? 0.0 : 1.0;
-                k.push_back({{e.second.x * 2.0 + half, g.r * std::sqrt(std::max(0.0, 1.0 - mu * mu))}, e.second});
-            }
-            std::stable_sort(k.begin(), k.end(), [](const auto &a, const auto &b) { return a.first < b.first; });
-            for (size_t i = 0; i < v.size(); ++i) v[i].second = k[i].second;
-        }
-        if (pass == P_SN && snXcd) {
-            // Workgroups are dealt round-robin to the 8 XCDs (each with its own L2);
-            // deal them so that XCD x runs a contiguous band of tiles (mu rows, or
-            // lines in line order), whose rays gather from overlapping parts of the
-            // dJ table.
-            const size_t nt = v.size(), chunk = (nt + kXcds - 1) / kXcds;
-            std::vector<std::pair<double, uint2>> w;
-            w.reserve(nt);
-            for (size_t p = 0; p < chunk * kXcds; ++p) {
-                const size_t src = (p % kXcds) * chunk + p / kXcds;
-                if (src < nt) w.push_back(v[src]);
-            }
-            v.swap(w);
-        }
         if (pass == P_J && jseg) {
             jseg->clear();
             for (size_t i = 0; i < v.size(); ++i) {
@@ -585,6 +621,17 @@ hipError_t launch_dj(const Plan &pl, const SetDesc *S, const uint2 *T, const cha
     for (const JSeg &g : pl.jseg) {
         hipError_t e = launch_inscatterS(S, T + pl.off[P_J] + g.off, g.cnt, o.spherical_samples, ch, pl.maxNU, pl.jx,
                                          dirs + pl.dirJT_off, dirs + pl.dirJW_off, first, lds, g.G, st);
+        if (e != hipSuccess) return e;
+    }
+    return hipSuccess;
+}
+
+// The dSn pass: one launch per row class.  S: descriptors; T: the pass's tiles.
+hipError_t launch_dsn(const SetDesc *S, const uint2 *T, const std::vector<NSeg> &segs, const atmo_options &o, int snCap,
+                      int sb, hipStream_t st) {
+    for (const NSeg &g : segs) {
+        hipError_t e = launch_inscatterN(S, T + g.off, g.cnt, o.inscatter_samples, snCap, sb, g.cls,
+                                         lds_inscatterN(g.rows, sb), lin_4(o), st);
         if (e != hipSuccess) return e;
     }
     return hipSuccess;
@@ -648,9 +695,7 @@ atmo_status launch_all(Plan &pl, hipStream_t st, PassTimer *tm = nullptr) {
                                   first ? pl.ldsE1 : pl.ldsEN, st));
         HIPCHK(t.end());
         HIPCHK(t.begin(5, order));
-        HIPCHK(launch_inscatterN(S, T + pl.off[P_SN], pl.cnt[P_SN], o.inscatter_samples, pl.snCap, pl.snSb,
-                                 lds_inscatterN(sn_max_row_texels(pl.params, pl.snCap), pl.snSb), lin_4(o),
-                                 st));
+        HIPCHK(launch_dsn(S, T + pl.off[P_SN], pl.nseg, o, pl.snCap, pl.snSb, st));
         HIPCHK(t.end());
     }
     return ATMO_OK;
@@ -762,20 +807,20 @@ atmo_status autotune(Plan &pl, hipStream_t st, Tuning &tu) {
     for (int si = 0; si < 3; ++si)
     for (int ci = 0; ci < 3; ++ci)
         for (int xo = 0; xo < 3; ++xo) {
-            const size_t lds = lds_inscatterN(sn_max_row_texels(pl.params, caps[ci]), sbs[si]);
+            std::vector<uint2> tiles;
+            std::vector<NSeg> segs;
+            int off[P_COUNT], cnt[P_COUNT];
+            build_tiles(pl.params, o, tiles, off, cnt, caps[ci], xo, nullptr, &segs);
+            const size_t lds = lds_inscatterN(sn_max_row_texels(segs), sbs[si]);
             if (lds + static_lds_inscatterN() > (size_t)maxLds) {  // does not fit this device's LDS
                 tu.msN[si * 9 + ci * 3 + xo] = -1.f;
                 continue;
             }
-            std::vector<uint2> tiles;
-            int off[P_COUNT], cnt[P_COUNT];
-            build_tiles(pl.params, o, tiles, off, cnt, caps[ci], xo);
             HIPCHK(dt.ensure(tiles.size() * sizeof(uint2)));
             HIPCHK(h2d(dt.p, tiles.data(), tiles.size() * sizeof(uint2), pl.xs));
             float ms = 0.f;
             atmo_status rc = time_launch(st, ms, [&]() {
-                return launch_inscatterN((const SetDesc *)ds.p, (const uint2 *)dt.p + off[P_SN], cnt[P_SN],
-                                         o.inscatter_samples, caps[ci], sbs[si], lds, lin_4(o), st);
+                return launch_dsn((const SetDesc *)ds.p, (const uint2 *)dt.p + off[P_SN], segs, o, caps[ci], sbs[si], st);
             });
             if (rc != ATMO_OK) return rc;
             tu.msN[si * 9 + ci * 3 + xo] = ms;
@@ -800,7 +845,7 @@ atmo_status apply_tuning(Plan &pl, const Tuning &tu) {
     pl.tuned = true;
     if (retile) {
         std::vector<uint2> tiles;
-        build_tiles(pl.params, pl.opts, tiles, pl.off, pl.cnt, pl.snCap, pl.snXcd, &pl.jseg);
+        build_tiles(pl.params, pl.opts, tiles, pl.off, pl.cnt, pl.snCap, pl.snXcd, &pl.jseg, &pl.nseg);
         HIPCHK(pl.dtiles.ensure(tiles.size() * sizeof(uint2)));
         HIPCHK(h2d(pl.dtiles.p, tiles.data(), tiles.size() * sizeof(uint2), pl.xs));
     }
@@ -871,7 +916,7 @@ atmo_status build_plan(hipStream_t xs, const atmo_params *sets, int nsets, const
     HIPCHK(R.get(pl->dsets, nsets * sizeof(SetDesc)));
     // tiles
     std::vector<uint2> tiles;
-    build_tiles(pl->params, o, tiles, pl->off, pl->cnt, pl->snCap, pl->snXcd, &pl->jseg);
+    build_tiles(pl->params, o, tiles, pl->off, pl->cnt, pl->snCap, pl->snXcd, &pl->jseg, &pl->nseg);
     HIPCHK(R.get(pl->dtiles, tiles.size() * sizeof(uint2)));
     HIPCHK(h2d(pl->dtiles.p, tiles.data(), tiles.size() * sizeof(uint2), pl->xs));
     HIPCHK(R.get(pl->dflags, nsets * sizeof(unsigned)));
@@ -1319,7 +1364,8 @@ static atmo_status pass_run(atmo_engine *e, const atmo_params *p, const atmo_opt
     std::vector<atmo_params> ps(1, *p);
     atmo_options ot = o;
     ot.orders = std::max(ot.orders, 2);  // every pass gets its tiles
-    build_tiles(ps, ot, tiles, off, cnt);
+    std::vector<NSeg> nseg;
+    build_tiles(ps, ot, tiles, off, cnt, 4, 1, nullptr, &nseg);
     HIPCHK(e->pass_tiles.ensure(tiles.size() * sizeof(uint2)));
     HIPCHK(h2d(e->pass_tiles.p, tiles.data(), tiles.size() * sizeof(uint2), e->cap));
     size_t oJT, oJW, oE;
@@ -1352,8 +1398,7 @@ static atmo_status pass_run(atmo_engine *e, const atmo_params *p, const atmo_opt
     }
     case P_SN: {
         const int sb = form_sb(o.inscatterN_form);
-        const size_t lds = lds_inscatterN(sn_max_row_texels(std::vector<atmo_params>(1, *p), 4), sb);
-        HIPCHK(launch_inscatterN(S, T + off[P_SN], cnt[P_SN], o.inscatter_samples, 4, sb, lds, lin_4(o), hs));
+        HIPCHK(launch_dsn(S, T + off[P_SN], nseg, o, 4, sb, hs));
         break;
     }
     }

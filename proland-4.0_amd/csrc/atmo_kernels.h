@@ -60,11 +60,13 @@ hipError_t launch_irradianceN(const SetDesc *sets, const uint2 *tiles, int ntile
 // rpw_cap: at most this many mu rows per workgroup (1, 2 or 4); the tile table
 // must have been built with the same cap.  sb = 0: direct gathers; sb > 0:
 // LDS-staged blended rows, sb samples per round, lds = lds_inscatterN(max over
-// the batch of rows-per-workgroup x RNU*RMU_S, sb) bytes of dynamic LDS.
+// the launch's sets of rows-per-workgroup x RNU*RMU_S, sb) bytes of dynamic LDS.
+// row_class: texels per thread of the launch's sets (one launch per class).
+inline int row_class(int W4) { return W4 <= 256 ? 1 : (W4 + 255) / 256; }   // 1 .. 4: W4 <= 1024
 size_t lds_inscatterN(int max_row_texels, int sb);
 size_t static_lds_inscatterN();   // bytes of k_inscatterN's static LDS
 hipError_t launch_inscatterN(const SetDesc *sets, const uint2 *tiles, int ntiles, int nsamp,
-                             int rpw_cap, int sb, size_t lds, bool lin4, hipStream_t st);
+                             int rpw_cap, int sb, int row_class, size_t lds, bool lin4, hipStream_t st);
 hipError_t launch_check(const SetDesc *sets, const uint2 *tiles, int ntiles, unsigned int *flags,
                         hipStream_t st);
 

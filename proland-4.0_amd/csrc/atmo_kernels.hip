@@ -1006,6 +1006,15 @@ __device__ __forceinline__ float sn_txs(const SetDesc &s, float nu, float mus, f
     return fmaf(atanf(arg), half * (1.0f / 1.1f), near ? txb : 0.74f * half);
 }
 
+// Waves per SIMD the register budget of a k_inscatterN instantiation is cut to.
+// The kernel waits on its row gathers and on a barrier per LDS round, so more
+// waves help until the budget spills.  Per order, rows of 256 texels
+// (32x128x32x8): 135 us at 4 and 5 waves, 138 at 6, 153 at 8; 48-set batch of
+// mixed classes: 13.96 ms at (5, 5, 4, 4) for 1-4 texels per thread, 14.08 at
+// (4, 3, 3, 3), 15.2 at (7, 4, 5, 3).  One kernel for all classes, at three
+// waves, took 170 us and 16.2 ms.
+constexpr int sn_waves(int NM) { return NM <= 2 ? 5 : 4; }
+
 // STAGED = false: each texel gathers its 8 taps per sample from dJ directly
 // (global loads).  STAGED = true: per sample the workgroup first blends the
 // 4 (r, mu) table rows of every row it covers into one row
@@ -1014,21 +1023,17 @@ __device__ __forceinline__ float sn_txs(const SetDesc &s, float nu, float mus, f
 // neighbours of B_i and lerps in x.  The direct form blends the two columns
 // it needs in the same order (sn_blend, sn_lerp), so both give the same bits.
 // `sb` samples are blended per LDS round (dynamic LDS: sb * rows * RNU*RMU_S
-// float4).  A workgroup covers rows of RNU*RMU_S <= 256 texels with one texel
-// per thread, or one row of more with 2-4 texels per thread: the staged form
-// has a path for each.  In the second, a sample whose 4 rows are those of the
-// sample before it in the same LDS round blends the loaded rows again (the
-// row starts are workgroup-uniform there, so the test is a scalar branch).
-// Three waves per SIMD (up to 168 VGPRs): at four (128 VGPRs) the staged form
-// spills 116 bytes per lane, whose traffic shows in the kernel's HBM counters,
-// and both builds run at the same speed (2.31 and 2.33 ms per launch at
-// 64x256x64x16), the loads of a thread's texels being in flight together.
-template <bool STAGED, bool LIN4>   // LIN4: linear inscatter parameterisation (per-sample mu_s)
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void k_inscatterN(const SetDesc *__restrict__ sets,
-                                                    const uint2 *__restrict__ tiles,
-                                                    int nsamp, int rpw_cap, int sb) {
-    __shared__ SnEntry ent[kNRows][kNChunk];   // exactly 16 KiB: two workgroups of 64 KiB
-                                               // dynamic staging fit one CU's 160 KiB
+// float4).  NM: texels per thread.  A workgroup covers rows of RNU*RMU_S <= 256
+// texels with one texel per thread (NM = 1), or one row of more (NM = 2 .. 4):
+// the staged form has a path for each, and each NM is its own instantiation and
+// launch, so that its registers are what its class needs.  With NM >= 2, a
+// sample whose 4 rows are those of the sample before it in the same LDS round
+// blends the loaded rows again (the row starts are workgroup-uniform there, so
+// the test is a scalar branch).
+template <bool STAGED, bool LIN4, int NM>   // LIN4: linear inscatter parameterisation (per-sample mu_s)
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(sn_waves(NM))))
+void k_inscatterN(const SetDesc *__restrict__ sets, const uint2 *__restrict__ tiles, int nsamp, int rpw_cap, int sb) {
+    __shared__ SnEntry ent[NM == 1 ? kNRows : 1][kNChunk];
     extern __shared__ float4 blend[];   // [sb][nrows * W4] (STAGED)
     const uint2 tl = tiles[blockIdx.x];
     const SetDesc &s = sets[tl.x];
@@ -1044,18 +1049,16 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void k
 
     // texels of this thread: rows yb.. (row-major, x fastest)
     const int per = nrows * s.W4;
-    const int nmine = (per + (int)blockDim.x - 1) / (int)blockDim.x;
-    constexpr int MAXT = 4;   // W4 <= 1024 (validated on the host)
-    float acc[MAXT][3];
-    float nuf[MAXT], muSr[MAXT], txb[MAXT], fk[MAXT];
-    int kq[MAXT];   // the texel's nu slice k0 (< RNU) | its row in the workgroup << 16
+    float acc[NM][3];
+    float nuf[NM], muSr[NM], txb[NM], fk[NM];
+    int kq[NM];   // the texel's nu slice k0 (< RNU) | its row in the workgroup << 16
 #pragma unroll
-    for (int j = 0; j < MAXT; ++j) {
+    for (int j = 0; j < NM; ++j) {
         acc[j][0] = acc[j][1] = acc[j][2] = 0.f;
         nuf[j] = muSr[j] = txb[j] = fk[j] = 0.f;
         kq[j] = 0;
         const int e = threadIdx.x + j * (int)blockDim.x;
-        if (j < nmine && e < per) {
+        if (e < per) {
             const int row = e / s.W4, x = e % s.W4;
             double mu, muS, nu;
             mu_mus_nu(s, L, x, yb + row, mu, muS, nu);
@@ -1131,10 +1134,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void k
             ent[row][js] = en;
         }
         __syncthreads();
-        if (!STAGED) {
+        if constexpr (!STAGED) {
 #pragma unroll
-            for (int j = 0; j < MAXT; ++j) {
-                if (j >= nmine) break;
+            for (int j = 0; j < NM; ++j) {
                 const int e = threadIdx.x + j * (int)blockDim.x;
                 if (e >= per) break;
                 const SnEntry *er = ent[kq[j] >> 16];
@@ -1167,91 +1169,85 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void k
                 }
                 acc[j][0] = a0; acc[j][1] = a1; acc[j][2] = a2;
             }
-        } else if (nmine >= 2) {
+        } else if constexpr (NM >= 2) {
             // Rows of more than 256 texels (one row per workgroup, 2-4 texels
             // per thread): every slot reads the same sample entries, so (a)
             // issues all 4 * NM table loads of a thread before blending any,
             // and (b) interleaves the NM independent lookups of a sample.  The
             // arithmetic of each texel-sample is that of the general path.
-            auto one_row = [&](auto nmc) {
-                constexpr int NM = decltype(nmc)::value;
-                for (int s0 = 0; s0 < nc; s0 += sb) {
-                    const int ns = min(sb, nc - s0);
-                    // the table rows of the last sample loaded in this round: a later
-                    // sample on the same 4 rows (same first and last row start, which fix
-                    // the two layers and the two mu rows) blends them again without
-                    // loading (kept within a round: carried over the lookups, t would
-                    // spill at three waves per SIMD)
-                    float3 t[NM][4];
-                    unsigned P0 = 0u, P3 = 0u;
-                    for (int k = 0; k < ns; ++k) {
-                        const float4 w = ent[0][s0 + k].w;
-                        const int4 base = ent[0][s0 + k].base;
-                        // the 4 row starts are the same for the whole workgroup: in
-                        // scalar registers, the loads take them as their base and
-                        // the thread's own column offset (fixed over the samples)
-                        const unsigned R0 = (unsigned)__builtin_amdgcn_readfirstlane(base.x);
-                        const unsigned R1 = (unsigned)__builtin_amdgcn_readfirstlane(base.y);
-                        const unsigned R2 = (unsigned)__builtin_amdgcn_readfirstlane(base.z);
-                        const unsigned R3 = (unsigned)__builtin_amdgcn_readfirstlane(base.w);
-                        if (k == 0 || R0 != P0 || R3 != P3) {
-                            P0 = R0;
-                            P3 = R3;
-#pragma unroll
-                            for (int j = 0; j < NM; ++j) {
-                                // past the row's end: a valid address, the blend is not stored
-                                const unsigned xo = (unsigned)min((int)threadIdx.x + j * (int)blockDim.x, per - 1) * jb;
-                                t[j][0] = ld3b(Jr, xo, R0);
-                                t[j][1] = ld3b(Jr, xo, R1);
-                                t[j][2] = ld3b(Jr, xo, R2);
-                                t[j][3] = ld3b(Jr, xo, R3);
-                            }
-                        }
+            for (int s0 = 0; s0 < nc; s0 += sb) {
+                const int ns = min(sb, nc - s0);
+                // the table rows of the last sample loaded in this round: a later
+                // sample on the same 4 rows (same first and last row start, which fix
+                // the two layers and the two mu rows) blends them again without
+                // loading (kept within a round: carried over the lookups, t would
+                // spill at three waves per SIMD)
+                float3 t[NM][4];
+                unsigned P0 = 0u, P3 = 0u;
+                for (int k = 0; k < ns; ++k) {
+                    const float4 w = ent[0][s0 + k].w;
+                    const int4 base = ent[0][s0 + k].base;
+                    // the 4 row starts are the same for the whole workgroup: in
+                    // scalar registers, the loads take them as their base and
+                    // the thread's own column offset (fixed over the samples)
+                    const unsigned R0 = (unsigned)__builtin_amdgcn_readfirstlane(base.x);
+                    const unsigned R1 = (unsigned)__builtin_amdgcn_readfirstlane(base.y);
+                    const unsigned R2 = (unsigned)__builtin_amdgcn_readfirstlane(base.z);
+                    const unsigned R3 = (unsigned)__builtin_amdgcn_readfirstlane(base.w);
+                    if (k == 0 || R0 != P0 || R3 != P3) {
+                        P0 = R0;
+                        P3 = R3;
 #pragma unroll
                         for (int j = 0; j < NM; ++j) {
-                            const int e = threadIdx.x + j * (int)blockDim.x;
-                            const float3 b = sn_blend(w, t[j][0], t[j][1], t[j][2], t[j][3]);
-                            if (e < per) blend[(size_t)k * per + e] = make_float4(b.x, b.y, b.z, 0.f);
+                            // past the row's end: a valid address, the blend is not stored
+                            const unsigned xo = (unsigned)min((int)threadIdx.x + j * (int)blockDim.x, per - 1) * jb;
+                            t[j][0] = ld3b(Jr, xo, R0);
+                            t[j][1] = ld3b(Jr, xo, R1);
+                            t[j][2] = ld3b(Jr, xo, R2);
+                            t[j][3] = ld3b(Jr, xo, R3);
                         }
                     }
-                    __syncthreads();
-                    for (int k = 0; k < ns; ++k) {
-                        const SnEntry en = ent[0][s0 + k];
-                        const float4 *B = blend + (size_t)k * per;
-                        float3 v[NM];
-                        unsigned i0[NM];
-                        float ax[NM];
 #pragma unroll
-                        for (int j = 0; j < NM; ++j) {
-                            // slots past the row's end (kq 0) read in-row values and are never stored
-                            const unsigned kbase = (unsigned)((kq[j] & 0xffff) * s.RMUS);
-                            const float txs = __builtin_amdgcn_fmed3f(sn_txs<LIN4>(s, nuf[j], muSr[j], txb[j], en), 0.0f,
-                                                                      (float)(W4m2 + 1 - kbase));
-                            const unsigned is = min(__float2uint_rz(txs), W4m2 - kbase);
-                            ax[j] = txs - (float)is;
-                            i0[j] = kbase + is;
-                            v[j] = sn_lerp(ax[j], f3(B[i0[j]]), f3(B[i0[j] + 1]));
-                        }
-#pragma unroll
-                        for (int j = 0; j < NM; ++j) {
-                            if (fk[j] != 0.0f) {  // off-grid nu: blend with the next slice (k0 + 1 <= RNU - 1)
-                                unsigned j0 = i0[j] + (unsigned)s.RMUS;
-                                float bx = ax[j];
-                                if (j0 > W4m2) { j0 = W4m2; bx = 1.0f; }   // past the row's last column
-                                v[j] = lerp3(v[j], sn_lerp(bx, f3(B[j0]), f3(B[j0 + 1])), fk[j]);
-                            }
-                            acc[j][0] = fmaf(v[j].x, en.tw.x, acc[j][0]);
-                            acc[j][1] = fmaf(v[j].y, en.tw.y, acc[j][1]);
-                            acc[j][2] = fmaf(v[j].z, en.tw.z, acc[j][2]);
-                        }
+                    for (int j = 0; j < NM; ++j) {
+                        const int e = threadIdx.x + j * (int)blockDim.x;
+                        const float3 b = sn_blend(w, t[j][0], t[j][1], t[j][2], t[j][3]);
+                        if (e < per) blend[(size_t)k * per + e] = make_float4(b.x, b.y, b.z, 0.f);
                     }
-                    __syncthreads();
                 }
-            };
-            if (nmine == 2) one_row(std::integral_constant<int, 2>{});
-            else if (nmine == 3) one_row(std::integral_constant<int, 3>{});
-            else one_row(std::integral_constant<int, MAXT>{});
-        } else if (nmine == 1) {
+                __syncthreads();
+                for (int k = 0; k < ns; ++k) {
+                    const SnEntry en = ent[0][s0 + k];
+                    const float4 *B = blend + (size_t)k * per;
+                    float3 v[NM];
+                    unsigned i0[NM];
+                    float ax[NM];
+#pragma unroll
+                    for (int j = 0; j < NM; ++j) {
+                        // slots past the row's end (kq 0) read in-row values and are never stored
+                        const unsigned kbase = (unsigned)((kq[j] & 0xffff) * s.RMUS);
+                        const float txs = __builtin_amdgcn_fmed3f(sn_txs<LIN4>(s, nuf[j], muSr[j], txb[j], en), 0.0f,
+                                                                  (float)(W4m2 + 1 - kbase));
+                        const unsigned is = min(__float2uint_rz(txs), W4m2 - kbase);
+                        ax[j] = txs - (float)is;
+                        i0[j] = kbase + is;
+                        v[j] = sn_lerp(ax[j], f3(B[i0[j]]), f3(B[i0[j] + 1]));
+                    }
+#pragma unroll
+                    for (int j = 0; j < NM; ++j) {
+                        if (fk[j] != 0.0f) {  // off-grid nu: blend with the next slice (k0 + 1 <= RNU - 1)
+                            unsigned j0 = i0[j] + (unsigned)s.RMUS;
+                            float bx = ax[j];
+                            if (j0 > W4m2) { j0 = W4m2; bx = 1.0f; }   // past the row's last column
+                            v[j] = lerp3(v[j], sn_lerp(bx, f3(B[j0]), f3(B[j0 + 1])), fk[j]);
+                        }
+                        acc[j][0] = fmaf(v[j].x, en.tw.x, acc[j][0]);
+                        acc[j][1] = fmaf(v[j].y, en.tw.y, acc[j][1]);
+                        acc[j][2] = fmaf(v[j].z, en.tw.z, acc[j][2]);
+                    }
+                }
+                __syncthreads();
+            }
+        } else {
             // Rows of at most 256 texels (one texel per thread): samples are
             // blended and looked up in pairs, so a thread has 8 table loads and
             // two independent lookups in flight; the accumulation keeps sample
@@ -1327,8 +1323,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void k
         }
     }
 #pragma unroll
-    for (int j = 0; j < MAXT; ++j) {
-        if (j >= nmine) break;
+    for (int j = 0; j < NM; ++j) {
         const int e = threadIdx.x + j * (int)blockDim.x;
         if (e >= per) break;
         const int row = e / s.W4, x = e % s.W4;
@@ -1561,17 +1556,28 @@ size_t static_lds_inscatterN() { return sizeof(SnEntry) * kNRows * kNChunk; }
 size_t lds_inscatterN(int max_row_texels, int sb) {
     return sb > 0 ? sizeof(float4) * (size_t)sb * (size_t)max_row_texels : 0;
 }
-hipError_t launch_inscatterN(const SetDesc *sets, const uint2 *tiles, int ntiles, int nsamp,
-                             int rpw_cap, int sb, size_t lds, bool lin4, hipStream_t st) {
-    if (ntiles <= 0) return hipSuccess;
+template <int NM>
+static void launch_sn(const SetDesc *sets, const uint2 *tiles, int ntiles, int nsamp, int rpw_cap, int sb,
+                      size_t lds, bool lin4, hipStream_t st) {
 #define ATMO_LN(S, L, LDS, SB) \
-    hipLaunchKernelGGL((k_inscatterN<S, L>), dim3(ntiles), dim3(256), LDS, st, sets, tiles, nsamp, rpw_cap, SB)
+    hipLaunchKernelGGL((k_inscatterN<S, L, NM>), dim3(ntiles), dim3(256), LDS, st, sets, tiles, nsamp, rpw_cap, SB)
     if (sb > 0) {
         if (lin4) ATMO_LN(true, true, lds, sb); else ATMO_LN(true, false, lds, sb);
     } else {
         if (lin4) ATMO_LN(false, true, 0, 0); else ATMO_LN(false, false, 0, 0);
     }
 #undef ATMO_LN
+}
+hipError_t launch_inscatterN(const SetDesc *sets, const uint2 *tiles, int ntiles, int nsamp, int rpw_cap, int sb,
+                             int row_class, size_t lds, bool lin4, hipStream_t st) {
+    if (ntiles <= 0) return hipSuccess;
+    switch (row_class) {
+    case 1: launch_sn<1>(sets, tiles, ntiles, nsamp, rpw_cap, sb, lds, lin4, st); break;
+    case 2: launch_sn<2>(sets, tiles, ntiles, nsamp, rpw_cap, sb, lds, lin4, st); break;
+    case 3: launch_sn<3>(sets, tiles, ntiles, nsamp, rpw_cap, sb, lds, lin4, st); break;
+    case 4: launch_sn<4>(sets, tiles, ntiles, nsamp, rpw_cap, sb, lds, lin4, st); break;
+    default: return hipErrorInvalidValue;
+    }
     return hipGetLastError();
 }
 hipError_t launch_check(const SetDesc *sets, const uint2 *tiles, int ntiles, unsigned int *flags,
