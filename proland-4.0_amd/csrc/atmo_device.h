@@ -29,6 +29,24 @@ struct LayerGeom {
     double dhdH[4];  // FP32 uniform dhdH
 };
 
+// A mu_s column's terms of the dSn samples' mu_s offsets (sn_txs): k mu_s,
+// k (mu_s - mu_b), k (-0.1975 - mu_b), k mu_b, 1 + (k mu_b)^2 and the column's own
+// texel offset, with mu_b = max(mu_s, -0.1975) and k = tan(1.386).  Linear
+// parameterisation: mu_s and, in txb, mu_s + 0.2.
+struct ColGeom {
+    float mus, ck, lo, kb, kb2, txb;
+};
+
+// A view-ray sample of the dSn pass (k_snview): what does not involve the sun.
+// The 4 dJ rows around it (2 layers x 2 mu rows) are named by the parities of
+// their layer and mu row, so that a row keeps its name from sample to sample.
+struct SnView {
+    float az, ay;    // bilinear weights of the odd layer and the odd mu row
+    int row;         // 8 (layer RMU + mu row) of the first row; + 1: second mu row is the next one,
+                     // + 2: second layer is the next one (else the same, at an edge), + 4: the layer is odd
+    float dr;        // (r_i - r) / r_i; sample 0, where that is 0: the trapezoid step of the ray
+};
+
 struct SetDesc {
     // FP32 parameters promoted to double
     double Rg, Rt, RL, HR, HM, mieG, alpha;
@@ -51,15 +69,17 @@ struct SetDesc {
     float4 *T4, *dE4, *E4, *dSR4, *dSM4, *dJ4, *S4;
     float4 *tau4;                   // optical depth -ln T of the T texels (rgb), or null
     // transmittances along the view ray of each (layer, mu row) at the inscatter
-    // samples, [RR][RMU][nsamp + 1], and from the ground point to each layer
+    // samples (trapezoid weights folded in), [RR][RMU][nsamp + 1] (w: the sample's t / r_i), and from the ground point to each layer
     // radius per theta row of the spherical integral, [RR][NS]; null: computed
     // inline from T (pass-level entry points)
     float4 *tview, *tground;
+    SnView *view;                   // [RR][RMU][nsamp + 1]; null: computed in k_inscatterN
     int dJb;                        // bytes per dJ texel: 16 (float4) or 12 (packed rgb)
     int hs;                         // 1: table values rounded to FP16 on store (q16)
     int linT, lin4;                 // 1: the linear transmittance / inscatter parameterisation
     float *outT, *outE;
     const LayerGeom *layers;
+    const ColGeom *cols;            // [RMUS]
 };
 
 // ---------------------------------------------------------------------------

@@ -51,7 +51,7 @@ atmo_status fail(atmo_status st, const char *fmt, ...) {
                         "%s: %s (%s:%d)", #expr, hipGetErrorString(e_), __FILE__, __LINE__); \
     } while (0)
 
-enum Pass { P_T = 0, P_E1, P_S1, P_J, P_EN, P_SN, P_CHECK, P_COUNT };
+enum Pass { P_T = 0, P_E1, P_S1, P_J, P_EN, P_SN, P_VIEW, P_CHECK, P_COUNT };
 
 constexpr size_t kXcds = 8;  // MI355X accelerator complex dies
 constexpr size_t kJBlock = 16;   // dJ tiles (mu_s columns) dealt to one XCD together
@@ -172,6 +172,18 @@ double row_mu(const atmo_params &p, const LayerGeom &g, int y) {
     return std::min(std::max(mu, -1.0), 1.0);
 }
 
+// The mu_s column terms of the dSn pass (ColGeom; texture4D's mu_s axis, common.glsl:149-173).
+ColGeom col_geom(const atmo_params &p, const atmo_options &o, int m) {
+    const bool lin = (o.flags & ATMO_FLAG_LINEAR_INSCATTER) != 0;
+    const double k = (double)(float)std::tan(1.26 * 1.1), f = m / (p.RES_MU_S - 1.0);
+    const double muS = lin ? -0.2 + f * 1.2 : std::tan((2.0 * f - 1.0 + 0.26) * 1.1) / std::tan(1.26 * 1.1);
+    const double mub = std::max(muS, -0.1975);
+    if (lin) return {(float)muS, 0.f, 0.f, 0.f, 0.f, (float)(muS + 0.2)};
+    return {(float)(k * muS), (float)(k * (muS - mub)), (float)(k * (-0.1975 - mub)), (float)(k * mub),
+            (float)(1.0 + k * mub * (k * mub)),
+            (float)((std::atan(mub * std::tan(1.26 * 1.1)) / 1.1 + (1.0 - 0.26)) * 0.5 * (p.RES_MU_S - 1.0))};
+}
+
 void fill_desc(SetDesc &s, const atmo_params &p) {
     memset(&s, 0, sizeof s);
     s.Rg = p.Rg; s.Rt = p.Rt; s.RL = p.RL;
@@ -211,14 +223,26 @@ SetSizes sizes(const atmo_params &p) {
     return {(size_t)p.TRANSMITTANCE_W * p.TRANSMITTANCE_H, (size_t)p.SKY_W * p.SKY_H,
             (size_t)p.RES_R * p.RES_MU * p.RES_MU_S * p.RES_NU};
 }
-// work tables per set: T4, dE4, E4, dSR4, dSM4, dJ4
-size_t work_bytes(const atmo_params &p, const atmo_options &o) {
+// The dSn passes' view-ray samples (SetDesc::view), 16 bytes each.  dSM4 is last
+// read by the order-2 dJ and dE passes, before the first dSn pass, so the table
+// takes its place where it fits (rows of more texels than a ray has samples) and
+// has its own memory otherwise.
+size_t view_bytes(const atmo_params &p, const atmo_options &o) {
+    return (size_t)p.RES_R * p.RES_MU * (o.inscatter_samples + 1) * sizeof(SnView);
+}
+size_t view_extra(const atmo_params &p, const atmo_options &o) {
+    const size_t b = view_bytes(p, o);
+    return o.orders < 2 || b <= sizes(p).n4 * 16 ? 0 : align256(b);
+}
+// work tables per set: T4, dE4, E4, dSR4, dSM4, dJ4; view: with SetDesc::view
+size_t work_bytes(const atmo_params &p, const atmo_options &o, bool view = true) {
     SetSizes z = sizes(p);
     size_t b = 2 * align256(z.nT * 16) + 2 * align256(z.nE * 16) + 2 * align256(z.n4 * 16);   // T, tau, ...
     b += align256((size_t)p.RES_R * p.RES_MU * (o.inscatter_samples + 1) * 16);   // tview
     if (o.orders >= 2) {
         b += align256(z.n4 * 12);                                         // dJ, packed rgb
         b += align256((size_t)p.RES_R * o.spherical_samples * 16);        // tground
+        if (view) b += view_extra(p, o);
     }
     return b;
 }
@@ -302,32 +326,21 @@ int jg_for_set(const atmo_params &p) {
 struct JSeg {   // a run of P_J tiles whose sets share one G
     int G, off, cnt;
 };
-struct NSeg {   // a run of P_SN tiles whose sets share one row class (texels per thread)
-    int cls, off, cnt;
-    int rows;   // largest rows-per-workgroup x RNU*RMU_S of its sets (k_inscatterN staging)
+struct NSeg {   // a run of P_SN tiles whose sets share one workgroup shape
+    SnShape sh;
+    int W4max, off, cnt;
 };
 
 // Kernel variants chosen by the autotuner, with the times measured for each.
 struct Tuning {
-    int jG = 4, snCap = 4, snXcd = 1, snSb = 2;   // jG = 0: per-set choice
+    int jG = 4, snXcd = 1, snForm = 1;   // jG = 0: per-set choice
     float msJ[5] = {0, 0, 0, 0, 0};  // G = 2, 3, 4, 8, per set (order-2 + order->=3 launches)
-    float msN[27] = {};   // [direct, staged 1, staged 2][caps 1, 2, 4][plain, XCD, XCD + line order]
+    float msN[6] = {};   // [direct, staged][plain, XCD, XCD + line order]
 };
 
-// staged samples per LDS round of a k_inscatterN form (1 direct: 0; 3: 1; 0, the
-// default before tuning, as form 2: rounds of two samples, the faster ones at
-// every class but 16x64x16x4 (32 against 30 us); 32x128x32x8: 149 against 167 us)
-int form_sb(int form) { return form == 1 ? 0 : (form == 3 ? 1 : 2); }
-// mu rows a k_inscatterN workgroup covers with the cap snCap
-int sn_rows(const atmo_params &p, int snCap) {
-    return std::max(1, std::min(std::min(snCap, 4), 256 / (p.RES_MU_S * p.RES_NU)));
-}
-// largest LDS row staging of a tile table's segments
-int sn_max_row_texels(const std::vector<NSeg> &segs) {
-    int m = 0;
-    for (const NSeg &g : segs) m = std::max(m, g.rows);
-    return m;
-}
+// launch_inscatterN form of an option (1 direct; 2, 3 and the default before
+// tuning: LDS-staged rows)
+int sn_form(int form) { return form == 1 ? 0 : 1; }
 
 struct Plan {
     std::vector<atmo_params> params;
@@ -347,9 +360,9 @@ struct Plan {
     int jG = 4;        // k_inscatterS texels per thread (0: per set, see jg_for_set)
     std::vector<JSeg> jseg;   // P_J tiles grouped by the per-set G
     std::vector<NSeg> nseg;   // P_SN tiles grouped by row class
-    int snCap = 4;     // k_inscatterN max mu rows per workgroup
+    bool view = true;  // the sets have SetDesc::view
     int snXcd = 1;     // k_inscatterN XCD-banded tile order
-    int snSb = 2;      // k_inscatterN: 0 direct gathers, > 0 LDS-staged rows (samples per round)
+    int snForm = 1;    // k_inscatterN: 0 direct gathers, 1 LDS-staged rows
     bool tuned = false;
     void drop_graph() {
         if (gexec) (void)hipGraphExecDestroy(gexec);
@@ -459,25 +472,27 @@ atmo_status upload_dirs(DevBuf &buf, hipStream_t xs, const atmo_options &o, size
     return ATMO_OK;
 }
 
-// The k_inscatterN tiles (workgroups of up to snCap mu rows) of a batch, grouped
-// by row class, most texels per thread first; appended to `tiles`.
-void build_sn_tiles(const std::vector<atmo_params> &ps, int snCap, int snXcd, std::vector<uint2> &tiles,
-                    std::vector<NSeg> &segs) {
+// The k_inscatterN tiles (mu rows) of a batch, grouped by workgroup shape, the
+// longest rows first; appended to `tiles`.
+void build_sn_tiles(const std::vector<atmo_params> &ps, int snXcd, std::vector<uint2> &tiles, std::vector<NSeg> &segs) {
     struct Key {
         uint32_t key, tile;
     };
     std::vector<Key> k, tmp;
     std::vector<uint2> v;
+    std::map<std::pair<int, int>, std::vector<int>> groups;   // sets by (texels, threads)
+    for (int i = 0; i < (int)ps.size(); ++i) {
+        const SnShape sh = sn_shape(ps[i].RES_MU_S * ps[i].RES_NU);
+        groups[{-sh.texels, -sh.threads}].push_back(i);
+    }
     const int base = (int)tiles.size();
-    for (int cls = 4; cls >= 1; --cls) {
-        NSeg seg{cls, (int)tiles.size() - base, 0, 0};
+    for (const auto &g : groups) {
+        NSeg seg{{-g.first.first, -g.first.second}, 0, (int)tiles.size() - base, 0};
         v.clear();
-        for (int i = 0; i < (int)ps.size(); ++i) {
+        for (int i : g.second) {
             const atmo_params &p = ps[i];
-            const int W4 = p.RES_MU_S * p.RES_NU;
-            if (row_class(W4) != cls) continue;
-            const int rpw = sn_rows(p, snCap), ngy = (p.RES_MU + rpw - 1) / rpw, nt = p.RES_R * ngy;
-            seg.rows = std::max(seg.rows, rpw * W4);
+            const int nt = p.RES_R * p.RES_MU;
+            seg.W4max = std::max(seg.W4max, p.RES_MU_S * p.RES_NU);
             if (snXcd == 2) {
                 // "line order": a view ray is a straight line, fixed by its impact
                 // parameter r sqrt(1 - mu^2) and its half (up / down); rays of different
@@ -487,12 +502,12 @@ void build_sn_tiles(const std::vector<atmo_params> &ps, int snCap, int snXcd, st
                 tmp.resize(nt);
                 for (int l = 0, t = 0; l < p.RES_R; ++l) {
                     const LayerGeom g = layer_geom(p, l);
-                    for (int y = 0; y < ngy; ++y, ++t) {
-                        const double mu = row_mu(p, g, y * rpw);
+                    for (int y = 0; y < p.RES_MU; ++y, ++t) {
+                        const double mu = row_mu(p, g, y);
                         const float b = (float)(g.r * std::sqrt(std::max(0.0, 1.0 - mu * mu)));
                         uint32_t u;
                         memcpy(&u, &b, 4);
-                        k[t] = {u | (y * rpw < p.RES_MU / 2 ? 0u : 0x80000000u), (uint32_t)t};
+                        k[t] = {u | (y < p.RES_MU / 2 ? 0u : 0x80000000u), (uint32_t)t};
                     }
                 }
                 for (int sh = 0; sh < 33; sh += 11) {
@@ -508,7 +523,6 @@ void build_sn_tiles(const std::vector<atmo_params> &ps, int snCap, int snXcd, st
             }
         }
         seg.cnt = (int)v.size();
-        if (!seg.cnt) continue;
         segs.push_back(seg);
         if (snXcd) {
             // Workgroups are dealt round-robin to the 8 XCDs (each with its own L2);
@@ -528,15 +542,15 @@ void build_sn_tiles(const std::vector<atmo_params> &ps, int snCap, int snXcd, st
 // Tile tables of every pass for a batch.  The spherical-integral passes list
 // the most expensive tiles first so mixed-resolution batches drain evenly.
 void build_tiles(const std::vector<atmo_params> &ps, const atmo_options &o,
-                 std::vector<uint2> &tiles, int off[P_COUNT], int cnt[P_COUNT], int snCap = 4,
-                 int snXcd = 1, std::vector<JSeg> *jseg = nullptr, std::vector<NSeg> *nseg = nullptr) {
+                 std::vector<uint2> &tiles, int off[P_COUNT], int cnt[P_COUNT], int snXcd = 1,
+                 std::vector<JSeg> *jseg = nullptr, std::vector<NSeg> *nseg = nullptr) {
     tiles.clear();
     const int n = (int)ps.size();
     for (int pass = 0; pass < P_COUNT; ++pass) {
         off[pass] = (int)tiles.size();
         if (pass == P_SN) {
             std::vector<NSeg> segs;
-            if (o.orders >= 2) build_sn_tiles(ps, snCap, snXcd, tiles, segs);
+            if (o.orders >= 2) build_sn_tiles(ps, snXcd, tiles, segs);
             cnt[pass] = (int)tiles.size() - off[pass];
             if (nseg) nseg->swap(segs);
             continue;
@@ -563,10 +577,12 @@ void build_tiles(const std::vector<atmo_params> &ps, const atmo_options &o,
                 cost = jg_for_set(p) * 1e12 + (double)p.RES_MU * p.RES_NU;
                 break;
             case P_EN: nt = (long long)z.nE; cost = (double)p.RES_NU; break;
+            case P_VIEW: nt = ((long long)p.RES_R * p.RES_MU * (o.inscatter_samples + 1) + 255) / 256; break;
             case P_CHECK: nt = (std::max(std::max(z.n4, z.nT), z.nE) + 255) / 256; break;
             }
             if (pass == P_J && o.orders < 2) nt = 0;
             if (pass == P_EN && o.orders < 2) nt = 0;
+            if (pass == P_VIEW && o.orders < 2) nt = 0;
             for (long long t = 0; t < nt; ++t) v.push_back({cost, make_uint2((unsigned)i, (unsigned)t)});
         }
         if (pass == P_J || pass == P_EN)
@@ -626,12 +642,13 @@ hipError_t launch_dj(const Plan &pl, const SetDesc *S, const uint2 *T, const cha
     return hipSuccess;
 }
 
-// The dSn pass: one launch per row class.  S: descriptors; T: the pass's tiles.
-hipError_t launch_dsn(const SetDesc *S, const uint2 *T, const std::vector<NSeg> &segs, const atmo_options &o, int snCap,
-                      int sb, hipStream_t st) {
+// The dSn pass: one launch per workgroup shape.  S: descriptors; T: the pass's
+// tiles; view: the sets have SetDesc::view.
+hipError_t launch_dsn(const SetDesc *S, const uint2 *T, const std::vector<NSeg> &segs, const atmo_options &o, int form,
+                      bool view, hipStream_t st) {
     for (const NSeg &g : segs) {
-        hipError_t e = launch_inscatterN(S, T + g.off, g.cnt, o.inscatter_samples, snCap, sb, g.cls,
-                                         lds_inscatterN(g.rows, sb), lin_4(o), st);
+        hipError_t e = launch_inscatterN(S, T + g.off, g.cnt, o.inscatter_samples, view ? form : 2, g.sh, g.W4max,
+                                         lin_4(o), st);
         if (e != hipSuccess) return e;
     }
     return hipSuccess;
@@ -695,7 +712,9 @@ atmo_status launch_all(Plan &pl, hipStream_t st, PassTimer *tm = nullptr) {
                                   first ? pl.ldsE1 : pl.ldsEN, st));
         HIPCHK(t.end());
         HIPCHK(t.begin(5, order));
-        HIPCHK(launch_dsn(S, T + pl.off[P_SN], pl.nseg, o, pl.snCap, pl.snSb, st));
+        if (first && pl.view)   // dSM4 has been read for the last time
+            HIPCHK(launch_snview(S, T + pl.off[P_VIEW], pl.cnt[P_VIEW], o.inscatter_samples, st));
+        HIPCHK(launch_dsn(S, T + pl.off[P_SN], pl.nseg, o, pl.snForm, pl.view, st));
         HIPCHK(t.end());
     }
     return ATMO_OK;
@@ -705,9 +724,9 @@ atmo_status launch_all(Plan &pl, hipStream_t st, PassTimer *tm = nullptr) {
 // Autotuner.  After the first run of a plan whose shape class has not been
 // tuned in this process, every variant of the two dominant passes is timed on
 // the plan's own (by then scratch) work tables: k_inscatterS with 2, 3, 4 or 8
-// texels per thread (orders 2 and >= 3), k_inscatterN in its three forms with
-// up to 1, 2 or 4 mu rows per workgroup and three tile orders (its
-// descriptors carry no S pointer, so the finished tables are not touched).
+// texels per thread (orders 2 and >= 3), k_inscatterN in its two forms and three
+// tile orders (its descriptors carry no S pointer, so the finished tables are
+// not touched).
 // Every variant computes bit-identical tables (the k_inscatterN forms blend the
 // same columns in the same FP32 order), so tuning changes the time only.  The
 // fastest is kept per shape class and applied before the first launch of any
@@ -799,53 +818,45 @@ atmo_status autotune(Plan &pl, hipStream_t st, Tuning &tu) {
     DevBuf ds, dt;
     HIPCHK(ds.ensure(hs.size() * sizeof(SetDesc)));
     HIPCHK(h2d(ds.p, hs.data(), hs.size() * sizeof(SetDesc), pl.xs));
-    const int caps[3] = {1, 2, 4}, sbs[3] = {0, 1, 2};   // sb: staged samples per LDS round
-    int dev = 0, maxLds = 0;
-    HIPCHK(hipGetDevice(&dev));
-    HIPCHK(hipDeviceGetAttribute(&maxLds, hipDeviceAttributeMaxSharedMemoryPerBlock, dev));
     float bestN = 1e30f;
-    for (int si = 0; si < 3; ++si)
-    for (int ci = 0; ci < 3; ++ci)
-        for (int xo = 0; xo < 3; ++xo) {
-            std::vector<uint2> tiles;
-            std::vector<NSeg> segs;
-            int off[P_COUNT], cnt[P_COUNT];
-            build_tiles(pl.params, o, tiles, off, cnt, caps[ci], xo, nullptr, &segs);
-            const size_t lds = lds_inscatterN(sn_max_row_texels(segs), sbs[si]);
-            if (lds + static_lds_inscatterN() > (size_t)maxLds) {  // does not fit this device's LDS
-                tu.msN[si * 9 + ci * 3 + xo] = -1.f;
+    for (int xo = 0; xo < 3; ++xo) {
+        std::vector<uint2> tiles;
+        std::vector<NSeg> segs;
+        build_sn_tiles(pl.params, xo, tiles, segs);
+        HIPCHK(dt.ensure(tiles.size() * sizeof(uint2)));
+        HIPCHK(h2d(dt.p, tiles.data(), tiles.size() * sizeof(uint2), pl.xs));
+        for (int form = 0; form < 2; ++form) {
+            float ms = 0.f;
+            if (form == 0 && !pl.view) {
+                tu.msN[form * 3 + xo] = -1.f;
                 continue;
             }
-            HIPCHK(dt.ensure(tiles.size() * sizeof(uint2)));
-            HIPCHK(h2d(dt.p, tiles.data(), tiles.size() * sizeof(uint2), pl.xs));
-            float ms = 0.f;
             atmo_status rc = time_launch(st, ms, [&]() {
-                return launch_dsn((const SetDesc *)ds.p, (const uint2 *)dt.p + off[P_SN], segs, o, caps[ci], sbs[si], st);
+                return launch_dsn((const SetDesc *)ds.p, (const uint2 *)dt.p, segs, o, form, pl.view, st);
             });
             if (rc != ATMO_OK) return rc;
-            tu.msN[si * 9 + ci * 3 + xo] = ms;
+            tu.msN[form * 3 + xo] = ms;
             if (ms < bestN) {
                 bestN = ms;
-                tu.snCap = caps[ci];
                 tu.snXcd = xo;
-                tu.snSb = sbs[si];
+                tu.snForm = form;
             }
         }
+    }
     return ATMO_OK;
 }
 
 // Applies a tuning to a plan: rebuilds the tile table if the k_inscatterN
 // variant changed and drops the captured graph.
 atmo_status apply_tuning(Plan &pl, const Tuning &tu) {
-    const bool retile = tu.snCap != pl.snCap || tu.snXcd != pl.snXcd;
+    const bool retile = tu.snXcd != pl.snXcd;
     pl.jG = pl.opts.texels_per_thread ? pl.opts.texels_per_thread : tu.jG;
-    pl.snCap = tu.snCap;
     pl.snXcd = tu.snXcd;
-    pl.snSb = pl.opts.inscatterN_form ? form_sb(pl.opts.inscatterN_form) : tu.snSb;
+    pl.snForm = pl.opts.inscatterN_form ? sn_form(pl.opts.inscatterN_form) : tu.snForm;
     pl.tuned = true;
     if (retile) {
         std::vector<uint2> tiles;
-        build_tiles(pl.params, pl.opts, tiles, pl.off, pl.cnt, pl.snCap, pl.snXcd, &pl.jseg, &pl.nseg);
+        build_tiles(pl.params, pl.opts, tiles, pl.off, pl.cnt, pl.snXcd, &pl.jseg, &pl.nseg);
         HIPCHK(pl.dtiles.ensure(tiles.size() * sizeof(uint2)));
         HIPCHK(h2d(pl.dtiles.p, tiles.data(), tiles.size() * sizeof(uint2), pl.xs));
     }
@@ -856,7 +867,8 @@ atmo_status apply_tuning(Plan &pl, const Tuning &tu) {
 // rg: where the device buffers come from (nullptr: hipMalloc); tu: kernel
 // variants to build the plan with (nullptr: the defaults, tuned later).
 atmo_status build_plan(hipStream_t xs, const atmo_params *sets, int nsets, const atmo_options &o,
-                       std::unique_ptr<Plan> &out, Region *rg = nullptr, const Tuning *tu = nullptr) {
+                       std::unique_ptr<Plan> &out, Region *rg = nullptr, const Tuning *tu = nullptr,
+                       bool view = true) {
     std::unique_ptr<Plan> pl(new Plan);
     Region heap;
     Region &R = rg ? *rg : heap;
@@ -864,12 +876,12 @@ atmo_status build_plan(hipStream_t xs, const atmo_params *sets, int nsets, const
     pl->params.assign(sets, sets + nsets);
     pl->opts = o;
     pl->jG = o.texels_per_thread;   // 0: each set with its own G until the tuner has run
-    pl->snSb = form_sb(o.inscatterN_form);
+    pl->snForm = sn_form(o.inscatterN_form);
+    pl->view = view;
     if (tu) {
         pl->jG = o.texels_per_thread ? o.texels_per_thread : tu->jG;
-        pl->snCap = tu->snCap;
         pl->snXcd = tu->snXcd;
-        pl->snSb = o.inscatterN_form ? form_sb(o.inscatterN_form) : tu->snSb;
+        pl->snForm = o.inscatterN_form ? sn_form(o.inscatterN_form) : tu->snForm;
         pl->tuned = true;
     }
     // work arena
@@ -877,18 +889,25 @@ atmo_status build_plan(hipStream_t xs, const atmo_params *sets, int nsets, const
     std::vector<size_t> base(nsets);
     for (int i = 0; i < nsets; ++i) {
         base[i] = total;
-        total += work_bytes(sets[i], o);
+        total += work_bytes(sets[i], o, view);
     }
     HIPCHK(R.get(pl->arena, total));
-    // layers
+    // layers, then the mu_s columns of every set
     std::vector<LayerGeom> layers;
-    std::vector<size_t> loff(nsets);
+    std::vector<ColGeom> cols;
+    std::vector<size_t> loff(nsets), coff(nsets);
     for (int i = 0; i < nsets; ++i) {
         loff[i] = layers.size();
+        coff[i] = cols.size();
         for (int l = 0; l < sets[i].RES_R; ++l) layers.push_back(layer_geom(sets[i], l));
+        for (int m = 0; m < sets[i].RES_MU_S; ++m) cols.push_back(col_geom(sets[i], o, m));
     }
-    HIPCHK(R.get(pl->dlayers, layers.size() * sizeof(LayerGeom)));
-    HIPCHK(h2d(pl->dlayers.p, layers.data(), layers.size() * sizeof(LayerGeom), pl->xs));
+    const size_t cols_off = align256(layers.size() * sizeof(LayerGeom));
+    std::vector<char> geom(cols_off + cols.size() * sizeof(ColGeom));
+    memcpy(geom.data(), layers.data(), layers.size() * sizeof(LayerGeom));
+    memcpy(geom.data() + cols_off, cols.data(), cols.size() * sizeof(ColGeom));
+    HIPCHK(R.get(pl->dlayers, geom.size()));
+    HIPCHK(h2d(pl->dlayers.p, geom.data(), geom.size(), pl->xs));
     // descriptors (output pointers are filled in per call)
     pl->hsets.resize(nsets);
     char *ar = (char *)pl->arena.p;
@@ -907,16 +926,18 @@ atmo_status build_plan(hipStream_t xs, const atmo_params *sets, int nsets, const
         s.dJ4 = o.orders >= 2 ? (float4 *)b : nullptr;
         if (o.orders >= 2) {
             b += align256(z.n4 * 12);
-            s.tground = (float4 *)b;
+            s.tground = (float4 *)b; b += align256((size_t)sets[i].RES_R * o.spherical_samples * 16);
+            s.view = !view ? nullptr : view_extra(sets[i], o) ? (SnView *)b : (SnView *)s.dSM4;
         }
         s.dJb = 12;  // the ray gathers of dSn read 12 bytes per texel
         set_table_flags(s, o);
         s.layers = (const LayerGeom *)pl->dlayers.p + loff[i];
+        s.cols = (const ColGeom *)((const char *)pl->dlayers.p + cols_off) + coff[i];
     }
     HIPCHK(R.get(pl->dsets, nsets * sizeof(SetDesc)));
     // tiles
     std::vector<uint2> tiles;
-    build_tiles(pl->params, o, tiles, pl->off, pl->cnt, pl->snCap, pl->snXcd, &pl->jseg, &pl->nseg);
+    build_tiles(pl->params, o, tiles, pl->off, pl->cnt, pl->snXcd, &pl->jseg, &pl->nseg);
     HIPCHK(R.get(pl->dtiles, tiles.size() * sizeof(uint2)));
     HIPCHK(h2d(pl->dtiles.p, tiles.data(), tiles.size() * sizeof(uint2), pl->xs));
     HIPCHK(R.get(pl->dflags, nsets * sizeof(unsigned)));
@@ -946,17 +967,18 @@ atmo_status build_plan(hipStream_t xs, const atmo_params *sets, int nsets, const
 
 // Device bytes build_plan takes from a Region for this batch (every part
 // rounded to 256 bytes, as Region::get does).
-size_t plan_bytes(const std::vector<atmo_params> &ps, const atmo_options &o, int snCap, int snXcd) {
-    size_t work = 0, nl = 0;
+size_t plan_bytes(const std::vector<atmo_params> &ps, const atmo_options &o, int snXcd, bool view) {
+    size_t work = 0, nl = 0, nc = 0;
     for (const atmo_params &p : ps) {
-        work += work_bytes(p, o);
+        work += work_bytes(p, o, view);
         nl += (size_t)p.RES_R;
+        nc += (size_t)p.RES_MU_S;
     }
     std::vector<uint2> tiles;
     int off[P_COUNT], cnt[P_COUNT];
-    build_tiles(ps, o, tiles, off, cnt, snCap, snXcd);
+    build_tiles(ps, o, tiles, off, cnt, snXcd);
     size_t a, b, c;
-    return align256(work) + align256(nl * sizeof(LayerGeom)) + align256(ps.size() * sizeof(SetDesc)) +
+    return align256(work) + align256(align256(nl * sizeof(LayerGeom)) + nc * sizeof(ColGeom)) + align256(ps.size() * sizeof(SetDesc)) +
            align256(tiles.size() * sizeof(uint2)) + align256(ps.size() * sizeof(unsigned)) +
            align256(dirs_bytes(o, a, b, c));
 }
@@ -1143,11 +1165,15 @@ atmo_status atmo_engine_tuning(atmo_engine *e, atmo_tuning *out) {
     memset(out, 0, sizeof *out);
     out->tuned = !e->last_key.empty();
     out->inscatterS_texels_per_thread = e->last_tuning.jG;
-    out->inscatterN_rows_per_workgroup = e->last_tuning.snCap;
+    out->inscatterN_rows_per_workgroup = 1;
     out->inscatterN_xcd_order = e->last_tuning.snXcd;
     for (int i = 0; i < 5; ++i) out->inscatterS_ms[i] = e->last_tuning.msJ[i];
-    for (int i = 0; i < 27; ++i) out->inscatterN_ms[i] = e->last_tuning.msN[i];
-    out->inscatterN_staged_samples = e->last_tuning.snSb;
+    for (int i = 0; i < 27; ++i) out->inscatterN_ms[i] = -1.f;
+    for (int x = 0; x < 3; ++x) {
+        out->inscatterN_ms[x] = e->last_tuning.msN[x];
+        out->inscatterN_ms[9 + x] = e->last_tuning.msN[3 + x];
+    }
+    out->inscatterN_staged_samples = e->last_tuning.snForm;
     return ATMO_OK;
 }
 
@@ -1184,7 +1210,10 @@ atmo_status atmo_engine_precompute(atmo_engine *e, const atmo_params *sets, int 
     if (!reuse) {
         HIPCHK(hipStreamSynchronize(hs));
         e->plan.reset();
-        if ((st = build_plan(e->cap, sets, nsets, o, e->plan)) != ATMO_OK) return st;
+        st = build_plan(e->cap, sets, nsets, o, e->plan);
+        if (st == ATMO_ERR_OUT_OF_MEMORY)   // without the table of view-ray samples
+            st = build_plan(e->cap, sets, nsets, o, e->plan, nullptr, nullptr, false);
+        if (st != ATMO_OK) return st;
     }
     Plan &pl = *e->plan;
     bool changed = !reuse;
@@ -1272,8 +1301,14 @@ atmo_status atmo_precompute_noalloc(const atmo_params *sets, int nsets, const at
             have = true;
         }
     }
-    const int snCap = have ? tu.snCap : 4, snXcd = have ? tu.snXcd : 1;
-    const size_t need = plan_bytes(ps, o, snCap, snXcd);
+    const int snXcd = have ? tu.snXcd : 1;
+    // without the table of view-ray samples where the array is too small for it
+    bool view = true;
+    size_t need = plan_bytes(ps, o, snXcd, true);
+    if (need > (size_t)ATMO_NOALLOC_MAX_BYTES) {
+        view = false;
+        need = plan_bytes(ps, o, snXcd, false);
+    }
     if (need > (size_t)ATMO_NOALLOC_MAX_BYTES)
         return fail(ATMO_ERR_INVALID_ARGUMENT,
                     "this batch needs %zu bytes of device work memory; the allocation-free precompute "
@@ -1288,7 +1323,7 @@ atmo_status atmo_precompute_noalloc(const atmo_params *sets, int nsets, const at
     rg.base = base;
     rg.cap = ATMO_NOALLOC_MAX_BYTES;
     std::unique_ptr<Plan> pl;
-    if ((st = build_plan(hs, sets, nsets, o, pl, &rg, have ? &tu : nullptr)) != ATMO_OK) return st;
+    if ((st = build_plan(hs, sets, nsets, o, pl, &rg, have ? &tu : nullptr, view)) != ATMO_OK) return st;
     for (int i = 0; i < nsets; ++i) {
         SetDesc &d = pl->hsets[i];
         d.S4 = (float4 *)out[i].inscatter;
@@ -1347,9 +1382,14 @@ static atmo_status pass_setup(atmo_engine *e, const atmo_params *p, const atmo_o
     set_table_flags(s, oo);
     std::vector<LayerGeom> layers;
     for (int l = 0; l < p->RES_R; ++l) layers.push_back(layer_geom(*p, l));
-    HIPCHK(e->pass_layers.ensure(layers.size() * sizeof(LayerGeom)));
+    std::vector<ColGeom> cols;
+    for (int m = 0; m < p->RES_MU_S; ++m) cols.push_back(col_geom(*p, oo, m));
+    const size_t cols_off = align256(layers.size() * sizeof(LayerGeom));
+    HIPCHK(e->pass_layers.ensure(cols_off + cols.size() * sizeof(ColGeom)));
     HIPCHK(h2d(e->pass_layers.p, layers.data(), layers.size() * sizeof(LayerGeom), e->cap));
     s.layers = (const LayerGeom *)e->pass_layers.p;
+    s.cols = (const ColGeom *)((char *)e->pass_layers.p + cols_off);
+    HIPCHK(h2d((char *)e->pass_layers.p + cols_off, cols.data(), cols.size() * sizeof(ColGeom), e->cap));
     return ATMO_OK;
 }
 
@@ -1365,7 +1405,7 @@ static atmo_status pass_run(atmo_engine *e, const atmo_params *p, const atmo_opt
     atmo_options ot = o;
     ot.orders = std::max(ot.orders, 2);  // every pass gets its tiles
     std::vector<NSeg> nseg;
-    build_tiles(ps, ot, tiles, off, cnt, 4, 1, nullptr, &nseg);
+    build_tiles(ps, ot, tiles, off, cnt, 1, nullptr, &nseg);
     HIPCHK(e->pass_tiles.ensure(tiles.size() * sizeof(uint2)));
     HIPCHK(h2d(e->pass_tiles.p, tiles.data(), tiles.size() * sizeof(uint2), e->cap));
     size_t oJT, oJW, oE;
@@ -1396,11 +1436,7 @@ static atmo_status pass_run(atmo_engine *e, const atmo_params *p, const atmo_opt
                                   first, lds, hs));
         break;
     }
-    case P_SN: {
-        const int sb = form_sb(o.inscatterN_form);
-        HIPCHK(launch_dsn(S, T + off[P_SN], nseg, o, 4, sb, hs));
-        break;
-    }
+    case P_SN: HIPCHK(launch_dsn(S, T + off[P_SN], nseg, o, sn_form(o.inscatterN_form), false, hs)); break;
     }
     HIPCHK(hipStreamSynchronize(hs));
     g_err.clear();

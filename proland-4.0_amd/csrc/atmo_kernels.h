@@ -57,16 +57,17 @@ hipError_t launch_inscatterS(const SetDesc *sets, const uint2 *tiles, int ntiles
                              hipStream_t st);
 hipError_t launch_irradianceN(const SetDesc *sets, const uint2 *tiles, int ntiles, int NI, int CH,
                               const void *dirs, bool first, size_t lds, hipStream_t st);
-// rpw_cap: at most this many mu rows per workgroup (1, 2 or 4); the tile table
-// must have been built with the same cap.  sb = 0: direct gathers; sb > 0:
-// LDS-staged blended rows, sb samples per round, lds = lds_inscatterN(max over
-// the launch's sets of rows-per-workgroup x RNU*RMU_S, sb) bytes of dynamic LDS.
-// row_class: texels per thread of the launch's sets (one launch per class).
-inline int row_class(int W4) { return W4 <= 256 ? 1 : (W4 + 255) / 256; }   // 1 .. 4: W4 <= 1024
-size_t lds_inscatterN(int max_row_texels, int sb);
-size_t static_lds_inscatterN();   // bytes of k_inscatterN's static LDS
-hipError_t launch_inscatterN(const SetDesc *sets, const uint2 *tiles, int ntiles, int nsamp,
-                             int rpw_cap, int sb, int row_class, size_t lds, bool lin4, hipStream_t st);
+// The dSn pass, one mu row (tile) per workgroup.  form: 0 direct gathers, 1
+// LDS-staged rows (both read SetDesc::view and tview), 2 LDS-staged rows without
+// SetDesc::view.  W4max: the most texels of a row of the launch's sets.
+struct SnShape {
+    int texels, threads;   // per thread (1 .. 3), per workgroup (a multiple of 64 up to 512)
+};
+SnShape sn_shape(int W4);   // W4 <= 1024
+hipError_t launch_inscatterN(const SetDesc *sets, const uint2 *tiles, int ntiles, int nsamp, int form, SnShape sh,
+                             int W4max, bool lin4, hipStream_t st);
+// SetDesc::view of every set, tiles of 256 consecutive samples
+hipError_t launch_snview(const SetDesc *sets, const uint2 *tiles, int ntiles, int nsamp, hipStream_t st);
 hipError_t launch_check(const SetDesc *sets, const uint2 *tiles, int ntiles, unsigned int *flags,
                         hipStream_t st);
 

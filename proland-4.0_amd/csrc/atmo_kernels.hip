@@ -101,13 +101,11 @@ __global__ __launch_bounds__(256) void k_irradiance1(const SetDesc *__restrict__
     }
 }
 
-constexpr int kNChunk = 64;   // samples staged per chunk
-constexpr int kNRows = 4;     // max mu rows per workgroup
+constexpr int kNChunk = 64;   // k_inscatterN form 2: samples staged per chunk
+constexpr int kNRows = 4;     // k_inscatter1: max mu rows per workgroup
 
-// rows per workgroup: as many whole rows as fit 256 threads, at most rpw_cap (<= 4)
-__device__ __forceinline__ int sn_rows_per_wg(int W4, int rpw_cap) {
-    return max(1, min(min(rpw_cap, kNRows), 256 / W4));
-}
+// mu rows per workgroup of k_inscatter1 and k_tview: as many whole rows as fit 256 threads, at most 4
+__device__ __forceinline__ int rows_per_wg(int W4) { return max(1, min(kNRows, 256 / W4)); }
 
 // ---------------------------------------------------------------------------
 // Pass dS1 — inscatter1.glsl:104-150 fused with copyInscatter1.glsl:104-109.
@@ -115,7 +113,7 @@ __device__ __forceinline__ int sn_rows_per_wg(int W4, int rpw_cap) {
 // an integration sample that does not involve the sun — its distance and
 // radius, the view-ray transmittance T(r, mu, t), the scale-height factors and
 // the r-row of the T(r_i, mu_s_i) lookup — is shared by the RNU x RMU_S texels
-// of the row.  A workgroup covers up to 4 rows (as k_inscatterN), stages those
+// of the row.  A workgroup covers up to 4 rows, stages those
 // terms (FP64 geometry) in LDS, and each thread then needs only the sun
 // visibility test, mu_s_i and the mu-axis half of the T lookup per sample.
 // ---------------------------------------------------------------------------
@@ -154,7 +152,7 @@ __global__ __launch_bounds__(256) void k_inscatter1(const SetDesc *__restrict__ 
     const float sc = (float)s.TW / 1.5f;
     if (tab)
         for (int k = threadIdx.x; k < s.TW; k += blockDim.x) xk[k] = tan(1.5 * (k + 0.5) / s.TW);
-    const int RPW = sn_rows_per_wg(s.W4, kNRows);
+    const int RPW = rows_per_wg(s.W4);
     const int ngy = (s.RMU + RPW - 1) / RPW;
     const int l = (int)tl.y / ngy;
     const int yb = ((int)tl.y % ngy) * RPW;
@@ -208,7 +206,7 @@ __global__ __launch_bounds__(256) void k_inscatter1(const SetDesc *__restrict__ 
             const float3 Tseg = s.tview ? ld3(gptr(s.tview) + ((size_t)l * s.RMU + yb + row) * (nsamp + 1) + i)
                               : up      ? T_ratio_lin(s, (float)(r - s.Rg), (float)mu, h1, mu1)
                                         : T_ratio_lin(s, h1, -mu1, (float)(r - s.Rg), (float)-mu);
-            const float w = (i == 0 || i == nsamp) ? 0.5f : 1.0f;
+            const float w = !s.tview && (i == 0 || i == nsamp) ? 0.5f : 1.0f;
             en.T[0] = Tseg.x * w; en.T[1] = Tseg.y * w; en.T[2] = Tseg.z * w;
             const double rid = sqrt(en.q + s.Rg2);
             en.iri = 1.0 / rid;
@@ -944,16 +942,63 @@ __global__ __launch_bounds__(256) void k_irradianceN(const SetDesc *__restrict__
 // every quantity of an integration sample that does not involve the sun
 // (sample radius and zenith cosine, the texture4D r and mu coordinates and
 // filter weights, the transmittance T(r, mu, t)) is shared by the
-// RNU x RMU_S texels of the row.  A workgroup covers up to 4 rows: it stages
-// those per-sample terms in LDS (FP64 geometry, in chunks of 64 samples) and
-// each thread then integrates its texels with only the mu_s-dependent work.
+// RNU x RMU_S texels of the row, which one workgroup covers: k_snview computes
+// those per-sample terms once per precompute (FP64 geometry), and each thread
+// integrates its texels with only the mu_s-dependent work.
 // ---------------------------------------------------------------------------
-struct SnEntry {
-    float4 w;     // bilinear (r, mu) weights of the 4 table rows
-    int4 base;    // offsets of the 4 rows (z0y0, z0y1, z1y0, z1y1)
-    float4 tw;    // T(r, mu, t) * trapezoid weight (rgb), t
-    float4 ir;    // 1 / r_i, r_i - r
-};
+// Sample i of the view ray of mu row y, layer l (FP64 geometry).
+__device__ __forceinline__ SnView sn_view(const SetDesc &s, const LayerGeom &L, int y, int i, int nsamp,
+                                          double &mu, double &h1, double &mu1, float &tr) {
+    const double r = L.r, rho2 = r * r - s.Rg2;
+    double muS_u, nu_u;
+    mu_mus_nu(s, L, 0, y, mu, muS_u, nu_u);
+    const double rmu = r * mu;
+    const double delta = rmu * rmu - rho2;            // constant along the ray
+    const double dx = limit_d(s, r, mu) / nsamp;
+    const double ti = i * dx;
+    const double q = rho2 + ti * (ti + 2.0 * rmu);    // ri^2 - Rg^2
+    const double rmui = rmu + ti;                     // ri * mui
+    const double ri = sqrt(q + s.Rg2);
+    const double rho = sqrt(fmax(q, 0.0));
+    double f, c;
+    if (rmui < 0.0 && delta > 0.0) {
+        f = -rho / (sqrt(delta) - rmui);
+        c = 0.5 - 0.5 / s.RMU;
+    } else {
+        f = (sqrt(fmax(delta + s.H * s.H, 0.0)) - rmui) / (rho + s.H);
+        c = 0.5 + 0.5 / s.RMU;
+    }
+    const double ty = s.lin4 ? (0.5 / s.RMU + (rmui / ri + 1.0) / 2.0 * (1.0 - 1.0 / s.RMU)) * s.RMU - 0.5
+                             : (c + f * (0.5 - 1.0 / s.RMU)) * s.RMU - 0.5;
+    const double tz = rho / s.H * (s.RR - 1.0);
+    int z0, z1, y0, y1;
+    float az, ay;
+    gl_axis_d(tz, s.RR, z0, z1, az);
+    gl_axis_d(ty, s.RMU, y0, y1, ay);
+    h1 = q / (ri + s.Rg);
+    mu1 = rmui / ri;
+    tr = (float)(ti / ri);
+    SnView v;
+    const bool dy = y1 != y0, dz = z1 != z0, oy = y0 & 1, oz = z0 & 1;
+    // weights of the odd ones; at an edge both taps are the same row, whose name takes it all
+    v.ay = dy ? (oy ? 1.f - ay : ay) : (oy ? 1.f : 0.f);
+    v.az = dz ? (oz ? 1.f - az : az) : (oz ? 1.f : 0.f);
+    v.row = 8 * (z0 * s.RMU + y0) + (dy ? 1 : 0) + (dz ? 2 : 0) + (oz ? 4 : 0);
+    v.dr = i == 0 ? (float)dx : (float)((ri - r) / ri);
+    return v;
+}
+// Row indices (layer RMU + mu row) of a sample: x even layer, even mu row; y even,
+// odd; z odd, even; w odd, odd.  (RMU is even, so an index has its mu row's parity.)
+__device__ __forceinline__ int4 sn_rows4(int RMU, int row) {
+    const int p = row >> 3, oy = p & 1, dy = row & 1, dz = (row & 2) ? RMU : 0;
+    const int ye = oy ? dy : 0, yo = oy ? 0 : dy;                     // from p to the even / odd mu row
+    const int ze = (row & 4) ? dz : 0, zo = (row & 4) ? 0 : dz;       // from p to the even / odd layer
+    return make_int4(p + ze + ye, p + ze + yo, p + zo + ye, p + zo + yo);
+}
+// Blend weights of the 4 rows in the order of sn_rows4.
+__device__ __forceinline__ float4 sn_weights(float az, float ay) {
+    return make_float4((1.f - az) * (1.f - ay), (1.f - az) * ay, az * (1.f - ay), az * ay);
+}
 
 // The (r, mu) blend of one table column x: sum_q w_q dJ[row_q][x], in one fixed
 // FP32 order.  Both forms of k_inscatterN (direct gathers, LDS-staged rows)
@@ -976,366 +1021,240 @@ __device__ __forceinline__ float3 sn_lerp(float ax, float3 b0, float3 b1) {
 // that move: an FP32 mu_s_i (~2e-8 absolute) put through the coordinate
 // formula (whose + 0.74, resp. + 0.2, cancels at the low end) would give it
 // only to a few 1e-3.  So:
-//   linear (:165), mus = (mu_s + 0.2) r per texel: offset proportional to
-//     mu_s_i + 0.2 = (nu t + (mu_s + 0.2) r + 0.2 (r_i - r)) / r_i;
-//   non-linear (:161), mus = mu_s and txb = the texel's own offset (FP64): with
+//   linear (:165): offset proportional to mu_s_i + 0.2 =
+//     nu t / r_i - mu_s (r_i - r) / r_i + (mu_s + 0.2);
+//   non-linear (:161), txb = the texel's own offset (FP64): with
 //     d = max(mu_s_i, -0.1975) - mu_b, mu_b = max(mu_s, -0.1975), and
 //     mu_s_i - mu_s = (nu t - mu_s (r_i - r)) / r_i,
 //     offset = txb + C atan(k d / (1 + k mu_b k (mu_b + d))), k = tan(1.386),
 //     C = 0.5 (RMUS - 1) / 1.1 (atan a - atan b = atan((a - b) / (1 + a b)),
-//     used while |k d| < 0.5, where 1 + a b > 0; larger moves take the
-//     reference's form, which has no cancellation there).
+//     used while |k d| < 0.5, where the argument is below 0.5334); larger moves
+//     take the reference's form, which has no cancellation there.
+// The per-column terms, k folded in (ColGeom), leave two FMAs for k d; the near
+// arctangent is its own odd polynomial (weighted least-squares fit of
+// (atan(x)/x - 1)/x^2 on |x| <= 0.534, 7.2e-8 relative in FP32 arithmetic) and
+// the far form is entered only by waves in which a lane needs it: 19 VALU
+// slots instead of 36 for a wave of near moves.  A lane's value does not depend
+// on its wave's vote.
+struct SnTexel {
+    float nu;    // k nu (linear: nu)
+    ColGeom c;
+};
 template <bool LIN4>
-__device__ __forceinline__ float sn_txs(const SetDesc &s, float nu, float mus, float txb,
-                                        const SnEntry &en) {
+__device__ __forceinline__ float sn_txs(const SetDesc &s, const SnTexel &x, float tr, float dr) {
     const float half = 0.5f * (float)(s.RMUS - 1);
-    if (LIN4)
-        return fmaxf(fmaf(nu, en.tw.w, fmaf(0.2f, en.ir.y, mus)) * en.ir.x, 0.0f) * (1.0f / 1.2f) *
-               (2.0f * half);
-    // Every sum of products is an explicit fmaf: left to contraction, the
-    // compiler fuses kb + kd as fma(k, d, kb) in one inlined copy and as
-    // fma(k, mub, kd) in another, and the paths of k_inscatterN must agree
-    // bit for bit.
-    const float mub = fmaxf(mus, -0.1975f);
-    // d = mu_s_i - mu_s + (mu_s - mu_b), dmu = (nu t - mu_s (r_i - r)) / r_i
-    const float d = fmaxf(fmaf(fmaf(nu, en.tw.w, -mus * en.ir.y), en.ir.x, mus - mub), -0.1975f - mub);
-    const float k = s.f_tMuS, kb = k * mub, kd = k * d;
-    const float kbd = fmaf(k, d, kb);   // kb + kd
+    // every sum of products is an explicit fmaf, so that the inlined copies of
+    // the kernel's forms agree bit for bit
+    if (LIN4) return fmaxf(fmaf(x.nu, tr, fmaf(-x.c.mus, dr, x.c.txb)), 0.0f) * (1.0f / 1.2f) * (2.0f * half);
+    const float c = half * (1.0f / 1.1f);
+    const float kd = fmaxf(fmaf(x.nu, tr, fmaf(-x.c.mus, dr, x.c.ck)), x.c.lo);
     const bool near = fabsf(kd) < 0.5f;
-    const float arg = near ? kd * __builtin_amdgcn_rcpf(fmaf(kb, kbd, 1.0f)) : kbd;
-    return fmaf(atanf(arg), half * (1.0f / 1.1f), near ? txb : 0.74f * half);
+    const float a = kd * __builtin_amdgcn_rcpf(fmaf(x.c.kb, kd, x.c.kb2));
+    const float z = a * a;
+    float p = fmaf(z, -0.04780794680118561f, 0.09955135732889175f);
+    p = fmaf(z, p, -0.14134405553340912f);
+    p = fmaf(z, p, 0.19991108775138855f);
+    p = fmaf(z, p, -0.3333316147327423f);
+    float o = fmaf(c, fmaf(a, z * p, a), x.c.txb);
+    if (!__all(near)) {
+        const float far = fmaf(c, atanf(x.c.kb + kd), 0.74f * half);
+        o = near ? o : far;
+    }
+    return o;
 }
 
-// Waves per SIMD the register budget of a k_inscatterN instantiation is cut to.
-// The kernel waits on its row gathers and on a barrier per LDS round, so more
-// waves help until the budget spills.  Per order, rows of 256 texels
-// (32x128x32x8): 135 us at 4 and 5 waves, 138 at 6, 153 at 8; 48-set batch of
-// mixed classes: 13.96 ms at (5, 5, 4, 4) for 1-4 texels per thread, 14.08 at
-// (4, 3, 3, 3), 15.2 at (7, 4, 5, 3).  One kernel for all classes, at three
-// waves, took 170 us and 16.2 ms.
-constexpr int sn_waves(int NM) { return NM <= 2 ? 5 : 4; }
+// Waves per SIMD the register budget of a k_inscatterN instantiation is cut to:
+// the most that need no spill (40, 70 and 108 VGPRs).  A spill in the sample loop
+// costs more than any number of waves gives: 3 texels per thread with 9 registers
+// spilled at five waves took 13.1 ms per order for the 48-set mixed batch,
+// without them at four 8.9 ms.
+// Form 2, whose FP64 terms need about 100 VGPRs, runs at four.
+constexpr int sn_waves(int form, int NM) { return form == 2 ? 4 : NM == 1 ? 8 : NM == 2 ? 6 : 4; }
 
-// STAGED = false: each texel gathers its 8 taps per sample from dJ directly
-// (global loads).  STAGED = true: per sample the workgroup first blends the
-// 4 (r, mu) table rows of every row it covers into one row
-// B_i[x] = sum_q w_q dJ[row_q][x] in LDS (coalesced loads, 4 per texel
-// instead of 8, shared by all texels that hit x), then each texel reads two
-// neighbours of B_i and lerps in x.  The direct form blends the two columns
-// it needs in the same order (sn_blend, sn_lerp), so both give the same bits.
-// `sb` samples are blended per LDS round (dynamic LDS: sb * rows * RNU*RMU_S
-// float4).  NM: texels per thread.  A workgroup covers rows of RNU*RMU_S <= 256
-// texels with one texel per thread (NM = 1), or one row of more (NM = 2 .. 4):
-// the staged form has a path for each, and each NM is its own instantiation and
-// launch, so that its registers are what its class needs.  With NM >= 2, a
-// sample whose 4 rows are those of the sample before it in the same LDS round
-// blends the loaded rows again (the row starts are workgroup-uniform there, so
-// the test is a scalar branch).
-template <bool STAGED, bool LIN4, int NM>   // LIN4: linear inscatter parameterisation (per-sample mu_s)
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(sn_waves(NM))))
-void k_inscatterN(const SetDesc *__restrict__ sets, const uint2 *__restrict__ tiles, int nsamp, int rpw_cap, int sb) {
-    __shared__ SnEntry ent[NM == 1 ? kNRows : 1][kNChunk];
-    extern __shared__ float4 blend[];   // [sb][nrows * W4] (STAGED)
+// One mu row of RNU*RMU_S texels per workgroup, NM texels per thread.  FORM:
+//   0  each texel gathers its 8 taps per sample from dJ directly (global loads);
+//   1  per sample the workgroup first blends the 4 (r, mu) table rows around it
+//      into one row B[x] = sum_q w_q dJ[row_q][x] in LDS (coalesced loads), then
+//      each texel reads two neighbours of B and lerps in x;
+//   2  as 1, without SetDesc::view: the workgroup computes the samples' terms
+//      into LDS itself, 64 at a time.
+// The direct form blends the two columns it needs in the same order (sn_blend,
+// sn_lerp), so all forms give the same bits.  The staged row is double-buffered:
+// a sample's rows are loaded during the lookups of the one before it, and there
+// is one barrier per sample.  A row that the sample before it had too (the same
+// layer and mu row, kept in registers under the parities of both) is not loaded
+// again: 1.6 of 4 rows per sample are loaded at 32x128x32x8, 2.6 at
+// 64x256x64x16.  The samples' terms are workgroup-uniform, in scalar registers.
+//
+// What it measured per order, before (several rows per workgroup, samples' terms
+// computed by each workgroup in every order, 4 row loads and two barriers per
+// sample, 77 VALU slots per texel-sample) and now (about 50): 32x128x32x8 170 ->
+// 99 us, 64x256x64x16 2.21 -> 1.51 ms, the 48-set mixed batch 16.2 -> 8.5 ms.  It
+// is held by its VALU (about 70 %) and the row loads between them.
+template <int FORM, bool LIN4, int NM>   // LIN4: linear inscatter parameterisation (per-sample mu_s)
+__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(sn_waves(FORM, NM))))
+void k_inscatterN(const SetDesc *__restrict__ sets, const uint2 *__restrict__ tiles, int nsamp) {
+    struct Entry {
+        SnView v;
+        float4 tw;   // T(r, mu, t) * trapezoid weight (rgb), t / r_i
+    };
+    __shared__ Entry ent[FORM == 2 ? kNChunk : 1];
+    extern __shared__ float4 blend[];   // [2][W4 + 1]
     const uint2 tl = tiles[blockIdx.x];
     const SetDesc &s = sets[tl.x];
-    const int RPW = sn_rows_per_wg(s.W4, rpw_cap);
-    const int ngy = (s.RMU + RPW - 1) / RPW;
-    const int l = (int)tl.y / ngy;
-    const int yb = ((int)tl.y % ngy) * RPW;
-    const int nrows = min(RPW, s.RMU - yb);
-    const LayerGeom L = s.layers[l];
-    const double r = L.r;
-    const double rho2 = r * r - s.Rg2;
-    const int HW = s.RMU * s.W4;
-
-    // texels of this thread: rows yb.. (row-major, x fastest)
-    const int per = nrows * s.W4;
+    const int l = (int)tl.y / s.RMU, y = (int)tl.y % s.RMU;
+    const int nthr = blockDim.x, W4 = s.W4;
     float acc[NM][3];
-    float nuf[NM], muSr[NM], txb[NM], fk[NM];
-    int kq[NM];   // the texel's nu slice k0 (< RNU) | its row in the workgroup << 16
+    SnTexel tx[NM];
+    unsigned kbase[NM];   // first column of the texel's nu slice
+    // nu = -1 + 2 k / (RNU - 1) is on slice k of the table, so the nu lerp of
+    // texture4D has weight 0 and a lookup reads slice k only
+    auto texel_nu = [&](int x) { return -1.0 + (double)(x / s.RMUS) / (s.RNU - 1.0) * 2.0; };
 #pragma unroll
     for (int j = 0; j < NM; ++j) {
         acc[j][0] = acc[j][1] = acc[j][2] = 0.f;
-        nuf[j] = muSr[j] = txb[j] = fk[j] = 0.f;
-        kq[j] = 0;
-        const int e = threadIdx.x + j * (int)blockDim.x;
-        if (e < per) {
-            const int row = e / s.W4, x = e % s.W4;
-            double mu, muS, nu;
-            mu_mus_nu(s, L, x, yb + row, mu, muS, nu);
-            // nu lies on a slice of the table: the nu lerp of texture4D has weight 0 or 1
-            double pos = (nu + 1.0) / 2.0 * (s.RNU - 1.0);
-            const double kr = rint(pos);
-            if (fabs(pos - kr) < 1e-9) pos = kr;
-            const double kfl = floor(pos);
-            fk[j] = (float)(pos - kfl);
-            kq[j] = (int)kfl | (row << 16);
-            nuf[j] = (float)nu;
-            // the texel's terms of its samples' mu_s offsets (sn_txs)
-            muSr[j] = (float)(LIN4 ? (muS + 0.2) * r : muS);
-            txb[j] = LIN4 ? 0.0f : (float)(tex4d_umus(s, muS) * s.RMUS - 0.5);
-        }
+        const int x = min((int)threadIdx.x + j * nthr, W4 - 1);   // past the row's end: nothing is stored
+        kbase[j] = (unsigned)(x / s.RMUS * s.RMUS);
+        tx[j].nu = (float)(LIN4 ? texel_nu(x) : (double)s.f_tMuS * texel_nu(x));
+        tx[j].c = s.cols[x % s.RMUS];
     }
-
     // the dJ table as a buffer (< 2^31 bytes: at most 2^27 texels of 16 bytes)
-    const __amdgpu_buffer_rsrc_t Jr = table_rsrc(s.dJ4, (unsigned)((size_t)s.RR * HW * s.dJb));
-    // A lookup's texel column is kbase + txs: kbase the first column of its nu
-    // slice, txs its offset, kept apart so that the fraction ax has full FP32
-    // precision.  txs runs past RMU_S - 1 into the next slice when mu_s_i > 1
-    // (as GL's coordinate does); only the row's last column clamps (CLAMP_TO_EDGE),
-    // and i0 = kbase + is <= W4 - 2 keeps both taps in the row.
-    const unsigned W4m2 = (unsigned)(s.W4 - 2);
-    const unsigned jb = (unsigned)s.dJb;   // bytes per dJ texel
-    for (int c0 = 0; c0 <= nsamp; c0 += kNChunk) {
-        const int nc = min(kNChunk, nsamp + 1 - c0);
+    const __amdgpu_buffer_rsrc_t Jr = table_rsrc(s.dJ4, (unsigned)((size_t)s.n4 * s.dJb));
+    const unsigned jb = (unsigned)s.dJb, rowb = (unsigned)W4 * jb;   // bytes per dJ texel and row
+
+    // sample i, as uniform values
+    typedef __attribute__((address_space(4))) const SnView cview;
+    typedef __attribute__((address_space(4))) const F4 cf4;
+    const size_t v0 = ((size_t)l * s.RMU + y) * (nsamp + 1);
+    const cview *gv = (const cview *)(s.view + v0);
+    const cf4 *gt = (const cf4 *)(s.tview + v0);
+    int c0 = 0;
+    float dx = 0.f;   // the row's trapezoid step
+    auto get = [&](int i) {
+        Entry e;
+        if constexpr (FORM == 2) {
+            const Entry &q = ent[i - c0];
+            auto u = [](float f) { return __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(f))); };
+            e.v.az = u(q.v.az); e.v.ay = u(q.v.ay); e.v.dr = u(q.v.dr);
+            e.v.row = __builtin_amdgcn_readfirstlane(q.v.row);
+            e.tw = make_float4(u(q.tw.x), u(q.tw.y), u(q.tw.z), u(q.tw.w));
+        } else {
+            e.v.az = gv[i].az; e.v.ay = gv[i].ay; e.v.row = gv[i].row; e.v.dr = gv[i].dr;
+            e.tw = make_float4(gt[i].x, gt[i].y, gt[i].z, gt[i].w);
+        }
+        if (i == 0) {
+            dx = e.v.dr;
+            e.v.dr = 0.f;
+        }
+        return e;
+    };
+    auto stage = [&](int c) {   // FORM 2: the terms of samples c .. c + 63
+        c0 = c;
         __syncthreads();
-        // stage the row-uniform terms of samples c0 .. c0+nc-1 (FP64 geometry)
-        for (int e = threadIdx.x; e < nrows * kNChunk; e += blockDim.x) {
-            const int row = e / kNChunk, js = e % kNChunk;
-            if (js >= nc) continue;
-            const int i = c0 + js;
-            double mu, muS_u, nu_u;
-            mu_mus_nu(s, L, 0, yb + row, mu, muS_u, nu_u);
-            const double rmu = r * mu;
-            const double delta = rmu * rmu - rho2;            // constant along the ray
-            const double dx = limit_d(s, r, mu) / nsamp;
-            const double ti = i * dx;
-            const double q = rho2 + ti * (ti + 2.0 * rmu);   // ri^2 - Rg^2
-            const double rmui = rmu + ti;                     // ri * mui
-            const double ri = sqrt(q + s.Rg2);
-            const double rho = sqrt(fmax(q, 0.0));
-            double f, c;
-            if (rmui < 0.0 && delta > 0.0) {
-                f = -rho / (sqrt(delta) - rmui);
-                c = 0.5 - 0.5 / s.RMU;
-            } else {
-                f = (sqrt(fmax(delta + s.H * s.H, 0.0)) - rmui) / (rho + s.H);
-                c = 0.5 + 0.5 / s.RMU;
+        for (int js = threadIdx.x; js < min(kNChunk, nsamp + 1 - c); js += nthr) {
+            const int i = c + js;
+            const LayerGeom &L = s.layers[l];
+            double mu, h1, mu1;
+            float tr;
+            Entry en;
+            en.v = sn_view(s, L, y, i, nsamp, mu, h1, mu1, tr);
+            if (s.tview) {
+                en.tw = s.tview[v0 + i];
+            } else {   // transmittance(r, mu, ti) (common.glsl:272-282)
+                const float hl = (float)(L.r - s.Rg), wt = (i == 0 || i == nsamp) ? 0.5f : 1.0f;
+                const float3 T = mu > 0.0 ? T_ratio_lin(s, hl, (float)mu, (float)h1, (float)mu1)
+                                          : T_ratio_lin(s, (float)h1, (float)-mu1, hl, (float)-mu);
+                en.tw = make_float4(T.x * wt, T.y * wt, T.z * wt, tr);
             }
-            const double ty = s.lin4 ? (0.5 / s.RMU + (rmui / ri + 1.0) / 2.0 * (1.0 - 1.0 / s.RMU)) * s.RMU - 0.5
-                                     : (c + f * (0.5 - 1.0 / s.RMU)) * s.RMU - 0.5;
-            const double tz = rho / s.H * (s.RR - 1.0);
-            int z0, z1, y0, y1;
-            float az, ay;
-            gl_axis_d(tz, s.RR, z0, z1, az);
-            gl_axis_d(ty, s.RMU, y0, y1, ay);
-            // transmittance(r, mu, ti) (common.glsl:272-282)
-            const float h1 = (float)(q / (ri + s.Rg));
-            const float mu1 = (float)(rmui / ri);
-            const float3 Tseg = s.tview ? ld3(gptr(s.tview) + ((size_t)l * s.RMU + yb + row) * (nsamp + 1) + i)
-                              : mu > 0.0 ? T_ratio_lin(s, (float)(r - s.Rg), (float)mu, h1, mu1)
-                                         : T_ratio_lin(s, h1, -mu1, (float)(r - s.Rg), (float)-mu);
-            const float wt = (i == 0 || i == nsamp) ? 0.5f : 1.0f;
-            SnEntry en;
-            en.w = make_float4((1.f - az) * (1.f - ay), (1.f - az) * ay, az * (1.f - ay), az * ay);
-            en.base = make_int4((z0 * HW + y0 * s.W4) * s.dJb, (z0 * HW + y1 * s.W4) * s.dJb,
-                                (z1 * HW + y0 * s.W4) * s.dJb, (z1 * HW + y1 * s.W4) * s.dJb);
-            en.tw = make_float4(Tseg.x * wt, Tseg.y * wt, Tseg.z * wt, (float)ti);
-            en.ir = make_float4((float)(1.0 / ri), (float)(ri - r), 0.f, 0.f);
-            ent[row][js] = en;
+            ent[js] = en;
         }
         __syncthreads();
-        if constexpr (!STAGED) {
+    };
+    // A lookup's texel column is kbase + txs, txs the offset inside the slice,
+    // kept apart so that the fraction ax has full FP32 precision.  txs runs past
+    // RMU_S - 1 into the next slice when mu_s_i > 1 (as GL's coordinate does);
+    // only the row's last column clamps (CLAMP_TO_EDGE): at txs = W4 - 1 - kbase
+    // the fraction is 0 and the second tap is the padding column W4, a copy of
+    // the last.
+    if constexpr (FORM == 0) {
+#pragma unroll
+        for (int j = 0; j < NM; ++j) {
+            const unsigned last = (unsigned)W4 - 1 - kbase[j];
+            for (int i = 0; i <= nsamp; ++i) {
+                const Entry en = get(i);
+                const float4 w = sn_weights(en.v.az, en.v.ay);
+                const int4 rows = sn_rows4(s.RMU, en.v.row);
+                const float txs = __builtin_amdgcn_fmed3f(sn_txs<LIN4>(s, tx[j], en.tw.w, en.v.dr), 0.0f, (float)last);
+                const unsigned is = __float2uint_rz(txs);
+                // the blended columns is and is + 1 (as the staged form's rows hold them)
+                auto column = [&](unsigned x) {
+                    const unsigned o = (kbase[j] + x) * jb;
+                    return sn_blend(w, ld3b(Jr, o, (unsigned)rows.x * rowb), ld3b(Jr, o, (unsigned)rows.y * rowb),
+                                    ld3b(Jr, o, (unsigned)rows.z * rowb), ld3b(Jr, o, (unsigned)rows.w * rowb));
+                };
+                const float3 v = sn_lerp(__builtin_amdgcn_fractf(txs), column(is), column(min(is + 1, last)));
+                acc[j][0] = fmaf(v.x, en.tw.x, acc[j][0]);
+                acc[j][1] = fmaf(v.y, en.tw.y, acc[j][1]);
+                acc[j][2] = fmaf(v.z, en.tw.z, acc[j][2]);
+            }
+        }
+    } else {
+        unsigned xo[NM];   // byte offset of each texel's column in a table row
+#pragma unroll
+        for (int j = 0; j < NM; ++j) xo[j] = (unsigned)min((int)threadIdx.x + j * nthr, W4 - 1) * jb;
+        float3 t[4][NM];
+        int held[4] = {-1, -1, -1, -1};
+        auto load_rows = [&](int row) {   // the rows that the registers do not hold yet
+            const int4 r4 = sn_rows4(s.RMU, row);
+            const int want[4] = {r4.x, r4.y, r4.z, r4.w};
+#pragma unroll
+            for (int q = 0; q < 4; ++q)
+                if (want[q] != held[q]) {
+                    held[q] = want[q];
+#pragma unroll
+                    for (int j = 0; j < NM; ++j) t[q][j] = ld3b(Jr, xo[j], (unsigned)want[q] * rowb);
+                }
+        };
+        if (FORM == 2) stage(0);
+        Entry cur = get(0);
+        load_rows(cur.v.row);
+        float4 *B = blend;
+        for (int i = 0; i <= nsamp; ++i) {
+            const float4 w = sn_weights(cur.v.az, cur.v.ay);
 #pragma unroll
             for (int j = 0; j < NM; ++j) {
-                const int e = threadIdx.x + j * (int)blockDim.x;
-                if (e >= per) break;
-                const SnEntry *er = ent[kq[j] >> 16];
-                const unsigned kbase = (unsigned)((kq[j] & 0xffff) * s.RMUS);
-                const float txmax = (float)(W4m2 + 1 - kbase);
-                const unsigned ismax = W4m2 - kbase;
-                float a0 = acc[j][0], a1 = acc[j][1], a2 = acc[j][2];
-                for (int js = 0; js < nc; ++js) {
-                    const SnEntry en = er[js];
-                    const float txs = __builtin_amdgcn_fmed3f(sn_txs<LIN4>(s, nuf[j], muSr[j], txb[j], en), 0.0f, txmax);
-                    const unsigned is = min(__float2uint_rz(txs), ismax);
-                    const float ax = txs - (float)is;
-                    const unsigned i0 = kbase + is;
-                    // the blended columns i0 and i0 + 1 (as the staged form's rows hold them)
-                    auto column = [&](unsigned x) {
-                        const unsigned o = x * jb;
-                        return sn_blend(en.w, ld3b(Jr, (unsigned)en.base.x + o, 0u), ld3b(Jr, (unsigned)en.base.y + o, 0u),
-                                        ld3b(Jr, (unsigned)en.base.z + o, 0u), ld3b(Jr, (unsigned)en.base.w + o, 0u));
-                    };
-                    float3 v = sn_lerp(ax, column(i0), column(i0 + 1));
-                    if (fk[j] != 0.0f) {  // off-grid nu: blend with the next slice (k0 + 1 <= RNU - 1)
-                        unsigned j0 = i0 + (unsigned)s.RMUS;
-                        float bx = ax;
-                        if (j0 > W4m2) { j0 = W4m2; bx = 1.0f; }   // past the row's last column
-                        v = lerp3(v, sn_lerp(bx, column(j0), column(j0 + 1)), fk[j]);
-                    }
-                    a0 = fmaf(v.x, en.tw.x, a0);
-                    a1 = fmaf(v.y, en.tw.y, a1);
-                    a2 = fmaf(v.z, en.tw.z, a2);
-                }
-                acc[j][0] = a0; acc[j][1] = a1; acc[j][2] = a2;
+                const int x = threadIdx.x + j * nthr;
+                const float3 b = sn_blend(w, t[0][j], t[1][j], t[2][j], t[3][j]);
+                if (x < W4) B[x] = make_float4(b.x, b.y, b.z, 0.f);
+                if (x == W4 - 1) B[W4] = make_float4(b.x, b.y, b.z, 0.f);
             }
-        } else if constexpr (NM >= 2) {
-            // Rows of more than 256 texels (one row per workgroup, 2-4 texels
-            // per thread): every slot reads the same sample entries, so (a)
-            // issues all 4 * NM table loads of a thread before blending any,
-            // and (b) interleaves the NM independent lookups of a sample.  The
-            // arithmetic of each texel-sample is that of the general path.
-            for (int s0 = 0; s0 < nc; s0 += sb) {
-                const int ns = min(sb, nc - s0);
-                // the table rows of the last sample loaded in this round: a later
-                // sample on the same 4 rows (same first and last row start, which fix
-                // the two layers and the two mu rows) blends them again without
-                // loading (kept within a round: carried over the lookups, t would
-                // spill at three waves per SIMD)
-                float3 t[NM][4];
-                unsigned P0 = 0u, P3 = 0u;
-                for (int k = 0; k < ns; ++k) {
-                    const float4 w = ent[0][s0 + k].w;
-                    const int4 base = ent[0][s0 + k].base;
-                    // the 4 row starts are the same for the whole workgroup: in
-                    // scalar registers, the loads take them as their base and
-                    // the thread's own column offset (fixed over the samples)
-                    const unsigned R0 = (unsigned)__builtin_amdgcn_readfirstlane(base.x);
-                    const unsigned R1 = (unsigned)__builtin_amdgcn_readfirstlane(base.y);
-                    const unsigned R2 = (unsigned)__builtin_amdgcn_readfirstlane(base.z);
-                    const unsigned R3 = (unsigned)__builtin_amdgcn_readfirstlane(base.w);
-                    if (k == 0 || R0 != P0 || R3 != P3) {
-                        P0 = R0;
-                        P3 = R3;
+            if (FORM == 2 && (i & (kNChunk - 1)) == kNChunk - 1 && i < nsamp) stage(i + 1);
+            const Entry nxt = get(min(i + 1, nsamp));
+            __syncthreads();
+            load_rows(nxt.v.row);   // in flight during the lookups
 #pragma unroll
-                        for (int j = 0; j < NM; ++j) {
-                            // past the row's end: a valid address, the blend is not stored
-                            const unsigned xo = (unsigned)min((int)threadIdx.x + j * (int)blockDim.x, per - 1) * jb;
-                            t[j][0] = ld3b(Jr, xo, R0);
-                            t[j][1] = ld3b(Jr, xo, R1);
-                            t[j][2] = ld3b(Jr, xo, R2);
-                            t[j][3] = ld3b(Jr, xo, R3);
-                        }
-                    }
-#pragma unroll
-                    for (int j = 0; j < NM; ++j) {
-                        const int e = threadIdx.x + j * (int)blockDim.x;
-                        const float3 b = sn_blend(w, t[j][0], t[j][1], t[j][2], t[j][3]);
-                        if (e < per) blend[(size_t)k * per + e] = make_float4(b.x, b.y, b.z, 0.f);
-                    }
-                }
-                __syncthreads();
-                for (int k = 0; k < ns; ++k) {
-                    const SnEntry en = ent[0][s0 + k];
-                    const float4 *B = blend + (size_t)k * per;
-                    float3 v[NM];
-                    unsigned i0[NM];
-                    float ax[NM];
-#pragma unroll
-                    for (int j = 0; j < NM; ++j) {
-                        // slots past the row's end (kq 0) read in-row values and are never stored
-                        const unsigned kbase = (unsigned)((kq[j] & 0xffff) * s.RMUS);
-                        const float txs = __builtin_amdgcn_fmed3f(sn_txs<LIN4>(s, nuf[j], muSr[j], txb[j], en), 0.0f,
-                                                                  (float)(W4m2 + 1 - kbase));
-                        const unsigned is = min(__float2uint_rz(txs), W4m2 - kbase);
-                        ax[j] = txs - (float)is;
-                        i0[j] = kbase + is;
-                        v[j] = sn_lerp(ax[j], f3(B[i0[j]]), f3(B[i0[j] + 1]));
-                    }
-#pragma unroll
-                    for (int j = 0; j < NM; ++j) {
-                        if (fk[j] != 0.0f) {  // off-grid nu: blend with the next slice (k0 + 1 <= RNU - 1)
-                            unsigned j0 = i0[j] + (unsigned)s.RMUS;
-                            float bx = ax[j];
-                            if (j0 > W4m2) { j0 = W4m2; bx = 1.0f; }   // past the row's last column
-                            v[j] = lerp3(v[j], sn_lerp(bx, f3(B[j0]), f3(B[j0 + 1])), fk[j]);
-                        }
-                        acc[j][0] = fmaf(v[j].x, en.tw.x, acc[j][0]);
-                        acc[j][1] = fmaf(v[j].y, en.tw.y, acc[j][1]);
-                        acc[j][2] = fmaf(v[j].z, en.tw.z, acc[j][2]);
-                    }
-                }
-                __syncthreads();
+            for (int j = 0; j < NM; ++j) {
+                const float txs = __builtin_amdgcn_fmed3f(sn_txs<LIN4>(s, tx[j], cur.tw.w, cur.v.dr), 0.0f,
+                                                          (float)(W4 - 1 - (int)kbase[j]));
+                const float4 *p = B + kbase[j] + __float2uint_rz(txs);
+                const float3 v = sn_lerp(__builtin_amdgcn_fractf(txs), f3(p[0]), f3(p[1]));
+                acc[j][0] = fmaf(v.x, cur.tw.x, acc[j][0]);
+                acc[j][1] = fmaf(v.y, cur.tw.y, acc[j][1]);
+                acc[j][2] = fmaf(v.z, cur.tw.z, acc[j][2]);
             }
-        } else {
-            // Rows of at most 256 texels (one texel per thread): samples are
-            // blended and looked up in pairs, so a thread has 8 table loads and
-            // two independent lookups in flight; the accumulation keeps sample
-            // order, and each texel-sample's arithmetic is the general path's.
-            const int e = threadIdx.x;
-            const bool live = e < per;
-            const int rowj = kq[0] >> 16;   // 0 past the rows' end: valid addresses, nothing stored
-            const SnEntry *er = ent[rowj];
-            const unsigned xo = (unsigned)(live ? e - rowj * s.W4 : 0) * jb;
-            const unsigned kbase = (unsigned)((kq[0] & 0xffff) * s.RMUS);
-            const float txmax = (float)(W4m2 + 1 - kbase);
-            const unsigned ismax = W4m2 - kbase;
-            const float4 *Brow = blend + rowj * s.W4;
-            auto group = [&](int s0, int k, auto pc) {   // samples s0+k .. s0+k+P-1
-                constexpr int P = decltype(pc)::value;
-                float3 t[P][4];
-#pragma unroll
-                for (int q = 0; q < P; ++q) {
-                    // the row starts differ between the rows of a workgroup: in the VGPR offset
-                    const int4 base = er[s0 + k + q].base;
-                    t[q][0] = ld3b(Jr, (unsigned)base.x + xo, 0u);
-                    t[q][1] = ld3b(Jr, (unsigned)base.y + xo, 0u);
-                    t[q][2] = ld3b(Jr, (unsigned)base.z + xo, 0u);
-                    t[q][3] = ld3b(Jr, (unsigned)base.w + xo, 0u);
-                }
-#pragma unroll
-                for (int q = 0; q < P; ++q) {
-                    const float3 b = sn_blend(er[s0 + k + q].w, t[q][0], t[q][1], t[q][2], t[q][3]);
-                    if (live) blend[(size_t)(k + q) * per + e] = make_float4(b.x, b.y, b.z, 0.f);
-                }
-            };
-            auto lookup = [&](int s0, int k, auto pc) {
-                constexpr int P = decltype(pc)::value;
-                float3 v[P];
-                unsigned i0[P];
-                float ax[P];
-#pragma unroll
-                for (int q = 0; q < P; ++q) {
-                    const float txs = __builtin_amdgcn_fmed3f(
-                        sn_txs<LIN4>(s, nuf[0], muSr[0], txb[0], er[s0 + k + q]), 0.0f, txmax);
-                    const unsigned is = min(__float2uint_rz(txs), ismax);
-                    ax[q] = txs - (float)is;
-                    i0[q] = kbase + is;
-                    const float4 *B = Brow + (size_t)(k + q) * per;
-                    v[q] = sn_lerp(ax[q], f3(B[i0[q]]), f3(B[i0[q] + 1]));
-                }
-#pragma unroll
-                for (int q = 0; q < P; ++q) {
-                    if (fk[0] != 0.0f) {  // off-grid nu: blend with the next slice (k0 + 1 <= RNU - 1)
-                        const float4 *B = Brow + (size_t)(k + q) * per;
-                        unsigned j0 = i0[q] + (unsigned)s.RMUS;
-                        float bx = ax[q];
-                        if (j0 > W4m2) { j0 = W4m2; bx = 1.0f; }   // past the row's last column
-                        v[q] = lerp3(v[q], sn_lerp(bx, f3(B[j0]), f3(B[j0 + 1])), fk[0]);
-                    }
-                    const float4 tw = er[s0 + k + q].tw;
-                    acc[0][0] = fmaf(v[q].x, tw.x, acc[0][0]);
-                    acc[0][1] = fmaf(v[q].y, tw.y, acc[0][1]);
-                    acc[0][2] = fmaf(v[q].z, tw.z, acc[0][2]);
-                }
-            };
-            for (int s0 = 0; s0 < nc; s0 += sb) {
-                const int ns = min(sb, nc - s0);
-                int k = 0;
-                for (; k + 1 < ns; k += 2) group(s0, k, std::integral_constant<int, 2>{});
-                if (k < ns) group(s0, k, std::integral_constant<int, 1>{});
-                __syncthreads();
-                k = 0;
-                for (; k + 1 < ns; k += 2) lookup(s0, k, std::integral_constant<int, 2>{});
-                if (k < ns) lookup(s0, k, std::integral_constant<int, 1>{});
-                __syncthreads();
-            }
+            cur = nxt;
+            B = B == blend ? blend + W4 + 1 : blend;
         }
     }
 #pragma unroll
     for (int j = 0; j < NM; ++j) {
-        const int e = threadIdx.x + j * (int)blockDim.x;
-        if (e >= per) break;
-        const int row = e / s.W4, x = e % s.W4;
-        const size_t t = ((size_t)l * s.RMU + yb + row) * s.W4 + x;
-        // the row's trapezoid step, as the sample staging computes it (mu depends on the row only)
-        double mu, muS_u, nu_u;
-        mu_mus_nu(s, L, 0, yb + row, mu, muS_u, nu_u);
-        const float dx = (float)(limit_d(s, r, mu) / nsamp);
+        const int x = threadIdx.x + j * nthr;
+        if (x >= W4) break;
+        const size_t t = ((size_t)l * s.RMU + y) * W4 + x;
         const float4 o = q16(make_float4(acc[j][0] * dx, acc[j][1] * dx, acc[j][2] * dx, 0.f), s.hs);
         s.dSR4[t] = o;
         if (s.S4) {
-            const double nu = nuf[j];
+            const double nu = (float)texel_nu(x);
             const float pr = (float)((3.0 / (16.0 * kPI)) * (1.0 + nu * nu));
             float4 S = s.S4[t];
             S.x += o.x / pr;
@@ -1346,11 +1265,26 @@ void k_inscatterN(const SetDesc *__restrict__ sets, const uint2 *__restrict__ ti
     }
 }
 
+// The view-ray samples' terms of the dSn passes (SetDesc::view), once per
+// precompute: they depend on the geometry only.  Inside k_inscatterN their FP64
+// chain runs on one wave of each workgroup while the others wait, in every order.
+__global__ __launch_bounds__(256) void k_snview(const SetDesc *__restrict__ sets, const uint2 *__restrict__ tiles,
+                                                int nsamp) {
+    const uint2 tl = tiles[blockIdx.x];
+    const SetDesc &s = sets[tl.x];
+    const size_t e = (size_t)tl.y * 256 + threadIdx.x;
+    const int row = (int)(e / (nsamp + 1));
+    if (row >= s.RR * s.RMU) return;
+    double mu, h1, mu1;
+    float tr;
+    s.view[e] = sn_view(s, s.layers[row / s.RMU], row % s.RMU, (int)(e % (nsamp + 1)), nsamp, mu, h1, mu1, tr);
+}
+
 // ---------------------------------------------------------------------------
 // Transmittance tables of one precompute (after the T pass, before the passes
 // that use them): every ratio T(x)/T(y) of common.glsl:272-282 the later passes
 // take depends only on the T table and the geometry, not on the order.
-//  k_tview:   T(r, mu, t_i) along the view ray of each (layer, mu row) at the
+//  k_tview:   T(r, mu, t_i), times the trapezoid weight of sample i, along the view ray of each (layer, mu row) at the
 //             inscatter samples t_i = i limit(r, mu) / nsamp (inscatter1.glsl,
 //             inscatterN.glsl), same tiles as k_inscatter1;
 //  k_tground: T from the ground point seen in direction theta to the layer
@@ -1363,7 +1297,7 @@ __global__ __launch_bounds__(256) void k_tview(const SetDesc *__restrict__ sets,
                                                const uint2 *__restrict__ tiles, int nsamp) {
     const uint2 tl = tiles[blockIdx.x];
     const SetDesc &s = sets[tl.x];
-    const int RPW = sn_rows_per_wg(s.W4, kNRows);
+    const int RPW = rows_per_wg(s.W4);
     const int ngy = (s.RMU + RPW - 1) / RPW;
     const int l = (int)tl.y / ngy;
     const int yb = ((int)tl.y % ngy) * RPW;
@@ -1383,7 +1317,9 @@ __global__ __launch_bounds__(256) void k_tview(const SetDesc *__restrict__ sets,
         const double mu1 = (rmu + ti) / ri;
         const float3 t = mu > 0.0 ? T_ratio_d(s, r - s.Rg, mu, h1, mu1)
                                   : T_ratio_d(s, h1, -mu1, r - s.Rg, -mu);
-        s.tview[((size_t)l * s.RMU + yb + row) * (nsamp + 1) + i] = make_float4(t.x, t.y, t.z, 0.f);
+        const float wt = (i == 0 || i == nsamp) ? 0.5f : 1.0f;   // trapezoid weight
+        s.tview[((size_t)l * s.RMU + yb + row) * (nsamp + 1) + i] =
+            make_float4(t.x * wt, t.y * wt, t.z * wt, (float)(ti / ri));
     }
 }
 
@@ -1552,32 +1488,50 @@ hipError_t launch_irradianceN(const SetDesc *sets, const uint2 *tiles, int ntile
                            CH, (const DirE *)dirs);
     return hipGetLastError();
 }
-size_t static_lds_inscatterN() { return sizeof(SnEntry) * kNRows * kNChunk; }
-size_t lds_inscatterN(int max_row_texels, int sb) {
-    return sb > 0 ? sizeof(float4) * (size_t)sb * (size_t)max_row_texels : 0;
+// Two texels per thread share a sample's uniform work and give a wave two
+// independent lookups: 32x128x32x8 (rows of 256 texels) 116 us per order with one
+// texel per thread, 99 with two, 145 with four (one wave per row); 1024 texels
+// 1.51 ms with two (512 threads), 1.60 with four; 135 texels 48 us with one, 47
+// with two.  Three where two leave 8 % or more of the threads' slots idle beyond
+// what three do: 576 texels (640 slots against 576) 9.5 ms with two, 8.5 with
+// three for the 48-set mixed batch.  Rows of at most a wave have one.
+SnShape sn_shape(int W4) {
+    const int t2 = 64 * ((W4 + 127) / 128), t3 = 64 * ((W4 + 191) / 192);
+    if (W4 <= 64) return {1, 64};
+    return W4 > 256 && 3 * t3 * 100 <= 2 * t2 * 92 ? SnShape{3, t3} : SnShape{2, t2};
 }
 template <int NM>
-static void launch_sn(const SetDesc *sets, const uint2 *tiles, int ntiles, int nsamp, int rpw_cap, int sb,
-                      size_t lds, bool lin4, hipStream_t st) {
-#define ATMO_LN(S, L, LDS, SB) \
-    hipLaunchKernelGGL((k_inscatterN<S, L, NM>), dim3(ntiles), dim3(256), LDS, st, sets, tiles, nsamp, rpw_cap, SB)
-    if (sb > 0) {
-        if (lin4) ATMO_LN(true, true, lds, sb); else ATMO_LN(true, false, lds, sb);
+static void launch_sn(const SetDesc *sets, const uint2 *tiles, int ntiles, int nsamp, int form, int threads, int W4max,
+                      bool lin4, hipStream_t st) {
+    const size_t lds = form == 0 ? 0 : sizeof(float4) * 2 * ((size_t)W4max + 1);
+#define ATMO_LN(F, L) \
+    hipLaunchKernelGGL((k_inscatterN<F, L, NM>), dim3(ntiles), dim3(threads), lds, st, sets, tiles, nsamp)
+    if (form == 0) {
+        if (lin4) ATMO_LN(0, true); else ATMO_LN(0, false);
+    } else if (form == 1) {
+        if (lin4) ATMO_LN(1, true); else ATMO_LN(1, false);
     } else {
-        if (lin4) ATMO_LN(false, true, 0, 0); else ATMO_LN(false, false, 0, 0);
+        if (lin4) ATMO_LN(2, true); else ATMO_LN(2, false);
     }
 #undef ATMO_LN
 }
-hipError_t launch_inscatterN(const SetDesc *sets, const uint2 *tiles, int ntiles, int nsamp, int rpw_cap, int sb,
-                             int row_class, size_t lds, bool lin4, hipStream_t st) {
+hipError_t launch_inscatterN(const SetDesc *sets, const uint2 *tiles, int ntiles, int nsamp, int form, SnShape sh,
+                             int W4max, bool lin4, hipStream_t st) {
     if (ntiles <= 0) return hipSuccess;
-    switch (row_class) {
-    case 1: launch_sn<1>(sets, tiles, ntiles, nsamp, rpw_cap, sb, lds, lin4, st); break;
-    case 2: launch_sn<2>(sets, tiles, ntiles, nsamp, rpw_cap, sb, lds, lin4, st); break;
-    case 3: launch_sn<3>(sets, tiles, ntiles, nsamp, rpw_cap, sb, lds, lin4, st); break;
-    case 4: launch_sn<4>(sets, tiles, ntiles, nsamp, rpw_cap, sb, lds, lin4, st); break;
+    if (form < 0 || form > 2 || sh.threads < 64 || sh.threads > 512 || sh.threads % 64 ||
+        W4max > sh.texels * sh.threads)
+        return hipErrorInvalidValue;
+    switch (sh.texels) {
+    case 1: launch_sn<1>(sets, tiles, ntiles, nsamp, form, sh.threads, W4max, lin4, st); break;
+    case 2: launch_sn<2>(sets, tiles, ntiles, nsamp, form, sh.threads, W4max, lin4, st); break;
+    case 3: launch_sn<3>(sets, tiles, ntiles, nsamp, form, sh.threads, W4max, lin4, st); break;
     default: return hipErrorInvalidValue;
     }
+    return hipGetLastError();
+}
+hipError_t launch_snview(const SetDesc *sets, const uint2 *tiles, int ntiles, int nsamp, hipStream_t st) {
+    if (ntiles <= 0) return hipSuccess;
+    hipLaunchKernelGGL(k_snview, dim3(ntiles), dim3(256), 0, st, sets, tiles, nsamp);
     return hipGetLastError();
 }
 hipError_t launch_check(const SetDesc *sets, const uint2 *tiles, int ntiles, unsigned int *flags,

@@ -827,6 +827,40 @@ def test_inscatterN_forms_agree_on_rows_of_more_than_256_texels(eng, res, lin):
         assert torch.equal(x, y) and torch.equal(y, z)
 
 
+@pytest.mark.parametrize("mus,nu,samples", [(8, 8, 50), (13, 5, 1), (32, 4, 63), (43, 3, 64), (64, 8, 12),
+                                            (57, 9, 12), (64, 16, 12)])
+def test_inscatterN_workgroup_shapes(eng, mus, nu, samples):
+    """Rows of 64, 65, 128, 129, 512, 513 and 1024 texels, the edges of the
+    k_inscatterN workgroup shapes (1 to 3 texels per thread, 64 to 512 threads),
+    with 2, 13, 51, 64 and 65 samples per ray: the staged and the direct form
+    bit for bit, the tables within the bar of the whole-chain tests."""
+    p = small(res=(4, 16, mus, nu))
+    kw = dict(orders=3, inscatter_samples=samples)
+    a = eng.precompute(p, options(flags=8, inscatterN_form=1, **kw))[0]
+    b = eng.precompute(p, options(flags=8, inscatterN_form=2, **kw))[0]
+    torch.cuda.synchronize()
+    for x, y in zip(a, b):
+        assert torch.equal(x, y)
+    oT, oE, oS = O.precompute(p, options(**kw))
+    _assert("S", b[2].double().cpu().numpy(), oS, TOL)
+
+
+@pytest.mark.parametrize("samples", [50, 70])
+def test_inscatterN_without_the_table_of_view_samples(eng, samples):
+    """A set whose work memory fits the allocation-free precompute's array only
+    without the table of view-ray samples (rows of 8 texels): k_inscatterN then
+    computes the samples' terms itself, in one and in two LDS rounds, and gives
+    the engine's bits."""
+    p = small(res=(70 if samples == 50 else 60, 512, 4, 2))
+    o = options(flags=FLAG_NO_AUTOTUNE, spherical_samples=4, inscatter_samples=samples)
+    assert L.workspace_size(p, o) > L.NOALLOC_MAX_BYTES
+    ref = eng.precompute(p, o)[0]
+    got = L.precompute_noalloc(p, o)[0]
+    torch.cuda.synchronize()
+    for x, y in zip(got, ref):
+        assert torch.equal(x, y)
+
+
 def test_precision_study_configuration(eng):
     """The precision-study workload (Earth, T 512x128, E 128x32, inscatter
     64x256x64x16, 32x64 directions, orders 1-8) against the FP64 oracle:
