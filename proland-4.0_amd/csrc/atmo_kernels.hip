@@ -337,6 +337,14 @@ __device__ __forceinline__ void stage_slice(const SetDesc &s, const float4 *cons
 // texel the lookup position is pos = (nu1 + 1)/2 (RNU - 1) + 1 =
 // posA s'.w + posB, with s' = posA s folded in per texel and the mu_s term
 // folded in per theta.
+//
+// Bound by vector instruction issue, then by LDS reads: at 64x256x64x16 and
+// 32 x 64 directions an order >= 3 takes 7.8 ms, 7.2 with the lookups' LDS reads
+// left out.  On gfx950 an add, multiply or FMA of registers and literals issues
+// in about 2 cycles per wave; with a scalar-register operand, and a conversion,
+// floor, shift or integer multiply-add, in 4.  So the loop keeps its operands in
+// vector registers and forms LDS addresses with FMAs (lds_entry): 8.6 -> 7.8 ms;
+// 16x64x16x4: order 2 130 -> 116 us, order 3 73 -> 60.
 // ---------------------------------------------------------------------------
 // Entries of padding in front of the staged ground-irradiance row: texel
 // coordinates down to -(0.8/1.2) SW - 0.5 (mu_s = -1) plus rounding.
@@ -346,10 +354,40 @@ __host__ __device__ __forceinline__ int e_pad(int SW) { return (2 * SW) / 3 + 3;
 // cover [kPosLo, RNU + kPosHi].
 constexpr float kPosLo = 1.0f - 1.0f / 256.0f, kPosHi = 1.0f / 256.0f;
 
-// The value at 0 of the line through (k, a) with slope d, a - k d, from FP64
-// and rounded once; a lookup at pos in [k, k + 1) is then fma(pos, d, .).
+// The staged rows are functions of a coordinate u = pos - 1/2 (ground row of
+// order 2: xg - 1/2), whose rounding to an integer is the entry k = floor(pos).
+// An entry holds its line's value at u = 0: with slope d through (pos = k, a),
+// a - (k - 1/2) d, from FP64 and rounded once; a lookup is then fma(u, d, .).
 __device__ __forceinline__ float at_zero(float a, float d, int k) {
-    return (float)((double)a - (double)k * (double)d);
+    return (float)((double)a - ((double)k - 0.5) * (double)d);
+}
+
+// LDS byte address of an entry in two FMA-class instructions (about 2 cycles per
+// wave on gfx950, where a conversion and a shift-add take 4 each).  u + kRound,
+// kRound = 1.5 2^23, is kRound + k with k = u rounded to the nearest integer;
+// times STRIDE 2^-149, plus (base - STRIDE kRound) 2^-149, it is the denormal
+// whose bit pattern is base + STRIDE k.  Exact: the addend is a multiple of
+// STRIDE below 2^24 STRIDE (base is a multiple of STRIDE), the result is an
+// integer below 2^23.  At a tie either neighbour may come out: the two lines meet
+// there.
+constexpr float kRound = 12582912.0f;
+template <int STRIDE>
+__device__ __forceinline__ float lds_addend(unsigned base) {   // (base - STRIDE kRound) 2^-149
+    return ((float)base - (float)STRIDE * kRound) * 1.40129846e-45f;
+}
+template <int STRIDE>
+__device__ __forceinline__ unsigned lds_entry(float u, float addend) {
+    return __float_as_uint(fmaf(u + kRound, (float)STRIDE * 1.40129846e-45f, addend));
+}
+__device__ __forceinline__ float4 lds4(unsigned a, int off = 0) {
+    typedef float v4 __attribute__((ext_vector_type(4)));
+    const v4 v = *(__attribute__((address_space(3))) const v4 *)(a + off);
+    return make_float4(v.x, v.y, v.z, v.w);
+}
+__device__ __forceinline__ float2 lds2(unsigned a, int off = 0) {
+    typedef float v2 __attribute__((ext_vector_type(2)));
+    const v2 v = *(__attribute__((address_space(3))) const v2 *)(a + off);
+    return make_float2(v.x, v.y);
 }
 
 struct DirJ {      // per-theta constants of the NS x 2NS grid
@@ -372,7 +410,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k
                                                     const float2 *__restrict__ dirW) {
     constexpr int NT = FIRST ? 2 : 1;
     constexpr int PW = FIRST ? 3 : 2;      // float4 per staged pair entry
-    extern __shared__ float4 lds[];
+    extern __shared__ __attribute__((aligned(32))) float4 lds[];   // lds_entry: 32-byte strides
     const uint2 tl = tiles[blockIdx.x];
     const SetDesc &s = sets[tl.x];
     const int l = (int)tl.y / s.RMUS;
@@ -386,6 +424,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k
     const int JXr = FIRST ? 0 : JX;
     const size_t npairs = (size_t)CH * NP + (size_t)JXr;
     __shared__ int s_jxmax;
+    __shared__ double s_u[4];   // mu_s, 1 - mu_s^2, sqrt(1 - mu_s^2), posA
     // order 2, unchunked: the entries' three float4 as planes kJ1Plane apart
     // (16-byte stride in each: a lookup's reads spread over the LDS banks, and
     // one address serves all three with immediate offsets); otherwise whole
@@ -396,7 +435,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k
     float4 *pairs = lds;                                   // rows of NP (+ JX) entries
     // [CH][NV][NT] slice values (the planes compute each entry's two directly)
     float4 *vtmp = pairs + (PLANES ? 2 * kJ1Plane + npairs : npairs * PW);
-    float4 *epair = vtmp + (PLANES ? 0 : (size_t)CH * NV * NT);   // [EPAD + SW + 1][2] (order 2)
+    // [EPAD + SW + 1][2] (order 2), 32-byte aligned
+    float4 *epair = lds + (((vtmp - lds) + (PLANES ? 0 : (size_t)CH * NV * NT) + 1) & ~(size_t)1);
     float4 *gdat = epair + (FIRST ? (size_t)(EPAD + s.SW + 1) * 2 : 0);   // [CH][3]
 
     const LayerGeom L = s.layers[l];
@@ -416,7 +456,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k
         const int k0 = min(max(k - EPAD, 0), s.SW - 1), k1 = min(max(k - EPAD + 1, 0), s.SW - 1);
         const float4 a = s.dE4[k0];
         const float4 b = s.dE4[k1];
-        // {a - k d, d}: the lookup at texel coordinate xg is fma(xg, d, a - k d)
+        // the lookup at texel coordinate xg is fma(xg - 1/2, d, .) (at_zero)
         const float dx = b.x - a.x, dy = b.y - a.y, dz = b.z - a.z;
         epair[2 * k] = make_float4(at_zero(a.x, dx, k), at_zero(a.y, dy, k), at_zero(a.z, dz, k), dx);
         epair[2 * k + 1] = make_float4(dy, dz, 0.f, 0.f);
@@ -427,10 +467,19 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k
     const float eR = (float)exp(-hr / s.HR), eM = (float)exp(-hr / s.HM);
     const float A0 = s.bR[0] * eR * s.kR, A1 = s.bR[1] * eR * s.kR, A2 = s.bR[2] * eR * s.kR;
     const float B0 = s.bMS[0] * eM * s.kM, B1 = s.bMS[1] * eM * s.kM, B2 = s.bMS[2] * eM * s.kM;
-    const float iposA = (float)(1.0 / posAd), nposBi = (float)(-posBd / posAd);
+    const float iposA = (float)(1.0 / posAd), nposBi = (float)((0.5 - posBd) / posAd);   // nu1 from u
     const float g2p1 = s.g2p1, m2g = s.m2g;
+    if (threadIdx.x == 0) {
+        s_u[0] = muS;
+        s_u[1] = fma(-muS, muS, 1.0);
+        s_u[2] = sqrt(s_u[1]);
+        s_u[3] = posAd;
+    }
     const int ngk = (NU + G - 1) / G;
     const int ngroups = s.RMU * ngk;
+    // LDS byte addresses of the staged rows
+    const unsigned pairs_b = (unsigned)(size_t)(__attribute__((address_space(3))) char *)pairs;
+    const float epb = lds_addend<32>((unsigned)(size_t)(__attribute__((address_space(3))) char *)epair);
 
     for (int c0 = 0; c0 < NS; c0 += CH) {
         const int nth = CHUNK ? min(CH, NS - c0) : NS;
@@ -477,22 +526,23 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k
                                               : T_ratio_lin(s, h1, (float)-mu1, 0.0f, (float)-mug);
                 const float gr = (float)(s.alpha / kPI);
                 g0 = make_float4(gr * tr.x, gr * tr.y, gr * tr.z, 1.0f);
-                // E texel coordinate ((r muS + dg nu1)/Rg + 0.2)/1.2 SW - 0.5 as c1 pos + ce0
+                // E texel coordinate ((r muS + dg nu1)/Rg + 0.2)/1.2 SW - 0.5 as c1 u + ce0
                 const double sc = s.SW / 1.2;
                 const double e1 = dg / s.Rg * sc, e0 = (r * muS / s.Rg + 0.2) * sc - 0.5 + EPAD;
                 c1 = e1 / posAd;
-                ce0 = e0 - e1 * posBd / posAd;
+                ce0 = e0 + e1 * (0.5 - posBd) / posAd;   // xg = c1 u + ce0
                 // E cells the lookups of this row can reach: positions [1, NU] up to rounding
                 const float fc1 = (float)c1, fce0 = (float)ce0;
-                jlo = (int)__float2uint_rz(fmaf(kPosLo, fc1, fce0));
-                jhi = (int)__float2uint_rz(fmaf((float)NU + kPosHi, fc1, fce0));
+                jlo = (int)__float2uint_rz(fmaf(kPosLo - 0.5f, fc1, fce0));
+                jhi = (int)__float2uint_rz(fmaf((float)NU + kPosHi - 0.5f, fc1, fce0));
                 // the lookups move xg by at most c1 (RNU - 1 + 2/256) <= 2.0158 e1
                 // (RNU >= 2): at most that many + 1 cells; the host sizes the rows
                 // with ceil(2.05 e1) + 2 per ground row (merged_extra)
                 jhi = min(jhi, jlo + (int)ceil(2.05 * e1) + 1);
             }
             gdat[3 * itl] = g0;
-            gdat[3 * itl + 1] = make_float4((float)c1, (float)ce0, (float)(posAd * muS * ct + posBd),
+            // order 2's ground lookup takes xg - 1/2 (its entries' coordinate)
+            gdat[3 * itl + 1] = make_float4((float)c1, (float)(FIRST ? ce0 - 0.5 : ce0), (float)(posAd * muS * ct + posBd - 0.5),
                                             (float)((kPI / NS) * (kPI / NS) * sin((it + 0.5) * (kPI / NS))));
             gdat[3 * itl + 2] = make_float4(__int_as_float(jlo), __int_as_float(jhi),
                                             __int_as_float(FIRST ? NP : NP + (jhi - jlo)), 0.f);
@@ -556,12 +606,12 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k
             }
         }
         // (4b) orders >= 3, ground rows: the lookup of a ground direction is
-        // S(pos) + g0 E(xg(pos)) with xg = c1 pos + ce0, two piecewise-linear
+        // S(pos) + g0 E(xg(pos)) with xg = c1 u + ce0, u = pos - 1/2, two piecewise-linear
         // functions of the same position, with knots at the integers (slices) and
         // where xg crosses an integer (E texels).  The merged row holds one entry
         // per segment between consecutive knots of either kind: the slope Q and
-        // P - p0 Q, where P is the value at the segment's start p0, so that a
-        // lookup is fma(pos, Q, P - p0 Q).  The segment of (kk, jg) = (floor(pos), floor(xg)) is
+        // the value at u = 0 of the line through (p0, P), the segment's start, so
+        // that a lookup is fma(u, Q, .).  The segment of (kk, jg) = (floor(pos), floor(xg)) is
         // entry kk + jg - jlo (each knot raises one of the two by one); segments
         // are found by intersecting every slice cell with every E cell of the row
         // (FP64), so entries of zero-length segments at coinciding knots exist too.
@@ -579,15 +629,15 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k
                 double lo = kk == 0 ? (double)kPosLo : (double)kk;
                 double hi = kk == NU ? (double)NU + kPosHi : kk + 1.0;
                 if (c1 > 0.0) {
-                    lo = fmax(lo, (jg - ce0) / c1);
-                    hi = fmin(hi, (jg + 1 - ce0) / c1);
+                    lo = fmax(lo, (jg - ce0) / c1 + 0.5);
+                    hi = fmin(hi, (jg + 1 - ce0) / c1 + 0.5);
                 }
                 if (lo > hi) continue;
                 const float4 a = vtmp[((size_t)itl * NV + kk) * NT];
                 const float4 b = vtmp[((size_t)itl * NV + kk + 1) * NT];
                 const float4 ea = s.dE4[min(max(jg - EPAD, 0), s.SW - 1)];
                 const float4 eb = s.dE4[min(max(jg + 1 - EPAD, 0), s.SW - 1)];
-                const double u = lo - kk, v = lo * c1 + ce0 - jg;   // fractions at p0
+                const double u = lo - kk, v = (lo - 0.5) * c1 + ce0 - jg;   // fractions at p0
                 const double dx = (double)b.x - a.x, dy = (double)b.y - a.y, dz = (double)b.z - a.z;
                 const double fx = (double)eb.x - ea.x, fy = (double)eb.y - ea.y, fz = (double)eb.z - ea.z;
                 const double Px = a.x + u * dx + g0.x * (ea.x + v * fx);
@@ -595,9 +645,10 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k
                 const double Pz = a.z + u * dz + g0.z * (ea.z + v * fz);
                 const float Qx = (float)(dx + g0.x * c1 * fx), Qy = (float)(dy + g0.y * c1 * fy),
                             Qz = (float)(dz + g0.z * c1 * fz);
-                // the FP32 slope's line through (p0, P), at pos = 0
+                // the FP32 slope's line through (p0, P), at u = 0
                 float4 *q = pairs + ((size_t)rowoff(itl) + kk + jj) * PW;
-                q[0] = make_float4((float)(Px - lo * Qx), (float)(Py - lo * Qy), (float)(Pz - lo * Qz), Qx);
+                const double l0 = lo - 0.5;
+                q[0] = make_float4((float)(Px - l0 * Qx), (float)(Py - l0 * Qy), (float)(Pz - l0 * Qz), Qx);
                 q[1] = make_float4(Qy, Qz, 0.f, 0.f);
             }
         }
@@ -605,26 +656,35 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k
 
         for (int grp = threadIdx.x; grp < ngroups; grp += blockDim.x) {
             const int y = grp % s.RMU, kb = (grp / s.RMU) * G;
-            float vx = 0.f, vz = 0.f;
-            float sxp[G], syp[G];
-    #pragma unroll
-            for (int g = 0; g < G; ++g) {
-                const int k = min(kb + g, NU - 1);
-                double mu, muS_t, nu;
-                mu_mus_nu(s, L, k * s.RMUS + m, y, mu, muS_t, nu);
-                // inscatterS.glsl:113-122 (FP64)
+            // the G texels' set-up (inscatterS.glsl:113-122, FP64); products rounded
+            // on their own and explicit fma: every G gives the same bits.  Its uniform
+            // terms are read from LDS by each group, so that no FP64 value takes a
+            // register over the direction loop.
+            float vx, vz, sxp[G], syp[G];
+            {
+                asm volatile("" ::: "memory");
+                const volatile double *us = s_u;
+                const double uS = us[0], uq = us[1], ur = us[2], up = us[3];
+                double mu, muS_t, nu0;
+                mu_mus_nu(s, s.layers[l], kb * s.RMUS + m, y, mu, muS_t, nu0);
                 mu = fmin(fmax(mu, -1.0), 1.0);
-                const double var = sqrt(1.0 - mu * mu) * sqrt(1.0 - muS * muS);
-                nu = fmin(fmax(nu, muS * mu - var), muS * mu + var);
-                const double vxd = sqrt(1.0 - mu * mu);
-                const double sxd = vxd == 0.0 ? 0.0 : (nu - muS * mu) / vxd;
-                const double syd = sqrt(fmax(0.0, 1.0 - sxd * sxd - muS * muS));
+                const double vxd = sqrt(fma(-mu, mu, 1.0)), var = __dmul_rn(vxd, ur), mm = __dmul_rn(uS, mu);
                 vx = (float)vxd;
                 vz = (float)mu;
-                sxp[g] = (float)(posAd * sxd);
-                syp[g] = (float)(posAd * syd);
+    #pragma unroll
+                for (int g = 0; g < G; ++g) {
+                    const int k = min(kb + g, NU - 1);
+                    double nu = -1.0 + (double)k / (s.RNU - 1.0) * 2.0;
+                    nu = fmin(fmax(nu, mm - var), mm + var);
+                    const double sxd = vxd == 0.0 ? 0.0 : (nu - mm) / vxd;
+                    const double syd = sqrt(fmax(0.0, fma(-sxd, sxd, uq)));
+                    sxp[g] = (float)(up * sxd);
+                    syp[g] = (float)(up * syd);
+                }
             }
             const float cx1 = m2g * vx;
+            int vzero;
+            asm("v_mov_b32 %0, 0" : "=v"(vzero));
             float acc[G][3];
     #pragma unroll
             for (int g = 0; g < G; ++g)
@@ -649,52 +709,64 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k
 
             // 4D lookup of one direction from the staged pairs: the clamp of the
             // nu slice is implicit, |s.w| <= 1 keeps pos in [1, RNU] (+ rounding)
-            // and kk = trunc(pos) in [0, RNU] = the staged pair range.
+            // and the entry in [0, RNU] = the staged pair range.
             // (order 2: the Rayleigh and Mie values weighted by the phase functions of
             // nu1 = s.w, as q1 (R + z1 M) with q1 = 1 + nu1^2, z1 = (1+g^2-2g nu1)^-3/2;
             // the caller applies q1, whose per-set constants are folded into the staging)
-            auto lookup = [&](const float4 *pt, float pos, float out[3], float &q1) {
-                const unsigned kk = __float2uint_rz(pos);
-                // ES = 3: a 24-bit multiply (full rate; kk <= RNU) instead of the
-                // 32-bit one the compiler picks; 2 and 1: a shift
-                const float4 *pp = pt + (ES == 3 ? __umul24(kk, (unsigned)ES) : kk * ES);
-                const float4 a = pp[0];
+            // Orders >= 3, ground direction: the merged sky + ground entry of the
+            // segment holding pos (4b).  floor(xg) is exact (v_floor): the row's cells
+            // are those of its floor, so a tie has to go up.
+            struct Tap {
+                float u;
+                float4 a, b, c;   // orders >= 3: a, b.xy
+            };
+            auto fetch = [&](auto gr, float pt, unsigned pi, float gb, float cg1, float cg0, float u) {
+                Tap t;
+                t.u = u;
+                unsigned pp;
+                if constexpr (!FIRST && decltype(gr)::value) {
+                    const float fg = floorf(fmaf(u, cg1, cg0));   // >= 0: EPAD is folded into cg0
+                    pp = __float_as_uint(fmaf(fg, 32.0f * 1.40129846e-45f, fmaf(u + kRound, 32.0f * 1.40129846e-45f, gb)));
+                } else if constexpr (ES == 3) {   // 48-byte entries: the addend has no exact FP32 form
+                    pp = pi + __umul24(__float2uint_rz(u + 0.5f), 48u);
+                } else {
+                    pp = lds_entry<16 * ES>(u, pt);
+                }
+                t.a = lds4(pp);
+                if (FIRST) {
+                    t.b = lds4(pp, 16 * CS);
+                    t.c = lds4(pp, 32 * CS);
+                } else {
+                    const float2 d = lds2(pp, 16);
+                    t.b.x = d.x;
+                    t.b.y = d.y;
+                }
+                return t;
+            };
+            auto value = [&](const Tap &t, float out[3], float &q1) {
+                const float u = t.u;
                 if (!FIRST) {
-                    const float2 d = *(const float2 *)(pp + 1);
-                    out[0] = fmaf(pos, a.w, a.x);
-                    out[1] = fmaf(pos, d.x, a.y);
-                    out[2] = fmaf(pos, d.y, a.z);
+                    out[0] = fmaf(u, t.a.w, t.a.x);
+                    out[1] = fmaf(u, t.b.x, t.a.y);
+                    out[2] = fmaf(u, t.b.y, t.a.z);
                     q1 = 1.0f;
                 } else {
-                    const float4 b = pp[CS], c2 = pp[2 * CS];
-                    const float nu1 = fmaf(pos, iposA, nposBi);
+                    const float nu1 = fmaf(u, iposA, nposBi);
                     q1 = fmaf(nu1, nu1, 1.0f);
                     const float y1 = __builtin_amdgcn_rsqf(fmaf(m2g, nu1, g2p1));
                     const float z1 = y1 * y1 * y1;
-                    const float m0 = fmaf(pos, c2.y, b.z), m1 = fmaf(pos, c2.z, b.w), m2 = fmaf(pos, c2.w, c2.x);
-                    out[0] = fmaf(m0, z1, fmaf(pos, a.w, a.x));
-                    out[1] = fmaf(m1, z1, fmaf(pos, b.x, a.y));
-                    out[2] = fmaf(m2, z1, fmaf(pos, b.y, a.z));
+                    const float m0 = fmaf(u, t.c.y, t.b.z), m1 = fmaf(u, t.c.z, t.b.w), m2 = fmaf(u, t.c.w, t.c.x);
+                    out[0] = fmaf(m0, z1, fmaf(u, t.a.w, t.a.x));
+                    out[1] = fmaf(m1, z1, fmaf(u, t.b.x, t.a.y));
+                    out[2] = fmaf(m2, z1, fmaf(u, t.b.y, t.a.z));
                 }
             };
-            // orders >= 3, ground direction: the merged sky + ground entry of the
-            // segment holding pos (4b)
-            auto glookup = [&](unsigned gb, float pos, float cg1, float cg0, float out[3]) {
-                const float xg = fmaf(pos, cg1, cg0);   // >= 0: EPAD is folded into cg0
-                const unsigned e = __float2uint_rz(pos) + __float2uint_rz(xg);
-                const float4 *pp = pairs + (gb + e * PW);
-                const float4 a = pp[0];
-                const float2 b = *(const float2 *)(pp + 1);
-                out[0] = fmaf(pos, a.w, a.x);
-                out[1] = fmaf(pos, b.x, a.y);
-                out[2] = fmaf(pos, b.y, a.z);
-            };
             // irradiance at the ground point seen in direction w, row 0 of dE
-            auto ground_e = [&](float pos, float cg1, float cg0, float out[3]) {
-                const float xg = fmaf(pos, cg1, cg0);   // >= 0: EPAD is folded into cg0
-                const unsigned kg = __float2uint_rz(xg);
-                const float4 ea = epair[2 * kg];
-                const float2 ed = *(const float2 *)(epair + 2 * kg + 1);
+            auto ground_e = [&](float u, float cg1, float cg0, float out[3]) {
+                const float xg = fmaf(u, cg1, cg0);   // texel coordinate - 1/2
+                const unsigned pe = lds_entry<32>(xg, epb);
+                const float4 ea = lds4(pe);
+                const float2 ed = lds2(pe, 16);
                 out[0] = fmaf(xg, ea.w, ea.x);
                 out[1] = fmaf(xg, ed.x, ea.y);
                 out[2] = fmaf(xg, ed.y, ea.z);
@@ -708,22 +780,37 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k
                 const float vzwz = vz * ct;
                 const float cx0 = fmaf(m2g, vzwz, g2p1);
                 const float dw = g1.w, cp = g1.z;
-                const float4 *pt = pairs + (size_t)rowoff(itl) * ES;
-                // merged ground row: entry (floor(pos) + floor(xg)) - jlo, as an
-                // index that wraps modulo 2^32 (jlo may exceed the row offset)
-                const unsigned gbase = (unsigned)(rowoff(itl) - __float_as_int(gdat[3 * itl + 2].x)) * PW;
-                const float2 *wrow = dirW + (size_t)it * 2 * NS;
+                const unsigned pi = pairs_b + (unsigned)rowoff(itl) * 16 * ES;
+                const float pt = lds_addend<16 * ES>(pi);
+                // merged ground row: entry (floor(pos) + floor(xg)) - jlo (the exact
+                // sum of the two products is base + 32 (k + floor(xg) - jlo))
+                const float gbase = ((float)(int)(pairs_b + 32 * (rowoff(itl) - __float_as_int(gdat[3 * itl + 2].x))) -
+                                     32.0f * kRound) * 1.40129846e-45f;
+                // through a vector address: in a scalar register, w would halve the
+                // rate of every FMA that takes it
+                const float2 *wrow = dirW + (size_t)it * 2 * NS + vzero;
                 // the directions of one theta row; GR: a merged ground row of orders
                 // >= 3 (a compile-time branch, so the lookups of all G texels stay
                 // one straight sequence)
                 auto phi_row = [&](auto gr) {
                     constexpr bool GR = decltype(gr)::value;
                     float2 wn = wrow[0];
+                    // Orders >= 3: the lookups of texel g + 1 are read while texel g's are
+                    // used; without the second set in flight four waves per SIMD do not
+                    // cover the LDS (8.6 against 7.9 ms per order, G = 8, 64x256x64x16).
+                    constexpr int AHEAD = FIRST ? 0 : 1;   // (order 2 has no registers for it)
+                    Tap ta[2], tb[2];
+                    auto fetch_pair = [&](int g, float2 w) {
+                        const float base = fmaf(sxp[g], w.x, cp);
+                        ta[g & 1] = fetch(gr, pt, pi, gbase, g1.x, g1.y, fmaf(syp[g], w.y, base));
+                        tb[g & 1] = fetch(gr, pt, pi, gbase, g1.x, g1.y, fmaf(-syp[g], w.y, base));
+                    };
                     // directions phi and 2 pi - phi together: same w.x, opposite w.y,
                     // hence the same nu2 = v.w (v has no y component) and weights
                     for (int ip = 0; ip < NS; ++ip) {
                         const float2 w = wn;
-                        if (ip + 1 < NS) wn = wrow[ip + 1];  // scalar prefetch of the next direction
+                        if (ip + 1 < NS) wn = wrow[ip + 1];  // prefetch of the next direction
+                        if (AHEAD) fetch_pair(0, w);
                         const float nu2 = fmaf(vx, w.x, vzwz);
                         const float q2 = fmaf(nu2 * dw, nu2, dw);
                         const float y2 = __builtin_amdgcn_rsqf(fmaf(cx1, w.x, cx0));
@@ -731,44 +818,32 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k
                         // betaR e^(-h/HR) pR(nu2) dw + betaMSca e^(-h/HM) pM(nu2) dw (:182-185)
                         const float W0 = fmaf(A0, q2, B0 * t2), W1 = fmaf(A1, q2, B1 * t2),
                                     W2 = fmaf(A2, q2, B2 * t2);
-                        float pa[G], pb[G], lv[G][3];
     #pragma unroll
                         for (int g = 0; g < G; ++g) {
-                            const float base = fmaf(sxp[g], w.x, cp);
-                            pa[g] = fmaf(syp[g], w.y, base);
-                            pb[g] = fmaf(-syp[g], w.y, base);
-                            float la[3], lb[3], qa, qb;
-                            if constexpr (!FIRST && GR) {
-                                glookup(gbase, pa[g], g1.x, g1.y, la);
-                                glookup(gbase, pb[g], g1.x, g1.y, lb);
-                            } else {
-                                lookup(pt, pa[g], la, qa);
-                                lookup(pt, pb[g], lb, qb);
-                            }
+                            if (g + AHEAD < G) fetch_pair(g + AHEAD, w);
+                            if (AHEAD) __builtin_amdgcn_sched_barrier(0);
+                            const Tap &a = ta[g & 1], &b = tb[g & 1];
+                            float la[3], lb[3], lv[3], qa, qb;
+                            value(a, la, qa);
+                            value(b, lb, qb);
                             if (FIRST) {
     #pragma unroll
-                                for (int c = 0; c < 3; ++c) lv[g][c] = fmaf(qa, la[c], qb * lb[c]);
+                                for (int c = 0; c < 3; ++c) lv[c] = fmaf(qa, la[c], qb * lb[c]);
                             } else {
     #pragma unroll
-                                for (int c = 0; c < 3; ++c) lv[g][c] = la[c] + lb[c];
+                                for (int c = 0; c < 3; ++c) lv[c] = la[c] + lb[c];
                             }
-                        }
-                        if (FIRST && ground) {   // order 2: the separate ground term (uniform branch)
-    #pragma unroll
-                            for (int g = 0; g < G; ++g) {
+                            if (FIRST && ground) {   // order 2: the separate ground term (uniform branch)
                                 float ea[3], eb[3];
-                                ground_e(pa[g], g1.x, g1.y, ea);
-                                ground_e(pb[g], g1.x, g1.y, eb);
-                                lv[g][0] = fmaf(g0.x, ea[0] + eb[0], lv[g][0]);
-                                lv[g][1] = fmaf(g0.y, ea[1] + eb[1], lv[g][1]);
-                                lv[g][2] = fmaf(g0.z, ea[2] + eb[2], lv[g][2]);
+                                ground_e(a.u, g1.x, g1.y, ea);
+                                ground_e(b.u, g1.x, g1.y, eb);
+                                lv[0] = fmaf(g0.x, ea[0] + eb[0], lv[0]);
+                                lv[1] = fmaf(g0.y, ea[1] + eb[1], lv[1]);
+                                lv[2] = fmaf(g0.z, ea[2] + eb[2], lv[2]);
                             }
-                        }
-    #pragma unroll
-                        for (int g = 0; g < G; ++g) {
-                            acc[g][0] = fmaf(lv[g][0], W0, acc[g][0]);
-                            acc[g][1] = fmaf(lv[g][1], W1, acc[g][1]);
-                            acc[g][2] = fmaf(lv[g][2], W2, acc[g][2]);
+                            acc[g][0] = fmaf(lv[0], W0, acc[g][0]);
+                            acc[g][1] = fmaf(lv[1], W1, acc[g][1]);
+                            acc[g][2] = fmaf(lv[2], W2, acc[g][2]);
                         }
                     }
                 };
@@ -1386,7 +1461,7 @@ size_t lds_inscatterS(int NS, int CH, int RNU, int SW, int JX, bool first) {
     const size_t npairs = (size_t)CH * (RNU + 1) + (first ? 0 : (size_t)JX);
     const bool planes = first && !inscatterS_chunked(NS, CH, RNU, first);
     return sizeof(float4) * ((planes ? 2 * (size_t)kJ1Plane + npairs : npairs * PW) +
-                             (planes ? 0 : (size_t)CH * (RNU + 2) * NT) +
+                             (planes ? 0 : (size_t)CH * (RNU + 2) * NT) + 1 +
                              (first ? (size_t)(e_pad(SW) + SW + 1) * 2 : 0) + (size_t)CH * 3);
 }
 int merged_row_extra(double r, double Rg, double Rt, int SW, int NS, int it) {

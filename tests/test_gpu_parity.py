@@ -779,6 +779,25 @@ def test_every_inscatterS_variant_gives_identical_tables(eng, res):
     _assert("S", outs[0][2].double().cpu().numpy(), S, TOL)
 
 
+@pytest.mark.parametrize("nu,sw,ns", [(2, 2, 3), (3, 7, 5), (4, 16, 2), (9, 50, 16), (15, 128, 31), (16, 33, 33),
+                                      (16, 64, 40)])
+def test_inscatterS_lookups_at_the_ends_of_their_rows(eng, nu, sw, ns):
+    """The fewest and most nu slices, ground rows of 2 to 128 texels, odd direction
+    grids (a direction on the horizon, positions on an entry's edge) and, at 40 and
+    33 x 66 directions of 16 slices, the chunked order 2: every texels-per-thread
+    variant bit for bit, the tables within the bar of the whole-chain tests."""
+    p = small(res=(4, 12, 6, nu), E=(sw, 4))
+    kw = dict(orders=3, spherical_samples=ns)
+    outs = [eng.precompute(p, options(flags=8, texels_per_thread=g, **kw))[0] for g in (2, 3, 4, 8)]
+    torch.cuda.synchronize()
+    for o in outs[1:]:
+        for a, b in zip(outs[0], o):
+            assert torch.equal(a, b)
+    T, E, S = O.precompute(p, options(**kw))
+    _assert("S", outs[0][2].double().cpu().numpy(), S, TOL)
+    _assert("E", outs[0][1].double().cpu().numpy(), E, TOL)
+
+
 @pytest.mark.parametrize("ci", range(len(CASES)))
 @pytest.mark.parametrize("form", [2, 3])
 def test_pass_inscatterN_staged_form(eng, ci, form):
