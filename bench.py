@@ -186,7 +186,7 @@ def main():
     # lookups; the third argument is the staging-in-rounds variant)
     later = [ms for name, order, ms in times if name == "inscatterS" and order >= 3]
     avg_ms = sum(later) / len(later)
-    kname = "k_inscatterS<false,%d,false>" % eng.tuning().get("inscatterS_texels_per_thread", 4)
+    kname = "k_inscatterS<false,%d,0>" % eng.tuning().get("inscatterS_texels_per_thread", 4)
     traffic = profiled(TRAFFIC_PROFILE, "traffic", kname)
     # FP32 FLOPs one launch executes (rocprofv3 SQ_INSTS_VALU_FLOPS_FP32 x 64 lanes,
     # FMA = 2) over its live launch time: the roofline figure

@@ -323,8 +323,41 @@ int jg_for_set(const atmo_params &p) {
     return best;
 }
 
-struct JSeg {   // a run of P_J tiles whose sets share one G
+// Slots k_inscatterS deals the theta rows of a set's workgroups to (1: none):
+// doubled while the set's own waves, counted with four texels per thread, stay
+// below two per SIMD (2048), where latency is no longer covered.  16x64x16x4 (256
+// workgroups of one wave), order 2 / order 3 in us: 1 slot 114 / 62, 2 62 / 36,
+// 4 44 / 27, 8 42 / 26, 16 44 / 27; 21x90x27x5 (1134 waves): 1 slot 134 / 66, 2
+// 129 / 65, 4 134 / 75.  A property of the set and the options alone, and not of
+// the texels per thread: the sums are added in slot order, so the bits of a
+// set's tables depend on the slots.
+int dj_split(const atmo_params &p, const atmo_options &o) {
+    const long waves = (long)p.RES_R * p.RES_MU_S * ((p.RES_MU * ((p.RES_NU + 3) / 4) + 63) / 64);
+    int ds = 1;
+    while (ds < 8 && 2 * ds <= o.spherical_samples && waves * ds < 2048) ds *= 2;
+    if (ds == 1) return 1;
+    // all theta rows staged at once, with room for the partial sums
+    const int NS = o.spherical_samples;
+    const size_t cap = kSphLdsBudget - sizeof(float) * 3 * kJSplitThreads;
+    if (inscatterS_chunked(NS, NS, p.RES_NU, true) || lds_inscatterS(NS, NS, p.RES_NU, p.SKY_W, 0, true) > cap) return 1;
+    const int jx = merged_extra(&p, 1, NS, NS);
+    return lds_inscatterS(NS, NS, p.RES_NU, p.SKY_W, jx, false) > cap ? 1 : ds;
+}
+
+// Threads of a k_inscatterS workgroup that deals its theta rows to ds slots:
+// every slot holds the set's groups of G texels, as far as they fit.
+int dj_threads(int RMU, int NU, int G, int ds) {
+    if (ds == 1) return 256;
+    const int waves = (RMU * ((NU + G - 1) / G) + 63) / 64;
+    return 64 * ds * std::min(waves, kJSplitThreads / 64 / ds);
+}
+
+struct JSeg {   // a run of P_J tiles whose sets share one G, or one split
     int G, off, cnt;
+    int DS = 1;               // slots (1: the plan's staging, 256 threads)
+    int RMU = 0, NU = 0, SW = 0;   // of a split's sets
+    int jx = 0;               // merged ground rows and LDS of a split's launches
+    size_t lds1 = 0, lds = 0;
 };
 struct NSeg {   // a run of P_SN tiles whose sets share one workgroup shape
     SnShape sh;
@@ -333,7 +366,7 @@ struct NSeg {   // a run of P_SN tiles whose sets share one workgroup shape
 
 // Kernel variants chosen by the autotuner, with the times measured for each.
 struct Tuning {
-    int jG = 4, snXcd = 1, snForm = 1;   // jG = 0: per-set choice
+    int jG = 4, jG1 = 4, snXcd = 1, snForm = 1;   // jG, jG1 = 0: per-set choice
     float msJ[5] = {0, 0, 0, 0, 0};  // G = 2, 3, 4, 8, per set (order-2 + order->=3 launches)
     float msN[6] = {};   // [direct, staged][plain, XCD, XCD + line order]
 };
@@ -357,7 +390,7 @@ struct Plan {
     hipGraph_t graph = nullptr;
     hipGraphExec_t gexec = nullptr;
     // kernel variants (picked by the autotuner)
-    int jG = 4;        // k_inscatterS texels per thread (0: per set, see jg_for_set)
+    int jG = 4, jG1 = 4;   // k_inscatterS texels per thread, orders >= 3 and order 2 (0: per set, see jg_for_set)
     std::vector<JSeg> jseg;   // P_J tiles grouped by the per-set G
     std::vector<NSeg> nseg;   // P_SN tiles grouped by row class
     bool view = true;  // the sets have SetDesc::view
@@ -575,6 +608,8 @@ void build_tiles(const std::vector<atmo_params> &ps, const atmo_options &o,
                 // grouped by the per-set G (descending), most expensive first inside a group
                 nt = (long long)p.RES_R * p.RES_MU_S;
                 cost = jg_for_set(p) * 1e12 + (double)p.RES_MU * p.RES_NU;
+                if (dj_split(p, o) > 1)   // behind the others, the sets of one split together
+                    cost = -((dj_split(p, o) * 1e4 + p.RES_MU) * 1e4 + p.RES_NU);
                 break;
             case P_EN: nt = (long long)z.nE; cost = (double)p.RES_NU; break;
             case P_VIEW: nt = ((long long)p.RES_R * p.RES_MU * (o.inscatter_samples + 1) + 255) / 256; break;
@@ -593,9 +628,28 @@ void build_tiles(const std::vector<atmo_params> &ps, const atmo_options &o,
         if (pass == P_J && jseg) {
             jseg->clear();
             for (size_t i = 0; i < v.size(); ++i) {
-                const int g = jg_for_set(ps[v[i].second.x]);
-                if (jseg->empty() || jseg->back().G != g) jseg->push_back({g, (int)i, 0});
+                const atmo_params &p = ps[v[i].second.x];
+                if (i && v[i].second.x == v[i - 1].second.x) {
+                    jseg->back().cnt += 1;
+                    continue;
+                }
+                JSeg g{jg_for_set(p), (int)i, 0, dj_split(p, o)};
+                if (g.DS > 1) {
+                    g.RMU = p.RES_MU;
+                    g.NU = p.RES_NU;
+                }
+                if (jseg->empty() || jseg->back().G != g.G || jseg->back().DS != g.DS || jseg->back().RMU != g.RMU ||
+                    jseg->back().NU != g.NU)
+                    jseg->push_back(g);
                 jseg->back().cnt += 1;
+                if (g.DS > 1) {
+                    const int NS = o.spherical_samples;
+                    JSeg &b = jseg->back();
+                    b.jx = std::max(b.jx, merged_extra(&p, 1, NS, NS));
+                    b.SW = std::max(b.SW, p.SKY_W);
+                    b.lds1 = lds_inscatterS(NS, NS, b.NU, b.SW, 0, true);
+                    b.lds = lds_inscatterS(NS, NS, b.NU, b.SW, b.jx, false);
+                }
             }
         }
         if (pass == P_J) {
@@ -629,17 +683,25 @@ void build_tiles(const std::vector<atmo_params> &ps, const atmo_options &o,
 hipError_t launch_dj(const Plan &pl, const SetDesc *S, const uint2 *T, const char *dirs, bool first, int G,
                      hipStream_t st) {
     const atmo_options &o = pl.opts;
-    const size_t lds = first ? pl.ldsJ1 : pl.ldsJ;
-    const int ch = first ? pl.chJ1 : pl.chJ;
-    if (G != 0)
-        return launch_inscatterS(S, T + pl.off[P_J], pl.cnt[P_J], o.spherical_samples, ch, pl.maxNU, pl.jx,
-                                 dirs + pl.dirJT_off, dirs + pl.dirJW_off, first, lds, G, st);
+    const int NS = o.spherical_samples;
+    auto run = [&](int off, int cnt, int ch, int NU, int jx, size_t lds, int g, int ds, int threads) {
+        return launch_inscatterS(S, T + pl.off[P_J] + off, cnt, NS, ch, NU, jx, dirs + pl.dirJT_off,
+                                 dirs + pl.dirJW_off, first, lds, g, ds, threads, st);
+    };
+    hipError_t e = hipSuccess;
+    int whole = 0;   // tiles of the sets that are not split: the first segments
     for (const JSeg &g : pl.jseg) {
-        hipError_t e = launch_inscatterS(S, T + pl.off[P_J] + g.off, g.cnt, o.spherical_samples, ch, pl.maxNU, pl.jx,
-                                         dirs + pl.dirJT_off, dirs + pl.dirJW_off, first, lds, g.G, st);
+        if (g.DS == 1) {
+            whole += g.cnt;
+            if (G == 0) e = run(g.off, g.cnt, first ? pl.chJ1 : pl.chJ, pl.maxNU, pl.jx, first ? pl.ldsJ1 : pl.ldsJ, g.G, 1, 256);
+        } else {
+            const int gg = G ? G : g.G;
+            e = run(g.off, g.cnt, NS, g.NU, g.jx, first ? g.lds1 : g.lds, gg, g.DS, dj_threads(g.RMU, g.NU, gg, g.DS));
+        }
         if (e != hipSuccess) return e;
     }
-    return hipSuccess;
+    if (G != 0) e = run(0, whole, first ? pl.chJ1 : pl.chJ, pl.maxNU, pl.jx, first ? pl.ldsJ1 : pl.ldsJ, G, 1, 256);
+    return e;
 }
 
 // The dSn pass: one launch per workgroup shape.  S: descriptors; T: the pass's
@@ -704,7 +766,7 @@ atmo_status launch_all(Plan &pl, hipStream_t st, PassTimer *tm = nullptr) {
     for (int order = 2; order <= o.orders; ++order) {
         const bool first = order == 2;
         HIPCHK(t.begin(3, order));
-        HIPCHK(launch_dj(pl, S, T, dirs, first, pl.jG, st));
+        HIPCHK(launch_dj(pl, S, T, dirs, first, first ? pl.jG1 : pl.jG, st));
         HIPCHK(t.end());
         HIPCHK(t.begin(4, order));
         HIPCHK(launch_irradianceN(S, T + pl.off[P_EN], pl.cnt[P_EN], o.irradiance_samples,
@@ -794,7 +856,7 @@ atmo_status autotune(Plan &pl, hipStream_t st, Tuning &tu) {
     // choices differ (otherwise it is the same launch as one of the others)
     const int Gs[5] = {2, 3, 4, 8, 0};
     const bool mixedG = pl.jseg.size() > 1;
-    float bestJ = 1e30f;
+    float bestJ = 1e30f, bestJ1 = 1e30f;
     for (int gi = 0; gi < 5; ++gi) {
         if (Gs[gi] == 0 && !mixedG) {
             tu.msJ[gi] = -1.f;
@@ -807,9 +869,13 @@ atmo_status autotune(Plan &pl, hipStream_t st, Tuning &tu) {
         if (rc != ATMO_OK) return rc;
         // weight: one order-2 launch, (orders - 2) later ones
         tu.msJ[gi] = m1 + m2 * std::max(0, o.orders - 2);
-        if (tu.msJ[gi] < bestJ) {
-            bestJ = tu.msJ[gi];
+        if (m2 < bestJ) {
+            bestJ = m2;
             tu.jG = Gs[gi];
+        }
+        if (m1 < bestJ1) {
+            bestJ1 = m1;
+            tu.jG1 = Gs[gi];
         }
     }
     // k_inscatterN variants: descriptors without S (the accumulation is skipped)
@@ -851,6 +917,7 @@ atmo_status autotune(Plan &pl, hipStream_t st, Tuning &tu) {
 atmo_status apply_tuning(Plan &pl, const Tuning &tu) {
     const bool retile = tu.snXcd != pl.snXcd;
     pl.jG = pl.opts.texels_per_thread ? pl.opts.texels_per_thread : tu.jG;
+    pl.jG1 = pl.opts.texels_per_thread ? pl.opts.texels_per_thread : tu.jG1;
     pl.snXcd = tu.snXcd;
     pl.snForm = pl.opts.inscatterN_form ? sn_form(pl.opts.inscatterN_form) : tu.snForm;
     pl.tuned = true;
@@ -875,11 +942,12 @@ atmo_status build_plan(hipStream_t xs, const atmo_params *sets, int nsets, const
     pl->xs = xs;
     pl->params.assign(sets, sets + nsets);
     pl->opts = o;
-    pl->jG = o.texels_per_thread;   // 0: each set with its own G until the tuner has run
+    pl->jG = pl->jG1 = o.texels_per_thread;   // 0: each set with its own G until the tuner has run
     pl->snForm = sn_form(o.inscatterN_form);
     pl->view = view;
     if (tu) {
         pl->jG = o.texels_per_thread ? o.texels_per_thread : tu->jG;
+        pl->jG1 = o.texels_per_thread ? o.texels_per_thread : tu->jG1;
         pl->snXcd = tu->snXcd;
         pl->snForm = o.inscatterN_form ? sn_form(o.inscatterN_form) : tu->snForm;
         pl->tuned = true;
@@ -1425,7 +1493,7 @@ static atmo_status pass_run(atmo_engine *e, const atmo_params *p, const atmo_opt
         const int jx = first ? 0 : jx_of_ch(ch);
         const size_t lds = lds_inscatterS(o.spherical_samples, ch, p->RES_NU, p->SKY_W, jx, first);
         HIPCHK(launch_inscatterS(S, T + off[P_J], cnt[P_J], o.spherical_samples, ch, p->RES_NU, jx, d + oJT, d + oJW, first,
-                                 lds, o.texels_per_thread ? o.texels_per_thread : jg_for_set(*p), hs));
+                                 lds, o.texels_per_thread ? o.texels_per_thread : jg_for_set(*p), 1, 256, hs));
         break;
     }
     case P_EN: {

@@ -32,6 +32,10 @@ constexpr size_t kSphLdsBudget = 64 * 1024;
 // RES_NU 16.  Chunked: CH < NS, or an order-2 round too large for a plane
 // (those launches use the chunked variant, also for a single round).
 constexpr int kJ1Plane = 544;
+// k_inscatterS forms: all theta rows staged at once, staged in chunks, or all
+// at once with the rows dealt to DS slots of a workgroup's threads
+constexpr int kJPlain = 0, kJChunk = 1, kJSplit = 2;
+constexpr int kJSplitThreads = 1024;
 bool inscatterS_chunked(int NS, int CH, int RNU, bool first);
 size_t lds_inscatterS(int NS, int CH, int RNU, int SW, int JX, bool first);
 // bound on the extra entries of theta row `it` (NS rows) of a layer at radius r
@@ -54,7 +58,7 @@ hipError_t launch_inscatter1(const SetDesc *sets, const uint2 *tiles, int ntiles
 // the largest RES_NU of the launch's sets
 hipError_t launch_inscatterS(const SetDesc *sets, const uint2 *tiles, int ntiles, int NS, int CH, int RNU,
                              int JX, const void *dirT, const void *dirW, bool first, size_t lds, int G,
-                             hipStream_t st);
+                             int DS, int threads, hipStream_t st);
 hipError_t launch_irradianceN(const SetDesc *sets, const uint2 *tiles, int ntiles, int NI, int CH,
                               const void *dirs, bool first, size_t lds, hipStream_t st);
 // The dSn pass, one mu row (tile) per workgroup.  form: 0 direct gathers, 1

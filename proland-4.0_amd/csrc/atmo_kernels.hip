@@ -344,7 +344,8 @@ __device__ __forceinline__ void stage_slice(const SetDesc &s, const float4 *cons
 // in about 2 cycles per wave; with a scalar-register operand, and a conversion,
 // floor, shift or integer multiply-add, in 4.  So the loop keeps its operands in
 // vector registers and forms LDS addresses with FMAs (lds_entry): 8.6 -> 7.8 ms;
-// 16x64x16x4: order 2 130 -> 116 us, order 3 73 -> 60.
+// 16x64x16x4 is bound by the latency of one wave per SIMD instead: order 2
+// 130 -> 116 us, order 3 73 -> 60, and 42 and 26 us with the theta rows split.
 // ---------------------------------------------------------------------------
 // Entries of padding in front of the staged ground-irradiance row: texel
 // coordinates down to -(0.8/1.2) SW - 0.5 (mu_s = -1) plus rounding.
@@ -403,11 +404,16 @@ struct DirJ {      // per-theta constants of the NS x 2NS grid
 // allows): G = 8 then keeps its direction loops free of spills (its per-group
 // set-up spills a few registers) and runs 2 % faster than G = 4 at 32 x 64
 // directions; at 166 VGPRs (three waves) it ran 14 % slower.
-template <bool FIRST, int G, bool CHUNK>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k_inscatterS(const SetDesc *__restrict__ sets,
-                                                    const uint2 *__restrict__ tiles, int NS, int CH,
-                                                    int JX, const DirJ *__restrict__ dirT,
-                                                    const float2 *__restrict__ dirW) {
+//
+// SPLIT: sets with too few columns to fill the chip (16x64x16x4 has 256
+// workgroups of 64 groups, one wave on a quarter of the SIMDs): the workgroup has
+// DS slots of threads for its groups, each takes every DS-th theta row, and the
+// slots' sums are added through LDS in slot order.
+template <bool FIRST, int G, int MODE>
+__global__ __launch_bounds__(MODE == kJSplit ? kJSplitThreads : 256) __attribute__((amdgpu_waves_per_eu(4))) void
+k_inscatterS(const SetDesc *__restrict__ sets, const uint2 *__restrict__ tiles, int NS, int CH, int JX, int DS,
+             const DirJ *__restrict__ dirT, const float2 *__restrict__ dirW) {
+    constexpr bool CHUNK = MODE == kJChunk, SPLIT = MODE == kJSplit;
     constexpr int NT = FIRST ? 2 : 1;
     constexpr int PW = FIRST ? 3 : 2;      // float4 per staged pair entry
     extern __shared__ __attribute__((aligned(32))) float4 lds[];   // lds_entry: 32-byte strides
@@ -438,6 +444,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k
     // [EPAD + SW + 1][2] (order 2), 32-byte aligned
     float4 *epair = lds + (((vtmp - lds) + (PLANES ? 0 : (size_t)CH * NV * NT) + 1) & ~(size_t)1);
     float4 *gdat = epair + (FIRST ? (size_t)(EPAD + s.SW + 1) * 2 : 0);   // [CH][3]
+    float *part = (float *)(gdat + 3 * CH);   // SPLIT: [DS - 1][3][threads / DS] partial sums
 
     const LayerGeom L = s.layers[l];
     const double r = fmin(fmax(L.r, s.Rg), s.Rt);          // inscatterS.glsl:112
@@ -654,7 +661,14 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k
         }
         __syncthreads();
 
-        for (int grp = threadIdx.x; grp < ngroups; grp += blockDim.x) {
+        // SPLIT: the threads are DS slots of gpi threads (whole waves); slot ds takes
+        // the theta rows ds, ds + DS, ... of the groups of all slots
+        const int gpi = SPLIT ? (int)blockDim.x / DS : (int)blockDim.x;
+        const int ds = SPLIT ? __builtin_amdgcn_readfirstlane((int)threadIdx.x / gpi) : 0;
+        const int gt = (int)threadIdx.x - ds * gpi;
+        for (int base = 0; base < ngroups; base += gpi) {
+            if (!SPLIT && base + gt >= ngroups) break;
+            const int grp = SPLIT ? min(base + gt, ngroups - 1) : base + gt;
             const int y = grp % s.RMU, kb = (grp / s.RMU) * G;
             // the G texels' set-up (inscatterS.glsl:113-122, FP64); products rounded
             // on their own and explicit fma: every G gives the same bits.  Its uniform
@@ -772,7 +786,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k
                 out[2] = fmaf(xg, ed.y, ea.z);
             };
 
-            for (int itl = 0; itl < nth; ++itl) {
+            for (int itl = SPLIT ? ds : 0; itl < nth; itl += SPLIT ? DS : 1) {
                 const int it = c0 + itl;
                 const float ct = dirT[it].ct;
                 const float4 g0 = gdat[3 * itl], g1 = gdat[3 * itl + 1];
@@ -793,7 +807,6 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k
                 // >= 3 (a compile-time branch, so the lookups of all G texels stay
                 // one straight sequence)
                 auto phi_row = [&](auto gr) {
-                    constexpr bool GR = decltype(gr)::value;
                     float2 wn = wrow[0];
                     // Orders >= 3: the lookups of texel g + 1 are read while texel g's are
                     // used; without the second set in flight four waves per SIMD do not
@@ -849,6 +862,23 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k
                 };
                 if (!FIRST && ground) phi_row(std::true_type{});
                 else phi_row(std::false_type{});
+            }
+            if (SPLIT) {   // the slots' sums, added in slot order
+    #pragma unroll
+                for (int g = 0; g < G; ++g) {
+                    float *q = part + ((ds - 1) * 3) * gpi + gt;
+                    if (ds > 0) {
+                        q[0] = acc[g][0]; q[gpi] = acc[g][1]; q[2 * gpi] = acc[g][2];
+                    }
+                    __syncthreads();
+                    for (int j = 0; ds == 0 && j < 3 * (DS - 1); j += 3) {
+                        acc[g][0] += part[j * gpi + gt];
+                        acc[g][1] += part[(j + 1) * gpi + gt];
+                        acc[g][2] += part[(j + 2) * gpi + gt];
+                    }
+                    __syncthreads();
+                }
+                if (ds > 0 || base + gt >= ngroups) continue;
             }
     #pragma unroll
             for (int g = 0; g < G; ++g) {
@@ -1528,26 +1558,32 @@ hipError_t launch_inscatter1(const SetDesc *sets, const uint2 *tiles, int ntiles
 }
 hipError_t launch_inscatterS(const SetDesc *sets, const uint2 *tiles, int ntiles, int NS, int CH, int RNU,
                              int JX, const void *dirT, const void *dirW, bool first, size_t lds, int G,
-                             hipStream_t st) {
+                             int DS, int threads, hipStream_t st) {
     if (ntiles <= 0) return hipSuccess;
     if (CH < 1 || CH > NS || JX < 0) return hipErrorInvalidValue;
-#define ATMO_LJ(F, GG, C)                                                                          \
-    hipLaunchKernelGGL((k_inscatterS<F, GG, C>), dim3(ntiles), dim3(256), lds, st, sets, tiles, NS, \
-                       CH, JX, (const DirJ *)dirT, (const float2 *)dirW)
     if (G != 2 && G != 3 && G != 4 && G != 8) return hipErrorInvalidValue;
-    if (inscatterS_chunked(NS, CH, RNU, first)) {   // chunked staging: one variant (all G give the same bits)
-        if (first) ATMO_LJ(true, 4, true); else ATMO_LJ(false, 4, true);
-    } else if (G == 2) {
-        if (first) ATMO_LJ(true, 2, false); else ATMO_LJ(false, 2, false);
-    } else if (G == 3) {
-        if (first) ATMO_LJ(true, 3, false); else ATMO_LJ(false, 3, false);
-    } else if (G == 4) {
-        if (first) ATMO_LJ(true, 4, false); else ATMO_LJ(false, 4, false);
-    } else if (G == 8) {
-        if (first) ATMO_LJ(true, 8, false); else ATMO_LJ(false, 8, false);
-    } else {
+    const bool chunked = inscatterS_chunked(NS, CH, RNU, first);
+    if (DS < 1 || threads < 64 || threads % (64 * DS) || threads > (DS > 1 ? kJSplitThreads : 256) || (DS > 1 && chunked))
         return hipErrorInvalidValue;
+    if (DS > 1) lds += sizeof(float) * 3 * (size_t)(threads - threads / DS);
+#define ATMO_LJ(F, GG, M)                                                                              \
+    hipLaunchKernelGGL((k_inscatterS<F, GG, M>), dim3(ntiles), dim3(threads), lds, st, sets, tiles, NS, \
+                       CH, JX, DS, (const DirJ *)dirT, (const float2 *)dirW)
+#define ATMO_LJG(F, M)                \
+    switch (G) {                      \
+    case 2: ATMO_LJ(F, 2, M); break;  \
+    case 3: ATMO_LJ(F, 3, M); break;  \
+    case 4: ATMO_LJ(F, 4, M); break;  \
+    default: ATMO_LJ(F, 8, M); break; \
     }
+    if (chunked) {   // chunked staging: one variant (all G give the same bits)
+        if (first) ATMO_LJ(true, 4, kJChunk); else ATMO_LJ(false, 4, kJChunk);
+    } else if (DS > 1) {
+        if (first) ATMO_LJG(true, kJSplit) else ATMO_LJG(false, kJSplit)
+    } else {
+        if (first) ATMO_LJG(true, kJPlain) else ATMO_LJG(false, kJPlain)
+    }
+#undef ATMO_LJG
 #undef ATMO_LJ
     return hipGetLastError();
 }

@@ -798,6 +798,26 @@ def test_inscatterS_lookups_at_the_ends_of_their_rows(eng, nu, sw, ns):
     _assert("E", outs[0][1].double().cpu().numpy(), E, TOL)
 
 
+@pytest.mark.parametrize("res,ns", [((4, 16, 6, 4), 16), ((4, 16, 6, 4), 5), ((4, 16, 6, 4), 3), ((8, 34, 40, 5), 16),
+                                    ((2, 256, 4, 9), 16)])
+def test_inscatterS_theta_rows_split_over_a_workgroup(eng, res, ns):
+    """Few columns: k_inscatterS deals the theta rows to 8 slots of threads (4 and
+    2 with 5 and 3 rows, 4 with 640 waves), once with more groups than a slot
+    holds.  Every texels-per-thread variant, and the set in a batch with one that
+    is not split, bit for bit; the tables within the bar of the whole-chain tests."""
+    p = small(res=res)
+    kw = dict(orders=3, spherical_samples=ns, flags=8)
+    outs = [eng.precompute(p, options(texels_per_thread=g, **kw))[0] for g in (2, 3, 4, 8)]
+    outs.append(eng.precompute([small(res=(32, 128, 20, 8)), p, small(res=(16, 16, 4, 4)), p], options(**kw))[3])
+    torch.cuda.synchronize()
+    for o in outs[1:]:
+        for a, b in zip(outs[0], o):
+            assert torch.equal(a, b)
+    T, E, S = O.precompute(p, options(**kw))
+    _assert("S", outs[0][2].double().cpu().numpy(), S, TOL)
+    _assert("E", outs[0][1].double().cpu().numpy(), E, TOL)
+
+
 @pytest.mark.parametrize("ci", range(len(CASES)))
 @pytest.mark.parametrize("form", [2, 3])
 def test_pass_inscatterN_staged_form(eng, ci, form):
