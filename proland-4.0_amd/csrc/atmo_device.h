@@ -35,6 +35,7 @@ struct LayerGeom {
 // parameterisation: mu_s and, in txb, mu_s + 0.2.
 struct ColGeom {
     float mus, ck, lo, kb, kb2, txb;
+    float hi, lo64;   // mu_s in two parts, for FP64 uses
 };
 
 // A view-ray sample of the dSn pass (k_snview): what does not involve the sun.

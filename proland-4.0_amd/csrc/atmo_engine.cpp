@@ -19,6 +19,7 @@
 #include <memory>
 #include <mutex>
 #include <string>
+#include <tuple>
 #include <vector>
 
 #include <sys/stat.h>
@@ -178,10 +179,11 @@ ColGeom col_geom(const atmo_params &p, const atmo_options &o, int m) {
     const double k = (double)(float)std::tan(1.26 * 1.1), f = m / (p.RES_MU_S - 1.0);
     const double muS = lin ? -0.2 + f * 1.2 : std::tan((2.0 * f - 1.0 + 0.26) * 1.1) / std::tan(1.26 * 1.1);
     const double mub = std::max(muS, -0.1975);
-    if (lin) return {(float)muS, 0.f, 0.f, 0.f, 0.f, (float)(muS + 0.2)};
+    const float hi = (float)muS, lo = (float)(muS - (double)hi);
+    if (lin) return {(float)muS, 0.f, 0.f, 0.f, 0.f, (float)(muS + 0.2), hi, lo};
     return {(float)(k * muS), (float)(k * (muS - mub)), (float)(k * (-0.1975 - mub)), (float)(k * mub),
             (float)(1.0 + k * mub * (k * mub)),
-            (float)((std::atan(mub * std::tan(1.26 * 1.1)) / 1.1 + (1.0 - 0.26)) * 0.5 * (p.RES_MU_S - 1.0))};
+            (float)((std::atan(mub * std::tan(1.26 * 1.1)) / 1.1 + (1.0 - 0.26)) * 0.5 * (p.RES_MU_S - 1.0)), hi, lo};
 }
 
 void fill_desc(SetDesc &s, const atmo_params &p) {
@@ -364,6 +366,16 @@ struct NSeg {   // a run of P_SN tiles whose sets share one workgroup shape
     int W4max, off, cnt;
 };
 
+struct S1Seg {   // a run of P_S1 tiles whose sets share one dS1 kernel and workgroup shape
+    S1Shape sh;
+    int TWmax, off, cnt;
+};
+struct Segs {   // the launches of a plan's passes
+    std::vector<JSeg> j;
+    std::vector<NSeg> n;
+    std::vector<S1Seg> s1;
+};
+
 // Kernel variants chosen by the autotuner, with the times measured for each.
 struct Tuning {
     int jG = 4, jG1 = 4, snXcd = 1, snForm = 1;   // jG, jG1 = 0: per-set choice
@@ -391,8 +403,7 @@ struct Plan {
     hipGraphExec_t gexec = nullptr;
     // kernel variants (picked by the autotuner)
     int jG = 4, jG1 = 4;   // k_inscatterS texels per thread, orders >= 3 and order 2 (0: per set, see jg_for_set)
-    std::vector<JSeg> jseg;   // P_J tiles grouped by the per-set G
-    std::vector<NSeg> nseg;   // P_SN tiles grouped by row class
+    Segs segs;
     bool view = true;  // the sets have SetDesc::view
     int snXcd = 1;     // k_inscatterN XCD-banded tile order
     int snForm = 1;    // k_inscatterN: 0 direct gathers, 1 LDS-staged rows
@@ -576,16 +587,37 @@ void build_sn_tiles(const std::vector<atmo_params> &ps, int snXcd, std::vector<u
 // the most expensive tiles first so mixed-resolution batches drain evenly.
 void build_tiles(const std::vector<atmo_params> &ps, const atmo_options &o,
                  std::vector<uint2> &tiles, int off[P_COUNT], int cnt[P_COUNT], int snXcd = 1,
-                 std::vector<JSeg> *jseg = nullptr, std::vector<NSeg> *nseg = nullptr) {
+                 Segs *out = nullptr) {
     tiles.clear();
+    Segs local;
+    Segs &sg = out ? *out : local;
+    sg = Segs();
     const int n = (int)ps.size();
     for (int pass = 0; pass < P_COUNT; ++pass) {
         off[pass] = (int)tiles.size();
         if (pass == P_SN) {
-            std::vector<NSeg> segs;
-            if (o.orders >= 2) build_sn_tiles(ps, snXcd, tiles, segs);
+            if (o.orders >= 2) build_sn_tiles(ps, snXcd, tiles, sg.n);
             cnt[pass] = (int)tiles.size() - off[pass];
-            if (nseg) nseg->swap(segs);
+            continue;
+        }
+        if (pass == P_S1) {   // a mu row each, the sets of one launch together
+            std::map<std::tuple<int, int, int, int>, std::vector<int>> groups;
+            for (int i = 0; i < n; ++i) {
+                const S1Shape sh = s1_shape(ps[i].RES_MU_S * ps[i].RES_NU, ps[i].TRANSMITTANCE_W, lin_t(o));
+                groups[{sh.axis, -sh.texels, sh.columns, -sh.threads}].push_back(i);
+            }
+            for (const auto &g : groups) {
+                const atmo_params &q = ps[g.second[0]];
+                S1Seg seg{s1_shape(q.RES_MU_S * q.RES_NU, q.TRANSMITTANCE_W, lin_t(o)), 0, (int)tiles.size() - off[pass], 0};
+                for (int i : g.second) {
+                    const int nt = (ps[i].RES_R * ps[i].RES_MU + kTileRows - 1) / kTileRows;
+                    seg.TWmax = std::max(seg.TWmax, ps[i].TRANSMITTANCE_W);
+                    for (int t = 0; t < nt; ++t) tiles.push_back(make_uint2((unsigned)i, (unsigned)t));
+                    seg.cnt += nt;
+                }
+                sg.s1.push_back(seg);
+            }
+            cnt[pass] = (int)tiles.size() - off[pass];
             continue;
         }
         std::vector<std::pair<double, uint2>> v;
@@ -595,15 +627,8 @@ void build_tiles(const std::vector<atmo_params> &ps, const atmo_options &o,
             long long nt = 0;
             double cost = 0;
             switch (pass) {
-            case P_T: nt = (z.nT + 15) / 16; break;
+            case P_T: nt = (z.nT + 16 * kTileY - 1) / (16 * kTileY); break;
             case P_E1: nt = (z.nE + 255) / 256; break;
-            case P_S1: {
-                // workgroups of up to 4 mu rows (k_inscatter1)
-                const int W4 = p.RES_MU_S * p.RES_NU;
-                const int rpw = std::max(1, std::min(4, 256 / W4));
-                nt = (long long)p.RES_R * ((p.RES_MU + rpw - 1) / rpw);
-                break;
-            }
             case P_J:
                 // grouped by the per-set G (descending), most expensive first inside a group
                 nt = (long long)p.RES_R * p.RES_MU_S;
@@ -612,12 +637,13 @@ void build_tiles(const std::vector<atmo_params> &ps, const atmo_options &o,
                     cost = -((dj_split(p, o) * 1e4 + p.RES_MU) * 1e4 + p.RES_NU);
                 break;
             case P_EN: nt = (long long)z.nE; cost = (double)p.RES_NU; break;
-            case P_VIEW: nt = ((long long)p.RES_R * p.RES_MU * (o.inscatter_samples + 1) + 255) / 256; break;
-            case P_CHECK: nt = (std::max(std::max(z.n4, z.nT), z.nE) + 255) / 256; break;
+            case P_VIEW:
+                nt = ((long long)p.RES_R * p.RES_MU * (o.inscatter_samples + 1) + 256 * kTileY - 1) / (256 * kTileY);
+                break;
+            case P_CHECK: nt = (std::max(std::max(z.n4, z.nT), z.nE) + 256 * kTileY - 1) / (256 * kTileY); break;
             }
             if (pass == P_J && o.orders < 2) nt = 0;
             if (pass == P_EN && o.orders < 2) nt = 0;
-            if (pass == P_VIEW && o.orders < 2) nt = 0;
             for (long long t = 0; t < nt; ++t) v.push_back({cost, make_uint2((unsigned)i, (unsigned)t)});
         }
         if (pass == P_J || pass == P_EN)
@@ -625,12 +651,11 @@ void build_tiles(const std::vector<atmo_params> &ps, const atmo_options &o,
                              [](const std::pair<double, uint2> &a, const std::pair<double, uint2> &b) {
                                  return a.first > b.first;
                              });
-        if (pass == P_J && jseg) {
-            jseg->clear();
+        if (pass == P_J) {
             for (size_t i = 0; i < v.size(); ++i) {
                 const atmo_params &p = ps[v[i].second.x];
                 if (i && v[i].second.x == v[i - 1].second.x) {
-                    jseg->back().cnt += 1;
+                    sg.j.back().cnt += 1;
                     continue;
                 }
                 JSeg g{jg_for_set(p), (int)i, 0, dj_split(p, o)};
@@ -638,13 +663,13 @@ void build_tiles(const std::vector<atmo_params> &ps, const atmo_options &o,
                     g.RMU = p.RES_MU;
                     g.NU = p.RES_NU;
                 }
-                if (jseg->empty() || jseg->back().G != g.G || jseg->back().DS != g.DS || jseg->back().RMU != g.RMU ||
-                    jseg->back().NU != g.NU)
-                    jseg->push_back(g);
-                jseg->back().cnt += 1;
+                if (sg.j.empty() || sg.j.back().G != g.G || sg.j.back().DS != g.DS || sg.j.back().RMU != g.RMU ||
+                    sg.j.back().NU != g.NU)
+                    sg.j.push_back(g);
+                sg.j.back().cnt += 1;
                 if (g.DS > 1) {
                     const int NS = o.spherical_samples;
-                    JSeg &b = jseg->back();
+                    JSeg &b = sg.j.back();
                     b.jx = std::max(b.jx, merged_extra(&p, 1, NS, NS));
                     b.SW = std::max(b.SW, p.SKY_W);
                     b.lds1 = lds_inscatterS(NS, NS, b.NU, b.SW, 0, true);
@@ -668,8 +693,8 @@ void build_tiles(const std::vector<atmo_params> &ps, const atmo_options &o,
                     for (size_t x = 0; x < kXcds; ++x)
                         if (k < q[x].size()) v[p++] = q[x][k];
             };
-            if (jseg && !jseg->empty())
-                for (const JSeg &g : *jseg) deal((size_t)g.off, (size_t)g.cnt);
+            if (!sg.j.empty())
+                for (const JSeg &g : sg.j) deal((size_t)g.off, (size_t)g.cnt);
             else
                 deal(0, v.size());
         }
@@ -690,7 +715,7 @@ hipError_t launch_dj(const Plan &pl, const SetDesc *S, const uint2 *T, const cha
     };
     hipError_t e = hipSuccess;
     int whole = 0;   // tiles of the sets that are not split: the first segments
-    for (const JSeg &g : pl.jseg) {
+    for (const JSeg &g : pl.segs.j) {
         if (g.DS == 1) {
             whole += g.cnt;
             if (G == 0) e = run(g.off, g.cnt, first ? pl.chJ1 : pl.chJ, pl.maxNU, pl.jx, first ? pl.ldsJ1 : pl.ldsJ, g.G, 1, 256);
@@ -702,6 +727,15 @@ hipError_t launch_dj(const Plan &pl, const SetDesc *S, const uint2 *T, const cha
     }
     if (G != 0) e = run(0, whole, first ? pl.chJ1 : pl.chJ, pl.maxNU, pl.jx, first ? pl.ldsJ1 : pl.ldsJ, G, 1, 256);
     return e;
+}
+
+// The dS1 pass: one launch per kernel and workgroup shape.
+hipError_t launch_ds1(const SetDesc *S, const uint2 *T, const std::vector<S1Seg> &segs, const atmo_options &o, hipStream_t st) {
+    for (const S1Seg &g : segs) {
+        const hipError_t e = launch_inscatter1(S, T + g.off, g.cnt, o.inscatter_samples, g.sh, g.TWmax, st);
+        if (e != hipSuccess) return e;
+    }
+    return hipSuccess;
 }
 
 // The dSn pass: one launch per workgroup shape.  S: descriptors; T: the pass's
@@ -754,14 +788,14 @@ atmo_status launch_all(Plan &pl, hipStream_t st, PassTimer *tm = nullptr) {
     HIPCHK(t.begin(0, 1));
     HIPCHK(launch_transmittance(S, T + pl.off[P_T], pl.cnt[P_T], o.transmittance_samples, st));
     // the transmittance tables of the later passes (timed with the T pass)
-    HIPCHK(launch_tview(S, T + pl.off[P_S1], pl.cnt[P_S1], o.inscatter_samples, st));
+    HIPCHK(launch_tview(S, T + pl.off[P_VIEW], pl.cnt[P_VIEW], o.inscatter_samples, st));
     if (o.orders >= 2) HIPCHK(launch_tground(S, T + pl.off[P_J], pl.cnt[P_J], o.spherical_samples, st));
     HIPCHK(t.end());
     HIPCHK(t.begin(1, 1));
     HIPCHK(launch_irradiance1(S, T + pl.off[P_E1], pl.cnt[P_E1], st));
     HIPCHK(t.end());
     HIPCHK(t.begin(2, 1));
-    HIPCHK(launch_inscatter1(S, T + pl.off[P_S1], pl.cnt[P_S1], o.inscatter_samples, lin_t(o), st));
+    HIPCHK(launch_ds1(S, T + pl.off[P_S1], pl.segs.s1, o, st));
     HIPCHK(t.end());
     for (int order = 2; order <= o.orders; ++order) {
         const bool first = order == 2;
@@ -776,7 +810,7 @@ atmo_status launch_all(Plan &pl, hipStream_t st, PassTimer *tm = nullptr) {
         HIPCHK(t.begin(5, order));
         if (first && pl.view)   // dSM4 has been read for the last time
             HIPCHK(launch_snview(S, T + pl.off[P_VIEW], pl.cnt[P_VIEW], o.inscatter_samples, st));
-        HIPCHK(launch_dsn(S, T + pl.off[P_SN], pl.nseg, o, pl.snForm, pl.view, st));
+        HIPCHK(launch_dsn(S, T + pl.off[P_SN], pl.segs.n, o, pl.snForm, pl.view, st));
         HIPCHK(t.end());
     }
     return ATMO_OK;
@@ -855,7 +889,7 @@ atmo_status autotune(Plan &pl, hipStream_t st, Tuning &tu) {
     // 0: each set with its own G (jg_for_set), a candidate only when the sets'
     // choices differ (otherwise it is the same launch as one of the others)
     const int Gs[5] = {2, 3, 4, 8, 0};
-    const bool mixedG = pl.jseg.size() > 1;
+    const bool mixedG = pl.segs.j.size() > 1;
     float bestJ = 1e30f, bestJ1 = 1e30f;
     for (int gi = 0; gi < 5; ++gi) {
         if (Gs[gi] == 0 && !mixedG) {
@@ -923,7 +957,7 @@ atmo_status apply_tuning(Plan &pl, const Tuning &tu) {
     pl.tuned = true;
     if (retile) {
         std::vector<uint2> tiles;
-        build_tiles(pl.params, pl.opts, tiles, pl.off, pl.cnt, pl.snXcd, &pl.jseg, &pl.nseg);
+        build_tiles(pl.params, pl.opts, tiles, pl.off, pl.cnt, pl.snXcd, &pl.segs);
         HIPCHK(pl.dtiles.ensure(tiles.size() * sizeof(uint2)));
         HIPCHK(h2d(pl.dtiles.p, tiles.data(), tiles.size() * sizeof(uint2), pl.xs));
     }
@@ -1005,7 +1039,7 @@ atmo_status build_plan(hipStream_t xs, const atmo_params *sets, int nsets, const
     HIPCHK(R.get(pl->dsets, nsets * sizeof(SetDesc)));
     // tiles
     std::vector<uint2> tiles;
-    build_tiles(pl->params, o, tiles, pl->off, pl->cnt, pl->snXcd, &pl->jseg, &pl->nseg);
+    build_tiles(pl->params, o, tiles, pl->off, pl->cnt, pl->snXcd, &pl->segs);
     HIPCHK(R.get(pl->dtiles, tiles.size() * sizeof(uint2)));
     HIPCHK(h2d(pl->dtiles.p, tiles.data(), tiles.size() * sizeof(uint2), pl->xs));
     HIPCHK(R.get(pl->dflags, nsets * sizeof(unsigned)));
@@ -1472,8 +1506,8 @@ static atmo_status pass_run(atmo_engine *e, const atmo_params *p, const atmo_opt
     std::vector<atmo_params> ps(1, *p);
     atmo_options ot = o;
     ot.orders = std::max(ot.orders, 2);  // every pass gets its tiles
-    std::vector<NSeg> nseg;
-    build_tiles(ps, ot, tiles, off, cnt, 1, nullptr, &nseg);
+    Segs segs;
+    build_tiles(ps, ot, tiles, off, cnt, 1, &segs);
     HIPCHK(e->pass_tiles.ensure(tiles.size() * sizeof(uint2)));
     HIPCHK(h2d(e->pass_tiles.p, tiles.data(), tiles.size() * sizeof(uint2), e->cap));
     size_t oJT, oJW, oE;
@@ -1485,7 +1519,7 @@ static atmo_status pass_run(atmo_engine *e, const atmo_params *p, const atmo_opt
     switch (pass) {
     case P_T: HIPCHK(launch_transmittance(S, T + off[P_T], cnt[P_T], o.transmittance_samples, hs)); break;
     case P_E1: HIPCHK(launch_irradiance1(S, T + off[P_E1], cnt[P_E1], hs)); break;
-    case P_S1: HIPCHK(launch_inscatter1(S, T + off[P_S1], cnt[P_S1], o.inscatter_samples, lin_t(o), hs)); break;
+    case P_S1: HIPCHK(launch_ds1(S, T + off[P_S1], segs.s1, o, hs)); break;
     case P_J: {
         auto jx_of_ch = [&](int c) { return merged_extra(p, 1, o.spherical_samples, c); };
         const int ch = chunk_inscatterS(o.spherical_samples, p->RES_NU, p->SKY_W, jx_of_ch, first);
@@ -1504,7 +1538,7 @@ static atmo_status pass_run(atmo_engine *e, const atmo_params *p, const atmo_opt
                                   first, lds, hs));
         break;
     }
-    case P_SN: HIPCHK(launch_dsn(S, T + off[P_SN], nseg, o, sn_form(o.inscatterN_form), false, hs)); break;
+    case P_SN: HIPCHK(launch_dsn(S, T + off[P_SN], segs.n, o, sn_form(o.inscatterN_form), false, hs)); break;
     }
     HIPCHK(hipStreamSynchronize(hs));
     g_err.clear();

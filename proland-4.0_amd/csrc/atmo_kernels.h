@@ -22,6 +22,9 @@ struct DirEHost {
 // a time: CH is the largest count (up to all of them) whose staging fits
 // kSphLdsBudget, the dynamic LDS a launch gets without raising the kernel's
 // limit; 0 = not even one row fits.  lds_* are the bytes for CH rows.
+// Workgroups (grid.y) per entry of the tile tables of T, the view-ray samples and
+// the numeric check, and mu rows per entry of dS1's: the tables stay small.
+constexpr int kTileY = 16, kTileRows = 4;
 constexpr size_t kSphLdsBudget = 64 * 1024;
 // JX: extra LDS entries of the merged ground rows of one staging round of the
 // orders >= 3 pass (the sum over its theta rows of merged_row_extra, maximum
@@ -52,10 +55,9 @@ hipError_t launch_irradiance1(const SetDesc *sets, const uint2 *tiles, int ntile
 hipError_t launch_tview(const SetDesc *sets, const uint2 *tiles, int ntiles, int nsamp, hipStream_t st);
 hipError_t launch_tground(const SetDesc *sets, const uint2 *tiles, int ntiles, int NS, hipStream_t st);
 // linT / lin4: the sets' parameterisation flags (one per batch), compiled in
-hipError_t launch_inscatter1(const SetDesc *sets, const uint2 *tiles, int ntiles, int nsamp,
-                             bool linT, hipStream_t st);
 // G: texels per thread (2, 3, 4 or 8); CH: theta rows per staging round; RNU:
-// the largest RES_NU of the launch's sets
+// the largest RES_NU of the launch's sets; DS: slots of the workgroup's threads the
+// theta rows are dealt to (1: none; more: all rows staged at once)
 hipError_t launch_inscatterS(const SetDesc *sets, const uint2 *tiles, int ntiles, int NS, int CH, int RNU,
                              int JX, const void *dirT, const void *dirW, bool first, size_t lds, int G,
                              int DS, int threads, hipStream_t st);
@@ -68,6 +70,18 @@ struct SnShape {
     int texels, threads;   // per thread (1 .. 3), per workgroup (a multiple of 64 up to 512)
 };
 SnShape sn_shape(int W4);   // W4 <= 1024
+// The dS1 pass, one mu row (tile) per workgroup.  sh: s1_shape of every set of the
+// launch; TWmax: the most T columns of its sets.
+constexpr int kXkMax = 2048;   // T columns whose centres are staged for the sun lookups
+struct S1Shape {
+    int axis;      // how the mu axis of the sun's T lookup is found
+    int texels;    // per thread, 1 to 3 with LDS-staged T rows, 0: gathers
+    int columns;   // T columns staged per thread (1, 2)
+    int threads;   // per workgroup
+};
+S1Shape s1_shape(int W4, int TW, bool linT);
+hipError_t launch_inscatter1(const SetDesc *sets, const uint2 *tiles, int ntiles, int nsamp, S1Shape sh, int TWmax,
+                             hipStream_t st);
 hipError_t launch_inscatterN(const SetDesc *sets, const uint2 *tiles, int ntiles, int nsamp, int form, SnShape sh,
                              int W4max, bool lin4, hipStream_t st);
 // SetDesc::view of every set, tiles of 256 consecutive samples

@@ -22,7 +22,7 @@ __global__ __launch_bounds__(256) void k_transmittance(const SetDesc *__restrict
     const uint2 tl = tiles[blockIdx.x];
     const SetDesc &s = sets[tl.x];
     const int lane = threadIdx.x & 15;
-    const int t = (int)tl.y * 16 + (threadIdx.x >> 4);
+    const int t = ((int)tl.y * kTileY + (int)blockIdx.y) * 16 + (threadIdx.x >> 4);
     const bool valid = t < s.TW * s.TH;
     const int tt = valid ? t : 0;
     const int i = tt % s.TW, j = tt / s.TW;
@@ -53,6 +53,9 @@ __global__ __launch_bounds__(256) void k_transmittance(const SetDesc *__restrict
         sM += __shfl_xor(sM, off, 16);
     }
     if (lane == 0 && valid) {
+        // sun_centres: tan(1.5 m), its leading part in row 0 and the rest in row 1
+        double c = j < 2 ? tan(1.5 * m) : 0.0;
+        const float ck = j == 0 ? (float)c : j == 1 ? (float)(c - (double)(float)c) : 0.0f;
         double q = s.Rg / r;
         bool below = mu < -sqrt(1.0 - q * q);
         double dR = below ? 1e9 : sR * dx;
@@ -67,7 +70,7 @@ __global__ __launch_bounds__(256) void k_transmittance(const SetDesc *__restrict
         if (s.tau4)
             s.tau4[t] = make_float4((float)((double)s.bR[0] * dR + (double)s.bME[0] * dM),
                                     (float)((double)s.bR[1] * dR + (double)s.bME[1] * dM),
-                                    (float)((double)s.bR[2] * dR + (double)s.bME[2] * dM), 0.0f);
+                                    (float)((double)s.bR[2] * dR + (double)s.bME[2] * dM), ck);
         if (s.outT) {
             s.outT[3 * t + 0] = o.x;
             s.outT[3 * t + 1] = o.y;
@@ -102,10 +105,33 @@ __global__ __launch_bounds__(256) void k_irradiance1(const SetDesc *__restrict__
 }
 
 constexpr int kNChunk = 64;   // k_inscatterN form 2: samples staged per chunk
-constexpr int kNRows = 4;     // k_inscatter1: max mu rows per workgroup
-
-// mu rows per workgroup of k_inscatter1 and k_tview: as many whole rows as fit 256 threads, at most 4
-__device__ __forceinline__ int rows_per_wg(int W4) { return max(1, min(kNRows, 256 / W4)); }
+// LDS byte address of an entry in two FMA-class instructions (about 2 cycles per
+// wave on gfx950, where a conversion and a shift-add take 4 each).  u + kRound,
+// kRound = 1.5 2^23, is kRound + k with k = u rounded to the nearest integer;
+// times STRIDE 2^-149, plus (base - STRIDE kRound) 2^-149, it is the denormal
+// whose bit pattern is base + STRIDE k.  Exact: the addend is a multiple of
+// STRIDE below 2^24 STRIDE (base is a multiple of STRIDE), the result is an
+// integer below 2^23.  At a tie either neighbour may come out: the two lines meet
+// there.
+constexpr float kRound = 12582912.0f;
+template <int STRIDE>
+__device__ __forceinline__ float lds_addend(unsigned base) {   // (base - STRIDE kRound) 2^-149
+    return ((float)base - (float)STRIDE * kRound) * 1.40129846e-45f;
+}
+template <int STRIDE>
+__device__ __forceinline__ unsigned lds_entry(float u, float addend) {
+    return __float_as_uint(fmaf(u + kRound, (float)STRIDE * 1.40129846e-45f, addend));
+}
+__device__ __forceinline__ float4 lds4(unsigned a, int off = 0) {
+    typedef float v4 __attribute__((ext_vector_type(4)));
+    const v4 v = *(__attribute__((address_space(3))) const v4 *)(size_t)(a + off);
+    return make_float4(v.x, v.y, v.z, v.w);
+}
+__device__ __forceinline__ float2 lds2(unsigned a, int off = 0) {
+    typedef float v2 __attribute__((ext_vector_type(2)));
+    const v2 v = *(__attribute__((address_space(3))) const v2 *)(size_t)(a + off);
+    return make_float2(v.x, v.y);
+}
 
 // ---------------------------------------------------------------------------
 // Pass dS1 — inscatter1.glsl:104-150 fused with copyInscatter1.glsl:104-109.
@@ -113,174 +139,374 @@ __device__ __forceinline__ int rows_per_wg(int W4) { return max(1, min(kNRows, 2
 // an integration sample that does not involve the sun — its distance and
 // radius, the view-ray transmittance T(r, mu, t), the scale-height factors and
 // the r-row of the T(r_i, mu_s_i) lookup — is shared by the RNU x RMU_S texels
-// of the row.  A workgroup covers up to 4 rows, stages those
-// terms (FP64 geometry) in LDS, and each thread then needs only the sun
-// visibility test, mu_s_i and the mu-axis half of the T lookup per sample.
+// of the row.  A workgroup computes those terms (FP64 geometry) for its row in LDS,
+// and a texel then needs only the sun's visibility, mu_s_i and the mu axis of the
+// T lookup per sample.
+//
+// Two forms.  k_inscatter1_rows: the two T rows of the sample, weighted by the
+// r fraction and by T(r, mu, t), are blended once into an LDS row that the row's
+// texels look up; the rows are loaded coalesced, one sample ahead, into registers by
+// the parity of the row number, so a step to the next row loads one.
+// k_inscatter1: every texel gathers its four T texels.  Gathers of 64 lanes cost
+// the texture path about 27 cycles each, a staged row costs 64 per CU for all its
+// texels: 32x128x32x8 (256 texels, 256 columns) 159 -> 105 us; 48 sets of the mixed
+// batch 14.9 -> 7.8 ms; 64x256x64x16 2.34 -> 1.14 ms.
 // ---------------------------------------------------------------------------
-struct S1Entry {
+struct __attribute__((aligned(16))) S1Entry {
     double ti;       // sample distance
-    double q;        // r_i^2 - Rg^2
-    double iri;      // 1 / r_i
-    float T[3];      // T(r, mu, t_i), trapezoid weight folded in
+    double thr;      // the sun is visible where r_i mu_s_i >= thr
+    double iri;      // 1 / r_i, times the factor of the mu axis' argument
     float eR, eM;    // exp(-h_i/HR), exp(-h_i/HM)
-    float b;         // T-table row weight of r_i
-    unsigned j0, j1; // T-table row offsets (bytes) of r_i
+    float p0[3];     // weights of the T row of even and of odd number: r fraction x T(r, mu, t_i) x
+    unsigned j0;     // trapezoid weight; rows of r_i (k_inscatter1: p0 without the r fraction, p1[0] the fraction)
+    float p1[3];
+    unsigned j1;
 };
 
 constexpr int kS1Chunk = 64;
-constexpr int kXkMax = 2048;   // T-table columns whose centres are staged for the sun lookups
+constexpr int kXkMin = 64;     // columns from which a few terms of the arctangent's series do
 
-template <bool LINT>   // linear transmittance parameterisation (the per-sample T lookup)
-__global__ __launch_bounds__(256) void k_inscatter1(const SetDesc *__restrict__ sets,
-                                                    const uint2 *__restrict__ tiles,
-                                                    int nsamp) {
-    __shared__ S1Entry ent[kNRows][kS1Chunk];
-    __shared__ float rowdx[kNRows];
-    __shared__ double xk[LINT ? 1 : kXkMax];
+// The mu axis of the sun's T lookup next to the horizon, where T is steep: an FP32
+// texel coordinate is good to ~3e-5 of a texel at TW = 512, which moves a grazing
+// sun's T by ~1e-4.  So the filter fraction is taken from a column centre x_k =
+// tan(1.5 (k + 0.5) / TW), staged once per workgroup:  u - u_k = (atan x - atan x_k)
+// / 1.5 = atan((x - x_k) / (1 + x x_k)) / 1.5, x = (mu_s_i + 0.15) tan(1.5) / 1.15 and
+// the difference in FP64; the centre is any within about a column of x (its column
+// comes from a fit of atan in x / (1 + |x|), good to 7.1e-4), the integer part of the
+// offset moves to the column, and the arctangent of the small offset is its series (three
+// terms, 6e-9 relative from kXkMin columns on; below, atanf).
+enum { kSunTab, kSunLin, kSunWide, kSunFew };   // centres; linear parameterisation; more than kXkMax columns
+                                                // (FP32); centres, fewer than kXkMin columns
+struct SunAxis {
+    double c;      // argument at mu_s_i = 0
+    double scale;  // argument per mu_s_i
+    float last, sc;   // TW - 1, TW / 1.5
+    float xk;      // LDS address of the centres (lds_addend form, base only)
+};
+template <int AX>
+__device__ __forceinline__ SunAxis sun_axis(const SetDesc &s, const double *xk) {
+    SunAxis x;
+    x.c = AX == kSunLin ? 0.15 / 1.15 * s.TW - 0.5 : 0.15 * s.tMu;
+    x.scale = AX == kSunLin ? s.TW / 1.15 : s.tMu;
+    x.last = (float)(s.TW - 1);
+    x.sc = (float)s.TW / 1.5f;
+    x.xk = (float)(unsigned)(size_t)(__attribute__((address_space(3))) const char *)xk * 1.40129846e-45f;
+    return x;
+}
+// The column (a whole number in [0, TW - 1]) and the fraction of r_i mu_s_i = num, in two
+// steps: the argument and a centre near it (an LDS read), then the offset from it.
+struct SunCell {
+    double x, xk;   // argument, centre
+    float xf, k;    // argument, column of the centre
+};
+template <int AX>
+__device__ __forceinline__ SunCell sun_cell(const SunAxis &x, double num, double iri) {
+    SunCell c;
+    c.x = fma(num, iri, x.c);
+    if constexpr (AX == kSunTab || AX == kSunFew) {
+        c.xf = (float)c.x;
+        const float t = c.xf * __builtin_amdgcn_rcpf(1.0f + fabsf(c.xf));
+        const float ta = __uint_as_float(__float_as_uint(t) & 0x7fffffffu);
+        float q = fmaf(ta, 2.434126615524292f, -6.0853166580200195f);
+        q = fmaf(ta, q, 3.8018410205841064f);
+        q = fmaf(ta, q, 0.38255468010902405f);
+        q = fmaf(ta, q, 1.0375903844833374f);
+        c.k = __builtin_amdgcn_fmed3f((fmaf(t * x.sc, q, -0.5f) + kRound) - kRound, 0.0f, x.last);
+        const unsigned xa = __float_as_uint(fmaf(c.k, 8.0f * 1.40129846e-45f, x.xk));
+        c.xk = *(__attribute__((address_space(3))) const double *)(size_t)xa;
+    }
+    return c;
+}
+template <int AX>
+__device__ __forceinline__ void sun_column(const SunAxis &x, const SunCell &c, float &col, float &a) {
+    if constexpr (AX == kSunLin) {
+        const double p = fmin(fmax(c.x, 0.0), (double)x.last), f = floor(p);
+        col = (float)f;
+        a = (float)(p - f);
+    } else if constexpr (AX == kSunWide) {
+        const float p = __builtin_amdgcn_fmed3f(fmaf(atanf((float)c.x), x.sc, -0.5f), 0.0f, x.last);
+        col = floorf(p);
+        a = p - col;
+    } else {
+        const float d = (float)(c.x - c.xk);
+        const float g = d * __builtin_amdgcn_rcpf(fmaf(c.xf, c.xf - d, 1.0f));
+        float o;   // offset from the centre, in columns
+        if constexpr (AX == kSunTab) {
+            const float z = g * g, e = g * x.sc;
+            o = fmaf(e, z * fmaf(z, 0.2f, -1.0f / 3.0f), e);
+        } else {
+            o = atanf(g) * x.sc;
+        }
+        o = __builtin_amdgcn_fmed3f(o, -c.k, x.last - c.k);   // CLAMP_TO_EDGE
+        const float f = floorf(o);
+        a = o - f;
+        col = c.k + f;
+    }
+}
+// Centres of the T table's columns: from the spare component of the first two rows of
+// optical depths (k_transmittance), high and low part, where there are any.
+__device__ __forceinline__ void sun_centres(const SetDesc &s, double *xk) {
+    for (int k = threadIdx.x; k < s.TW; k += blockDim.x)
+        xk[k] = s.tau4 ? (double)s.tau4[k].w + (double)s.tau4[s.TW + k].w : tan(1.5 * (k + 0.5) / s.TW);
+}
+// nu and r mu_s of the texel in column x
+__device__ __forceinline__ void s1_texel(const SetDesc &s, int x, double r, double &nu, double &muSr) {
+    const ColGeom c = s.cols[x % s.RMUS];
+    nu = -1.0 + (double)(x / s.RMUS) / (s.RNU - 1.0) * 2.0;
+    muSr = ((double)c.hi + (double)c.lo64) * r;
+}
+// The terms of sample i of the row (l, y); BY_PARITY: row weights for k_inscatter1_rows.
+// Stores the row's sample distance in dx.
+template <bool BY_PARITY>
+__device__ __forceinline__ S1Entry s1_entry(const SetDesc &s, int l, int y, int i, int nsamp, const SunAxis &ax, float &sdx) {
+    const double r = s.layers[l].r;
+    double mu, muS_u, nu_u;
+    mu_mus_nu(s, s.layers[l], 0, y, mu, muS_u, nu_u);
+    const double dx = limit_d(s, r, mu) / nsamp;
+    if (i == 0) sdx = (float)dx;
+    const double rho2 = r * r - s.Rg2;
+    const double rmu = r * mu;
+    const bool up = mu > 0.0;
+    S1Entry en;
+    en.ti = i * dx;
+    const double q = rho2 + en.ti * (en.ti + 2.0 * rmu);       // ri^2 - Rg^2
+    // muSi >= -sqrt(1 - Rg^2 / max(Rg, ri)^2)  <=>  ri muSi >= -sqrt(ri^2 - Rg^2)
+    en.thr = q > 0.0 ? -sqrt(q) : 0.0;
+    const float ri = sqrtf((float)(q + s.Rg2));
+    const float h1 = (float)q / (ri + s.f_Rg);                 // ri - Rg (< 0 at a ground hit)
+    const float mu1 = (float)(rmu + en.ti) / ri;
+    // transmittance(r, mu, t_i) (common.glsl:272-282)
+    const float3 Tseg = s.tview ? ld3(gptr(s.tview) + ((size_t)l * s.RMU + y) * (nsamp + 1) + i)
+                      : up      ? T_ratio_lin(s, (float)(r - s.Rg), (float)mu, h1, mu1)
+                                : T_ratio_lin(s, h1, -mu1, (float)(r - s.Rg), (float)-mu);
+    const float w = !s.tview && (i == 0 || i == nsamp) ? 0.5f : 1.0f;
+    const float T[3] = {Tseg.x * w, Tseg.y * w, Tseg.z * w};
+    const double rid = sqrt(q + s.Rg2);
+    en.iri = ax.scale / rid;
+    const float hc = fmaxf(h1, 0.0f);                          // ri = max(Rg, ri)
+    en.eR = __expf(-hc * (float)(1.0 / s.HR));
+    en.eM = __expf(-hc * (float)(1.0 / s.HM));
+    // r axis of T(max(Rg, ri), muSi): common.glsl:114-124 (FP64 coordinate)
+    int j0, j1;
+    double bd;
+    gl_axis_dd(T_ur_d(s, q / (rid + s.Rg)) * s.TH - 0.5, s.TH, j0, j1, bd);
+    const float b = (float)bd;
+    if (BY_PARITY) {   // rows j0 and j0 + 1, or the one row of an edge
+        const float w0 = j1 == j0 ? 1.0f : 1.0f - b, w1 = j1 == j0 ? 0.0f : b;
+        const float we = j0 & 1 ? w1 : w0, wo = j0 & 1 ? w0 : w1;
+#pragma unroll
+        for (int c = 0; c < 3; ++c) { en.p0[c] = we * T[c]; en.p1[c] = wo * T[c]; }
+        en.j0 = (unsigned)(j0 & 1 ? j1 : j0);   // even (an edge's: either parity, weight 0)
+        en.j1 = (unsigned)(j0 & 1 ? j0 : j1);
+    } else {
+#pragma unroll
+        for (int c = 0; c < 3; ++c) en.p0[c] = T[c];
+        en.p1[0] = b; en.p1[1] = en.p1[2] = 0.f;
+        en.j0 = (unsigned)(j0 * s.TW) * 16u;
+        en.j1 = (unsigned)(j1 * s.TW) * 16u;
+    }
+    return en;
+}
+__device__ __forceinline__ void s1_store(const SetDesc &s, size_t t, float fdx, const float r[3], const float m[3]) {
+    const float4 oR = q16(make_float4(r[0] * fdx * s.bR[0], r[1] * fdx * s.bR[1], r[2] * fdx * s.bR[2], 0.f), s.hs);
+    const float4 oM = q16(make_float4(m[0] * fdx * s.bMS[0], m[1] * fdx * s.bMS[1], m[2] * fdx * s.bMS[2], 0.f), s.hs);
+    s.dSR4[t] = oR;
+    s.dSM4[t] = oM;
+    if (s.S4) s.S4[t] = make_float4(oR.x, oR.y, oR.z, oM.x);
+}
+
+// One mu row per workgroup, NM texels and NC T columns per thread.  Dynamic LDS:
+// [2][NC threads + 1] row entries (the last one zero: the second tap of the last
+// column, whose fraction is 0), [TW] centres.
+template <int AX, int NM, int NC>
+__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(NM >= 3 ? 4 : 5))) void
+k_inscatter1_rows(const SetDesc *__restrict__ sets, const uint2 *__restrict__ tiles, int nsamp) {
+    extern __shared__ __attribute__((aligned(32))) float4 lds[];
+    __shared__ __attribute__((aligned(16))) S1Entry ent[kS1Chunk];
+    __shared__ float s_dx;
     const uint2 tl = tiles[blockIdx.x];
     const SetDesc &s = sets[tl.x];
-    // The sun's T lookups at mu_s_i next to the horizon, where T is steep:
-    // an FP32 texel coordinate (atanf, then * TW) is good to ~3e-5 of a texel
-    // at TW = 512, which moves a grazing sun's T by ~1e-4.  So the filter
-    // fraction is taken from the centre of the column the FP32 coordinate
-    // falls in, u - u_k = (atan x - atan x_k) / 1.5 with
-    // atan x - atan x_k = atan((x - x_k) / (1 + x x_k)) (less than 1.5 / TW,
-    // FP32 is exact enough there), x = (mu_s_i + 0.15) tan(1.5) / 1.15 in FP64
-    // and x_k = tan(1.5 (k + 0.5) / TW) staged once per workgroup (tables of at
-    // most kXkMax columns; wider ones keep the FP32 coordinate).
-    const bool tab = !LINT && s.TW <= kXkMax;
-    const float sc = (float)s.TW / 1.5f;
-    if (tab)
-        for (int k = threadIdx.x; k < s.TW; k += blockDim.x) xk[k] = tan(1.5 * (k + 0.5) / s.TW);
-    const int RPW = rows_per_wg(s.W4);
-    const int ngy = (s.RMU + RPW - 1) / RPW;
-    const int l = (int)tl.y / ngy;
-    const int yb = ((int)tl.y % ngy) * RPW;
-    const int nrows = min(RPW, s.RMU - yb);
-    const LayerGeom L = s.layers[l];
-    const double r = L.r;
-    const double rho2 = r * r - s.Rg2;
-    const int per = nrows * s.W4;
-    const int nmine = (per + (int)blockDim.x - 1) / (int)blockDim.x;
-    constexpr int MAXT = 4;   // W4 <= 1024 (validated on the host)
-    float aR[MAXT][3], aM[MAXT][3];
-    double nud[MAXT], muSr[MAXT];
-    int rowi[MAXT];
+    const int TW = s.TW, W4 = s.W4, nthr = (int)blockDim.x;
+    const int RS = NC * nthr + 1;
+    double *xk = (double *)(lds + 2 * RS);
+    if (AX == kSunTab) sun_centres(s, xk);
+    if (threadIdx.x < 2) lds[threadIdx.x * RS + RS - 1] = make_float4(0.f, 0.f, 0.f, 0.f);
+    const SunAxis ax = sun_axis<AX>(s, xk);
+    const int line = (int)tl.y * kTileRows + (int)blockIdx.y;
+    if (line >= s.RR * s.RMU) return;
+    const int l = line / s.RMU, y = line % s.RMU;
+    const double r = s.layers[l].r;
+    double nud[NM], muSr[NM];
+    float aR[NM][3], aM[NM][3];
 #pragma unroll
-    for (int j = 0; j < MAXT; ++j) {
-        aR[j][0] = aR[j][1] = aR[j][2] = aM[j][0] = aM[j][1] = aM[j][2] = 0.f;
-        nud[j] = muSr[j] = 0.0;
-        rowi[j] = 0;
-        const int e = threadIdx.x + j * (int)blockDim.x;
-        if (j < nmine && e < per) {
-            const int row = e / s.W4, x = e % s.W4;
-            double mu, muS, nu;
-            mu_mus_nu(s, L, x, yb + row, mu, muS, nu);
-            nud[j] = nu;
-            muSr[j] = muS * r;
-            rowi[j] = row;
-        }
+    for (int j = 0; j < NM; ++j) {
+        s1_texel(s, min((int)threadIdx.x + j * nthr, W4 - 1), r, nud[j], muSr[j]);
+#pragma unroll
+        for (int c = 0; c < 3; ++c) aR[j][c] = aM[j][c] = 0.f;
     }
-    const float iHR = (float)(1.0 / s.HR), iHM = (float)(1.0 / s.HM);
-    const __amdgpu_buffer_rsrc_t Tr = table_rsrc(s.T4, (unsigned)((size_t)s.TW * s.TH * sizeof(float4)));
+    const __amdgpu_buffer_rsrc_t Tr = table_rsrc(s.T4, (unsigned)((size_t)TW * s.TH * sizeof(float4)));
+    unsigned xo[NC];
+#pragma unroll
+    for (int c = 0; c < NC; ++c) xo[c] = (unsigned)min((int)threadIdx.x + c * nthr, TW - 1) * 16u;
+    float3 t0[NC], t1[NC];   // the held rows of even and of odd number
+#pragma unroll
+    for (int c = 0; c < NC; ++c) t0[c] = t1[c] = make_float3(0.f, 0.f, 0.f);
+    int held0 = -1, held1 = -1;
+    struct Stage {   // S1Entry's part for the staging
+        float4 p0, p1;
+    } st;
+    auto get_stage = [&](int js) {
+        const float4 *q = (const float4 *)&ent[js];
+        st.p0 = q[2];
+        st.p1 = q[3];
+    };
+    auto load_rows = [&]() {   // those that the registers do not hold yet
+        const int j0 = __builtin_amdgcn_readfirstlane(__float_as_int(st.p0.w)), j1 = __builtin_amdgcn_readfirstlane(__float_as_int(st.p1.w));
+        auto load = [&](int j, float3 t[NC]) {
+#pragma unroll
+            for (int c = 0; c < NC; ++c) t[c] = ld3b(Tr, xo[c], (unsigned)(j * TW) * 16u);
+        };
+        if (j0 != held0) load(held0 = j0, t0);
+        if (j1 != held1) load(held1 = j1, t1);
+    };
     for (int c0 = 0; c0 <= nsamp; c0 += kS1Chunk) {
         const int nc = min(kS1Chunk, nsamp + 1 - c0);
+        if (c0 > 0) __syncthreads();
+        for (int js = threadIdx.x; js < nc; js += nthr) ent[js] = s1_entry<true>(s, l, y, c0 + js, nsamp, ax, s_dx);
         __syncthreads();
-        for (int e = threadIdx.x; e < nrows * kS1Chunk; e += blockDim.x) {
-            const int row = e / kS1Chunk, js = e % kS1Chunk;
-            if (js >= nc) continue;
-            const int i = c0 + js;
-            double mu, muS_u, nu_u;
-            mu_mus_nu(s, L, 0, yb + row, mu, muS_u, nu_u);
-            const double rmu = r * mu;
-            const double dx = limit_d(s, r, mu) / nsamp;
-            if (i == 0) rowdx[row] = (float)dx;
-            const bool up = mu > 0.0;
-            S1Entry en;
-            en.ti = i * dx;
-            en.q = rho2 + en.ti * (en.ti + 2.0 * rmu);                 // ri^2 - Rg^2
-            const float ri = sqrtf((float)(en.q + s.Rg2));
-            const float h1 = (float)en.q / (ri + s.f_Rg);              // ri - Rg (< 0 at a ground hit)
-            const float mu1 = (float)(rmu + en.ti) / ri;
-            // transmittance(r, mu, t_i) (common.glsl:272-282)
-            const float3 Tseg = s.tview ? ld3(gptr(s.tview) + ((size_t)l * s.RMU + yb + row) * (nsamp + 1) + i)
-                              : up      ? T_ratio_lin(s, (float)(r - s.Rg), (float)mu, h1, mu1)
-                                        : T_ratio_lin(s, h1, -mu1, (float)(r - s.Rg), (float)-mu);
-            const float w = !s.tview && (i == 0 || i == nsamp) ? 0.5f : 1.0f;
-            en.T[0] = Tseg.x * w; en.T[1] = Tseg.y * w; en.T[2] = Tseg.z * w;
-            const double rid = sqrt(en.q + s.Rg2);
-            en.iri = 1.0 / rid;
-            const float hc = fmaxf(h1, 0.0f);                          // ri = max(Rg, ri)
-            en.eR = __expf(-hc * iHR);
-            en.eM = __expf(-hc * iHM);
-            // r axis of T(max(Rg, ri), muSi): common.glsl:114-124 (FP64 coordinate)
-            int j0, j1;
-            double bd;
-            gl_axis_dd(T_ur_d(s, en.q / (rid + s.Rg)) * s.TH - 0.5, s.TH, j0, j1, bd);
-            en.b = (float)bd;
-            en.j0 = (unsigned)(j0 * s.TW) * 16u;
-            en.j1 = (unsigned)(j1 * s.TW) * 16u;
-            ent[row][js] = en;
+        get_stage(0);
+        load_rows();
+        for (int js = 0; js < nc; ++js) {
+            float4 *row = lds + (js & 1) * RS;
+#pragma unroll
+            for (int c = 0; c < NC; ++c)
+                row[(int)threadIdx.x + c * nthr] =
+                    make_float4(fmaf(t0[c].x, st.p0.x, t1[c].x * st.p1.x), fmaf(t0[c].y, st.p0.y, t1[c].y * st.p1.y),
+                                fmaf(t0[c].z, st.p0.z, t1[c].z * st.p1.z), 0.f);
+            // this sample's terms and the next one's rows, read before the barrier
+            const double ti = ent[js].ti, thr = ent[js].thr, iri = ent[js].iri;
+            const float eR = ent[js].eR, eM = ent[js].eM;
+            get_stage(min(js + 1, nc - 1));
+            __syncthreads();
+            if (js + 1 < nc) load_rows();
+            const float rb = (float)(unsigned)(size_t)(__attribute__((address_space(3))) const char *)row * 1.40129846e-45f;
+            // the texels step by step together: a step's LDS reads are in flight at once
+            SunCell cell[NM];
+            float vis[NM], col[NM], a[NM];
+            float4 v0[NM], v1[NM];
+#pragma unroll
+            for (int j = 0; j < NM; ++j) {
+                const double num = fma(nud[j], ti, muSr[j]);        // ri * muSi
+                vis[j] = num >= thr ? 1.0f : 0.0f;
+                cell[j] = sun_cell<AX>(ax, num, iri);
+            }
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int j = 0; j < NM; ++j) {
+                sun_column<AX>(ax, cell[j], col[j], a[j]);
+                const unsigned p = __float_as_uint(fmaf(col[j], 16.0f * 1.40129846e-45f, rb));
+                v0[j] = lds4(p);
+                v1[j] = lds4(p, 16);
+            }
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int j = 0; j < NM; ++j) {
+                const float wR = vis[j] * eR, wM = vis[j] * eM;
+                const float3 v = lerp3(f3(v0[j]), f3(v1[j]), a[j]);
+                aR[j][0] = fmaf(v.x, wR, aR[j][0]); aR[j][1] = fmaf(v.y, wR, aR[j][1]); aR[j][2] = fmaf(v.z, wR, aR[j][2]);
+                aM[j][0] = fmaf(v.x, wM, aM[j][0]); aM[j][1] = fmaf(v.y, wM, aM[j][1]); aM[j][2] = fmaf(v.z, wM, aM[j][2]);
+            }
         }
+    }
+#pragma unroll
+    for (int j = 0; j < NM; ++j) {
+        const int x = (int)threadIdx.x + j * nthr;
+        if (x < W4) s1_store(s, ((size_t)l * s.RMU + y) * W4 + x, s_dx, aR[j], aM[j]);
+    }
+}
+
+// One mu row per workgroup.  Rows of at most 128 texels deal their samples to 4
+// (at most 64 texels) or 2 slots of threads, whose sums are added through LDS in slot
+// order: 16x64x16x4, whose 1024 rows would give a SIMD one wave, takes 20 us instead of 35.
+// Dynamic LDS: [TW] centres.
+template <int AX>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void
+k_inscatter1(const SetDesc *__restrict__ sets, const uint2 *__restrict__ tiles, int nsamp) {
+    extern __shared__ __attribute__((aligned(32))) float4 lds[];
+    __shared__ __attribute__((aligned(16))) S1Entry ent[kS1Chunk];
+    __shared__ float s_dx;
+    __shared__ float part[6][192];
+    const uint2 tl = tiles[blockIdx.x];
+    const SetDesc &s = sets[tl.x];
+    const int TW = s.TW, W4 = s.W4;
+    double *xk = (double *)lds;
+    if (AX == kSunTab || AX == kSunFew) sun_centres(s, xk);
+    const SunAxis ax = sun_axis<AX>(s, xk);
+    const int line = (int)tl.y * kTileRows + (int)blockIdx.y;
+    if (line >= s.RR * s.RMU) return;
+    const int l = line / s.RMU, y = line % s.RMU;
+    const double r = s.layers[l].r;
+    const int slots = W4 <= 64 ? 4 : W4 <= 128 ? 2 : 1, nthr = 256 / slots;
+    const int slot = __builtin_amdgcn_readfirstlane((int)threadIdx.x / nthr), lane = (int)threadIdx.x - slot * nthr;
+    constexpr int MAXT = 4;   // W4 <= 1024 (validated on the host)
+    double nud[MAXT], muSr[MAXT];
+    float aR[MAXT][3], aM[MAXT][3];
+#pragma unroll
+    for (int j = 0; j < MAXT; ++j) {
+#pragma unroll
+        for (int c = 0; c < 3; ++c) aR[j][c] = aM[j][c] = 0.f;
+        nud[j] = muSr[j] = 0.0;
+        if (j * nthr < W4) s1_texel(s, min(lane + j * nthr, W4 - 1), r, nud[j], muSr[j]);
+    }
+    const __amdgpu_buffer_rsrc_t Tr = table_rsrc(s.T4, (unsigned)((size_t)TW * s.TH * sizeof(float4)));
+    const unsigned lastb = (unsigned)(TW - 1) * 16u;
+    for (int c0 = 0; c0 <= nsamp; c0 += kS1Chunk) {   // a multiple of the slots
+        const int nc = min(kS1Chunk, nsamp + 1 - c0);
+        __syncthreads();
+        for (int js = threadIdx.x; js < nc; js += blockDim.x) ent[js] = s1_entry<false>(s, l, y, c0 + js, nsamp, ax, s_dx);
         __syncthreads();
 #pragma unroll
         for (int j = 0; j < MAXT; ++j) {
-            if (j >= nmine) break;
-            const int e = threadIdx.x + j * (int)blockDim.x;
-            if (e >= per) break;
-            const S1Entry *er = ent[rowi[j]];
-            float r0 = aR[j][0], r1 = aR[j][1], r2 = aR[j][2];
-            float m0 = aM[j][0], m1 = aM[j][1], m2 = aM[j][2];
-            for (int js = 0; js < nc; ++js) {
-                const S1Entry &en = er[js];
+            if (j * nthr >= W4) break;
+#pragma unroll 2
+            for (int js = slot; js < nc; js += slots) {
+                const S1Entry &en = ent[js];
                 const double num = fma(nud[j], en.ti, muSr[j]);        // ri * muSi
-                // muSi >= -sqrt(1 - Rg^2 / max(Rg, ri)^2)  <=>  num >= 0 or num^2 <= ri^2 - Rg^2
-                if (!(num >= 0.0 || num * num <= en.q)) continue;
-                const double mus = num * en.iri;   // mu_s_i
-                int i0, i1;
-                float a;
-                if (tab) {
-                    gl_axis(T_umu_t<false>(s, (float)mus) * s.TW - 0.5f, s.TW, i0, i1, a);
-                    if (i1 == i0 + 1) {   // between two columns (not clamped to an edge)
-                        const double x = (mus + 0.15) * s.tMu, x0 = xk[i0];
-                        const float d = (float)(x - x0) * __builtin_amdgcn_rcpf(fmaf((float)x, (float)x0, 1.0f));
-                        // the FP64 coordinate can sit a rounding outside the FP32
-                        // cell: keep the filter weight in [0, 1] (a convex lerp)
-                        a = __builtin_amdgcn_fmed3f(atanf(d) * sc, 0.0f, 1.0f);
-                    }
-                } else if (LINT) {   // (mu_s_i + 0.15) / 1.15: FP64 is cheap here
-                    double ad;
-                    gl_axis_dd(T_umu_d<true>(s, mus) * s.TW - 0.5, s.TW, i0, i1, ad);
-                    a = (float)ad;
-                } else {   // more than kXkMax columns: the FP32 coordinate
-                    gl_axis(T_umu_t<false>(s, (float)mus) * s.TW - 0.5f, s.TW, i0, i1, a);
-                }
-                // buffer loads at byte offsets (i0, i1 >= 0: clamped to the table)
-                const unsigned o0 = (unsigned)i0 << 4, o1 = (unsigned)i1 << 4;
+                const float vis = num >= en.thr ? 1.0f : 0.0f;
+                float col, a;
+                sun_column<AX>(ax, sun_cell<AX>(ax, num, en.iri), col, a);
+                const unsigned o0 = __float2uint_rz(col) * 16u, o1 = min(o0 + 16u, lastb);
                 const float3 t00 = ld3b(Tr, en.j0 + o0, 0u), t01 = ld3b(Tr, en.j0 + o1, 0u);
                 const float3 t10 = ld3b(Tr, en.j1 + o0, 0u), t11 = ld3b(Tr, en.j1 + o1, 0u);
-                const float3 Ts = lerp3(lerp3(t00, t01, a), lerp3(t10, t11, a), en.b);
-                const float tx = en.T[0] * Ts.x, ty = en.T[1] * Ts.y, tz = en.T[2] * Ts.z;
-                r0 = fmaf(tx, en.eR, r0); r1 = fmaf(ty, en.eR, r1); r2 = fmaf(tz, en.eR, r2);
-                m0 = fmaf(tx, en.eM, m0); m1 = fmaf(ty, en.eM, m1); m2 = fmaf(tz, en.eM, m2);
+                const float3 Ts = lerp3(lerp3(t00, t01, a), lerp3(t10, t11, a), en.p1[0]);
+                const float wR = vis * en.eR, wM = vis * en.eM;
+                const float tx = en.p0[0] * Ts.x, ty = en.p0[1] * Ts.y, tz = en.p0[2] * Ts.z;
+                aR[j][0] = fmaf(tx, wR, aR[j][0]); aR[j][1] = fmaf(ty, wR, aR[j][1]); aR[j][2] = fmaf(tz, wR, aR[j][2]);
+                aM[j][0] = fmaf(tx, wM, aM[j][0]); aM[j][1] = fmaf(ty, wM, aM[j][1]); aM[j][2] = fmaf(tz, wM, aM[j][2]);
             }
-            aR[j][0] = r0; aR[j][1] = r1; aR[j][2] = r2;
-            aM[j][0] = m0; aM[j][1] = m1; aM[j][2] = m2;
         }
+    }
+    if (slots > 1) {
+        if (slot > 0) {
+#pragma unroll
+            for (int c = 0; c < 3; ++c) {
+                part[c][threadIdx.x - nthr] = aR[0][c];
+                part[3 + c][threadIdx.x - nthr] = aM[0][c];
+            }
+        }
+        __syncthreads();
+        if (slot > 0) return;
+        for (int q = 0; q + 1 < slots; ++q)
+#pragma unroll
+            for (int c = 0; c < 3; ++c) {
+                aR[0][c] += part[c][q * nthr + lane];
+                aM[0][c] += part[3 + c][q * nthr + lane];
+            }
     }
 #pragma unroll
     for (int j = 0; j < MAXT; ++j) {
-        if (j >= nmine) break;
-        const int e = threadIdx.x + j * (int)blockDim.x;
-        if (e >= per) break;
-        const int row = e / s.W4, x = e % s.W4;
-        const size_t t = ((size_t)l * s.RMU + yb + row) * s.W4 + x;
-        const float fdx = rowdx[row];
-        const float4 oR = q16(make_float4(aR[j][0] * fdx * s.bR[0], aR[j][1] * fdx * s.bR[1], aR[j][2] * fdx * s.bR[2], 0.f), s.hs);
-        const float4 oM = q16(make_float4(aM[j][0] * fdx * s.bMS[0], aM[j][1] * fdx * s.bMS[1], aM[j][2] * fdx * s.bMS[2], 0.f), s.hs);
-        s.dSR4[t] = oR;
-        s.dSM4[t] = oM;
-        if (s.S4) s.S4[t] = make_float4(oR.x, oR.y, oR.z, oM.x);
+        const int x = lane + j * nthr;
+        if (x < W4 && j * nthr < W4) s1_store(s, ((size_t)l * s.RMU + y) * W4 + x, s_dx, aR[j], aM[j]);
     }
 }
 
@@ -361,34 +587,6 @@ constexpr float kPosLo = 1.0f - 1.0f / 256.0f, kPosHi = 1.0f / 256.0f;
 // a - (k - 1/2) d, from FP64 and rounded once; a lookup is then fma(u, d, .).
 __device__ __forceinline__ float at_zero(float a, float d, int k) {
     return (float)((double)a - ((double)k - 0.5) * (double)d);
-}
-
-// LDS byte address of an entry in two FMA-class instructions (about 2 cycles per
-// wave on gfx950, where a conversion and a shift-add take 4 each).  u + kRound,
-// kRound = 1.5 2^23, is kRound + k with k = u rounded to the nearest integer;
-// times STRIDE 2^-149, plus (base - STRIDE kRound) 2^-149, it is the denormal
-// whose bit pattern is base + STRIDE k.  Exact: the addend is a multiple of
-// STRIDE below 2^24 STRIDE (base is a multiple of STRIDE), the result is an
-// integer below 2^23.  At a tie either neighbour may come out: the two lines meet
-// there.
-constexpr float kRound = 12582912.0f;
-template <int STRIDE>
-__device__ __forceinline__ float lds_addend(unsigned base) {   // (base - STRIDE kRound) 2^-149
-    return ((float)base - (float)STRIDE * kRound) * 1.40129846e-45f;
-}
-template <int STRIDE>
-__device__ __forceinline__ unsigned lds_entry(float u, float addend) {
-    return __float_as_uint(fmaf(u + kRound, (float)STRIDE * 1.40129846e-45f, addend));
-}
-__device__ __forceinline__ float4 lds4(unsigned a, int off = 0) {
-    typedef float v4 __attribute__((ext_vector_type(4)));
-    const v4 v = *(__attribute__((address_space(3))) const v4 *)(a + off);
-    return make_float4(v.x, v.y, v.z, v.w);
-}
-__device__ __forceinline__ float2 lds2(unsigned a, int off = 0) {
-    typedef float v2 __attribute__((ext_vector_type(2)));
-    const v2 v = *(__attribute__((address_space(3))) const v2 *)(a + off);
-    return make_float2(v.x, v.y);
 }
 
 struct DirJ {      // per-theta constants of the NS x 2NS grid
@@ -1377,7 +1575,7 @@ __global__ __launch_bounds__(256) void k_snview(const SetDesc *__restrict__ sets
                                                 int nsamp) {
     const uint2 tl = tiles[blockIdx.x];
     const SetDesc &s = sets[tl.x];
-    const size_t e = (size_t)tl.y * 256 + threadIdx.x;
+    const size_t e = ((size_t)tl.y * kTileY + blockIdx.y) * 256 + threadIdx.x;
     const int row = (int)(e / (nsamp + 1));
     if (row >= s.RR * s.RMU) return;
     double mu, h1, mu1;
@@ -1402,30 +1600,24 @@ __global__ __launch_bounds__(256) void k_tview(const SetDesc *__restrict__ sets,
                                                const uint2 *__restrict__ tiles, int nsamp) {
     const uint2 tl = tiles[blockIdx.x];
     const SetDesc &s = sets[tl.x];
-    const int RPW = rows_per_wg(s.W4);
-    const int ngy = (s.RMU + RPW - 1) / RPW;
-    const int l = (int)tl.y / ngy;
-    const int yb = ((int)tl.y % ngy) * RPW;
-    const int nrows = min(RPW, s.RMU - yb);
-    const LayerGeom L = s.layers[l];
+    const size_t e = ((size_t)tl.y * kTileY + blockIdx.y) * 256 + threadIdx.x;
+    const int line = (int)(e / (nsamp + 1)), i = (int)(e % (nsamp + 1));
+    if (line >= s.RR * s.RMU) return;
+    const LayerGeom L = s.layers[line / s.RMU];
     const double r = L.r;
     const double rho2 = r * r - s.Rg2;
-    for (int e = threadIdx.x; e < nrows * (nsamp + 1); e += blockDim.x) {
-        const int row = e / (nsamp + 1), i = e % (nsamp + 1);
-        double mu, muS_u, nu_u;
-        mu_mus_nu(s, L, 0, yb + row, mu, muS_u, nu_u);
-        const double rmu = r * mu;
-        const double ti = i * (limit_d(s, r, mu) / nsamp);
-        const double q = rho2 + ti * (ti + 2.0 * rmu);   // ri^2 - Rg^2
-        const double ri = sqrt(q + s.Rg2);
-        const double h1 = q / (ri + s.Rg);
-        const double mu1 = (rmu + ti) / ri;
-        const float3 t = mu > 0.0 ? T_ratio_d(s, r - s.Rg, mu, h1, mu1)
-                                  : T_ratio_d(s, h1, -mu1, r - s.Rg, -mu);
-        const float wt = (i == 0 || i == nsamp) ? 0.5f : 1.0f;   // trapezoid weight
-        s.tview[((size_t)l * s.RMU + yb + row) * (nsamp + 1) + i] =
-            make_float4(t.x * wt, t.y * wt, t.z * wt, (float)(ti / ri));
-    }
+    double mu, muS_u, nu_u;
+    mu_mus_nu(s, L, 0, line % s.RMU, mu, muS_u, nu_u);
+    const double rmu = r * mu;
+    const double ti = i * (limit_d(s, r, mu) / nsamp);
+    const double q = rho2 + ti * (ti + 2.0 * rmu);   // ri^2 - Rg^2
+    const double ri = sqrt(q + s.Rg2);
+    const double h1 = q / (ri + s.Rg);
+    const double mu1 = (rmu + ti) / ri;
+    const float3 t = mu > 0.0 ? T_ratio_d(s, r - s.Rg, mu, h1, mu1)
+                              : T_ratio_d(s, h1, -mu1, r - s.Rg, -mu);
+    const float wt = (i == 0 || i == nsamp) ? 0.5f : 1.0f;   // trapezoid weight
+    s.tview[e] = make_float4(t.x * wt, t.y * wt, t.z * wt, (float)(ti / ri));
 }
 
 __global__ __launch_bounds__(256) void k_tground(const SetDesc *__restrict__ sets,
@@ -1461,7 +1653,7 @@ __global__ __launch_bounds__(256) void k_check(const SetDesc *__restrict__ sets,
                                                unsigned int *__restrict__ flags) {
     const uint2 tl = tiles[blockIdx.x];
     const SetDesc &s = sets[tl.x];
-    const int t = (int)tl.y * 256 + threadIdx.x;
+    const int t = ((int)tl.y * kTileY + (int)blockIdx.y) * 256 + (int)threadIdx.x;
     bool bad = false;
     if (t < s.n4) {
         float4 v = s.S4[t];
@@ -1528,12 +1720,12 @@ int chunk_irradianceN(int NI, int RNU, bool first) {
 hipError_t launch_transmittance(const SetDesc *sets, const uint2 *tiles, int ntiles, int nsamp,
                                 hipStream_t st) {
     if (ntiles <= 0) return hipSuccess;
-    hipLaunchKernelGGL(k_transmittance, dim3(ntiles), dim3(256), 0, st, sets, tiles, nsamp);
+    hipLaunchKernelGGL(k_transmittance, dim3(ntiles, kTileY), dim3(256), 0, st, sets, tiles, nsamp);
     return hipGetLastError();
 }
 hipError_t launch_tview(const SetDesc *sets, const uint2 *tiles, int ntiles, int nsamp, hipStream_t st) {
     if (ntiles <= 0) return hipSuccess;
-    hipLaunchKernelGGL(k_tview, dim3(ntiles), dim3(256), 0, st, sets, tiles, nsamp);
+    hipLaunchKernelGGL(k_tview, dim3(ntiles, kTileY), dim3(256), 0, st, sets, tiles, nsamp);
     return hipGetLastError();
 }
 hipError_t launch_tground(const SetDesc *sets, const uint2 *tiles, int ntiles, int NS, hipStream_t st) {
@@ -1547,13 +1739,59 @@ hipError_t launch_irradiance1(const SetDesc *sets, const uint2 *tiles, int ntile
     hipLaunchKernelGGL(k_irradiance1, dim3(ntiles), dim3(256), 0, st, sets, tiles);
     return hipGetLastError();
 }
-hipError_t launch_inscatter1(const SetDesc *sets, const uint2 *tiles, int ntiles, int nsamp,
-                             bool linT, hipStream_t st) {
+// The texels per thread of k_inscatter1_rows with the least waves x (5 texels + 4 + T
+// columns per thread): a texel costs a wave about 150 issue cycles per sample, the
+// sample's own terms and the barrier 120, a staged column 30.  us at 51 samples, with 1 /
+// 2 / 3 / 4 texels: 32x128x32x8 (rows of 256) 119 / 103 / 125 / 190 (spills),
+// 21x90x27x5 (135) 58 / 54 / 48 / 85 (spills), 64x256x64x16 (1024, 512 columns)
+// - / 1434 / 1932 / 1143.  So: four columns per thread only where no spill
+// comes with them (three texels).  More columns than that cost more than the gathers
+// they save, and rows of at most 64 texels gather (k_inscatter1's slots).
+S1Shape s1_shape(int W4, int TW, bool linT) {
+    const int ax = linT ? kSunLin : TW > kXkMax ? kSunWide : TW < kXkMin ? kSunFew : kSunTab;
+    S1Shape best = {ax, 0, 0, 256};
+    if (W4 <= 64 || ax == kSunFew) return best;
+    int least = 1 << 30;
+    for (int n = 1; n <= 4; ++n) {
+        const int waves = (W4 + 64 * n - 1) / (64 * n), nc = (TW + 64 * waves - 1) / (64 * waves);
+        if (waves > 8 || nc > (n == 3 ? 4 : 2)) continue;
+        const int columns = nc > 2 ? 4 : nc, cost = waves * (5 * n + 4 + columns);
+        if (cost < least) {
+            least = cost;
+            best = {ax, n, columns, 64 * waves};
+        }
+    }
+    return best;
+}
+hipError_t launch_inscatter1(const SetDesc *sets, const uint2 *tiles, int ntiles, int nsamp, S1Shape sh, int TWmax,
+                             hipStream_t st) {
     if (ntiles <= 0) return hipSuccess;
-    if (linT)
-        hipLaunchKernelGGL(k_inscatter1<true>, dim3(ntiles), dim3(256), 0, st, sets, tiles, nsamp);
-    else
-        hipLaunchKernelGGL(k_inscatter1<false>, dim3(ntiles), dim3(256), 0, st, sets, tiles, nsamp);
+    if (sh.texels > 0 && (sh.threads > 512 || sh.columns * sh.threads < TWmax)) return hipErrorInvalidValue;
+    const size_t tab = sh.axis == kSunLin || sh.axis == kSunWide ? 0 : sizeof(double) * TWmax;
+    const size_t lds = tab + (sh.texels ? 2 * sizeof(float4) * (sh.columns * sh.threads + 1) : 0);
+#define ATMO_L1(...) hipLaunchKernelGGL((__VA_ARGS__), dim3(ntiles, kTileRows), dim3(sh.threads), lds, st, sets, tiles, nsamp)
+#define ATMO_L1C(NM, NC)                                                                   \
+    if (sh.axis == kSunLin) ATMO_L1(k_inscatter1_rows<kSunLin, NM, NC>);                   \
+    else ATMO_L1(k_inscatter1_rows<kSunTab, NM, NC>)
+#define ATMO_L1R(NM) \
+    if (sh.columns == 1) { ATMO_L1C(NM, 1); } else { ATMO_L1C(NM, 2); }
+    if (sh.texels == 0) {
+        if (sh.axis == kSunLin) ATMO_L1(k_inscatter1<kSunLin>);
+        else if (sh.axis == kSunWide) ATMO_L1(k_inscatter1<kSunWide>);
+        else if (sh.axis == kSunFew) ATMO_L1(k_inscatter1<kSunFew>);
+        else ATMO_L1(k_inscatter1<kSunTab>);
+    } else if (sh.texels == 1) {
+        ATMO_L1R(1)
+    } else if (sh.texels == 2) {
+        ATMO_L1R(2)
+    } else if (sh.texels == 3) {
+        if (sh.columns == 4) { ATMO_L1C(3, 4); } else { ATMO_L1R(3) }
+    } else {
+        ATMO_L1R(4)
+    }
+#undef ATMO_L1C
+#undef ATMO_L1R
+#undef ATMO_L1
     return hipGetLastError();
 }
 hipError_t launch_inscatterS(const SetDesc *sets, const uint2 *tiles, int ntiles, int NS, int CH, int RNU,
@@ -1642,13 +1880,13 @@ hipError_t launch_inscatterN(const SetDesc *sets, const uint2 *tiles, int ntiles
 }
 hipError_t launch_snview(const SetDesc *sets, const uint2 *tiles, int ntiles, int nsamp, hipStream_t st) {
     if (ntiles <= 0) return hipSuccess;
-    hipLaunchKernelGGL(k_snview, dim3(ntiles), dim3(256), 0, st, sets, tiles, nsamp);
+    hipLaunchKernelGGL(k_snview, dim3(ntiles, kTileY), dim3(256), 0, st, sets, tiles, nsamp);
     return hipGetLastError();
 }
 hipError_t launch_check(const SetDesc *sets, const uint2 *tiles, int ntiles, unsigned int *flags,
                         hipStream_t st) {
     if (ntiles <= 0) return hipSuccess;
-    hipLaunchKernelGGL(k_check, dim3(ntiles), dim3(256), 0, st, sets, tiles, flags);
+    hipLaunchKernelGGL(k_check, dim3(ntiles, kTileY), dim3(256), 0, st, sets, tiles, flags);
     return hipGetLastError();
 }
 

@@ -818,6 +818,28 @@ def test_inscatterS_theta_rows_split_over_a_workgroup(eng, res, ns):
     _assert("E", outs[0][1].double().cpu().numpy(), E, TOL)
 
 
+@pytest.mark.parametrize("lin", [0, FLAG_LINEAR_TRANSMITTANCE])
+@pytest.mark.parametrize("res,tw,samples", [((4, 16, 8, 8), 256, 50), ((4, 16, 3, 2), 64, 2), ((4, 18, 13, 5), 64, 63),
+                                            ((4, 16, 10, 10), 200, 64), ((3, 18, 27, 5), 256, 130), ((4, 16, 64, 4), 512, 12),
+                                            ((4, 16, 64, 4), 100, 12), ((4, 16, 64, 9), 256, 1), ((2, 16, 64, 16), 512, 12),
+                                            ((2, 16, 64, 16), 1024, 12), ((4, 16, 40, 5), 48, 50), ((4, 16, 13, 8), 600, 50),
+                                            ((4, 16, 40, 5), 2100, 50)])
+def test_inscatter1_workgroup_shapes(eng, res, tw, samples, lin):
+    """Rows of 6 to 1024 texels over 48 to 2100 T columns: the staged form with 1 to 4
+    texels and 1, 2 and 4 columns per thread, the gathers with 4, 2 and 1 slots of
+    samples, below and above the columns whose centres are staged, around a chunk of
+    64 samples; alone and in one batch, within the bar of the whole-chain tests."""
+    p = small(res=res, T=(tw, 12))
+    kw = dict(orders=1, inscatter_samples=samples, transmittance_samples=100, flags=8 | lin)
+    a = eng.precompute(p, options(**kw))[0]
+    b = eng.precompute([small(), p, small(res=(4, 16, 16, 8)), p], options(**kw))
+    torch.cuda.synchronize()
+    for x, y, z in zip(a, b[1], b[3]):
+        assert torch.equal(x, y) and torch.equal(x, z)
+    T, E, S = O.precompute(p, options(**kw))
+    _assert("S", a[2].double().cpu().numpy(), S, TOL)
+
+
 @pytest.mark.parametrize("ci", range(len(CASES)))
 @pytest.mark.parametrize("form", [2, 3])
 def test_pass_inscatterN_staged_form(eng, ci, form):
