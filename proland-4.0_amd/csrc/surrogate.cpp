@@ -119,9 +119,9 @@ struct atmo_surrogate {
     int exact_orders = 1;     // orders computed by the plain passes; the network predicts the rest
     Buf Xa, Ta;
     size_t nrows = 0;
-    // work buffers: X, T, H, Y for `cap` rows; Z, dZ, dY for `zcap` rows
+    // work buffers: X, T, H, Y for `cap` rows; dZ for `zcap` rows
     int cap = 0, zcap = 0;
-    Buf X, T, Z, H, dZa, dZb, dZ1, Y, dY, part, loss;
+    Buf X, T, H, dZa, dZb, Y, part, loss;
     atmo_engine *e1 = nullptr, *ej = nullptr, *ef = nullptr;
     ~atmo_surrogate() {
         if (e1) atmo_engine_destroy(e1);
@@ -131,7 +131,6 @@ struct atmo_surrogate {
     }
     __bf16 *Wb(int L) { return wb.as<__bf16>() + (size_t)(L - 2) * kNH * kNH; }
     __bf16 *Wt(int L) { return wt.as<__bf16>() + (size_t)(L - 2) * kNH * kNH; }
-    float *Zl(int i) { return Z.as<float>() + (size_t)i * zcap * kNH; }      // i = 0..kNL-1: Z1..Z_kNL
     __bf16 *Hl(int i) { return H.as<__bf16>() + (size_t)i * cap * kNH; }     // H1..H_kNL
 };
 
@@ -148,11 +147,8 @@ atmo_status ensure_cap(atmo_surrogate *s, int rows, bool train) {
     }
     if (train && rows > s->zcap) {
         const int c = rows;
-        HIPCHK(s->Z.ensure((size_t)kNL * c * kNH * 4));
         HIPCHK(s->dZa.ensure((size_t)c * kNH * 2));
         HIPCHK(s->dZb.ensure((size_t)c * kNH * 2));
-        HIPCHK(s->dZ1.ensure((size_t)c * kNH * 4));
-        HIPCHK(s->dY.ensure((size_t)c * kNOUT * 4));
         s->zcap = c;
     }
     return ATMO_OK;
@@ -183,42 +179,25 @@ atmo_status refresh_bf16(atmo_surrogate *s) {
     return ATMO_OK;
 }
 
-// Forward over `rows` rows of s->X (rows % 128 == 0).  train: keeps Z, and
-// computes the loss against s->T into loss_slot and dY.
-atmo_status forward(atmo_surrogate *s, int rows, bool train, float *loss_slot, float *Yout) {
+// Predictions for `rows` rows of s->X (rows % 128 == 0).
+atmo_status forward(atmo_surrogate *s, int rows, float *Yout) {
     const float *P = s->p.as<float>();
-    HIPCHK(layer1_fwd(s->X.as<float>(), P + OFF_W1, P + OFF_B1, rows, train ? s->Zl(0) : nullptr,
-                      s->Hl(0), s->st));
-    for (int L = 2; L <= kNL; ++L) {
-        GemmEpi ep{P + offB(L), nullptr, train ? s->Zl(L - 1) : nullptr, s->Hl(L - 1)};
-        HIPCHK(gemm(false, true, train ? EPI_FWD : EPI_FWD_INF, s->Hl(L - 2), s->Wt(L), rows, kNH, kNH,
-                    1, ep, s->st));
-    }
-    HIPCHK(layer5(s->Hl(kNL - 1), P + OFF_W5, P + OFF_B5, s->T.as<float>(), rows, train ? 0 : 1,
-                  Yout, s->dY.as<float>(), loss_slot, s->st));
+    HIPCHK(layer1_fwd(s->X.as<float>(), P + OFF_W1, P + OFF_B1, rows, s->Hl(0), s->st));
+    for (int L = 2; L <= kNL; ++L)
+        HIPCHK(gemm_act(s->Hl(L - 2), s->Wt(L), rows, kNH, kNH, P + offB(L), s->Hl(L - 1), s->st));
+    HIPCHK(layer5(s->Hl(kNL - 1), P + OFF_W5, P + OFF_B5, rows, Yout, s->st));
     return ATMO_OK;
 }
 
-atmo_status backward(atmo_surrogate *s, int rows) {
+// Loss and gradients (s->g) of `rows` rows of s->X against s->T.
+atmo_status forward_backward(atmo_surrogate *s, int rows, float *loss_slot) {
+    static_assert(kNL == 3, "train_pass has two hidden products");
     const float *P = s->p.as<float>();
-    float *G = s->g.as<float>();
-    HIPCHK(hipMemsetAsync(G, 0, NPARAM * 4, s->st));
-    __bf16 *cur = s->dZa.as<__bf16>(), *nxt = s->dZb.as<__bf16>();
-    HIPCHK(layer5_bwd(s->Hl(kNL - 1), s->Zl(kNL - 1), P + OFF_W5, s->dY.as<float>(), rows, G + OFF_W5, G + OFF_B5,
-                      cur, s->st));
-    const int nsplit = std::max(1, std::min(64, rows / 1024));
-    const int ns = (rows / nsplit) % 32 == 0 ? nsplit : 1;
-    HIPCHK(s->part.ensure((size_t)ns * kNH * kNH * 4));
-    for (int L = kNL; L >= 2; --L) {
-        GemmEpi ew{nullptr, nullptr, s->part.as<float>(), nullptr};
-        HIPCHK(gemm(true, false, EPI_PARTIAL, s->Hl(L - 2), cur, kNH, kNH, rows, ns, ew, s->st));
-        HIPCHK(reduce_partials(s->part.as<float>(), ns, kNH * kNH, G + offW(L), s->st));
-        HIPCHK(colsum(cur, rows, G + offB(L), s->st));
-        GemmEpi ex{nullptr, s->Zl(L - 2), L == 2 ? s->dZ1.as<float>() : nullptr, nxt};
-        HIPCHK(gemm(false, true, EPI_DX, cur, s->Wb(L), rows, kNH, kNH, 1, ex, s->st));
-        std::swap(cur, nxt);
-    }
-    HIPCHK(layer1_bwd(s->X.as<float>(), s->dZ1.as<float>(), rows, G + OFF_W1, G + OFF_B1, s->st));
+    HIPCHK(s->part.ensure(train_scratch(rows)));
+    TrainArgs a{s->X.as<float>(), s->T.as<float>(), s->Wt(2), s->Wt(3), s->Wb(2), s->Wb(3),
+                P + OFF_W1, P + OFF_B1, P + offB(2), P + offB(3), P + OFF_W5, P + OFF_B5,
+                s->Hl(0), s->Hl(1), s->dZa.as<__bf16>(), s->dZb.as<__bf16>(), nullptr, nullptr, rows};
+    HIPCHK(train_pass(a, s->part.as<float>(), s->g.as<float>(), loss_slot, s->st));
     return ATMO_OK;
 }
 
@@ -436,14 +415,12 @@ atmo_status atmo_surrogate_train(atmo_surrogate *s, int steps, int batch, float 
     STCHK(ensure_cap(s, batch, true));
     Buf lbuf;
     HIPCHK(lbuf.ensure((size_t)steps * 4));
-    HIPCHK(hipMemsetAsync(lbuf.p, 0, (size_t)steps * 4, s->st));
     for (int k = 0; k < steps; ++k) {
         const double c = 0.5 * (1.0 + std::cos(M_PI * k / std::max(1, steps - 1)));
         const float lrk = (float)(lr_end + (lr - lr_end) * c);
         HIPCHK(gather(s->Xa.as<float>(), s->Ta.as<float>(), s->nrows, batch, seed * 1000003ull + k,
                       s->X.as<float>(), s->T.as<float>(), s->st));
-        STCHK(forward(s, batch, true, lbuf.as<float>() + k, nullptr));
-        STCHK(backward(s, batch));
+        STCHK(forward_backward(s, batch, lbuf.as<float>() + k));
         STCHK(adam_step(s, lrk));
     }
     HIPCHK(hipStreamSynchronize(s->st));
@@ -459,9 +436,7 @@ atmo_status atmo_surrogate_loss_grad(atmo_surrogate *s, const float *X, const fl
     STCHK(ensure_cap(s, B, true));
     HIPCHK(hipMemcpyAsync(s->X.p, X, (size_t)B * kXS * 4, hipMemcpyDeviceToDevice, s->st));
     HIPCHK(hipMemcpyAsync(s->T.p, T, (size_t)B * kNOUT * 4, hipMemcpyDeviceToDevice, s->st));
-    HIPCHK(hipMemsetAsync(s->loss.p, 0, 4, s->st));
-    STCHK(forward(s, B, true, s->loss.as<float>(), nullptr));
-    STCHK(backward(s, B));
+    STCHK(forward_backward(s, B, s->loss.as<float>()));
     HIPCHK(hipStreamSynchronize(s->st));
     HIPCHK(hipMemcpy(loss, s->loss.p, 4, hipMemcpyDeviceToHost));
     HIPCHK(hipMemcpy(grad, s->g.p, NPARAM * 4, hipMemcpyDeviceToHost));
@@ -475,7 +450,7 @@ atmo_status atmo_surrogate_predict(atmo_surrogate *s, const float *X, int B, flo
     STCHK(ensure_cap(s, Bp, false));
     HIPCHK(hipMemsetAsync(s->X.p, 0, (size_t)Bp * kXS * 4, s->st));
     HIPCHK(hipMemcpyAsync(s->X.p, X, (size_t)B * kXS * 4, hipMemcpyDeviceToDevice, s->st));
-    STCHK(forward(s, Bp, false, nullptr, s->Y.as<float>()));
+    STCHK(forward(s, Bp, s->Y.as<float>()));
     HIPCHK(hipMemcpyAsync(Y, s->Y.p, (size_t)B * kNOUT * 4, hipMemcpyDeviceToDevice, s->st));
     HIPCHK(hipStreamSynchronize(s->st));
     return ATMO_OK;

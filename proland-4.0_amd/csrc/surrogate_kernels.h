@@ -13,13 +13,16 @@ constexpr int kNL = 3;     // hidden layers (H1 .. H_kNL)
 constexpr int kNG = kNL - 1;   // hidden 256x256 layers (layers 2 .. kNL, on the matrix cores)
 constexpr int kNOUT = 4;   // outputs (rgb + an always-zero alpha)
 
-enum { EPI_FWD = 0, EPI_FWD_INF = 1, EPI_DX = 2, EPI_PARTIAL = 3 };
-
-struct GemmEpi {
-    const float *bias;   // EPI_FWD*: bias[N]
-    const float *zin;    // EPI_DX: pre-activations of the layer below
-    float *zout;         // EPI_FWD: pre-activations; EPI_DX: optional FP32 copy; EPI_PARTIAL: partials
-    __bf16 *hout;        // EPI_FWD*: activations; EPI_DX: gradients
+// A training pass over `rows` rows (a multiple of 32).  Weights: bf16 [out][in] (t) and
+// [in][out] (b); h1 .. d2: rows x 256 bf16 each, the activations and gradients as
+// operand fragments; part1, part5: set by train_pass.
+struct TrainArgs {
+    const float *X, *T;
+    const __bf16 *w2t, *w3t, *w2b, *w3b;
+    const float *W1, *b1, *b2, *b3, *W5, *b5;
+    __bf16 *h1, *h2, *d3, *d2;
+    float *part1, *part5;
+    int rows;
 };
 
 struct FeatSet {
@@ -50,18 +53,12 @@ struct InferSet {
     float *E;
 };
 
-hipError_t gemm(bool ta, bool tb, int epi, const __bf16 *A, const __bf16 *B, int M, int N, int K,
-                int nsplit, const GemmEpi &ep, hipStream_t st);
-hipError_t layer1_fwd(const float *X, const float *W1, const float *b1, int rows, float *Z1,
-                      __bf16 *H1, hipStream_t st);
-hipError_t layer5(const __bf16 *H4, const float *W5, const float *b5, const float *Tg, int rows,
-                  int mode, float *Y, float *dY, float *loss, hipStream_t st);
-hipError_t layer5_bwd(const __bf16 *H4, const float *Z4, const float *W5, const float *dY, int rows,
-                      float *gW5, float *gb5, __bf16 *dZ4, hipStream_t st);
-hipError_t layer1_bwd(const float *X, const float *dZ1, int rows, float *gW1, float *gb1,
-                      hipStream_t st);
-hipError_t colsum(const __bf16 *D, int rows, float *g, hipStream_t st);
-hipError_t reduce_partials(const float *P, int nsplit, int n, float *g, hipStream_t st);
+hipError_t gemm_act(const __bf16 *A, const __bf16 *B, int M, int N, int K, const float *bias, __bf16 *hout, hipStream_t st);
+hipError_t layer1_fwd(const float *X, const float *W1, const float *b1, int rows, __bf16 *H1, hipStream_t st);
+hipError_t layer5(const __bf16 *H4, const float *W5, const float *b5, int rows, float *Y, hipStream_t st);
+// Gradients of every parameter (flat order) and the loss; scratch: train_scratch(rows) bytes, 16-byte aligned
+size_t train_scratch(int rows);
+hipError_t train_pass(TrainArgs a, float *scratch, float *g, float *loss, hipStream_t st);
 hipError_t adam(float *p, const float *g, float *m, float *v, int n, float lr, float b1, float b2,
                 float eps, float c1, float c2, hipStream_t st);
 hipError_t to_bf16(const float *W, __bf16 *Wb, __bf16 *Wt, hipStream_t st);

@@ -9,6 +9,7 @@
 // layers, the loss, the reductions and Adam are FP32 vector code.
 #include "surrogate_kernels.h"
 
+#include <algorithm>
 #include <mutex>
 
 namespace atmo {
@@ -37,21 +38,16 @@ __device__ __forceinline__ float dact(float z) {
 }
 
 // ---------------------------------------------------------------------------
-// C[M x N] = op(A)[M x K] . op(B)[K x N], bf16 in, FP32 accumulate.
-//   TA = false: A stored [M][K] (lda = K);  TA = true: A stored [K][M] (lda = M)
-//   TB = true : B stored [N][K] (ldb = K);  TB = false: B stored [K][N] (ldb = N)
-// Tile 128 x 128 x 32, 4 waves of 64 x 64 (2 x 2 MFMA 32x32 tiles).  blockIdx.z
-// splits K into chunks of kchunk (EPI_PARTIAL writes one partial per chunk).
-// M, N multiples of 128, K and kchunk multiples of 32 (checked by the host).
+// H_out[M x 256] = act(A[M x 256] . B^T + bias), bf16 in and out, FP32 accumulate; B
+// stored [N][K].  Tile 128 x 128 x 32, 4 waves of 64 x 64 (2 x 2 MFMA 32x32 tiles).
+// M, N multiples of 128, K a multiple of 32 (checked by the host).
 // ---------------------------------------------------------------------------
-template <bool TA, bool TB, int EPI>
-__global__ __launch_bounds__(256) void k_gemm(const __bf16 *__restrict__ A,
-                                              const __bf16 *__restrict__ Bm, int M, int N, int K,
-                                              int kchunk, GemmEpi ep) {
+__global__ __launch_bounds__(256) void k_gemm_act(const __bf16 *__restrict__ A, const __bf16 *__restrict__ Bm, int M,
+                                                  int N, int K, const float *__restrict__ bias,
+                                                  __bf16 *__restrict__ hout) {
     __shared__ __attribute__((aligned(16))) __bf16 As[128][40];
     __shared__ __attribute__((aligned(16))) __bf16 Bs[128][40];
     const int n0 = blockIdx.x * 128, m0 = blockIdx.y * 128;
-    const int kb = blockIdx.z * kchunk, ke = min(K, kb + kchunk);
     const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6, wm = w >> 1, wn = w & 1;
     f32x16 acc[2][2];
 #pragma unroll
@@ -61,33 +57,13 @@ __global__ __launch_bounds__(256) void k_gemm(const __bf16 *__restrict__ A,
 #pragma unroll
             for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.0f;
 
-    for (int k0 = kb; k0 < ke; k0 += 32) {
+    for (int k0 = 0; k0 < K; k0 += 32) {
         __syncthreads();
 #pragma unroll
         for (int i = 0; i < 2; ++i) {
-            const int c = tid + i * 256;
-            if (!TA) {
-                const int row = c >> 2, kc = (c & 3) * 8;
-                const uint4 v = *(const uint4 *)(A + (size_t)(m0 + row) * K + k0 + kc);
-                *(uint4 *)&As[row][kc] = v;
-            } else {
-                const int kr = c >> 4, mc = (c & 15) * 8;
-                const uint4 v = *(const uint4 *)(A + (size_t)(k0 + kr) * M + m0 + mc);
-                const __bf16 *pv = (const __bf16 *)&v;
-#pragma unroll
-                for (int j = 0; j < 8; ++j) As[mc + j][kr] = pv[j];
-            }
-            if (TB) {
-                const int n = c >> 2, kc = (c & 3) * 8;
-                const uint4 v = *(const uint4 *)(Bm + (size_t)(n0 + n) * K + k0 + kc);
-                *(uint4 *)&Bs[n][kc] = v;
-            } else {
-                const int kr = c >> 4, nc = (c & 15) * 8;
-                const uint4 v = *(const uint4 *)(Bm + (size_t)(k0 + kr) * N + n0 + nc);
-                const __bf16 *pv = (const __bf16 *)&v;
-#pragma unroll
-                for (int j = 0; j < 8; ++j) Bs[nc + j][kr] = pv[j];
-            }
+            const int c = tid + i * 256, row = c >> 2, kc = (c & 3) * 8;
+            *(uint4 *)&As[row][kc] = *(const uint4 *)(A + (size_t)(m0 + row) * K + k0 + kc);
+            *(uint4 *)&Bs[row][kc] = *(const uint4 *)(Bm + (size_t)(n0 + row) * K + k0 + kc);
         }
         __syncthreads();
 #pragma unroll
@@ -115,32 +91,18 @@ __global__ __launch_bounds__(256) void k_gemm(const __bf16 *__restrict__ A,
             for (int r = 0; r < 16; ++r) {
                 const int row = m0 + wm * 64 + i * 32 + 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3);
                 const int col = n0 + wn * 64 + j * 32 + (lane & 31);
-                const size_t o = (size_t)row * N + col;
-                const float v = acc[i][j][r];
-                if (EPI == EPI_FWD) {
-                    const float z = v + ep.bias[col];
-                    ep.zout[o] = z;
-                    ep.hout[o] = (__bf16)act(z);
-                } else if (EPI == EPI_FWD_INF) {
-                    ep.hout[o] = (__bf16)act(v + ep.bias[col]);
-                } else if (EPI == EPI_DX) {
-                    const float g = v * dact(ep.zin[o]);
-                    ep.hout[o] = (__bf16)g;
-                    if (ep.zout) ep.zout[o] = g;
-                } else {  // EPI_PARTIAL
-                    ep.zout[(size_t)blockIdx.z * M * N + o] = v;
-                }
+                hout[(size_t)row * N + col] = (__bf16)act(acc[i][j][r] + bias[col]);
             }
 }
 
 // ---------------------------------------------------------------------------
-// Layer 1 (14 -> 256), FP32: Z1 = X W1 + b1, H1 = act(Z1).  X rows are 16
+// Layer 1 (14 -> 256), FP32: H1 = act(X W1 + b1).  X rows are 16
 // floats (14 used).  One thread per (row, column).
 // ---------------------------------------------------------------------------
 __global__ __launch_bounds__(256) void k_layer1_fwd(const float *__restrict__ X,
                                                     const float *__restrict__ W1,
                                                     const float *__restrict__ b1, int rows,
-                                                    float *__restrict__ Z1, __bf16 *__restrict__ H1) {
+                                                    __bf16 *__restrict__ H1) {
     const size_t t = (size_t)blockIdx.x * 256 + threadIdx.x;
     if (t >= (size_t)rows * kNH) return;
     const int n = (int)(t % kNH);
@@ -148,29 +110,18 @@ __global__ __launch_bounds__(256) void k_layer1_fwd(const float *__restrict__ X,
     float z = b1[n];
 #pragma unroll
     for (int i = 0; i < kNIN; ++i) z = fmaf(X[b * kXS + i], W1[i * kNH + n], z);
-    if (Z1) Z1[t] = z;
     H1[t] = (__bf16)act(z);
 }
 
 // ---------------------------------------------------------------------------
-// Layer 5 (256 -> 4), FP32 from bf16 H4, fused with the loss: a wave takes a
-// row at a time (16 rows), each lane 4 of the 256 inputs, shuffles for the
-// dot products.
-//   mode 0 (train):   dY = 2 (Y - T) / (rows * 4), loss += sum (Y - T)^2 / (rows * 4)
-//   mode 1 (predict): Y written
+// Layer 5 (256 -> 4), FP32 from bf16 H4: a wave takes a row at a time (16 rows), each
+// lane 4 of the 256 inputs, shuffles for the dot products.
 // ---------------------------------------------------------------------------
 __global__ __launch_bounds__(256) void k_layer5(const __bf16 *__restrict__ H4,
                                                 const float *__restrict__ W5,
-                                                const float *__restrict__ b5,
-                                                const float *__restrict__ Tg, int rows, int mode,
-                                                float *__restrict__ Y, float *__restrict__ dY,
-                                                float *__restrict__ loss) {
-    // a block takes 64 rows, 16 per wave; the loss of its rows is summed in the
-    // block and added with one atomic (one per row serialised on the loss word)
-    __shared__ float lsum[4];
+                                                const float *__restrict__ b5, int rows,
+                                                float *__restrict__ Y) {
     const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-    const float inv = 1.0f / ((float)rows * kNOUT);
-    float l = 0.f;
     for (int rr = 0; rr < 16; ++rr) {
         const size_t b = (size_t)blockIdx.x * 64 + wv * 16 + rr;
         if (b >= (size_t)rows) break;
@@ -188,107 +139,9 @@ __global__ __launch_bounds__(256) void k_layer5(const __bf16 *__restrict__ H4,
             for (int off = 32; off > 0; off >>= 1) acc[o] += __shfl_xor(acc[o], off, 64);
         if (lane == 0) {
 #pragma unroll
-            for (int o = 0; o < kNOUT; ++o) {
-                const float y = acc[o] + b5[o];
-                if (mode == 0) {
-                    const float d = y - Tg[b * kNOUT + o];
-                    dY[b * kNOUT + o] = 2.0f * d * inv;
-                    l += d * d;
-                } else {
-                    Y[b * kNOUT + o] = y;
-                }
-            }
+            for (int o = 0; o < kNOUT; ++o) Y[b * kNOUT + o] = acc[o] + b5[o];
         }
     }
-    if (mode != 0) return;
-    if (lane == 0) lsum[wv] = l;
-    __syncthreads();
-    if (threadIdx.x == 0) atomicAdd(loss, (lsum[0] + lsum[1] + lsum[2] + lsum[3]) * inv);
-}
-
-// Layer 5 backward: dW5 += H4^T dY, db5 += sum dY, dZ4 = (dY W5^T) * act'(Z4).
-// A wave per row at a time as in the forward.
-__global__ __launch_bounds__(256) void k_layer5_bwd(const __bf16 *__restrict__ H4,
-                                                    const float *__restrict__ Z4,
-                                                    const float *__restrict__ W5,
-                                                    const float *__restrict__ dY, int rows,
-                                                    float *__restrict__ gW5, float *__restrict__ gb5,
-                                                    __bf16 *__restrict__ dZ4) {
-    __shared__ float part[4][kNH * kNOUT];
-    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-    for (int i = threadIdx.x; i < 4 * kNH * kNOUT; i += 256) (&part[0][0])[i] = 0.f;
-    __syncthreads();
-    // each block handles 64 rows (16 per wave)
-    float dsum = 0.f;  // lane o < 4: sum of dY[., o] over this wave's rows
-    for (int rr = 0; rr < 16; ++rr) {
-        const size_t b = (size_t)blockIdx.x * 64 + wv * 16 + rr;
-        if (b >= (size_t)rows) break;
-        float d[kNOUT];
-#pragma unroll
-        for (int o = 0; o < kNOUT; ++o) d[o] = dY[b * kNOUT + o];
-        dsum += lane == 0 ? d[0] : lane == 1 ? d[1] : lane == 2 ? d[2] : lane == 3 ? d[3] : 0.f;
-#pragma unroll
-        for (int q = 0; q < 4; ++q) {
-            const int k = lane * 4 + q;
-            const size_t idx = b * kNH + k;
-            const float h = (float)H4[idx];
-            float g = 0.f;
-#pragma unroll
-            for (int o = 0; o < kNOUT; ++o) {
-                part[wv][k * kNOUT + o] += h * d[o];
-                g = fmaf(d[o], W5[k * kNOUT + o], g);
-            }
-            dZ4[idx] = (__bf16)(g * dact(Z4[idx]));
-        }
-    }
-    if (lane < kNOUT) atomicAdd(&gb5[lane], dsum);
-    __syncthreads();
-    for (int i = threadIdx.x; i < kNH * kNOUT; i += 256)
-        atomicAdd(&gW5[i], part[0][i] + part[1][i] + part[2][i] + part[3][i]);
-}
-
-// Layer 1 backward: dW1 += X^T dZ1 (11 x 256), db1 += sum dZ1.  Block = 256
-// columns x a chunk of rows.
-__global__ __launch_bounds__(256) void k_layer1_bwd(const float *__restrict__ X,
-                                                    const float *__restrict__ dZ1, int rows,
-                                                    int chunk, float *__restrict__ gW1,
-                                                    float *__restrict__ gb1) {
-    const int n = threadIdx.x;
-    const size_t r0 = (size_t)blockIdx.x * chunk;
-    const size_t r1 = min((size_t)rows, r0 + chunk);
-    float a[kNIN], s = 0.f;
-#pragma unroll
-    for (int i = 0; i < kNIN; ++i) a[i] = 0.f;
-    for (size_t b = r0; b < r1; ++b) {
-        const float g = dZ1[b * kNH + n];
-        s += g;
-#pragma unroll
-        for (int i = 0; i < kNIN; ++i) a[i] = fmaf(X[b * kXS + i], g, a[i]);
-    }
-#pragma unroll
-    for (int i = 0; i < kNIN; ++i) atomicAdd(&gW1[i * kNH + n], a[i]);
-    atomicAdd(&gb1[n], s);
-}
-
-// Column sums of a bf16 [rows x 256] matrix into g (bias gradients).
-__global__ __launch_bounds__(256) void k_colsum(const __bf16 *__restrict__ D, int rows, int chunk,
-                                                float *__restrict__ g) {
-    const int n = threadIdx.x;
-    const size_t r0 = (size_t)blockIdx.x * chunk;
-    const size_t r1 = min((size_t)rows, r0 + chunk);
-    float s = 0.f;
-    for (size_t b = r0; b < r1; ++b) s += (float)D[b * kNH + n];
-    atomicAdd(&g[n], s);
-}
-
-// g[i] += sum over nsplit partials P[s][i].
-__global__ __launch_bounds__(256) void k_reduce_partials(const float *__restrict__ P, int nsplit,
-                                                         int n, float *__restrict__ g) {
-    const int i = blockIdx.x * 256 + threadIdx.x;
-    if (i >= n) return;
-    float s = 0.f;
-    for (int k = 0; k < nsplit; ++k) s += P[(size_t)k * n + i];
-    g[i] += s;
 }
 
 // Adam (bias-corrected) on the flat FP32 parameter vector.
@@ -816,6 +669,446 @@ __global__ __launch_bounds__(64 * NW) void k_mlp_infer(const InferSet *__restric
     }
 }
 
+// ---------------------------------------------------------------------------
+// Training pass, forward and backward of a batch in one kernel (k_train_rows), the
+// hidden layers' weight gradients in a second (k_train_dw) and the sums over
+// workgroups in a third (k_train_reduce).
+//
+// k_train_rows keeps 32 rows per wave in registers as k_mlp_infer does (products
+// transposed, D = W^T H^T, bf16 weights of one or two layers staged in LDS) and
+// recomputes pre-activations where the backward pass needs them instead of storing
+// them: layer 3's when its output gradient is known, layer 2's beside the products
+// that make its gradient, layer 1's likewise.  Two more 256x256 products per row cost
+// less than 400 MB of FP32 pre-activations and gradients written and read.  Every
+// value is rounded where a layer-by-layer pass rounds it (bf16 activations and
+// gradients, FP32 pre-activations) and summed in its order: k ascending on the matrix
+// cores, layer 1 as an FMA chain from the bias (v_mfma_f32_32x32x2_f32 gives an FMA
+// chain's bits), layer 5 over the butterfly's tree.
+//
+// The activations and gradients that the weight gradients contract over the rows
+// leave it transposed, as operand fragments: a product with the identity turns a
+// register tile (lane = row) into lane = feature, 16 rows per lane, exactly; each
+// store is one contiguous KB per wave and k_train_dw loads fragments straight into
+// registers.  The row order inside a block of 16 is the C layout's (8q + 4h + t) for
+// both operands of a product, so it cancels.
+//
+// 65,536 rows: 133 us, k_train_dw 46, k_train_reduce 20; the layer-by-layer kernels took 790
+// (GEMMs 420, bias sums 80, layers 1 and 5 250, sums 34).
+// ---------------------------------------------------------------------------
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+constexpr int kTrainWaves = 8;
+constexpr int kPart5 = kNH * kNOUT + 8;   // dW5, db5, loss of a wave
+struct TrainLds {
+    __bf16 w[kNH * kRowPad];              // staged weights; at the end the FP32 transposes and sums
+    float w1[kNIN * kNH], b[3 * kNH];     // layer 1's weights; b1, b2, b3
+    float4 w5[kNH];
+    float4 dy[kTrainWaves][32];
+};
+
+// D tile (features x 32 rows, FP32) -> bf16 B operands of k blocks 2nt (lo), 2nt + 1 (hi): tile_to_b's relayout
+__device__ __forceinline__ void tile_to_bf16(const float (&v)[16], bf16x8 &lo, bf16x8 &hi) {
+    typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+    unsigned P[4][2];
+#pragma unroll
+    for (int q = 0; q < 4; ++q)
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+            const bf16x2 p = {(__bf16)v[4 * q + 2 * i], (__bf16)v[4 * q + 2 * i + 1]};
+            P[q][i] = __builtin_bit_cast(unsigned, p);
+        }
+    u32x4 L, H;
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+        const auto a = __builtin_amdgcn_permlane32_swap(P[0][i], P[1][i], false, false);
+        const auto b = __builtin_amdgcn_permlane32_swap(P[2][i], P[3][i], false, false);
+        L[i] = a[0]; L[2 + i] = a[1]; H[i] = b[0]; H[2 + i] = b[1];
+    }
+    lo = __builtin_bit_cast(bf16x8, L);
+    hi = __builtin_bit_cast(bf16x8, H);
+}
+// The identity's 16 x 32 halves as B operands
+__device__ __forceinline__ bf16x8 identity(int c, int h, int half) {
+    bf16x8 v;
+#pragma unroll
+    for (int j = 0; j < 8; ++j) v[j] = (__bf16)(c == 16 * half + 8 * h + j ? 1.0f : 0.0f);
+    return v;
+}
+// tile (lane = row) -> lane = feature c, rows 8q + 4h + t in elements 4q + t
+__device__ __forceinline__ f32x16 transpose_tile(const bf16x8 &lo, const bf16x8 &hi, int c, int h) {
+    f32x16 acc;
+#pragma unroll
+    for (int r = 0; r < 16; ++r) acc[r] = 0.0f;
+    acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(lo, identity(c, h, 0), acc, 0, 0, 0);
+    return __builtin_amdgcn_mfma_f32_32x32x16_bf16(hi, identity(c, h, 1), acc, 0, 0, 0);
+}
+// fragments of feature tile nt of a 32-row block: two k blocks of 16 rows, 16 B per lane each
+__device__ __forceinline__ void store_fragments(__bf16 *out, int rb, int nt, int lane, const f32x16 &t) {
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+        u32x4 v;
+#pragma unroll
+        for (int i = 0; i < 4; ++i)   // exact bf16 values: their upper halves
+            v[i] = __builtin_amdgcn_perm(__float_as_uint(t[8 * u + 2 * i + 1]), __float_as_uint(t[8 * u + 2 * i]), 0x07060302u);
+        *(u32x4 *)(out + ((((size_t)rb * 8 + nt) * 2 + u) * 64 + lane) * 8) = v;
+    }
+}
+// tile nt of a 256x256 product from staged weight rows (row 0 of `w` is row 0 of the tile's half)
+__device__ __forceinline__ f32x16 train_tile(const __bf16 *w, int nt, int c, int h, const bf16x8 (&H)[16]) {
+    f32x16 acc;
+#pragma unroll
+    for (int r = 0; r < 16; ++r) acc[r] = 0.0f;
+    const __bf16 *row = w + (32 * nt + c) * kRowPad + 8 * h;
+#pragma unroll
+    for (int kb = 0; kb < 16; ++kb)
+        acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(*(const bf16x8 *)(row + 16 * kb), H[kb], acc, 0, 0, 0);
+    return acc;
+}
+// pre-activations of layer 1's tile nt: b1 + the chain over the inputs
+__device__ __forceinline__ f32x16 layer1_tile(const TrainLds &S, int nt, int c, int h, const float (&xf)[7]) {
+    f32x16 acc;
+#pragma unroll
+    for (int r = 0; r < 16; ++r) acc[r] = S.b[32 * nt + 8 * (r >> 2) + 4 * h + (r & 3)];
+#pragma unroll
+    for (int k = 0; k < 7; ++k)
+        acc = __builtin_amdgcn_mfma_f32_32x32x2f32(S.w1[(2 * k + h) * kNH + 32 * nt + c], xf[k], acc, 0, 0, 0);
+    return acc;
+}
+__device__ __forceinline__ void stage_train(const __bf16 *W, __bf16 *wl, int r0, int wv, int lane) {
+    stage_half_async<kTrainWaves>((const _Float16 *)W, (_Float16 *)wl, r0, wv, lane);
+}
+
+__global__ __launch_bounds__(64 * kTrainWaves) void k_train_rows(TrainArgs a) {
+    static_assert(kNL == 3 && kNIN == 14 && kNOUT == 4 && kNH == 256, "the layer sequence is written out");
+    extern __shared__ __attribute__((aligned(16))) char smem[];
+    TrainLds &S = *(TrainLds *)smem;
+    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6, h = lane >> 5, c = lane & 31;
+    const int row0 = (blockIdx.x * kTrainWaves + wv) * 32;
+    const bool active = row0 < a.rows;   // rows is a multiple of 32: whole waves
+    const int row = min(row0, a.rows - 32) + c, rb = row0 / 32;
+    __bf16 *wA = S.w, *wB = S.w + 128 * kRowPad;
+    for (int i = threadIdx.x; i < kNIN * kNH; i += 64 * kTrainWaves) S.w1[i] = a.W1[i];
+    for (int i = threadIdx.x; i < kNH; i += 64 * kTrainWaves) {
+        S.b[i] = a.b1[i];
+        S.b[kNH + i] = a.b2[i];
+        S.b[2 * kNH + i] = a.b3[i];
+        S.w5[i] = make_float4(a.W5[4 * i], a.W5[4 * i + 1], a.W5[4 * i + 2], a.W5[4 * i + 3]);
+    }
+    float xf[7];
+#pragma unroll
+    for (int k = 0; k < 7; ++k) xf[k] = a.X[(size_t)row * kXS + 2 * k + h];
+    __syncthreads();
+    stage_train(a.w2t, wA, 0, wv, lane);
+    stage_train(a.w2t, wA, 128, wv, lane);
+    const float *b2 = S.b + kNH, *b3 = S.b + 2 * kNH;
+
+    bf16x8 H1[16], H2[16];
+#pragma unroll
+    for (int nt = 0; nt < 8; ++nt) {   // layer 1
+        const f32x16 z = layer1_tile(S, nt, c, h, xf);
+        float v[16];
+#pragma unroll
+        for (int r = 0; r < 16; ++r) v[r] = act(z[r]);
+        tile_to_bf16(v, H1[2 * nt], H1[2 * nt + 1]);
+        const f32x16 t = transpose_tile(H1[2 * nt], H1[2 * nt + 1], c, h);
+        if (active) store_fragments(a.h1, rb, nt, lane, t);
+    }
+    wait_all_and_sync();
+    auto forward_tile = [&](const float *bias, int nt, const bf16x8 (&In)[16], bf16x8 &lo, bf16x8 &hi) {
+        const f32x16 z = train_tile(S.w, nt, c, h, In);
+        float v[16];
+#pragma unroll
+        for (int r = 0; r < 16; ++r) v[r] = act(z[r] + bias[32 * nt + 8 * (r >> 2) + 4 * h + (r & 3)]);
+        tile_to_bf16(v, lo, hi);
+    };
+#pragma unroll
+    for (int nt = 0; nt < 8; ++nt) {   // layer 2
+        if (nt == 4) {
+            wait_all_and_sync();
+            stage_train(a.w3t, wA, 0, wv, lane);
+        }
+        forward_tile(b2, nt, H1, H2[2 * nt], H2[2 * nt + 1]);
+        const f32x16 t = transpose_tile(H2[2 * nt], H2[2 * nt + 1], c, h);
+        if (active) store_fragments(a.h2, rb, nt, lane, t);
+    }
+    wait_all_and_sync();
+    stage_train(a.w3t, wA, 128, wv, lane);
+    float4 dy;
+    float *part5 = a.part5 + (size_t)rb * kPart5;
+    {
+        bf16x8 H3[16];
+#pragma unroll
+        for (int nt = 0; nt < 8; ++nt) {   // layer 3
+            if (nt == 4) wait_all_and_sync();
+            forward_tile(b3, nt, H2, H3[2 * nt], H3[2 * nt + 1]);
+        }
+        // layer 5: 4-input chains, then the tree of a 64-lane butterfly (chain L = features 4L ..
+        // 4L + 3 with L + 32, 16, 8, 4, 2, 1); L = 4 kb + 2h + j
+        float y[2][4];
+#pragma unroll
+        for (int j = 0; j < 2; ++j) {
+            float s[16][4];
+#pragma unroll
+            for (int kb = 0; kb < 16; ++kb) {
+#pragma unroll
+                for (int o = 0; o < 4; ++o) s[kb][o] = 0.f;
+#pragma unroll
+                for (int q = 0; q < 4; ++q) {
+                    const float hv = (float)H3[kb][4 * j + q];
+                    const float4 w = S.w5[16 * kb + 8 * h + 4 * j + q];
+                    s[kb][0] = fmaf(hv, w.x, s[kb][0]);
+                    s[kb][1] = fmaf(hv, w.y, s[kb][1]);
+                    s[kb][2] = fmaf(hv, w.z, s[kb][2]);
+                    s[kb][3] = fmaf(hv, w.w, s[kb][3]);
+                }
+                // combine as soon as the partners of a level are there
+                if (kb >= 8) {
+#pragma unroll
+                    for (int o = 0; o < 4; ++o) s[kb - 8][o] += s[kb][o];
+                }
+            }
+#pragma unroll
+            for (int off = 4; off > 0; off >>= 1)
+#pragma unroll
+                for (int kb = 0; kb < off; ++kb)
+#pragma unroll
+                    for (int o = 0; o < 4; ++o) s[kb][o] += s[kb + off][o];
+#pragma unroll
+            for (int o = 0; o < 4; ++o) y[j][o] = s[0][o] + __shfl_xor(s[0][o], 32, 64);
+        }
+        const float inv = 1.0f / ((float)a.rows * kNOUT);
+        float d[5];
+        d[4] = 0.f;
+#pragma unroll
+        for (int o = 0; o < 4; ++o) {
+            const float e = (y[0][o] + y[1][o]) + a.b5[o] - a.T[(size_t)row * kNOUT + o];
+            d[o] = 2.0f * e * inv;
+            d[4] += e * e;
+        }
+        dy = make_float4(d[0], d[1], d[2], d[3]);
+        if (h == 0) S.dy[wv][c] = dy;
+        __builtin_amdgcn_wave_barrier();
+        // dW5 = H3^T dY over this wave's rows, db5 and the loss
+#pragma unroll
+        for (int nt = 0; nt < 8; ++nt) {
+            const f32x16 t = transpose_tile(H3[2 * nt], H3[2 * nt + 1], c, h);
+            float g[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int r = 0; r < 16; ++r) {
+                const float4 e = S.dy[wv][8 * (r >> 2) + 4 * h + (r & 3)];
+                g[0] = fmaf(t[r], e.x, g[0]); g[1] = fmaf(t[r], e.y, g[1]);
+                g[2] = fmaf(t[r], e.z, g[2]); g[3] = fmaf(t[r], e.w, g[3]);
+            }
+#pragma unroll
+            for (int o = 0; o < 4; ++o) g[o] += __shfl_xor(g[o], 32, 64);
+            if (active && h == 0) *(float4 *)(part5 + 4 * (32 * nt + c)) = make_float4(g[0], g[1], g[2], g[3]);
+        }
+#pragma unroll
+        for (int o = 0; o < 5; ++o) {
+#pragma unroll
+            for (int off = 16; off > 0; off >>= 1) d[o] += __shfl_xor(d[o], off, 64);
+            if (active && lane == 0) part5[kNH * kNOUT + o] = o < 4 ? d[o] : d[o] * inv;
+        }
+    }
+    bf16x8 D3[16];
+#pragma unroll
+    for (int nt = 0; nt < 8; ++nt) {   // dZ3 = (dY W5^T) act'(Z3), Z3 again
+        if (nt == 4) {
+            wait_all_and_sync();
+            stage_train(a.w3b, wA, 0, wv, lane);
+        }
+        const f32x16 z = train_tile(S.w, nt, c, h, H2);
+        float v[16];
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+            const int f = 32 * nt + 8 * (r >> 2) + 4 * h + (r & 3);
+            const float4 w = S.w5[f];
+            float g = 0.f;
+            g = fmaf(dy.x, w.x, g); g = fmaf(dy.y, w.y, g); g = fmaf(dy.z, w.z, g); g = fmaf(dy.w, w.w, g);
+            v[r] = g * dact(z[r] + b3[f]);
+        }
+        tile_to_bf16(v, D3[2 * nt], D3[2 * nt + 1]);
+        const f32x16 t = transpose_tile(D3[2 * nt], D3[2 * nt + 1], c, h);
+        if (active) store_fragments(a.d3, rb, nt, lane, t);
+    }
+    bf16x8 D2[16];
+#pragma unroll
+    for (int half = 0; half < 2; ++half) {   // dZ2 = (dZ3 W3^T) act'(Z2), Z2 again
+        wait_all_and_sync();
+        if (half == 1) stage_train(a.w3b + 128 * kNH, wA, 0, wv, lane);
+        stage_train(a.w2t + 128 * half * kNH, wB, 0, wv, lane);
+        wait_all_and_sync();
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const int nt = 4 * half + i;
+            const f32x16 z = train_tile(wB, i, c, h, H1), p = train_tile(wA, i, c, h, D3);
+            float v[16];
+#pragma unroll
+            for (int r = 0; r < 16; ++r) v[r] = p[r] * dact(z[r] + b2[32 * nt + 8 * (r >> 2) + 4 * h + (r & 3)]);
+            tile_to_bf16(v, D2[2 * nt], D2[2 * nt + 1]);
+            const f32x16 t = transpose_tile(D2[2 * nt], D2[2 * nt + 1], c, h);
+            if (active) store_fragments(a.d2, rb, nt, lane, t);
+        }
+    }
+    wait_all_and_sync();
+    stage_train(a.w2b, wA, 0, wv, lane);
+    stage_train(a.w2b, wA, 128, wv, lane);
+    wait_all_and_sync();
+    float g1[8][16];
+#pragma unroll
+    for (int nt = 0; nt < 8; ++nt) {   // dZ1 = (dZ2 W2^T) act'(Z1), Z1 again; FP32
+        const f32x16 p = train_tile(S.w, nt, c, h, D2), z = layer1_tile(S, nt, c, h, xf);
+#pragma unroll
+        for (int r = 0; r < 16; ++r) g1[nt][r] = p[r] * dact(z[r]);
+    }
+    // dW1 and db1 (input 14 is 1) over this wave's rows: dZ1 through LDS (rows of 132
+    // floats), two halves of the features, FP32 products on the matrix cores
+    float xa[8];
+    const int m = lane & 15, k4 = lane >> 4;
+#pragma unroll
+    for (int k = 0; k < 8; ++k) {
+        const float x = m < kNIN ? a.X[(size_t)(min(row0, a.rows - 32) + 4 * k + k4) * kXS + m] : m == kNIN ? 1.0f : 0.0f;
+        xa[k] = active ? x : 0.0f;
+    }
+    __syncthreads();
+    float *tw = (float *)S.w + wv * (32 * 132);
+    f32x4 dw[16];
+#pragma unroll
+    for (int half = 0; half < 2; ++half) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+#pragma unroll
+            for (int q = 0; q < 4; ++q)
+                *(float4 *)(tw + c * 132 + 32 * i + 8 * q + 4 * h) =
+                    make_float4(g1[4 * half + i][4 * q], g1[4 * half + i][4 * q + 1], g1[4 * half + i][4 * q + 2], g1[4 * half + i][4 * q + 3]);
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+#pragma unroll
+        for (int n = 0; n < 8; ++n) {
+            f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int k = 0; k < 8; ++k)
+                acc = __builtin_amdgcn_mfma_f32_16x16x4f32(xa[k], tw[(4 * k + k4) * 132 + 16 * n + m], acc, 0, 0, 0);
+            dw[8 * half + n] = acc;
+        }
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+    }
+    __syncthreads();
+    float *ws = (float *)S.w;   // [wave][16][256]
+#pragma unroll
+    for (int n = 0; n < 16; ++n)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) ws[(wv * 16 + 4 * k4 + r) * kNH + 16 * n + m] = dw[n][r];
+    __syncthreads();
+    for (int e = threadIdx.x; e < 15 * kNH; e += 64 * kTrainWaves) {
+        float sum = 0.f;
+#pragma unroll
+        for (int w = 0; w < kTrainWaves; ++w) sum += ws[w * 16 * kNH + e];
+        a.part1[(size_t)blockIdx.x * 15 * kNH + e] = sum;
+    }
+}
+
+// dW = H^T dZ of layers 2 (blockIdx.z 0) and 3 over a range of 32-row blocks, one
+// 128 x 128 tile per workgroup (blockIdx.y), 64 x 64 per wave, straight from the
+// fragments; db = the column sums of dZ as products with ones.  A tile's fragments are
+// read by two waves of a workgroup and two workgroups, which share an XCD's L2 (the
+// range is blockIdx.x, a multiple of 8 of them where there are that many).
+__global__ __launch_bounds__(256) void k_train_dw(const __bf16 *h1, const __bf16 *d2, const __bf16 *h2, const __bf16 *d3,
+                                                  int nrb, float *__restrict__ part, float *__restrict__ partb) {
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, h = lane >> 5, c = lane & 31;
+    const __bf16 *A = blockIdx.z ? h2 : h1, *B = blockIdx.z ? d3 : d2;
+    const int mt = (blockIdx.y >> 1) * 4 + (w >> 1) * 2, nt = (blockIdx.y & 1) * 4 + (w & 1) * 2;
+    const int ns = gridDim.x, rb0 = (int)((long long)nrb * blockIdx.x / ns), rb1 = (int)((long long)nrb * (blockIdx.x + 1) / ns);
+    const bool bias = mt == 0;
+    f32x16 acc[2][2], sum[2];
+#pragma unroll
+    for (int r = 0; r < 16; ++r) acc[0][0][r] = acc[0][1][r] = acc[1][0][r] = acc[1][1][r] = sum[0][r] = sum[1][r] = 0.0f;
+    bf16x8 ones;
+#pragma unroll
+    for (int j = 0; j < 8; ++j) ones[j] = (__bf16)1.0f;
+    struct Frag {
+        bf16x8 a[2][2], b[2][2];   // [tile][k block]
+    };
+    auto load = [&](int rb) {
+        Frag f;
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+#pragma unroll
+            for (int u = 0; u < 2; ++u) {
+                f.a[i][u] = *(const bf16x8 *)(A + ((((size_t)rb * 8 + mt + i) * 2 + u) * 64 + lane) * 8);
+                f.b[i][u] = *(const bf16x8 *)(B + ((((size_t)rb * 8 + nt + i) * 2 + u) * 64 + lane) * 8);
+            }
+        return f;
+    };
+    Frag f0 = load(rb0), f1 = load(min(rb0 + 1, rb1 - 1));
+    for (int rb = rb0; rb < rb1; ++rb) {
+        const Frag f = f0;
+        f0 = f1;
+        f1 = load(min(rb + 2, rb1 - 1));
+#pragma unroll
+        for (int u = 0; u < 2; ++u) {
+#pragma unroll
+            for (int i = 0; i < 2; ++i)
+#pragma unroll
+                for (int j = 0; j < 2; ++j)
+                    acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(f.a[i][u], f.b[j][u], acc[i][j], 0, 0, 0);
+            if (bias) {
+#pragma unroll
+                for (int j = 0; j < 2; ++j) sum[j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ones, f.b[j][u], sum[j], 0, 0, 0);
+            }
+        }
+    }
+    const size_t split = (size_t)blockIdx.z * ns + blockIdx.x;
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int j = 0; j < 2; ++j)
+#pragma unroll
+            for (int r = 0; r < 16; ++r)
+                part[split * kNH * kNH + (size_t)(32 * (mt + i) + 8 * (r >> 2) + 4 * h + (r & 3)) * kNH + 32 * (nt + j) + c] = acc[i][j][r];
+    if (bias && h == 0) {
+#pragma unroll
+        for (int j = 0; j < 2; ++j) partb[split * kNH + 32 * (nt + j) + c] = sum[j][0];
+    }
+}
+
+// Gradient e (and, behind the parameters, the loss) = the sum of its partials; 64
+// values per workgroup, 16 threads each.  Parameters: W1, b1 (partials of
+// workgroups), W2, b2, W3, b3 (of row ranges), W5, b5 (of waves).
+__global__ __launch_bounds__(1024) void k_train_reduce(const float *__restrict__ part1, int nwg, const float *__restrict__ part,
+                                                       const float *__restrict__ partb, int ns, const float *__restrict__ part5,
+                                                       int nwave, float *__restrict__ g, float *__restrict__ loss) {
+    __shared__ float s[16][64];
+    const int x = threadIdx.x & 63, k0 = threadIdx.x >> 6;
+    constexpr int L1 = 15 * kNH, LH = kNH * kNH + kNH, N = L1 + kNG * LH + kNH * kNOUT + kNOUT;
+    const int e = blockIdx.x * 64 + x;
+    const float *p = part1 + e;
+    int count = nwg;
+    size_t stride = L1;
+    if (e >= L1 + kNG * LH) {
+        p = part5 + (e - L1 - kNG * LH);
+        count = nwave;
+        stride = kPart5;
+    } else if (e >= L1) {
+        const int L = (e - L1) / LH, i = (e - L1) % LH;
+        count = ns;
+        stride = i < kNH * kNH ? kNH * kNH : kNH;
+        p = (i < kNH * kNH ? part + i : partb + (i - kNH * kNH)) + (size_t)L * ns * stride;
+    }
+    float v = 0.f;
+    if (e <= N)
+#pragma unroll 4
+        for (int k = k0; k < count; k += 16) v += p[k * stride];
+    s[k0][x] = v;
+    __syncthreads();
+    if (k0 == 0 && e <= N) {
+#pragma unroll
+        for (int k = 1; k < 16; ++k) v += s[k][x];
+        if (e < N) g[e] = v;
+        else *loss = v;
+    }
+}
+
 // Weights of the fused kernel from the FP32 parameters: layer 1 (+ bias in
 // column 14) split into bf16 hi/lo, layer 5 into FP16 hi/lo, the hidden
 // weights as FP16 [out][in] and their biases packed.
@@ -850,50 +1143,20 @@ __global__ __launch_bounds__(256) void k_prep_fused(const float *__restrict__ W1
 // ---------------------------------------------------------------------------
 // launchers
 // ---------------------------------------------------------------------------
-hipError_t gemm(bool ta, bool tb, int epi, const __bf16 *A, const __bf16 *B, int M, int N, int K,
-                int nsplit, const GemmEpi &ep, hipStream_t st) {
-    if (M % 128 || N % 128 || K % 32 || nsplit < 1 || (K / nsplit) % 32) return hipErrorInvalidValue;
-    dim3 grid(N / 128, M / 128, nsplit);
-    const int kc = K / nsplit;
-#define SG_L(TA_, TB_, E_) hipLaunchKernelGGL((k_gemm<TA_, TB_, E_>), grid, dim3(256), 0, st, A, B, M, N, K, kc, ep)
-    if (!ta && tb && epi == EPI_FWD) SG_L(false, true, EPI_FWD);
-    else if (!ta && tb && epi == EPI_FWD_INF) SG_L(false, true, EPI_FWD_INF);
-    else if (!ta && tb && epi == EPI_DX) SG_L(false, true, EPI_DX);
-    else if (ta && !tb && epi == EPI_PARTIAL) SG_L(true, false, EPI_PARTIAL);
-    else return hipErrorInvalidValue;
-#undef SG_L
+hipError_t gemm_act(const __bf16 *A, const __bf16 *B, int M, int N, int K, const float *bias, __bf16 *hout, hipStream_t st) {
+    if (M % 128 || N % 128 || K % 32) return hipErrorInvalidValue;
+    hipLaunchKernelGGL(k_gemm_act, dim3(N / 128, M / 128), dim3(256), 0, st, A, B, M, N, K, bias, hout);
     return hipGetLastError();
 }
 
 static unsigned blocks(size_t n) { return (unsigned)((n + 255) / 256); }
 
-hipError_t layer1_fwd(const float *X, const float *W1, const float *b1, int rows, float *Z1, __bf16 *H1,
-                      hipStream_t st) {
-    hipLaunchKernelGGL(k_layer1_fwd, dim3(blocks((size_t)rows * kNH)), dim3(256), 0, st, X, W1, b1, rows, Z1, H1);
+hipError_t layer1_fwd(const float *X, const float *W1, const float *b1, int rows, __bf16 *H1, hipStream_t st) {
+    hipLaunchKernelGGL(k_layer1_fwd, dim3(blocks((size_t)rows * kNH)), dim3(256), 0, st, X, W1, b1, rows, H1);
     return hipGetLastError();
 }
-hipError_t layer5(const __bf16 *H4, const float *W5, const float *b5, const float *Tg, int rows, int mode,
-                  float *Y, float *dY, float *loss, hipStream_t st) {
-    hipLaunchKernelGGL(k_layer5, dim3((rows + 63) / 64), dim3(256), 0, st, H4, W5, b5, Tg, rows, mode, Y, dY, loss);
-    return hipGetLastError();
-}
-hipError_t layer5_bwd(const __bf16 *H4, const float *Z4, const float *W5, const float *dY, int rows,
-                      float *gW5, float *gb5, __bf16 *dZ4, hipStream_t st) {
-    hipLaunchKernelGGL(k_layer5_bwd, dim3((rows + 63) / 64), dim3(256), 0, st, H4, Z4, W5, dY, rows, gW5, gb5, dZ4);
-    return hipGetLastError();
-}
-hipError_t layer1_bwd(const float *X, const float *dZ1, int rows, float *gW1, float *gb1, hipStream_t st) {
-    const int chunk = 64;   // 1024 workgroups at the training batch
-    hipLaunchKernelGGL(k_layer1_bwd, dim3((rows + chunk - 1) / chunk), dim3(256), 0, st, X, dZ1, rows, chunk, gW1, gb1);
-    return hipGetLastError();
-}
-hipError_t colsum(const __bf16 *D, int rows, float *g, hipStream_t st) {
-    const int chunk = 64;   // 1024 workgroups at the training batch
-    hipLaunchKernelGGL(k_colsum, dim3((rows + chunk - 1) / chunk), dim3(256), 0, st, D, rows, chunk, g);
-    return hipGetLastError();
-}
-hipError_t reduce_partials(const float *P, int nsplit, int n, float *g, hipStream_t st) {
-    hipLaunchKernelGGL(k_reduce_partials, dim3(blocks(n)), dim3(256), 0, st, P, nsplit, n, g);
+hipError_t layer5(const __bf16 *H4, const float *W5, const float *b5, int rows, float *Y, hipStream_t st) {
+    hipLaunchKernelGGL(k_layer5, dim3((rows + 63) / 64), dim3(256), 0, st, H4, W5, b5, rows, Y);
     return hipGetLastError();
 }
 hipError_t adam(float *p, const float *g, float *m, float *v, int n, float lr, float b1, float b2,
@@ -955,25 +1218,51 @@ hipError_t prep_fused(const float *W1, const float *b1, const float *W5, const f
                        wt, a5h, a5l, bh);
     return hipGetLastError();
 }
-hipError_t mlp_infer(const InferSet *sets, int nsets, int ntiles, const FusedWeights &fw, const TargetNorm &tn,
-                     hipStream_t st) {
-    if (nsets <= 0 || ntiles <= 0) return hipSuccess;
-    // the kernel takes more dynamic LDS than the default limit: raise it once per device
+// Kernels that take more dynamic LDS than the default limit: raised once per device.
+static hipError_t raise_lds(const void *kernel, size_t bytes, unsigned long long &done) {
     static std::mutex mu;
-    static unsigned long long done = 0;
     int dev = 0;
     hipError_t e = hipGetDevice(&dev);
     if (e != hipSuccess) return e;
     if (dev < 0 || dev >= 64) return hipErrorInvalidDevice;
-    {
-        std::lock_guard<std::mutex> lk(mu);
-        if (!(done & (1ull << dev))) {
-            e = hipFuncSetAttribute((const void *)k_mlp_infer<kFusedRBW, kFusedNW>,
-                                    hipFuncAttributeMaxDynamicSharedMemorySize, (int)fused_lds());
-            if (e != hipSuccess) return e;
-            done |= 1ull << dev;
-        }
+    std::lock_guard<std::mutex> lk(mu);
+    if (!(done & (1ull << dev))) {
+        e = hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes);
+        if (e != hipSuccess) return e;
+        done |= 1ull << dev;
     }
+    return hipSuccess;
+}
+
+// Row ranges of k_train_dw: at least 4 blocks of 32 rows each, at most 64 (512 workgroups)
+static int dw_ranges(int rows) { return std::max(1, std::min(64, rows / 128)); }
+size_t train_scratch(int rows) {
+    const size_t nwg = (rows + 255) / 256, ns = dw_ranges(rows);
+    return sizeof(float) * (nwg * 15 * kNH + (size_t)(rows / 32) * kPart5 + 2 * ns * ((size_t)kNH * kNH + kNH));
+}
+hipError_t train_pass(TrainArgs a, float *scratch, float *g, float *loss, hipStream_t st) {
+    if (a.rows <= 0 || a.rows % 32) return hipErrorInvalidValue;
+    const int nwg = (a.rows + 255) / 256, ns = dw_ranges(a.rows), nrb = a.rows / 32;
+    a.part5 = scratch;   // 16-byte stores
+    a.part1 = a.part5 + (size_t)nrb * kPart5;
+    float *part = a.part1 + (size_t)nwg * 15 * kNH, *partb = part + (size_t)2 * ns * kNH * kNH;
+    static unsigned long long done = 0;
+    hipError_t e = raise_lds((const void *)k_train_rows, sizeof(TrainLds), done);
+    if (e != hipSuccess) return e;
+    hipLaunchKernelGGL(k_train_rows, dim3(nwg), dim3(64 * kTrainWaves), sizeof(TrainLds), st, a);
+    if ((e = hipGetLastError()) != hipSuccess) return e;
+    hipLaunchKernelGGL(k_train_dw, dim3(ns, 4, 2), dim3(256), 0, st, a.h1, a.d2, a.h2, a.d3, nrb, part, partb);
+    if ((e = hipGetLastError()) != hipSuccess) return e;
+    constexpr int N = 15 * kNH + kNG * (kNH * kNH + kNH) + kNH * kNOUT + kNOUT + 1;
+    hipLaunchKernelGGL(k_train_reduce, dim3((N + 63) / 64), dim3(1024), 0, st, a.part1, nwg, part, partb, ns, a.part5, nrb, g, loss);
+    return hipGetLastError();
+}
+hipError_t mlp_infer(const InferSet *sets, int nsets, int ntiles, const FusedWeights &fw, const TargetNorm &tn,
+                     hipStream_t st) {
+    if (nsets <= 0 || ntiles <= 0) return hipSuccess;
+    static unsigned long long done = 0;
+    const hipError_t e = raise_lds((const void *)k_mlp_infer<kFusedRBW, kFusedNW>, fused_lds(), done);
+    if (e != hipSuccess) return e;
     hipLaunchKernelGGL((k_mlp_infer<kFusedRBW, kFusedNW>), dim3(ntiles), dim3(64 * kFusedNW), fused_lds(), st, sets,
                        nsets, fw, tn);
     return hipGetLastError();

@@ -59,6 +59,25 @@ def test_gradients_match_oracle(sur, B):
         assert rel < 3e-2 and cos > 0.999, k
 
 
+@pytest.mark.parametrize("B", [256, 384, 640, 16512])
+def test_training_pass_sizes(sur, B):
+    """Whole workgroups of 256 rows and one of 128, one and more row ranges of the
+    weight-gradient products (128 rows each, 64 from 8192 rows on): the gradients to the
+    bar of test_gradients_match_oracle, and twice the same bits."""
+    X, T = rows(B, 2 + B)
+    dX, dT = torch.from_numpy(X).cuda(), torch.from_numpy(T).cuda()
+    loss, g = sur.loss_grad(dX, dT)
+    again, g2 = sur.loss_grad(dX, dT)
+    assert loss == again and np.array_equal(g, g2)
+    lo, go = M.loss_grad(sur.get_params().astype(np.float64), X, T, emulate_bf16=True)
+    assert loss == pytest.approx(lo, rel=2e-3)
+    gb, ob = blocks(g.astype(np.float64)), blocks(go)
+    for k in gb:
+        rel = np.linalg.norm(gb[k] - ob[k]) / max(np.linalg.norm(ob[k]), 1e-30)
+        cos = np.dot(gb[k], ob[k]) / max(np.linalg.norm(gb[k]) * np.linalg.norm(ob[k]), 1e-30)
+        assert rel < 3e-2 and cos > 0.999, k
+
+
 def _log_ray(p, l, y):
     """The mu-row coordinate: the row's ray length (getMuMuSNu with the setLayer
     radius) on a log scale from 1 m to 2 sqrt(Rt^2 - Rg^2)."""
