@@ -692,7 +692,7 @@ __global__ __launch_bounds__(64 * NW) void k_mlp_infer(const InferSet *__restric
 // registers.  The row order inside a block of 16 is the C layout's (8q + 4h + t) for
 // both operands of a product, so it cancels.
 //
-// 65,536 rows: 133 us, k_train_dw 46, k_train_reduce 20; the layer-by-layer kernels took 790
+// 65,536 rows: 103 us, k_train_dw 35, k_train_reduce 18; the layer-by-layer kernels took 790
 // (GEMMs 420, bias sums 80, layers 1 and 5 250, sums 34).
 // ---------------------------------------------------------------------------
 typedef float f32x4 __attribute__((ext_vector_type(4)));
@@ -741,16 +741,21 @@ __device__ __forceinline__ f32x16 transpose_tile(const bf16x8 &lo, const bf16x8 
     acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(lo, identity(c, h, 0), acc, 0, 0, 0);
     return __builtin_amdgcn_mfma_f32_32x32x16_bf16(hi, identity(c, h, 1), acc, 0, 0, 0);
 }
-// fragments of feature tile nt of a 32-row block: two k blocks of 16 rows, 16 B per lane each
-__device__ __forceinline__ void store_fragments(__bf16 *out, int rb, int nt, int lane, const f32x16 &t) {
+// k block u of a transposed tile (16 rows): exact bf16 values, their upper halves
+__device__ __forceinline__ u32x4 fragment(const f32x16 &t, int u) {
+    u32x4 v;
 #pragma unroll
-    for (int u = 0; u < 2; ++u) {
-        u32x4 v;
+    for (int i = 0; i < 4; ++i)
+        v[i] = __builtin_amdgcn_perm(__float_as_uint(t[8 * u + 2 * i + 1]), __float_as_uint(t[8 * u + 2 * i]), 0x07060302u);
+    return v;
+}
+// fragments of feature tile nt of a 32-row block (`out`, scalar): two k blocks of 16 rows, 16 B
+// per lane each.  Global stores with a scalar base: after a buffer store with a scalar
+// offset the compiler lets the next instruction overwrite the data registers, and under
+// load stores then wrote the new values.
+__device__ __forceinline__ void store_fragments(__bf16 *out, int nt, int lane, const f32x16 &t) {
 #pragma unroll
-        for (int i = 0; i < 4; ++i)   // exact bf16 values: their upper halves
-            v[i] = __builtin_amdgcn_perm(__float_as_uint(t[8 * u + 2 * i + 1]), __float_as_uint(t[8 * u + 2 * i]), 0x07060302u);
-        *(u32x4 *)(out + ((((size_t)rb * 8 + nt) * 2 + u) * 64 + lane) * 8) = v;
-    }
+    for (int u = 0; u < 2; ++u) *(u32x4 *)((char *)out + (unsigned)((nt * 2 + u) * 1024 + lane * 16)) = fragment(t, u);
 }
 // tile nt of a 256x256 product from staged weight rows (row 0 of `w` is row 0 of the tile's half)
 __device__ __forceinline__ f32x16 train_tile(const __bf16 *w, int nt, int c, int h, const bf16x8 (&H)[16]) {
@@ -773,16 +778,25 @@ __device__ __forceinline__ f32x16 layer1_tile(const TrainLds &S, int nt, int c, 
         acc = __builtin_amdgcn_mfma_f32_32x32x2f32(S.w1[(2 * k + h) * kNH + 32 * nt + c], xf[k], acc, 0, 0, 0);
     return acc;
 }
+// Asynchronous copy of 128 rows of a weight, from row r0, into the LDS image (stage_half_async
+// with scalar row addresses, which take no vector registers)
 __device__ __forceinline__ void stage_train(const __bf16 *W, __bf16 *wl, int r0, int wv, int lane) {
-    stage_half_async<kTrainWaves>((const _Float16 *)W, (_Float16 *)wl, r0, wv, lane);
+    const __amdgpu_buffer_rsrc_t r = __builtin_amdgcn_make_buffer_rsrc((void *)W, (short)0, kNH * kNH * 2, 0x00020000);
+    if (lane < 32) {
+#pragma unroll 1   // (unrolled, its row addresses would take 64 scalar registers)
+        for (int i = 0; i < 128 / kTrainWaves; ++i) {
+            const int row = r0 + 128 / kTrainWaves * wv + i;
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (lds_void *)(wl + row * kRowPad), 16, lane * 16, row * kNH * 2, 0, 0);
+        }
+    }
 }
 
 __global__ __launch_bounds__(64 * kTrainWaves) void k_train_rows(TrainArgs a) {
     static_assert(kNL == 3 && kNIN == 14 && kNOUT == 4 && kNH == 256, "the layer sequence is written out");
     extern __shared__ __attribute__((aligned(16))) char smem[];
     TrainLds &S = *(TrainLds *)smem;
-    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6, h = lane >> 5, c = lane & 31;
-    const int row0 = (blockIdx.x * kTrainWaves + wv) * 32;
+    const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), h = lane >> 5, c = lane & 31;
+    const int row0 = ((int)blockIdx.x * kTrainWaves + wv) * 32;
     const bool active = row0 < a.rows;   // rows is a multiple of 32: whole waves
     const int row = min(row0, a.rows - 32) + c, rb = row0 / 32;
     __bf16 *wA = S.w, *wB = S.w + 128 * kRowPad;
@@ -810,7 +824,7 @@ __global__ __launch_bounds__(64 * kTrainWaves) void k_train_rows(TrainArgs a) {
         for (int r = 0; r < 16; ++r) v[r] = act(z[r]);
         tile_to_bf16(v, H1[2 * nt], H1[2 * nt + 1]);
         const f32x16 t = transpose_tile(H1[2 * nt], H1[2 * nt + 1], c, h);
-        if (active) store_fragments(a.h1, rb, nt, lane, t);
+        if (active) store_fragments(a.h1 + (size_t)rb * 32 * kNH, nt, lane, t);
     }
     wait_all_and_sync();
     auto forward_tile = [&](const float *bias, int nt, const bf16x8 (&In)[16], bf16x8 &lo, bf16x8 &hi) {
@@ -828,11 +842,11 @@ __global__ __launch_bounds__(64 * kTrainWaves) void k_train_rows(TrainArgs a) {
         }
         forward_tile(b2, nt, H1, H2[2 * nt], H2[2 * nt + 1]);
         const f32x16 t = transpose_tile(H2[2 * nt], H2[2 * nt + 1], c, h);
-        if (active) store_fragments(a.h2, rb, nt, lane, t);
+        if (active) store_fragments(a.h2 + (size_t)rb * 32 * kNH, nt, lane, t);
     }
     wait_all_and_sync();
     stage_train(a.w3t, wA, 128, wv, lane);
-    float4 dy;
+    float dyf[2];   // this lane's half of the output gradients
     float *part5 = a.part5 + (size_t)rb * kPart5;
     {
         bf16x8 H3[16];
@@ -884,23 +898,44 @@ __global__ __launch_bounds__(64 * kTrainWaves) void k_train_rows(TrainArgs a) {
             d[o] = 2.0f * e * inv;
             d[4] += e * e;
         }
-        dy = make_float4(d[0], d[1], d[2], d[3]);
-        if (h == 0) S.dy[wv][c] = dy;
+        dyf[0] = h ? d[1] : d[0];
+        dyf[1] = h ? d[3] : d[2];
+        if (h == 0) S.dy[wv][c] = make_float4(d[0], d[1], d[2], d[3]);
         __builtin_amdgcn_wave_barrier();
-        // dW5 = H3^T dY over this wave's rows, db5 and the loss
+        // dW5 = H3^T dY over this wave's rows on the bf16 matrix cores: dY is exactly the sum of
+        // three bf16 numbers, columns o, 4 + o and 8 + o of the right operand, whose products
+        // add up in FP32; db5 and the loss
+        bf16x8 dyb[2];
+#pragma unroll
+        for (int u = 0; u < 2; ++u)
+#pragma unroll
+            for (int j = 0; j < 8; ++j) {
+                const float v = ((const float *)&S.dy[wv][8 * (2 * u + (j >> 2)) + 4 * h + (j & 3)])[c & 3];
+                const __bf16 hi = (__bf16)v, mid = (__bf16)(v - (float)hi), lo = (__bf16)((v - (float)hi) - (float)mid);
+                dyb[u][j] = c < 4 ? hi : c < 8 ? mid : c < 12 ? lo : (__bf16)0.0f;
+            }
 #pragma unroll
         for (int nt = 0; nt < 8; ++nt) {
             const f32x16 t = transpose_tile(H3[2 * nt], H3[2 * nt + 1], c, h);
-            float g[4] = {0.f, 0.f, 0.f, 0.f};
+            f32x16 g;
 #pragma unroll
-            for (int r = 0; r < 16; ++r) {
-                const float4 e = S.dy[wv][8 * (r >> 2) + 4 * h + (r & 3)];
-                g[0] = fmaf(t[r], e.x, g[0]); g[1] = fmaf(t[r], e.y, g[1]);
-                g[2] = fmaf(t[r], e.z, g[2]); g[3] = fmaf(t[r], e.w, g[3]);
+            for (int r = 0; r < 16; ++r) g[r] = 0.0f;
+#pragma unroll
+            for (int u = 0; u < 2; ++u)
+                g = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, fragment(t, u)), dyb[u], g, 0, 0, 0);
+            float w[16];
+#pragma unroll
+            for (int r = 0; r < 16; ++r) {   // columns o + (4 + o) + (8 + o) (row_shl by 4 and by 8 lanes)
+                const int v = __float_as_int(g[r]);
+                w[r] = g[r] + (__int_as_float(__builtin_amdgcn_update_dpp(0, v, 0x104, 0xf, 0xf, true)) +
+                               __int_as_float(__builtin_amdgcn_update_dpp(0, v, 0x108, 0xf, 0xf, true)));
             }
+            if (active && c < 4) {
 #pragma unroll
-            for (int o = 0; o < 4; ++o) g[o] += __shfl_xor(g[o], 32, 64);
-            if (active && h == 0) *(float4 *)(part5 + 4 * (32 * nt + c)) = make_float4(g[0], g[1], g[2], g[3]);
+                for (int q = 0; q < 4; ++q)
+                    *(float4 *)(part5 + kNH * c + 32 * nt + 8 * q + 4 * h) =
+                        make_float4(w[4 * q], w[4 * q + 1], w[4 * q + 2], w[4 * q + 3]);
+            }
         }
 #pragma unroll
         for (int o = 0; o < 5; ++o) {
@@ -917,25 +952,25 @@ __global__ __launch_bounds__(64 * kTrainWaves) void k_train_rows(TrainArgs a) {
             stage_train(a.w3b, wA, 0, wv, lane);
         }
         const f32x16 z = train_tile(S.w, nt, c, h, H2);
+        f32x16 g;   // dY W5^T, an FMA chain over the outputs
+#pragma unroll
+        for (int r = 0; r < 16; ++r) g[r] = 0.0f;
+#pragma unroll
+        for (int k = 0; k < 2; ++k)
+            g = __builtin_amdgcn_mfma_f32_32x32x2f32(((const float *)&S.w5[32 * nt + c])[2 * k + h], dyf[k], g, 0, 0, 0);
         float v[16];
 #pragma unroll
-        for (int r = 0; r < 16; ++r) {
-            const int f = 32 * nt + 8 * (r >> 2) + 4 * h + (r & 3);
-            const float4 w = S.w5[f];
-            float g = 0.f;
-            g = fmaf(dy.x, w.x, g); g = fmaf(dy.y, w.y, g); g = fmaf(dy.z, w.z, g); g = fmaf(dy.w, w.w, g);
-            v[r] = g * dact(z[r] + b3[f]);
-        }
+        for (int r = 0; r < 16; ++r) v[r] = g[r] * dact(z[r] + b3[32 * nt + 8 * (r >> 2) + 4 * h + (r & 3)]);
         tile_to_bf16(v, D3[2 * nt], D3[2 * nt + 1]);
         const f32x16 t = transpose_tile(D3[2 * nt], D3[2 * nt + 1], c, h);
-        if (active) store_fragments(a.d3, rb, nt, lane, t);
+        if (active) store_fragments(a.d3 + (size_t)rb * 32 * kNH, nt, lane, t);
     }
     bf16x8 D2[16];
 #pragma unroll
     for (int half = 0; half < 2; ++half) {   // dZ2 = (dZ3 W3^T) act'(Z2), Z2 again
         wait_all_and_sync();
-        if (half == 1) stage_train(a.w3b + 128 * kNH, wA, 0, wv, lane);
-        stage_train(a.w2t + 128 * half * kNH, wB, 0, wv, lane);
+        if (half == 1) stage_train(a.w3b, wA - 128 * kRowPad, 128, wv, lane);
+        stage_train(a.w2t, wB - 128 * half * kRowPad, 128 * half, wv, lane);
         wait_all_and_sync();
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
@@ -946,22 +981,17 @@ __global__ __launch_bounds__(64 * kTrainWaves) void k_train_rows(TrainArgs a) {
             for (int r = 0; r < 16; ++r) v[r] = p[r] * dact(z[r] + b2[32 * nt + 8 * (r >> 2) + 4 * h + (r & 3)]);
             tile_to_bf16(v, D2[2 * nt], D2[2 * nt + 1]);
             const f32x16 t = transpose_tile(D2[2 * nt], D2[2 * nt + 1], c, h);
-            if (active) store_fragments(a.d2, rb, nt, lane, t);
+            if (active) store_fragments(a.d2 + (size_t)rb * 32 * kNH, nt, lane, t);
         }
     }
     wait_all_and_sync();
     stage_train(a.w2b, wA, 0, wv, lane);
     stage_train(a.w2b, wA, 128, wv, lane);
     wait_all_and_sync();
-    float g1[8][16];
-#pragma unroll
-    for (int nt = 0; nt < 8; ++nt) {   // dZ1 = (dZ2 W2^T) act'(Z1), Z1 again; FP32
-        const f32x16 p = train_tile(S.w, nt, c, h, D2), z = layer1_tile(S, nt, c, h, xf);
-#pragma unroll
-        for (int r = 0; r < 16; ++r) g1[nt][r] = p[r] * dact(z[r]);
-    }
-    // dW1 and db1 (input 14 is 1) over this wave's rows: dZ1 through LDS (rows of 132
-    // floats), two halves of the features, FP32 products on the matrix cores
+    // dZ1 = (dZ2 W2^T) act'(Z1), Z1 again, FP32; dW1 and db1 (input 14 is 1) over this wave's
+    // rows: dZ1 through LDS, 64 features at a time, FP32 products on the matrix cores.  The
+    // transposes go where the first half of the weight was; a row's float4 e is at
+    // e ^ (4 (row % 4) + row / 4 % 4), which spreads writes and reads over the banks.
     float xa[8];
     const int m = lane & 15, k4 = lane >> 4;
 #pragma unroll
@@ -969,29 +999,42 @@ __global__ __launch_bounds__(64 * kTrainWaves) void k_train_rows(TrainArgs a) {
         const float x = m < kNIN ? a.X[(size_t)(min(row0, a.rows - 32) + 4 * k + k4) * kXS + m] : m == kNIN ? 1.0f : 0.0f;
         xa[k] = active ? x : 0.0f;
     }
-    __syncthreads();
-    float *tw = (float *)S.w + wv * (32 * 132);
+    float *tw = (float *)S.w + wv * (32 * 64);
     f32x4 dw[16];
 #pragma unroll
     for (int half = 0; half < 2; ++half) {
+        float g1[4][16];
 #pragma unroll
-        for (int i = 0; i < 4; ++i)
+        for (int i = 0; i < 4; ++i) {
+            const f32x16 z = layer1_tile(S, 4 * half + i, c, h, xf), p = train_tile(S.w, 4 * half + i, c, h, D2);
 #pragma unroll
-            for (int q = 0; q < 4; ++q)
-                *(float4 *)(tw + c * 132 + 32 * i + 8 * q + 4 * h) =
-                    make_float4(g1[4 * half + i][4 * q], g1[4 * half + i][4 * q + 1], g1[4 * half + i][4 * q + 2], g1[4 * half + i][4 * q + 3]);
-        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-        __builtin_amdgcn_wave_barrier();
-#pragma unroll
-        for (int n = 0; n < 8; ++n) {
-            f32x4 acc = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-            for (int k = 0; k < 8; ++k)
-                acc = __builtin_amdgcn_mfma_f32_16x16x4f32(xa[k], tw[(4 * k + k4) * 132 + 16 * n + m], acc, 0, 0, 0);
-            dw[8 * half + n] = acc;
+            for (int r = 0; r < 16; ++r) g1[i][r] = p[r] * dact(z[r]);
         }
-        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-        __builtin_amdgcn_wave_barrier();
+        if (half == 0) __syncthreads();   // every wave is done with the first half
+#pragma unroll
+        for (int pair = 0; pair < 2; ++pair) {
+#pragma unroll
+            for (int i = 0; i < 2; ++i)
+#pragma unroll
+                for (int q = 0; q < 4; ++q) {
+                    const float (&g)[16] = g1[2 * pair + i];
+                    *(float4 *)(tw + c * 64 + 4 * ((8 * i + 2 * q + h) ^ (4 * (c & 3) + ((c >> 2) & 3)))) =
+                        make_float4(g[4 * q], g[4 * q + 1], g[4 * q + 2], g[4 * q + 3]);
+                }
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+            __builtin_amdgcn_wave_barrier();
+#pragma unroll
+            for (int n = 0; n < 4; ++n) {
+                f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+                for (int k = 0; k < 8; ++k)   // row 4 k + k4, feature 16 n + m
+                    acc = __builtin_amdgcn_mfma_f32_16x16x4f32(
+                        xa[k], tw[(4 * k + k4) * 64 + 4 * ((4 * n + (m >> 2)) ^ (4 * k4 + (k & 3))) + (m & 3)], acc, 0, 0, 0);
+                dw[8 * half + 4 * pair + n] = acc;
+            }
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+            __builtin_amdgcn_wave_barrier();
+        }
     }
     __syncthreads();
     float *ws = (float *)S.w;   // [wave][16][256]
@@ -1072,39 +1115,50 @@ __global__ __launch_bounds__(256) void k_train_dw(const __bf16 *h1, const __bf16
     }
 }
 
-// Gradient e (and, behind the parameters, the loss) = the sum of its partials; 64
-// values per workgroup, 16 threads each.  Parameters: W1, b1 (partials of
-// workgroups), W2, b2, W3, b3 (of row ranges), W5, b5 (of waves).
-__global__ __launch_bounds__(1024) void k_train_reduce(const float *__restrict__ part1, int nwg, const float *__restrict__ part,
-                                                       const float *__restrict__ partb, int ns, const float *__restrict__ part5,
-                                                       int nwave, float *__restrict__ g, float *__restrict__ loss) {
-    __shared__ float s[16][64];
-    const int x = threadIdx.x & 63, k0 = threadIdx.x >> 6;
-    constexpr int L1 = 15 * kNH, LH = kNH * kNH + kNH, N = L1 + kNG * LH + kNH * kNOUT + kNOUT;
-    const int e = blockIdx.x * 64 + x;
+// Gradient e (and, behind the parameters, the loss) = the sum of its partials, with 4 threads
+// per value (16 for the waves' partials, of which there are 8 times as many as of workgroups),
+// up to 16 loads in flight each: 24 us with 16 threads per value everywhere, 18 so.
+// Parameters: W1, b1 (partials of workgroups), W2, b2, W3, b3 (of row ranges), W5, b5, loss (of waves).
+constexpr int kRedL1 = 15 * kNH, kRedLH = kNH * kNH + kNH, kRed5 = kRedL1 + kNG * kRedLH, kRedN = kRed5 + kNH * kNOUT + kNOUT;
+__global__ __launch_bounds__(256) void k_train_reduce(const float *__restrict__ part1, int nwg, const float *__restrict__ part,
+                                                      const float *__restrict__ partb, int ns, const float *__restrict__ part5,
+                                                      int nwave, float *__restrict__ g, float *__restrict__ loss) {
+    static_assert(kRed5 % 64 == 0, "a workgroup's values have one kind of partials");
+    __shared__ float s[256];
+    const bool waves = blockIdx.x >= kRed5 / 64;
+    const int E = waves ? 16 : 64, S = 256 / E, x = threadIdx.x % E, k0 = threadIdx.x / E;
+    const int e = waves ? kRed5 + ((int)blockIdx.x - kRed5 / 64) * 16 + x : (int)blockIdx.x * 64 + x;
     const float *p = part1 + e;
     int count = nwg;
-    size_t stride = L1;
-    if (e >= L1 + kNG * LH) {
-        p = part5 + (e - L1 - kNG * LH);
+    size_t stride = kRedL1;
+    if (waves) {
+        const int i = e - kRed5;   // W5 as [output][256] there
+        p = part5 + (i < kNH * kNOUT ? (i % kNOUT) * kNH + i / kNOUT : i);
         count = nwave;
         stride = kPart5;
-    } else if (e >= L1) {
-        const int L = (e - L1) / LH, i = (e - L1) % LH;
+    } else if (e >= kRedL1) {
+        const int L = (e - kRedL1) / kRedLH, i = (e - kRedL1) % kRedLH;
         count = ns;
         stride = i < kNH * kNH ? kNH * kNH : kNH;
         p = (i < kNH * kNH ? part + i : partb + (i - kNH * kNH)) + (size_t)L * ns * stride;
     }
     float v = 0.f;
-    if (e <= N)
-#pragma unroll 4
-        for (int k = k0; k < count; k += 16) v += p[k * stride];
-    s[k0][x] = v;
-    __syncthreads();
-    if (k0 == 0 && e <= N) {
+    if (e <= kRedN) {
+        int k = k0;
+        for (; k + 15 * S < count; k += 16 * S) {
+            float y[16];
 #pragma unroll
-        for (int k = 1; k < 16; ++k) v += s[k][x];
-        if (e < N) g[e] = v;
+            for (int i = 0; i < 16; ++i) y[i] = p[(k + i * S) * stride];
+#pragma unroll
+            for (int i = 0; i < 16; ++i) v += y[i];
+        }
+        for (; k < count; k += S) v += p[k * stride];
+    }
+    s[threadIdx.x] = v;
+    __syncthreads();
+    if (k0 == 0 && e <= kRedN) {
+        for (int k = 1; k < S; ++k) v += s[k * E + x];
+        if (e < kRedN) g[e] = v;
         else *loss = v;
     }
 }
@@ -1253,8 +1307,8 @@ hipError_t train_pass(TrainArgs a, float *scratch, float *g, float *loss, hipStr
     if ((e = hipGetLastError()) != hipSuccess) return e;
     hipLaunchKernelGGL(k_train_dw, dim3(ns, 4, 2), dim3(256), 0, st, a.h1, a.d2, a.h2, a.d3, nrb, part, partb);
     if ((e = hipGetLastError()) != hipSuccess) return e;
-    constexpr int N = 15 * kNH + kNG * (kNH * kNH + kNH) + kNH * kNOUT + kNOUT + 1;
-    hipLaunchKernelGGL(k_train_reduce, dim3((N + 63) / 64), dim3(1024), 0, st, a.part1, nwg, part, partb, ns, a.part5, nrb, g, loss);
+    hipLaunchKernelGGL(k_train_reduce, dim3(kRed5 / 64 + (kRedN + 1 - kRed5 + 15) / 16), dim3(256), 0, st, a.part1, nwg, part, partb, ns,
+                       a.part5, nrb, g, loss);
     return hipGetLastError();
 }
 hipError_t mlp_infer(const InferSet *sets, int nsets, int ntiles, const FusedWeights &fw, const TargetNorm &tn,
