@@ -113,7 +113,7 @@ struct atmo_surrogate {
     hipStream_t st = nullptr;
     Buf p, g, m, v, wb, wt;   // FP32 params/grads/Adam; bf16 W and W^T of layers 2..kNL
     Buf fz;                   // fused-inference weights (prep_fused)
-    Buf iset;                 // InferSet array of the last fused launch
+    Buf iset, imu;            // InferSet array and row coordinates of the last fused launch
     TargetNorm tn{{0, 0, 0}, {1, 1, 1}, 1e-6f};
     int adam_t = 0;
     int exact_orders = 1;     // orders computed by the plain passes; the network predicts the rest
@@ -494,9 +494,16 @@ atmo_status atmo_surrogate_precompute(atmo_surrogate *s, const atmo_params *sets
     {
         std::vector<InferSet> hs(nsets);
         const int rpb = fused_rows_per_block();
-        int tiles = 0;
+        int tiles = 0, maxrows = 0;
+        size_t rows = 0;
+        for (int i = 0; i < nsets; ++i) rows += (size_t)sets[i].RES_R * sets[i].RES_MU;
+        HIPCHK(s->imu.ensure(rows * sizeof(float)));
+        float *mu = s->imu.as<float>();
         for (int i = 0; i < nsets; ++i) {
             hs[i].fs = feat_set(sets[i]);
+            hs[i].mu = mu;
+            mu += hs[i].fs.RR * hs[i].fs.RMU;
+            maxrows = std::max(maxrows, hs[i].fs.RR * hs[i].fs.RMU);
             hs[i].tile0 = tiles;
             hs[i].S = (float4 *)out[i].inscatter;
             hs[i].E = out[i].irradiance;
@@ -504,7 +511,7 @@ atmo_status atmo_surrogate_precompute(atmo_surrogate *s, const atmo_params *sets
         }
         HIPCHK(s->iset.ensure(hs.size() * sizeof(InferSet)));
         HIPCHK(hipMemcpyAsync(s->iset.p, hs.data(), hs.size() * sizeof(InferSet), hipMemcpyHostToDevice, s->st));
-        HIPCHK(mlp_infer((const InferSet *)s->iset.p, nsets, tiles, fused_weights(s), s->tn, s->st));
+        HIPCHK(mlp_infer((const InferSet *)s->iset.p, nsets, tiles, maxrows, fused_weights(s), s->tn, s->st));
         HIPCHK(hipStreamSynchronize(s->st));  // hs must outlive the copy
     }
     HIPCHK(hipEventRecord(ev[2], s->st));

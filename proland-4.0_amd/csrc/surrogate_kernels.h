@@ -44,13 +44,14 @@ struct FusedWeights {
     const float *b5;             // [4]
 };
 
-// One set of a fused inference launch: its features, its first workgroup
+// One set of a fused inference launch: its features, its first tile
 // (tiles of fused_rows_per_block() rows: S texels, then E texels) and outputs.
 struct InferSet {
     FeatSet fs;
     int tile0, pad[3];
     float4 *S;
     float *E;
+    float *mu;   // [RR * RMU] row coordinates, written by mlp_infer
 };
 
 hipError_t gemm_act(const __bf16 *A, const __bf16 *B, int M, int N, int K, const float *bias, __bf16 *hout, hipStream_t st);
@@ -78,10 +79,10 @@ hipError_t prep_fused(const float *W1, const float *b1, const float *W5, const f
                       size_t bstride, __bf16 *a1h, __bf16 *a1l, _Float16 *wt, _Float16 *a5h, _Float16 *a5l,
                       float *bh, hipStream_t st);
 // Fused inference of every S and E texel of a batch of sets (device array
-// `sets`, tile0 ascending, ntiles workgroups in all): adds the predicted
-// higher orders to S.rgb and E.
+// `sets`, tile0 ascending, ntiles tiles in all, at most maxrows RR x RMU rows a set):
+// adds the predicted higher orders to S.rgb and E.
 int fused_rows_per_block();
-hipError_t mlp_infer(const InferSet *sets, int nsets, int ntiles, const FusedWeights &fw, const TargetNorm &tn,
+hipError_t mlp_infer(const InferSet *sets, int nsets, int ntiles, int maxrows, const FusedWeights &fw, const TargetNorm &tn,
                      hipStream_t st);
 hipError_t gather(const float *Xa, const float *Ta, size_t n, int B, unsigned long long seed,
                   float *X, float *Tg, hipStream_t st);

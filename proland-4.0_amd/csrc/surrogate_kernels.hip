@@ -175,6 +175,40 @@ __global__ __launch_bounds__(256) void k_to_bf16(const float *__restrict__ W, __
 // ---------------------------------------------------------------------------
 constexpr float kHorizonGap = 0.25f;
 
+// The mu coordinate of row y of layer l.
+__device__ __forceinline__ float row_coordinate(const FeatSet &fs, int l, int y) {
+    // mu rows: the row's ray length d (getMuMuSNu, common.glsl:175-190, with
+    // the layer radius of setLayer, PreprocessAtmo.cpp:255-271) on one log
+    // scale for the whole set, from 1 m (the shortest ray of the table: up
+    // from the highest layer) to 2 sqrt(Rt^2 - Rg^2) (longer than any ray),
+    // the ground-ray half in [-1, -kHorizonGap] and the sky half in
+    // [kHorizonGap, 1].  The table rows are linear in d up to a clamp at the
+    // shortest ray of a layer (10 m down from the lowest layer), where the
+    // inscatter, proportional to d, drops by 10-100x from one row to the
+    // next; on a log scale common to all layers that drop is the same slope
+    // everywhere, and the gap separates the straight-down and straight-up
+    // rows, which are neighbours in the table only.
+    const int half = fs.RMU / 2;
+    const double Rg = fs.Rg, Rt = fs.Rt, Rg2 = Rg * Rg;
+    double rl = (double)l / (fs.RR - 1);
+    rl = sqrt(Rg2 + rl * rl * (Rt * Rt - Rg2)) + (l == 0 ? 0.01 : (l == fs.RR - 1 ? -0.001 : 0.0));
+    const double rho = sqrt(fmax(rl * rl - Rg2, 0.0)), H = sqrt(Rt * Rt - Rg2);
+    double dmin, dmax, d;
+    if (y < half) {
+        dmin = rl - Rg;
+        dmax = 0.999 * rho;
+        d = (1.0 - (double)y / (half - 1)) * rho;
+    } else {
+        dmin = Rt - rl;
+        dmax = 0.999 * (rho + H);
+        d = (double)(y - half) / (half - 1) * (rho + H);
+    }
+    d = fmin(fmax(d, dmin), dmax);
+    const double dlo = 1e-3, dhi = 2.0 * H;   // in the parameters' length unit (km)
+    const float t = (float)fmin(fmax(log(d / dlo) / log(dhi / dlo), 0.0), 1.0);
+    return y < half ? fmaf(-(1.f - kHorizonGap), t, -kHorizonGap) : fmaf(1.f - kHorizonGap, t, kHorizonGap);
+}
+
 // Resolution-independent texel coordinates in [-1, 1] (the arguments of
 // getMuMuSNu, common.glsl:175-201), the 7 normalised atmosphere features, and
 // the exactly computed orders' value at the texel (ex: S.rgb of an inscatter
@@ -183,7 +217,9 @@ constexpr float kHorizonGap = 0.25f;
 // ones closely (where the view ray meets the ground, where the sun sets), so
 // the network learns them relative to what the exact part already resolves.
 // E texels use the irradiance coordinates in slots 0 and 2 and -2 in 1 and 3.
-__device__ __forceinline__ void texel_features(const FeatSet &fs, unsigned code, const float *ex, float *x) {
+// mu: row_coordinate of every (layer, row), or nullptr.
+__device__ __forceinline__ void texel_features(const FeatSet &fs, unsigned code, const float *ex, float *x,
+                                               const float *mu = nullptr) {
     if (code & 0x80000000u) {
         const unsigned t = code & 0x7fffffffu;
         const int i = t % fs.SW, j = t / fs.SW;
@@ -194,37 +230,8 @@ __device__ __forceinline__ void texel_features(const FeatSet &fs, unsigned code,
     } else {
         const int W4 = fs.RMUS * fs.RNU;
         const int xx = code % W4, y = (code / W4) % fs.RMU, l = code / (W4 * fs.RMU);
-        // mu rows: the row's ray length d (getMuMuSNu, common.glsl:175-190, with
-        // the layer radius of setLayer, PreprocessAtmo.cpp:255-271) on one log
-        // scale for the whole set, from 1 m (the shortest ray of the table: up
-        // from the highest layer) to 2 sqrt(Rt^2 - Rg^2) (longer than any ray),
-        // the ground-ray half in [-1, -kHorizonGap] and the sky half in
-        // [kHorizonGap, 1].  The table rows are linear in d up to a clamp at the
-        // shortest ray of a layer (10 m down from the lowest layer), where the
-        // inscatter, proportional to d, drops by 10-100x from one row to the
-        // next; on a log scale common to all layers that drop is the same slope
-        // everywhere, and the gap separates the straight-down and straight-up
-        // rows, which are neighbours in the table only.
-        const int half = fs.RMU / 2;
-        const double Rg = fs.Rg, Rt = fs.Rt, Rg2 = Rg * Rg;
-        double rl = (double)l / (fs.RR - 1);
-        rl = sqrt(Rg2 + rl * rl * (Rt * Rt - Rg2)) + (l == 0 ? 0.01 : (l == fs.RR - 1 ? -0.001 : 0.0));
-        const double rho = sqrt(fmax(rl * rl - Rg2, 0.0)), H = sqrt(Rt * Rt - Rg2);
-        double dmin, dmax, d;
-        if (y < half) {
-            dmin = rl - Rg;
-            dmax = 0.999 * rho;
-            d = (1.0 - (double)y / (half - 1)) * rho;
-        } else {
-            dmin = Rt - rl;
-            dmax = 0.999 * (rho + H);
-            d = (double)(y - half) / (half - 1) * (rho + H);
-        }
-        d = fmin(fmax(d, dmin), dmax);
-        const double dlo = 1e-3, dhi = 2.0 * H;   // in the parameters' length unit (km)
-        const float t = (float)fmin(fmax(log(d / dlo) / log(dhi / dlo), 0.0), 1.0);
         x[0] = 2.f * l / (fs.RR - 1) - 1.f;
-        x[1] = y < half ? fmaf(-(1.f - kHorizonGap), t, -kHorizonGap) : fmaf(1.f - kHorizonGap, t, kHorizonGap);
+        x[1] = mu ? mu[code / W4] : row_coordinate(fs, l, y);
         x[2] = 2.f * (xx % fs.RMUS) / (fs.RMUS - 1) - 1.f;
         x[3] = 2.f * (xx / fs.RMUS) / (fs.RNU - 1) - 1.f;
     }
@@ -443,19 +450,14 @@ __device__ __forceinline__ unsigned act_pk(float a, float b) {
     return __builtin_bit_cast(unsigned, z * (t * t * u));
 }
 
-// D tile (features x 32 rows) -> act(D + bias) as the FP16 B operands of k
-// blocks 2nt (lo) and 2nt + 1 (hi).  bias: the tile's 32 biases or nullptr.
-__device__ __forceinline__ void tile_to_b(const f32x16 &acc, const float *bias, int h, f16x8 &lo,
-                                          f16x8 &hi) {
+// D tile (features x 32 rows) -> act(D) as the FP16 B operands of k blocks 2nt (lo)
+// and 2nt + 1 (hi).
+__device__ __forceinline__ void tile_to_b(const f32x16 &acc, int h, f16x8 &lo, f16x8 &hi) {
     unsigned P[4][2];
 #pragma unroll
     for (int q = 0; q < 4; ++q) {
-        float z[4];
-#pragma unroll
-        for (int t = 0; t < 4; ++t)   // (no "+ 0.0f" without a bias: it would be kept, -0 + 0 = +0)
-            z[t] = bias ? acc[4 * q + t] + bias[8 * q + 4 * h + t] : acc[4 * q + t];
-        P[q][0] = act_pk(z[0], z[1]);
-        P[q][1] = act_pk(z[2], z[3]);
+        P[q][0] = act_pk(acc[4 * q], acc[4 * q + 1]);
+        P[q][1] = act_pk(acc[4 * q + 2], acc[4 * q + 3]);
     }
     // lane h = 0 keeps features 0-3, 16-19 and needs 4-7, 20-23 from lane l^32;
     // lane h = 1 keeps 12-15, 28-31 and needs 8-11, 24-27.  v_permlane32_swap
@@ -479,60 +481,72 @@ __device__ __forceinline__ void tile_to_b(const f32x16 &acc, const float *bias, 
 
 typedef __attribute__((address_space(3))) void lds_void;
 
-// Asynchronous copy of rows [r0, r0 + 128) of a [256][256] FP16 weight into
-// the padded LDS image (global_load_lds_dwordx4: each active lane moves 16 B
+// Asynchronous copy of 128 rows of 256 FP16 weights into a
+// padded LDS image (global_load_lds_dwordx4: each active lane moves 16 B
 // straight into LDS; one row = 32 lanes).  Each of the NW waves moves 128/NW rows.
 template <int NW>
-__device__ __forceinline__ void stage_half_async(const _Float16 *W, _Float16 *wl, int r0, int wv, int lane) {
+__device__ __forceinline__ void stage_half_async(const _Float16 *W, _Float16 *wl, int wv, int lane) {
     constexpr int RPWV = 128 / NW;
     if (lane < 32) {
 #pragma unroll 8
         for (int r = 0; r < RPWV; ++r) {
-            const int row = r0 + RPWV * wv + r;
+            const int row = RPWV * wv + r;
             __builtin_amdgcn_global_load_lds((const void *)(W + row * kNH + lane * 8),
                                              (lds_void *)(wl + row * kRowPad), 16, 0, 0);
         }
     }
 }
 
-// Output tiles nt0 .. nt0+3 of one hidden layer from the staged weight rows,
-// software-pipelined: the matrix-core products of tile nt run while the
-// vector units apply act and relayout tile nt - 1.  The accumulators start at
-// the tile's biases (element 4q + t of lane (c, h) is feature 8q + 4h + t).
-template <int RBW>
-__device__ __forceinline__ void tile_mfma(const _Float16 *wl, const float *bias, int nt, int c, int h,
-                                          const f16x8 (&H)[RBW][16], f32x16 (&acc)[RBW]) {
-    const float4 *bq = (const float4 *)(bias + 32 * nt + 4 * h);
-#pragma unroll
-    for (int q = 0; q < 4; ++q) {
-        const float4 b = bq[2 * q];
-#pragma unroll
-        for (int rb = 0; rb < RBW; ++rb) {
-            acc[rb][4 * q] = b.x; acc[rb][4 * q + 1] = b.y; acc[rb][4 * q + 2] = b.z; acc[rb][4 * q + 3] = b.w;
-        }
-    }
-    const _Float16 *wrow = wl + (32 * nt + c) * kRowPad + 8 * h;
-#pragma unroll
-    for (int kb = 0; kb < 16; ++kb) {
-        const f16x8 a = *(const f16x8 *)(wrow + 16 * kb);
-#pragma unroll
-        for (int rb = 0; rb < RBW; ++rb)
-            acc[rb] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a, H[rb][kb], acc[rb], 0, 0, 0);
-    }
-}
+// Output tiles nt0 .. nt0+3 of one hidden layer from the staged weight rows.  The
+// weight operands are read kAhead products ahead and tile nt - 1's activations are
+// dealt over tile nt's products (the group barriers: one product, one or two reads, a
+// few vector instructions).  The first product's addend is the tile's biases (element
+// 4q + t of lane (c, h) is feature 8q + 4h + t).
+constexpr int kAhead = 8;
 
-template <int RBW>
+#define ATMO_SG_PRODUCT(READS, VALU)                        \
+    __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);     \
+    __builtin_amdgcn_sched_group_barrier(0x100, READS, 0); \
+    __builtin_amdgcn_sched_group_barrier(0x002, VALU, 0)
+
 __device__ __forceinline__ void hidden_half(const _Float16 *wl, const float *bias, int nt0, int c, int h,
-                                            const f16x8 (&H)[RBW][16], f16x8 (&Hn)[RBW][16]) {
-    f32x16 acc[2][RBW];
-    tile_mfma<RBW>(wl, bias, nt0, c, h, H, acc[0]);
+                                            const f16x8 (&H)[16], f16x8 (&Hn)[16]) {
+    f32x16 acc[2], bq[2];
+    f16x8 a[kAhead];
+    const _Float16 *wrow = wl + c * kRowPad + 8 * h;
+    auto bias_tile = [&](int i) {
+        const float4 *p = (const float4 *)(bias + 32 * (nt0 + i) + 4 * h);
 #pragma unroll
-    for (int i = 1; i <= 4; ++i) {
-        if (i < 4) tile_mfma<RBW>(wl, bias, nt0 + i, c, h, H, acc[i & 1]);
-        const int nt = nt0 + i - 1;
+        for (int q = 0; q < 4; ++q) {
+            const float4 v = p[2 * q];
+            bq[i & 1][4 * q] = v.x; bq[i & 1][4 * q + 1] = v.y; bq[i & 1][4 * q + 2] = v.z; bq[i & 1][4 * q + 3] = v.w;
+        }
+    };
+    auto read = [&](int st) { a[st % kAhead] = *(const f16x8 *)(wrow + 32 * (st / 16) * kRowPad + 16 * (st % 16)); };
+    bias_tile(0);
 #pragma unroll
-        for (int rb = 0; rb < RBW; ++rb)
-            tile_to_b(acc[(i - 1) & 1][rb], nullptr, h, Hn[rb][2 * nt], Hn[rb][2 * nt + 1]);
+    for (int st = 0; st < kAhead; ++st) read(st);
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int i = 0; i < 5; ++i) {
+        if (i < 4) {
+#pragma unroll
+            for (int kb = 0; kb < 16; ++kb) {
+                const int st = 16 * i + kb;
+                acc[i & 1] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a[st % kAhead], H[kb], kb == 0 ? bq[i & 1] : acc[i & 1], 0, 0, 0);
+                if (st + kAhead < 64) read(st + kAhead);
+            }
+            if (i < 3) bias_tile(i + 1);
+        }
+        if (i > 0) {
+            const int nt = nt0 + i - 1;
+            tile_to_b(acc[(i - 1) & 1], h, Hn[2 * nt], Hn[2 * nt + 1]);
+        }
+        ATMO_SG_PRODUCT(1, 0); ATMO_SG_PRODUCT(1, 0); ATMO_SG_PRODUCT(1, 4); ATMO_SG_PRODUCT(1, 4);
+        ATMO_SG_PRODUCT(1, 4); ATMO_SG_PRODUCT(1, 4); ATMO_SG_PRODUCT(1, 4); ATMO_SG_PRODUCT(1, 4);
+        ATMO_SG_PRODUCT(1, 4); ATMO_SG_PRODUCT(1, 4); ATMO_SG_PRODUCT(1, 4); ATMO_SG_PRODUCT(1, 4);
+        ATMO_SG_PRODUCT(2, 4); ATMO_SG_PRODUCT(2, 4); ATMO_SG_PRODUCT(2, 4); ATMO_SG_PRODUCT(2, 4);
+        __builtin_amdgcn_sched_barrier(0);
     }
 }
 
@@ -541,131 +555,139 @@ __device__ __forceinline__ void wait_all_and_sync() {
     __syncthreads();
 }
 
-// LDS image: rows 0..127 of the current weight ("A") and rows 128..255 ("B"),
-// 528-byte rows.  While one half is read by the matrix cores the other is
-// being refilled for the next step, so every weight load after the first
-// overlaps compute.  Layer 1's weights (16 KB) sit in B before layer 2's
-// second half arrives; layer 5's (4 KB) in A after layer 4's first half.
-template <int RBW, int NW>
-__global__ __launch_bounds__(64 * NW) void k_mlp_infer(const InferSet *__restrict__ sets, int nsets,
+// row_coordinate of every layer and row of every set, into its mu table.
+__global__ __launch_bounds__(256) void k_infer_rows(const InferSet *__restrict__ sets) {
+    const InferSet &is = sets[blockIdx.y];
+    const int t = blockIdx.x * 256 + threadIdx.x;
+    if (t < is.fs.RR * is.fs.RMU) is.mu[t] = row_coordinate(is.fs, t / is.fs.RMU, t % is.fs.RMU);
+}
+
+// A workgroup stays on its CU and walks the tiles of 256 rows (blockIdx.x, + gridDim.x,
+// ...): the weights of layers 1 and 5 and the biases are staged once, a tile's exact
+// values and the first half of its layer 2 are loaded during the tile before.  LDS:
+// rows 0..127 of the current weight in wA, rows 128..255 in wB (528-byte rows), while
+// one half is read by the matrix cores the other is refilled for the next step; two
+// arrays, not one, so that the compiler does not wait for the one before it reads the
+// other.  24 sets of 32x128x32x8 (6.8 TFLOP): a workgroup per tile, with its own
+// search, staging, FP64 row coordinates and second read of S, spent 3.0 of 8.2 ms
+// outside the hidden layers; the whole call, exact part included, takes 10.15 ms
+// against 11.1.  64 rows per wave and 4 waves (half the LDS reads) took 12.4.
+template <int NW>
+__global__ __launch_bounds__(64 * NW) void k_mlp_infer(const InferSet *__restrict__ sets, int nsets, int ntiles,
                                                        FusedWeights fw, TargetNorm tn) {
-    extern __shared__ __attribute__((aligned(16))) _Float16 wl[];   // [256][kRowPad] (layer 1: bf16 bits)
+    static_assert(kNG == 2, "the layers alternate between two register arrays");
+    __shared__ __attribute__((aligned(16))) _Float16 wA[128 * kRowPad], wB[128 * kRowPad];
+    __shared__ __attribute__((aligned(16))) __bf16 w1[2 * kNH * 16];           // hi, lo: [256][16]
+    __shared__ __attribute__((aligned(16))) _Float16 w5[2 * kNOUT * kRowPad];   // hi rows, lo rows
     __shared__ float bs[kNG][kNH];
     const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6, h = lane >> 5, c = lane & 31;
-    // the set of this workgroup: last set whose first tile <= blockIdx.x
-    int lo = 0, hi = nsets - 1;
-    while (lo < hi) {
-        const int mid = (lo + hi + 1) >> 1;
-        if (sets[mid].tile0 <= (int)blockIdx.x) lo = mid; else hi = mid - 1;
-    }
-    const InferSet &is = sets[lo];
-    const FeatSet fs = is.fs;
-    const int row0 = 0, n = fs.n4 + fs.SW * fs.SH;
-    float4 *__restrict__ S = is.S;
-    float *__restrict__ E = is.E;
-    const int rw = ((int)blockIdx.x - is.tile0) * (32 * RBW * NW) + wv * (32 * RBW);    // first row of this wave
-    _Float16 *wB = wl + 128 * kRowPad;
-
-    // layer-1 weights (hi then lo, [256][16]) into B, hidden biases; layer 2's first half -> A
     for (int i = threadIdx.x; i < 1024; i += 64 * NW)
-        *(uint4 *)(wB + i * 8) = *(const uint4 *)((i < 512 ? fw.a1h : fw.a1l) + (i & 511) * 8);
+        *(uint4 *)(w1 + i * 8) = *(const uint4 *)((i < 512 ? fw.a1h : fw.a1l) + (i & 511) * 8);
+    for (int i = threadIdx.x; i < 256; i += 64 * NW)
+        *(uint4 *)(w5 + (i >> 5) * kRowPad + (i & 31) * 8) = *(const uint4 *)((i < 128 ? fw.a5h : fw.a5l) + (i & 127) * 8);
     for (int i = threadIdx.x; i < kNG * kNH; i += 64 * NW) (&bs[0][0])[i] = fw.bh[i];
     __syncthreads();
-    stage_half_async<NW>(fw.wt, wl, 0, wv, lane);
+    stage_half_async<NW>(fw.wt, wA, wv, lane);
 
-    f16x8 H[RBW][16];
-    // (1) features and layer 1
-#pragma unroll
-    for (int rb = 0; rb < RBW; ++rb) {
-        const int r = min(rw + 32 * rb + c, n - 1) + row0;
-        const unsigned code = r < fs.n4 ? (unsigned)r : (0x80000000u | (unsigned)(r - fs.n4));
-        float ex[3], x[kNIN];
-        exact_value(fs, code, is.S, is.E, ex);   // the exact part, before this kernel adds to it
-        texel_features(fs, code, ex, x);
-        float xe[16];
-#pragma unroll
-        for (int k = 0; k < 16; ++k) xe[k] = k < kNIN ? x[k] : (k == kNIN ? 1.0f : 0.0f);
-        bf16x8 xh, xl;
-        const unsigned hm = 0u - (unsigned)h;  // all ones on lanes 32..63
-#pragma unroll
-        for (int i = 0; i < 8; ++i) {
-            // lane half h takes input columns 8h .. 8h+7 (bit select, no indexed array)
-            const float v = __uint_as_float((__float_as_uint(xe[i]) & ~hm) | (__float_as_uint(xe[8 + i]) & hm));
-            const __bf16 vh = (__bf16)v;
-            xh[i] = vh;
-            xl[i] = (__bf16)(v - (float)vh);
-        }
-#pragma unroll
-        for (int nt = 0; nt < 8; ++nt) {
-            const bf16x8 ah = *(const bf16x8 *)(wB + (32 * nt + c) * 16 + 8 * h);   // bf16 bits
-            const bf16x8 al = *(const bf16x8 *)(wB + 4096 + (32 * nt + c) * 16 + 8 * h);
-            f32x16 acc;
-#pragma unroll
-            for (int j = 0; j < 16; ++j) acc[j] = 0.0f;
-            acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ah, xh, acc, 0, 0, 0);
-            acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(al, xh, acc, 0, 0, 0);
-            acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ah, xl, acc, 0, 0, 0);
-            tile_to_b(acc, nullptr, h, H[rb][2 * nt], H[rb][2 * nt + 1]);
-        }
+    int tile = blockIdx.x, si = 0;   // si: the last set whose first tile is at most `tile`
+    for (int hi = nsets - 1; si < hi;) {
+        const int mid = (si + hi + 1) >> 1;
+        if (sets[mid].tile0 <= tile) si = mid; else hi = mid - 1;
     }
-    // (2) hidden layers 2..kNL
-#pragma unroll 1
-    for (int L = 0; L < kNG; ++L) {
-        const _Float16 *W = fw.wt + (size_t)L * kNH * kNH;
-        wait_all_and_sync();                          // A holds rows 0..127; B is free
-        stage_half_async<NW>(W, wl, 128, wv, lane);   // B <- rows 128..255
-        f16x8 Hn[RBW][16];
-        hidden_half<RBW>(wl, bs[L], 0, c, h, H, Hn);
-        wait_all_and_sync();                          // B holds rows 128..255; A is free
-        if (L < kNG - 1) {
-            stage_half_async<NW>(W + (size_t)kNH * kNH, wl, 0, wv, lane);   // A <- next layer's rows 0..127
-        } else if (threadIdx.x < 256) {               // A <- layer 5 (hi then lo, [4][256])
-            *(uint4 *)(wl + threadIdx.x * 8) = *(const uint4 *)((threadIdx.x < 128 ? fw.a5h : fw.a5l) +
-                                                               (threadIdx.x & 127) * 8);
+    // this lane's row of a tile, its code and the exact part there, before this kernel adds to it
+    auto row_of = [&](const InferSet &is, int tl) { return (tl - is.tile0) * (32 * NW) + wv * 32 + c; };
+    auto code_of = [&](const FeatSet &fs, int r) {
+        r = min(r, fs.n4 + fs.SW * fs.SH - 1);
+        return r < fs.n4 ? (unsigned)r : (0x80000000u | (unsigned)(r - fs.n4));
+    };
+    auto exact_of = [&](const InferSet &is, int tl) {
+        const unsigned code = code_of(is.fs, row_of(is, tl));
+        if (!(code & 0x80000000u)) return is.S[code];
+        const float *e = is.E + 3 * (size_t)(code & 0x7fffffffu);
+        return make_float4(e[0], e[1], e[2], 0.f);
+    };
+    float4 ex = exact_of(sets[si], tile);
+    for (;;) {
+        const InferSet &is = sets[si];
+        const int next = tile + (int)gridDim.x;
+        const bool more = next < ntiles;
+        int sn = si;
+        while (more && sn + 1 < nsets && sets[sn + 1].tile0 <= next) ++sn;
+        f16x8 H[16], Hn[16];
+        // (1) features and layer 1
+        {
+            const FeatSet fs = is.fs;
+            const float e3[3] = {ex.x, ex.y, ex.z};
+            float x[kNIN];
+            texel_features(fs, code_of(fs, row_of(is, tile)), e3, x, is.mu);
+            float xe[16];
+#pragma unroll
+            for (int k = 0; k < 16; ++k) xe[k] = k < kNIN ? x[k] : (k == kNIN ? 1.0f : 0.0f);
+            bf16x8 xh, xl;
+            const unsigned hm = 0u - (unsigned)h;  // all ones on lanes 32..63
+#pragma unroll
+            for (int i = 0; i < 8; ++i) {
+                // lane half h takes input columns 8h .. 8h+7 (bit select, no indexed array)
+                const float v = __uint_as_float((__float_as_uint(xe[i]) & ~hm) | (__float_as_uint(xe[8 + i]) & hm));
+                const __bf16 vh = (__bf16)v;
+                xh[i] = vh;
+                xl[i] = (__bf16)(v - (float)vh);
+            }
+#pragma unroll
+            for (int nt = 0; nt < 8; ++nt) {
+                const bf16x8 ah = *(const bf16x8 *)(w1 + (32 * nt + c) * 16 + 8 * h);
+                const bf16x8 al = *(const bf16x8 *)(w1 + kNH * 16 + (32 * nt + c) * 16 + 8 * h);
+                f32x16 acc;
+#pragma unroll
+                for (int j = 0; j < 16; ++j) acc[j] = 0.0f;
+                acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ah, xh, acc, 0, 0, 0);
+                acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(al, xh, acc, 0, 0, 0);
+                acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ah, xl, acc, 0, 0, 0);
+                tile_to_b(acc, h, H[2 * nt], H[2 * nt + 1]);
+            }
         }
-        hidden_half<RBW>(wl, bs[L], 4, c, h, H, Hn);
+        // (2) hidden layers 2 and 3
+        float4 exn = ex;
 #pragma unroll
-        for (int rb = 0; rb < RBW; ++rb)
-#pragma unroll
-            for (int kb = 0; kb < 16; ++kb) H[rb][kb] = Hn[rb][kb];
-    }
-    // (3) layer 5 and the combination with the exact part
-    wait_all_and_sync();
-#pragma unroll
-    for (int rb = 0; rb < RBW; ++rb) {
+        for (int L = 0; L < kNG; ++L) {
+            const _Float16 *W = fw.wt + (size_t)L * kNH * kNH;
+            wait_all_and_sync();                                        // wA holds rows 0..127; wB is free
+            stage_half_async<NW>(W + 128 * kNH, wB, wv, lane);
+            hidden_half(wA, bs[L], 0, c, h, L ? Hn : H, L ? H : Hn);
+            wait_all_and_sync();                                        // wB holds rows 128..255; wA is free
+            if (L < kNG - 1) {
+                stage_half_async<NW>(W + (size_t)kNH * kNH, wA, wv, lane);
+            } else if (more) {   // for the next tile
+                stage_half_async<NW>(fw.wt, wA, wv, lane);
+                exn = exact_of(sets[sn], next);
+            }
+            hidden_half(wB, bs[L], 4, c, h, L ? Hn : H, L ? H : Hn);
+        }
+        // (3) layer 5, its hi rows in D rows 0..3 and its lo rows in 4..7 (the other rows repeat
+        // them and are not used), and the combination with the exact part
         f32x16 acc;
 #pragma unroll
         for (int j = 0; j < 16; ++j) acc[j] = 0.0f;
 #pragma unroll
-        for (int kb = 0; kb < 16; ++kb) {
-            f16x8 ah, al;
-            if (c < kNOUT) {
-                ah = *(const f16x8 *)(wl + c * kNH + 16 * kb + 8 * h);
-                al = *(const f16x8 *)(wl + 1024 + c * kNH + 16 * kb + 8 * h);
-            } else {
+        for (int kb = 0; kb < 16; ++kb)
+            acc = __builtin_amdgcn_mfma_f32_32x32x16_f16(*(const f16x8 *)(w5 + (c & 7) * kRowPad + 16 * kb + 8 * h), H[kb], acc, 0, 0, 0);
+        const int r = row_of(is, tile);
+        float v[3];
 #pragma unroll
-                for (int i = 0; i < 8; ++i) ah[i] = al[i] = (_Float16)0.0f;
-            }
-            acc = __builtin_amdgcn_mfma_f32_32x32x16_f16(ah, H[rb][kb], acc, 0, 0, 0);
-            acc = __builtin_amdgcn_mfma_f32_32x32x16_f16(al, H[rb][kb], acc, 0, 0, 0);
+        for (int k = 0; k < 3; ++k) {   // lanes h = 0: hi rows in acc[0..3], lanes h = 1: lo rows
+            const float y = acc[k] + __shfl_xor(acc[k], 32, 64);
+            v[k] = fmaxf(__expf((y + fw.b5[k]) * tn.sd[k] + tn.mu[k]) - tn.eps, 0.f);
         }
-        // lanes h = 0 hold outputs 0..3 of row c in acc[0..3]
-        const int rr = rw + 32 * rb + c;
-        if (h == 0 && rr < n) {
-            const int r = row0 + rr;
-            float v[3];
-#pragma unroll
-            for (int k = 0; k < 3; ++k)
-                v[k] = fmaxf(__expf((acc[k] + fw.b5[k]) * tn.sd[k] + tn.mu[k]) - tn.eps, 0.f);
-            if (r < fs.n4) {
-                float4 sv = S[r];
-                sv.x += v[0]; sv.y += v[1]; sv.z += v[2];
-                S[r] = sv;
-            } else {
-                const int e = r - fs.n4;
-                E[3 * e] += v[0]; E[3 * e + 1] += v[1]; E[3 * e + 2] += v[2];
-            }
+        if (h == 0 && r < is.fs.n4) {
+            is.S[r] = make_float4(ex.x + v[0], ex.y + v[1], ex.z + v[2], ex.w);
+        } else if (h == 0 && r < is.fs.n4 + is.fs.SW * is.fs.SH) {
+            float *e = is.E + 3 * (size_t)(r - is.fs.n4);
+            e[0] = ex.x + v[0]; e[1] = ex.y + v[1]; e[2] = ex.z + v[2];
         }
+        if (!more) break;
+        tile = next;
+        si = sn;
+        ex = exn;
     }
 }
 
@@ -1261,9 +1283,8 @@ hipError_t absmax(const float *a, size_t n, int stride, int ncomp, unsigned *out
 
 namespace atmo {
 namespace sg {
-constexpr int kFusedRBW = 1, kFusedNW = 8;
-size_t fused_lds() { return (size_t)kNH * kRowPad * sizeof(__bf16); }
-int fused_rows_per_block() { return 32 * kFusedRBW * kFusedNW; }
+constexpr int kFusedNW = 8;
+int fused_rows_per_block() { return 32 * kFusedNW; }
 hipError_t prep_fused(const float *W1, const float *b1, const float *W5, const float *Wh0, const float *bh0,
                       size_t bstride, __bf16 *a1h, __bf16 *a1l, _Float16 *wt, _Float16 *a5h, _Float16 *a5l,
                       float *bh, hipStream_t st) {
@@ -1311,14 +1332,19 @@ hipError_t train_pass(TrainArgs a, float *scratch, float *g, float *loss, hipStr
                        a.part5, nrb, g, loss);
     return hipGetLastError();
 }
-hipError_t mlp_infer(const InferSet *sets, int nsets, int ntiles, const FusedWeights &fw, const TargetNorm &tn,
+hipError_t mlp_infer(const InferSet *sets, int nsets, int ntiles, int maxrows, const FusedWeights &fw, const TargetNorm &tn,
                      hipStream_t st) {
     if (nsets <= 0 || ntiles <= 0) return hipSuccess;
-    static unsigned long long done = 0;
-    const hipError_t e = raise_lds((const void *)k_mlp_infer<kFusedRBW, kFusedNW>, fused_lds(), done);
+    int dev = 0, cus = 0;
+    hipError_t e = hipGetDevice(&dev);
+    if (e == hipSuccess) e = hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
     if (e != hipSuccess) return e;
-    hipLaunchKernelGGL((k_mlp_infer<kFusedRBW, kFusedNW>), dim3(ntiles), dim3(64 * kFusedNW), fused_lds(), st, sets,
-                       nsets, fw, tn);
+    for (int i = 0; i < nsets; i += 65535)   // grid limit in y
+        hipLaunchKernelGGL(k_infer_rows, dim3(blocks(maxrows), std::min(nsets - i, 65535)), dim3(256), 0, st, sets + i);
+    if ((e = hipGetLastError()) != hipSuccess) return e;
+    // one workgroup per CU (its LDS holds no second one)
+    hipLaunchKernelGGL(k_mlp_infer<kFusedNW>, dim3(std::min(ntiles, std::max(cus, 1))), dim3(64 * kFusedNW), 0, st, sets,
+                       nsets, ntiles, fw, tn);
     return hipGetLastError();
 }
 }  // namespace sg

@@ -236,6 +236,26 @@ def test_fused_inference_matches_the_network(sur):
         sur.set_norm(mu0, sd0, eps0)
 
 
+@pytest.mark.parametrize("nsets", [1, 45])
+def test_fused_inference_of_a_batch_is_that_of_its_sets(sur, nsets):
+    """A workgroup of the fused kernel walks tiles of several sets (45 sets of at
+    most 43 tiles: about 7 tiles each on 256 CUs, every one in another set; the last
+    tile of a set is partly filled).  Every set's tables are, bit for bit, those of a
+    call with that set alone."""
+    sets = small_sets(nsets, seed=SEED_BATCH + 9)
+    for i, p in enumerate(sets):
+        if i % 2:
+            p.RES_R, p.RES_MU, p.RES_MU_S, p.RES_NU = 9, 34, 7, 5
+    outs, rep = sur.precompute(sets, options(), judge_fraction=0.0)
+    torch.cuda.synchronize()
+    assert rep["judged"] == 0
+    for i in range(0, nsets, 11):
+        (one,), _ = sur.precompute([sets[i]], options(), judge_fraction=0.0)
+        torch.cuda.synchronize()
+        for a, b in zip(outs[i], one):
+            assert torch.equal(a, b), i
+
+
 def test_trained_network_gains_over_single_scattering_only():
     """What the learned part adds: after a short training on plain-method
     tables, the surrogate inscatter tables (exact single scattering + predicted
