@@ -272,6 +272,11 @@ struct DevBuf {
     void *p = nullptr;
     size_t n = 0;
     bool owned = true;   // false: a part of memory the buffer neither frees nor grows
+    void swap(DevBuf &o) {
+        std::swap(p, o.p);
+        std::swap(n, o.n);
+        std::swap(owned, o.owned);
+    }
     ~DevBuf() {
         if (p && owned) (void)hipFree(p);
     }
@@ -408,13 +413,33 @@ struct Plan {
     int snXcd = 1;     // k_inscatterN XCD-banded tile order
     int snForm = 1;    // k_inscatterN: 0 direct gathers, 1 LDS-staged rows
     bool tuned = false;
+    int runs = 0;                  // run_plan calls
+    hipEvent_t done = nullptr;     // behind the launches of the first run, while runs == 1
+    std::vector<std::vector<char>> staged;   // host sides of the uploads in flight on xs
+    // Asynchronous upload; complete once xs has been waited for (uploaded()).
+    template <class T>
+    hipError_t upload(DevBuf &b, const std::vector<T> &v) {
+        const char *p = (const char *)v.data();
+        staged.emplace_back(p, p + v.size() * sizeof(T));
+        return hipMemcpyAsync(b.p, staged.back().data(), staged.back().size(), hipMemcpyHostToDevice, xs);
+    }
+    void uploaded() { staged.clear(); }
+    // The buffers (and event) of a plan whose device work is done.
+    void recycle(Plan &o) {
+        for (auto m : {&Plan::dsets, &Plan::dlayers, &Plan::dtiles, &Plan::ddirs, &Plan::dflags}) (this->*m).swap(o.*m);
+        std::swap(done, o.done);
+    }
     void drop_graph() {
         if (gexec) (void)hipGraphExecDestroy(gexec);
         if (graph) (void)hipGraphDestroy(graph);
         gexec = nullptr;
         graph = nullptr;
     }
-    ~Plan() { drop_graph(); }
+    ~Plan() {
+        if (!staged.empty()) (void)hipStreamSynchronize(xs);
+        drop_graph();
+        if (done) (void)hipEventDestroy(done);
+    }
 };
 
 }  // namespace
@@ -431,6 +456,7 @@ struct atmo_engine {
     int device = 0;
     hipStream_t cap = nullptr;  // capture stream
     std::unique_ptr<Plan> plan;
+    std::unique_ptr<Plan> prev;   // the plan before, whose device work may not be done (change_plan)
     DevBuf pass_sets, pass_layers, pass_tiles, pass_dirs;
     std::vector<atmo_pass_time> times;
     Tuning last_tuning;
@@ -499,20 +525,22 @@ size_t dirs_bytes(const atmo_options &o, size_t &offJT, size_t &offJW, size_t &o
     return offE + align256(2 * NI * (NI / 2) * sizeof(DirEHost));
 }
 
-atmo_status upload_dirs(DevBuf &buf, hipStream_t xs, const atmo_options &o, size_t &offJT, size_t &offJW,
-                        size_t &offE, Region *rg = nullptr) {
+std::vector<char> pack_dirs(const atmo_options &o, size_t &offJT, size_t &offJW, size_t &offE) {
     std::vector<DirJHost> jt;
     std::vector<float> jw;
     std::vector<DirEHost> de;
     build_dirs(o.spherical_samples, o.irradiance_samples, jt, jw, de);
-    const size_t total = dirs_bytes(o, offJT, offJW, offE);
-    Region none;
-    HIPCHK((rg ? rg : &none)->get(buf, total));
-    std::vector<char> h(total, 0);
+    std::vector<char> h(dirs_bytes(o, offJT, offJW, offE), 0);
     memcpy(h.data() + offJT, jt.data(), jt.size() * sizeof(DirJHost));
     memcpy(h.data() + offJW, jw.data(), jw.size() * sizeof(float));
     memcpy(h.data() + offE, de.data(), de.size() * sizeof(DirEHost));
-    HIPCHK(h2d(buf.p, h.data(), total, xs));
+    return h;
+}
+
+atmo_status upload_dirs(DevBuf &buf, hipStream_t xs, const atmo_options &o, size_t &offJT, size_t &offJW, size_t &offE) {
+    const std::vector<char> h = pack_dirs(o, offJT, offJW, offE);
+    HIPCHK(buf.ensure(h.size()));
+    HIPCHK(h2d(buf.p, h.data(), h.size(), xs));
     return ATMO_OK;
 }
 
@@ -966,11 +994,13 @@ atmo_status apply_tuning(Plan &pl, const Tuning &tu) {
 }
 
 // rg: where the device buffers come from (nullptr: hipMalloc); tu: kernel
-// variants to build the plan with (nullptr: the defaults, tuned later).
+// variants to build the plan with (nullptr: the defaults, tuned later); into: an
+// empty plan with buffers to use, or nullptr.  The uploads are in flight on xs when
+// it returns.
 atmo_status build_plan(hipStream_t xs, const atmo_params *sets, int nsets, const atmo_options &o,
                        std::unique_ptr<Plan> &out, Region *rg = nullptr, const Tuning *tu = nullptr,
-                       bool view = true) {
-    std::unique_ptr<Plan> pl(new Plan);
+                       bool view = true, std::unique_ptr<Plan> into = nullptr) {
+    std::unique_ptr<Plan> pl(into ? std::move(into) : std::unique_ptr<Plan>(new Plan));
     Region heap;
     Region &R = rg ? *rg : heap;
     pl->xs = xs;
@@ -1009,7 +1039,7 @@ atmo_status build_plan(hipStream_t xs, const atmo_params *sets, int nsets, const
     memcpy(geom.data(), layers.data(), layers.size() * sizeof(LayerGeom));
     memcpy(geom.data() + cols_off, cols.data(), cols.size() * sizeof(ColGeom));
     HIPCHK(R.get(pl->dlayers, geom.size()));
-    HIPCHK(h2d(pl->dlayers.p, geom.data(), geom.size(), pl->xs));
+    HIPCHK(pl->upload(pl->dlayers, geom));
     // descriptors (output pointers are filled in per call)
     pl->hsets.resize(nsets);
     char *ar = (char *)pl->arena.p;
@@ -1041,10 +1071,11 @@ atmo_status build_plan(hipStream_t xs, const atmo_params *sets, int nsets, const
     std::vector<uint2> tiles;
     build_tiles(pl->params, o, tiles, pl->off, pl->cnt, pl->snXcd, &pl->segs);
     HIPCHK(R.get(pl->dtiles, tiles.size() * sizeof(uint2)));
-    HIPCHK(h2d(pl->dtiles.p, tiles.data(), tiles.size() * sizeof(uint2), pl->xs));
+    HIPCHK(pl->upload(pl->dtiles, tiles));
     HIPCHK(R.get(pl->dflags, nsets * sizeof(unsigned)));
-    atmo_status st = upload_dirs(pl->ddirs, pl->xs, o, pl->dirJT_off, pl->dirJW_off, pl->dirE_off, &R);
-    if (st != ATMO_OK) return st;
+    const std::vector<char> dirs = pack_dirs(o, pl->dirJT_off, pl->dirJW_off, pl->dirE_off);
+    HIPCHK(R.get(pl->ddirs, dirs.size()));
+    HIPCHK(pl->upload(pl->ddirs, dirs));
     int maxNU = 0, maxSW = 0;
     for (int i = 0; i < nsets; ++i) {
         maxNU = std::max(maxNU, sets[i].RES_NU);
@@ -1086,10 +1117,14 @@ size_t plan_bytes(const std::vector<atmo_params> &ps, const atmo_options &o, int
 }
 
 // Runs every pass of a plan on the caller's stream: with pass timing (eager
-// launches between hipEvent pairs), eagerly, or by replaying the plan's graph
-// (captured on first use).
+// launches between hipEvent pairs), eagerly, or by replaying the plan's graph.  The
+// first run is eager (a plan that runs once saves the capture, about 90 us of a
+// 32x128x32x8 set's 1.1 ms, and its launches hide behind the first kernels) and
+// leaves Plan::done behind; the graph is captured on the second.
 atmo_status run_plan(atmo_engine *e, Plan &pl, const atmo_options &o, hipStream_t hs) {
     atmo_status st;
+    const bool first = pl.runs == 0;
+    pl.runs = std::min(pl.runs, 2) + 1;
     if (o.flags & ATMO_FLAG_TIME_PASSES) {
         PassTimer tm;
         tm.on = true;
@@ -1101,11 +1136,17 @@ atmo_status run_plan(atmo_engine *e, Plan &pl, const atmo_options &o, hipStream_
             HIPCHK(hipEventElapsedTime(&ms, r.a, r.b));
             e->times.push_back({r.pass, r.order, ms});
         }
-    } else if (o.flags & ATMO_FLAG_NO_GRAPH) {
+    } else if (first || (o.flags & ATMO_FLAG_NO_GRAPH)) {
         if ((st = launch_all(pl, hs)) != ATMO_OK) return st;
+        if (first) {
+            if (!pl.done) HIPCHK(hipEventCreateWithFlags(&pl.done, hipEventDisableTiming));
+            HIPCHK(hipEventRecord(pl.done, hs));
+        }
     } else {
-        bool eager = false;
-        if (!pl.gexec) {
+        hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+        if (!pl.gexec && hs) HIPCHK(hipStreamIsCapturing(hs, &cap));
+        bool eager = cap != hipStreamCaptureStatusNone;   // no capture inside the caller's
+        if (!pl.gexec && !eager) {
             HIPCHK(hipStreamBeginCapture(e->cap, hipStreamCaptureModeThreadLocal));
             atmo_status cs = launch_all(pl, e->cap);
             hipGraph_t g = nullptr;
@@ -1134,6 +1175,45 @@ atmo_status run_plan(atmo_engine *e, Plan &pl, const atmo_options &o, hipStream_
         }
     }
     return ATMO_OK;
+}
+
+// Replaces the engine's plan.  A plan that has run once, eagerly, may still be at work
+// (a caller that changes its parameters on every call): the new one is built while it
+// is, takes over its work arena (ordered by its event) and the small buffers of the
+// plan before it (waited for), so that the device does not idle while the host builds:
+// two 32x128x32x8 sets, other ones in every pass, 2.93 -> 2.38 ms (of it 2.25 of kernels).
+// Any other plan, or an arena that is too small or more than twice too large, is
+// waited for and freed.
+atmo_status change_plan(atmo_engine *e, const atmo_params *sets, int nsets, const atmo_options &o, const Tuning *tu, hipStream_t hs) {
+    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+    if (hs) HIPCHK(hipStreamIsCapturing(hs, &cap));
+    if (cap != hipStreamCaptureStatusNone)
+        return fail(ATMO_ERR_DEVICE, "other sets or options than the engine's last call's, on a stream in capture");
+    size_t total = 0;
+    for (int i = 0; i < nsets; ++i) total += work_bytes(sets[i], o, true);
+    Plan *old = e->plan.get();
+    std::unique_ptr<Plan> into;
+    if (old && old->runs == 1 && old->done && total <= old->arena.n && old->arena.n / 2 <= total) {
+        into.reset(new Plan);
+        if (e->prev) {
+            HIPCHK(hipEventSynchronize(e->prev->done));
+            into->recycle(*e->prev);
+        }
+        HIPCHK(hipStreamWaitEvent(hs, old->done, 0));
+        into->arena.swap(old->arena);
+        e->prev = std::move(e->plan);
+    } else {
+        HIPCHK(hipStreamSynchronize(hs));
+        e->prev.reset();
+        e->plan.reset();
+    }
+    atmo_status st = build_plan(e->cap, sets, nsets, o, e->plan, nullptr, tu, true, std::move(into));
+    if (st == ATMO_ERR_OUT_OF_MEMORY) {   // without the table of view-ray samples
+        HIPCHK(hipStreamSynchronize(hs));
+        e->prev.reset();
+        st = build_plan(e->cap, sets, nsets, o, e->plan, nullptr, tu, false);
+    }
+    return st;
 }
 
 atmo_status check_out(const atmo_tables &t, int i) {
@@ -1247,6 +1327,7 @@ atmo_status atmo_engine_destroy(atmo_engine *e) {
     if (!e) return ATMO_OK;
     (void)hipSetDevice(e->device);
     (void)hipDeviceSynchronize();
+    e->prev.reset();
     e->plan.reset();
     if (e->cap) (void)hipStreamDestroy(e->cap);
     delete e;
@@ -1309,13 +1390,22 @@ atmo_status atmo_engine_precompute(atmo_engine *e, const atmo_params *sets, int 
     bool reuse = e->plan && (int)e->plan->params.size() == nsets && same_opts(e->plan->opts, o);
     if (reuse)
         for (int i = 0; i < nsets && reuse; ++i) reuse = same_params(e->plan->params[i], sets[i]);
+    // A new plan takes the cached tuning of its shape class, if there is one
+    Tuning tu;
+    std::string key;
+    bool have = false;
+    auto cached_tuning = [&](const std::vector<atmo_params> &ps) {
+        if (o.orders < 2 || (o.flags & ATMO_FLAG_NO_AUTOTUNE)) return;
+        key = shape_key(ps, o);
+        std::lock_guard<std::mutex> lk(tuning_mutex());
+        auto it = tuning_cache().find(key);
+        if (it == tuning_cache().end()) return;
+        tu = it->second;
+        have = true;
+    };
     if (!reuse) {
-        HIPCHK(hipStreamSynchronize(hs));
-        e->plan.reset();
-        st = build_plan(e->cap, sets, nsets, o, e->plan);
-        if (st == ATMO_ERR_OUT_OF_MEMORY)   // without the table of view-ray samples
-            st = build_plan(e->cap, sets, nsets, o, e->plan, nullptr, nullptr, false);
-        if (st != ATMO_OK) return st;
+        cached_tuning(std::vector<atmo_params>(sets, sets + nsets));
+        if ((st = change_plan(e, sets, nsets, o, have ? &tu : nullptr, hs)) != ATMO_OK) return st;
     }
     Plan &pl = *e->plan;
     bool changed = !reuse;
@@ -1330,36 +1420,28 @@ atmo_status atmo_engine_precompute(atmo_engine *e, const atmo_params *sets, int 
         }
     }
     if (changed) {
-        HIPCHK(hipStreamSynchronize(hs));
+        if (reuse) HIPCHK(hipStreamSynchronize(hs));   // nothing on the device reads a new plan's descriptors yet
         HIPCHK(h2d(pl.dsets.p, pl.hsets.data(), nsets * sizeof(SetDesc), e->cap));
+        pl.uploaded();   // the plan's other uploads, earlier on the same stream
     }
     // A plan that has not been tuned takes the cached tuning of its shape class
-    // before its first launch; with none cached, it is tuned after this run.
+    // before a launch; with none cached, it is tuned after this run.
     bool tune_after = false;
-    std::string key;
-    if (!pl.tuned && (o.orders >= 2) && !(o.flags & ATMO_FLAG_NO_AUTOTUNE)) {
-        key = shape_key(pl.params, o);
-        Tuning tu;
-        bool have = false;
-        {
-            std::lock_guard<std::mutex> lk(tuning_mutex());
-            auto it = tuning_cache().find(key);
-            if (it != tuning_cache().end()) {
-                tu = it->second;
-                have = true;
-            }
-        }
+    if (have) {
+        e->last_tuning = tu;
+        e->last_key = key;
+    } else if (!pl.tuned) {
+        if (reuse) cached_tuning(pl.params);
         if (have) {
             if ((st = apply_tuning(pl, tu)) != ATMO_OK) return st;
             e->last_tuning = tu;
             e->last_key = key;
         } else {
-            tune_after = true;
+            tune_after = !key.empty();
         }
     }
     if ((st = run_plan(e, pl, o, hs)) != ATMO_OK) return st;
     if (tune_after) {
-        Tuning tu;
         if ((st = autotune(pl, hs, tu)) != ATMO_OK) return st;
         {
             std::lock_guard<std::mutex> lk(tuning_mutex());
@@ -1433,6 +1515,7 @@ atmo_status atmo_precompute_noalloc(const atmo_params *sets, int nsets, const at
         d.outE = out[i].irradiance;
     }
     HIPCHK(h2d(pl->dsets.p, pl->hsets.data(), nsets * sizeof(SetDesc), hs));
+    pl->uploaded();
     if ((st = launch_all(*pl, hs)) != ATMO_OK) return st;
     if (o.flags & ATMO_FLAG_CHECK_NUMERICS)
         if ((st = check_numerics(*pl, hs)) != ATMO_OK) return st;

@@ -700,6 +700,40 @@ def test_graph_replays_match_eager(eng):
             assert np.array_equal(a, b), rep
 
 
+@pytest.mark.parametrize("streams", [1, 2])
+def test_sets_that_change_on_every_call(streams):
+    """A new plan is built while the last one's single run is at work, in its arena:
+    sets of the same and of other sizes (an arena that is kept, too small, more than
+    twice too large), repeats (the graph) and another stream, without a wait between
+    the calls, give the tables of engines of their own."""
+    shapes = [(6, 16, 6, 4), (6, 16, 6, 4), (8, 32, 16, 8), (6, 16, 8, 4), (6, 16, 6, 4), (4, 8, 4, 3), (6, 16, 6, 4)]
+    sets = []
+    for i, r in enumerate(shapes):
+        p = small(res=r)
+        p.HR = 6.0 + 0.5 * i
+        sets.append(p)
+    order = [0, 1, 0, 1, 3, 2, 2, 2, 1, 0, 5, 4, 6, 0, 0, 1]
+    want = []
+    for p in sets:
+        e = L.Engine(0)
+        want.append([t.clone() for t in e.precompute(p, options(flags=8))[0]])
+        torch.cuda.synchronize()
+        e.close()
+    st = [torch.cuda.Stream() for _ in range(streams)]
+    outs = [L.alloc_outputs(sets[i]) for i in order]
+    torch.cuda.synchronize()
+    e = L.Engine(0)
+    k = 0
+    for n, i in enumerate(order):
+        k += n > 0 and order[n - 1] != i   # repeats of a set stay on their stream
+        e.precompute(sets[i], options(flags=8), outs=[outs[n]], stream=st[k % streams])
+    torch.cuda.synchronize()
+    e.close()
+    for n, i in enumerate(order):
+        for x, y in zip(outs[n], want[i]):
+            assert torch.equal(x, y), (n, i)
+
+
 def test_numeric_check_flag_passes_on_valid_tables(eng):
     p = small()
     eng.precompute(p, options(flags=1))
