@@ -74,17 +74,8 @@ __device__ __forceinline__ float3 T_at(const CDesc &d, double r, double mu) {
     return rgb_bilinear(d.T, d.TW, d.TH, uMu * d.TW - 0.5f, uR * d.TH - 0.5f);
 }
 
-// sqrt (x >= 0) and 1/x in FP64 from the hardware estimates and Newton steps, a few
-// ulp: what follows rounds to a texel coordinate
-__device__ __forceinline__ double sqrt64(double x) {
-    x = fmax(x, 1e-280);
-    const double y = __builtin_amdgcn_rsq(x);
-    double g = x * y, h = 0.5 * y;
-    const double e = fma(-h, g, 0.5);
-    g = fma(g, e, g);
-    h = fma(h, e, h);
-    return fma(fma(-g, g, x), h, g);
-}
+// 1/x in FP64 from the hardware estimate and Newton steps, a few ulp (as sqrt64): what
+// follows rounds to a texel coordinate
 __device__ __forceinline__ double rcp64(double x) {
     double y = __builtin_amdgcn_rcp(x);
     y = fma(y, fma(-x, y, 1.0), y);

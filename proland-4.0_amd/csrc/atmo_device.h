@@ -306,6 +306,17 @@ __device__ __forceinline__ float phaseM(const SetDesc &s, float mu) {
 }
 
 // common.glsl:209-219 limit(r, mu), FP64.
+// sqrt (x >= 0) in FP64 from the hardware estimate and Newton steps, a few ulp
+__device__ __forceinline__ double sqrt64(double x) {
+    x = fmax(x, 1e-280);
+    const double y = __builtin_amdgcn_rsq(x);
+    double g = x * y, h = 0.5 * y;
+    const double e = fma(-h, g, 0.5);
+    g = fma(g, e, g);
+    h = fma(h, e, h);
+    return fma(fma(-g, g, x), h, g);
+}
+
 __device__ __forceinline__ double limit_d(const SetDesc &s, double r, double mu) {
     double rr1 = r * r * (mu * mu - 1.0);
     double dout = -r * mu + sqrt(rr1 + s.RL2);

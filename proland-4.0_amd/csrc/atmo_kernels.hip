@@ -11,10 +11,58 @@
 
 namespace atmo {
 
+// 2^y for y <= 1000, at least 2^-1000, 1.4e-14 relative: a polynomial in the fraction
+// (degree 9, fitted to the relative error on |f| <= 1/2), the integer part added to the
+// exponent.
+constexpr double kLog2e = 1.4426950408889634;
+__device__ __forceinline__ double exp2_64(double y) {
+    constexpr double kRound64 = 6755399441055744.0;   // 1.5 2^52
+    y = fmax(y, -1000.0);
+    const double t = y + kRound64, f = y - (t - kRound64);
+    double p = fma(f, 1.0150099678576792e-07, 1.3259402170656473e-06);
+    p = fma(f, p, 1.5252986067042296e-05);
+    p = fma(f, p, 0.00015403434961948063);
+    p = fma(f, p, 0.001333355761545632);
+    p = fma(f, p, 0.009618129192050495);
+    p = fma(f, p, 0.055504108668700244);
+    p = fma(f, p, 0.24022650695649567);
+    p = fma(f, p, 0.6931471805598719);
+    p = fma(f, p, 1.0000000000000133);
+    return __hiloint2double(__double2hiint(p) + (__double2loint(t) << 20), __double2loint(p));
+}
+
+// tan x for x in [0, 1.5], 4e-15 relative: from the Taylor series of sine and cosine at x / 2
+// (terms below 1e-18 left out).  A tenth of the library's code, which reduces any argument.
+__device__ __forceinline__ double tan_col(double x) {
+    const double y = 0.5 * x, z = y * y;
+    double s = fma(z, 2.8114572543455206e-15, -7.647163731819816e-13);
+    s = fma(z, s, 1.6059043836821613e-10);
+    s = fma(z, s, -2.505210838544172e-08);
+    s = fma(z, s, 2.7557319223985893e-06);
+    s = fma(z, s, -0.0001984126984126984);
+    s = fma(z, s, 0.008333333333333333);
+    s = fma(z, s, -0.16666666666666666);
+    s = fma(y * z, s, y);
+    double c = fma(z, 4.779477332387385e-14, -1.1470745597729725e-11);
+    c = fma(z, c, 2.08767569878681e-09);
+    c = fma(z, c, -2.755731922398589e-07);
+    c = fma(z, c, 2.48015873015873e-05);
+    c = fma(z, c, -0.001388888888888889);
+    c = fma(z, c, 0.041666666666666664);
+    c = fma(z, c, -0.5);
+    c = fma(z, c, 1.0);
+    return 2.0 * s * c / fma(-s, s, c * c);
+}
+
 // ---------------------------------------------------------------------------
 // Pass T — transmittance.glsl:78-98.  FP64 trapezoid of exp(-h/H) for both
 // scale heights at once; 16 lanes share one texel's samples.
-// tile = 16 consecutive texels.
+// tile = 16 consecutive texels.  Bound by FP64 issue: the library's exp and square
+// root take about 95 instructions a sample, exp2_64 and sqrt64 50, and the tables are
+// FP32 (256x64 texels, 500 samples: 28 -> 21 us); nearly half of the texels of the
+// tangent parameterisation look at the ground and need no samples, and straight code
+// without the library's argument reductions is fetched in time (-> 19.4; 24 sets 515 ->
+// 290 us).  A single set is left with its latency: 4 waves per SIMD, half of them idle.
 // ---------------------------------------------------------------------------
 __global__ __launch_bounds__(256) void k_transmittance(const SetDesc *__restrict__ sets,
                                                        const uint2 *__restrict__ tiles,
@@ -30,22 +78,26 @@ __global__ __launch_bounds__(256) void k_transmittance(const SetDesc *__restrict
     double rr = (j + 0.5) / s.TH;
     double m = (i + 0.5) / s.TW;
     double r, mu;
+    const double tm = tan_col(1.5 * m);
     if (s.linT) {
         r = s.Rg + rr * (s.Rt - s.Rg);
         mu = -0.15 + m * (1.0 + 0.15);
     } else {
         r = s.Rg + rr * rr * (s.Rt - s.Rg);
-        mu = -0.15 + tan(1.5 * m) / tan(1.5) * (1.0 + 0.15);
+        mu = -0.15 + tm * (1.15 / 14.101419947171719);   // tan(1.5)
     }
     double dx = limit_d(s, r, mu) / nsamp;
     double sR = 0.0, sM = 0.0;
-    const double iHR = 1.0 / s.HR, iHM = 1.0 / s.HM;
-    for (int k = lane; k <= nsamp; k += 16) {
-        double x = k * dx;
-        double h = sqrt(r * r + x * x + 2.0 * x * r * mu) - s.Rg;
-        double w = (k == 0 || k == nsamp) ? 0.5 : 1.0;
-        sR += w * exp(-h * iHR);
-        sM += w * exp(-h * iHM);
+    const double eR = -kLog2e / s.HR, eM = -kLog2e / s.HM;
+    const double r2 = r * r, rmu2 = 2.0 * r * mu;
+    const double q = s.Rg / r;
+    const bool below = mu < -sqrt(1.0 - q * q);   // the ground is in the way: no integral
+    for (int k = below ? nsamp + 1 : lane; k <= nsamp; k += 16) {
+        const double x = k * dx;
+        const double h = sqrt64(fma(x, x + rmu2, r2)) - s.Rg;   // >= 0: the ray ends at the ground
+        const double w = (k == 0 || k == nsamp) ? 0.5 : 1.0;
+        sR = fma(w, exp2_64(h * eR), sR);
+        sM = fma(w, exp2_64(h * eM), sM);
     }
 #pragma unroll
     for (int off = 8; off > 0; off >>= 1) {
@@ -54,23 +106,22 @@ __global__ __launch_bounds__(256) void k_transmittance(const SetDesc *__restrict
     }
     if (lane == 0 && valid) {
         // sun_centres: tan(1.5 m), its leading part in row 0 and the rest in row 1
-        double c = j < 2 ? tan(1.5 * m) : 0.0;
+        double c = j < 2 ? tm : 0.0;
         const float ck = j == 0 ? (float)c : j == 1 ? (float)(c - (double)(float)c) : 0.0f;
-        double q = s.Rg / r;
-        bool below = mu < -sqrt(1.0 - q * q);
         double dR = below ? 1e9 : sR * dx;
         double dM = below ? 1e9 : sM * dx;
+        double tau[3];
+#pragma unroll
+        for (int k = 0; k < 3; ++k) tau[k] = (double)s.bR[k] * dR + (double)s.bME[k] * dM;
         float4 o;
-        o.x = (float)exp(-((double)s.bR[0] * dR + (double)s.bME[0] * dM));
-        o.y = (float)exp(-((double)s.bR[1] * dR + (double)s.bME[1] * dM));
-        o.z = (float)exp(-((double)s.bR[2] * dR + (double)s.bME[2] * dM));
+        o.x = (float)exp2_64(tau[0] * -kLog2e);
+        o.y = (float)exp2_64(tau[1] * -kLog2e);
+        o.z = (float)exp2_64(tau[2] * -kLog2e);
         o.w = 0.0f;
         o = q16(o, s.hs);
         s.T4[t] = o;
         if (s.tau4)
-            s.tau4[t] = make_float4((float)((double)s.bR[0] * dR + (double)s.bME[0] * dM),
-                                    (float)((double)s.bR[1] * dR + (double)s.bME[1] * dM),
-                                    (float)((double)s.bR[2] * dR + (double)s.bME[2] * dM), ck);
+            s.tau4[t] = make_float4((float)tau[0], (float)tau[1], (float)tau[2], ck);
         if (s.outT) {
             s.outT[3 * t + 0] = o.x;
             s.outT[3 * t + 1] = o.y;

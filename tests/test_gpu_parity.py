@@ -684,6 +684,24 @@ def test_two_engines_on_two_threads(flags):
             assert np.array_equal(x, y), name
 
 
+@pytest.mark.parametrize("HR,HM,Rt,flags", [(8.0, 1.2, 6420.0, 0), (0.05, 0.01, 6480.0, 0), (40.0, 30.0, 6361.0, 0),
+                                            (8.0, 1.2, 6420.0, 32)])
+def test_transmittance_pass_follows_the_oracle(HR, HM, Rt, flags):
+    """The FP64 exponentials, roots and tangent of the T pass at their ends: scale
+    heights of a few metres (2^y far below its clamp) and of most of the atmosphere, a
+    thin one, both parameterisations (flag 32).  The oracle evaluates the same sums in
+    FP64: within one FP32 rounding (2^-23), and 1e-13 of 1 where T vanishes."""
+    p = small(res=(4, 8, 4, 3))
+    p.HR, p.HM, p.Rt, p.RL = HR, HM, Rt, Rt + 1.0
+    p.TRANSMITTANCE_W, p.TRANSMITTANCE_H = 67, 13
+    e = L.Engine(0)
+    o = options(flags=8 | flags, orders=1)
+    T = e.precompute(p, o)[0][0].double().cpu().numpy()
+    e.close()
+    oT = O.precompute(p, o)[0]
+    assert np.all(np.abs(T - oT) <= 2.0 ** -23 * np.abs(oT) * 1.01 + 1e-13)
+
+
 def test_graph_replays_match_eager(eng):
     p = small()
     eager = _chain(eng, p, options(flags=2))
