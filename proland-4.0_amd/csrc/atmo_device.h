@@ -48,6 +48,20 @@ struct SnView {
     float dr;        // (r_i - r) / r_i; sample 0, where that is 0: the trapezoid step of the ray
 };
 
+// A theta row of a spherical integral (dJ: per layer, dE: per irradiance row), what does
+// not involve the sun, and the sun's part, per mu_s column (dJ) or irradiance column (dE).
+// FP64 geometry, once per precompute (k_geometry).
+struct __attribute__((aligned(16))) ThetaRow {
+    double ct, e1;      // cos theta; ground row of dJ: E texels per unit of nu1 (else 0)
+    int base, dy, dz;   // first texel of the row's four table rows, steps to the next mu row and layer
+    float ay, az;       // their weights
+    float dw;           // dJ: dtheta dphi sin theta
+    float eR, eM;       // dJ: exp(-h/HR), exp(-h/HM) of the layer
+};
+struct __attribute__((aligned(16))) SunColumn {
+    double mus, txs;    // mu_s of the column and its texel offset in a nu slice
+};
+
 struct SetDesc {
     // FP32 parameters promoted to double
     double Rg, Rt, RL, HR, HM, mieG, alpha;
@@ -75,6 +89,9 @@ struct SetDesc {
     // inline from T (pass-level entry points)
     float4 *tview, *tground;
     SnView *view;                   // [RR][RMU][nsamp + 1]; null: computed in k_inscatterN
+    // [RR][NS] and [SH][NI/2]; [RMUS] and [SW]; null: computed in the dJ and dE kernels
+    ThetaRow *rowJ, *rowE;
+    SunColumn *sunJ, *sunE;
     int dJb;                        // bytes per dJ texel: 16 (float4) or 12 (packed rgb)
     int hs;                         // 1: table values rounded to FP16 on store (q16)
     int linT, lin4;                 // 1: the linear transmittance / inscatter parameterisation
@@ -221,7 +238,7 @@ __device__ __forceinline__ float3 T_ratio_lin(const SetDesc &s, float hx, float 
     return make_float3(fminf(a.x / b.x, 1.f), fminf(a.y / b.y, 1.f), fminf(a.z / b.z, 1.f));
 }
 
-// T_ratio_d is the form of the precompute's ratio tables (k_tview, k_tground:
+// T_ratio_d is the form of the precompute's ratio tables (k_geometry:
 // one ratio per layer, mu row and view-ray sample, and per layer and theta
 // row, evaluated once per precompute).  Its texel coordinates and filter
 // weights are computed in FP64: along a grazing view ray the ratio divides two

@@ -236,7 +236,12 @@ size_t view_extra(const atmo_params &p, const atmo_options &o) {
     const size_t b = view_bytes(p, o);
     return o.orders < 2 || b <= sizes(p).n4 * 16 ? 0 : align256(b);
 }
-// work tables per set: T4, dE4, E4, dSR4, dSM4, dJ4; view: with SetDesc::view
+// Theta rows and sun columns of the dJ and dE passes (SetDesc::rowJ ... sunE).
+size_t theta_bytes(const atmo_params &p, const atmo_options &o) {
+    const size_t rows = (size_t)p.RES_R * o.spherical_samples + (size_t)p.SKY_H * (o.irradiance_samples / 2);
+    return align256(rows * sizeof(ThetaRow) + ((size_t)p.RES_MU_S + p.SKY_W) * sizeof(SunColumn));
+}
+// work tables per set: T4, dE4, E4, dSR4, dSM4, dJ4; view: with SetDesc::view and the theta rows
 size_t work_bytes(const atmo_params &p, const atmo_options &o, bool view = true) {
     SetSizes z = sizes(p);
     size_t b = 2 * align256(z.nT * 16) + 2 * align256(z.nE * 16) + 2 * align256(z.n4 * 16);   // T, tau, ...
@@ -244,7 +249,7 @@ size_t work_bytes(const atmo_params &p, const atmo_options &o, bool view = true)
     if (o.orders >= 2) {
         b += align256(z.n4 * 12);                                         // dJ, packed rgb
         b += align256((size_t)p.RES_R * o.spherical_samples * 16);        // tground
-        if (view) b += view_extra(p, o);
+        if (view) b += view_extra(p, o) + theta_bytes(p, o);
     }
     return b;
 }
@@ -815,9 +820,13 @@ atmo_status launch_all(Plan &pl, hipStream_t st, PassTimer *tm = nullptr) {
     const char *dirs = (const char *)pl.ddirs.p;
     HIPCHK(t.begin(0, 1));
     HIPCHK(launch_transmittance(S, T + pl.off[P_T], pl.cnt[P_T], o.transmittance_samples, st));
-    // the transmittance tables of the later passes (timed with the T pass)
-    HIPCHK(launch_tview(S, T + pl.off[P_VIEW], pl.cnt[P_VIEW], o.inscatter_samples, st));
-    if (o.orders >= 2) HIPCHK(launch_tground(S, T + pl.off[P_J], pl.cnt[P_J], o.spherical_samples, st));
+    // the tables of the later passes (timed with the T pass)
+    int wpt = 0;
+    for (const atmo_params &p : pl.params)
+        if (o.orders >= 2)
+            wpt = std::max(wpt, theta_workgroups(p.RES_R, p.RES_MU_S, p.SKY_W, p.SKY_H, o.spherical_samples, o.irradiance_samples));
+    HIPCHK(launch_geometry(S, (int)pl.params.size(), wpt, T + pl.off[P_VIEW], pl.cnt[P_VIEW], o.inscatter_samples,
+                           o.spherical_samples, o.irradiance_samples, st));
     HIPCHK(t.end());
     HIPCHK(t.begin(1, 1));
     HIPCHK(launch_irradiance1(S, T + pl.off[P_E1], pl.cnt[P_E1], st));
@@ -1060,6 +1069,13 @@ atmo_status build_plan(hipStream_t xs, const atmo_params *sets, int nsets, const
             b += align256(z.n4 * 12);
             s.tground = (float4 *)b; b += align256((size_t)sets[i].RES_R * o.spherical_samples * 16);
             s.view = !view ? nullptr : view_extra(sets[i], o) ? (SnView *)b : (SnView *)s.dSM4;
+            if (view) {
+                b += view_extra(sets[i], o);
+                s.rowJ = (ThetaRow *)b;
+                s.rowE = s.rowJ + (size_t)sets[i].RES_R * o.spherical_samples;
+                s.sunJ = (SunColumn *)(s.rowE + (size_t)sets[i].SKY_H * (o.irradiance_samples / 2));
+                s.sunE = s.sunJ + sets[i].RES_MU_S;
+            }
         }
         s.dJb = 12;  // the ray gathers of dSn read 12 bytes per texel
         set_table_flags(s, o);

@@ -50,10 +50,11 @@ int chunk_irradianceN(int NI, int RNU, bool first);
 hipError_t launch_transmittance(const SetDesc *sets, const uint2 *tiles, int ntiles, int nsamp,
                                 hipStream_t st);
 hipError_t launch_irradiance1(const SetDesc *sets, const uint2 *tiles, int ntiles, hipStream_t st);
-// transmittance tables of a precompute (SetDesc::tview on the inscatter1 tiles,
-// SetDesc::tground on the dJ tiles), after the T pass
-hipError_t launch_tview(const SetDesc *sets, const uint2 *tiles, int ntiles, int nsamp, hipStream_t st);
-hipError_t launch_tground(const SetDesc *sets, const uint2 *tiles, int ntiles, int NS, hipStream_t st);
+// geometry and transmittance tables of a precompute (SetDesc::tview on nview tiles, tground,
+// theta rows and sun columns with wpt workgroups per set, 0: none), after the T pass
+int theta_workgroups(int RR, int RMUS, int SW, int SH, int NS, int NI);
+hipError_t launch_geometry(const SetDesc *sets, int nsets, int wpt, const uint2 *tiles, int nview, int nsamp, int NS, int NI,
+                           hipStream_t st);
 // linT / lin4: the sets' parameterisation flags (one per batch), compiled in
 // G: texels per thread (2, 3, 4 or 8); CH: theta rows per staging round; RNU:
 // the largest RES_NU of the launch's sets; DS: slots of the workgroup's threads the

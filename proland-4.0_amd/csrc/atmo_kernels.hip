@@ -561,6 +561,19 @@ k_inscatter1(const SetDesc *__restrict__ sets, const uint2 *__restrict__ tiles, 
     }
 }
 
+// The table rows of theta row `it` of N at radius r (squared height over the ground's: rho2).
+__device__ __forceinline__ void theta_taps(const SetDesc &s, double r, double rho2, double ct, ThetaRow &row) {
+    const double rmu = r * ct;
+    double tz, ty;
+    tex4d_rmu(s, rho2, rmu, rmu * rmu - rho2, ct, tz, ty);
+    int z0, z1, y0, y1;
+    gl_axis_d(tz, s.RR, z0, z1, row.az);
+    gl_axis_d(ty, s.RMU, y0, y1, row.ay);
+    row.base = (z0 * s.RMU + y0) * s.W4;
+    row.dy = (y1 - y0) * s.W4;
+    row.dz = (z1 - z0) * s.RMU * s.W4;
+}
+
 // ---------------------------------------------------------------------------
 // Shared staging of the spherical integrals (inscatterS, irradianceN).
 //
@@ -579,21 +592,18 @@ k_inscatter1(const SetDesc *__restrict__ sets, const uint2 *__restrict__ tiles, 
 // ---------------------------------------------------------------------------
 template <int NT>
 __device__ __forceinline__ void stage_slice(const SetDesc &s, const float4 *const *tabs,
-                                            double tz, double ty, double txs, int k,
+                                            const ThetaRow &row, double txs, int k,
                                             float4 *out) {
-    int z0, z1, y0, y1, x0, x1;
-    float az, ay, ax;
-    gl_axis_d(tz, s.RR, z0, z1, az);
-    gl_axis_d(ty, s.RMU, y0, y1, ay);
+    int x0, x1;
+    float ax;
+    const float ay = row.ay, az = row.az;
     gl_axis_d((double)k * s.RMUS + txs, s.W4, x0, x1, ax);
-    const size_t W = s.W4, HW = (size_t)s.RMU * s.W4;
 #pragma unroll
     for (int n = 0; n < NT; ++n) {
         const gfloat4 *tb = gptr(tabs[n]);
-        float3 c000 = ld3(tb + z0 * HW + y0 * W + x0), c001 = ld3(tb + z0 * HW + y0 * W + x1);
-        float3 c010 = ld3(tb + z0 * HW + y1 * W + x0), c011 = ld3(tb + z0 * HW + y1 * W + x1);
-        float3 c100 = ld3(tb + z1 * HW + y0 * W + x0), c101 = ld3(tb + z1 * HW + y0 * W + x1);
-        float3 c110 = ld3(tb + z1 * HW + y1 * W + x0), c111 = ld3(tb + z1 * HW + y1 * W + x1);
+        const gfloat4 *t0 = tb + row.base, *t1 = t0 + row.dz;
+        float3 c000 = ld3(t0 + x0), c001 = ld3(t0 + x1), c010 = ld3(t0 + row.dy + x0), c011 = ld3(t0 + row.dy + x1);
+        float3 c100 = ld3(t1 + x0), c101 = ld3(t1 + x1), c110 = ld3(t1 + row.dy + x0), c111 = ld3(t1 + row.dy + x1);
         float3 v = lerp3(lerp3(lerp3(c000, c001, ax), lerp3(c010, c011, ax), ay),
                          lerp3(lerp3(c100, c101, ax), lerp3(c110, c111, ax), ay), az);
         out[n] = make_float4(v.x, v.y, v.z, 0.f);
@@ -697,9 +707,18 @@ k_inscatterS(const SetDesc *__restrict__ sets, const uint2 *__restrict__ tiles, 
 
     const LayerGeom L = s.layers[l];
     const double r = fmin(fmax(L.r, s.Rg), s.Rt);          // inscatterS.glsl:112
-    const double muS = fmin(fmax(texel_mus(s, m), -1.0), 1.0);   // :114
     const double rho2 = r * r - s.Rg2;
-    const double txs = tex4d_umus(s, muS) * s.RMUS - 0.5;
+    // rows and the sun's column from the tables, where there are any (k_geometry): their FP64
+    // terms, 2,500 instructions of straight code, were half of a workgroup's set-up
+    const ThetaRow *rowJ = s.rowJ ? s.rowJ + (size_t)l * NS : nullptr;
+    double muS, txs;
+    if (rowJ) {
+        muS = s.sunJ[m].mus;
+        txs = s.sunJ[m].txs;
+    } else {
+        muS = fmin(fmax(texel_mus(s, m), -1.0), 1.0);   // :114
+        txs = tex4d_umus(s, muS) * s.RMUS - 0.5;
+    }
     const float4 *tabs[2] = {s.dSR4, s.dSM4};
     const double posAd = 0.5 * (NU - 1), posBd = posAd + 1.0;
 
@@ -720,7 +739,7 @@ k_inscatterS(const SetDesc *__restrict__ sets, const uint2 *__restrict__ tiles, 
 
     // per-layer scattering coefficients (phase constants folded in)
     const double hr = r - s.Rg;
-    const float eR = (float)exp(-hr / s.HR), eM = (float)exp(-hr / s.HM);
+    const float eR = rowJ ? rowJ[0].eR : (float)exp(-hr / s.HR), eM = rowJ ? rowJ[0].eM : (float)exp(-hr / s.HM);
     const float A0 = s.bR[0] * eR * s.kR, A1 = s.bR[1] * eR * s.kR, A2 = s.bR[2] * eR * s.kR;
     const float B0 = s.bMS[0] * eM * s.kM, B1 = s.bMS[1] * eM * s.kM, B2 = s.bMS[2] * eM * s.kM;
     const float iposA = (float)(1.0 / posAd), nposBi = (float)((0.5 - posBd) / posAd);   // nu1 from u
@@ -743,11 +762,10 @@ k_inscatterS(const SetDesc *__restrict__ sets, const uint2 *__restrict__ tiles, 
         if (CHUNK && c0 > 0) __syncthreads();   // every thread is done with the previous chunk's rows
         // (1) slice values V[it][kk], kk = slice + 1
         auto slice_value = [&](int it, int kk, float4 v[NT]) {
-            const double ct = cos((it + 0.5) * (kPI / NS));
-            const double rmu = r * ct;
-            double tz, ty;
-            tex4d_rmu(s, rho2, rmu, rmu * rmu - rho2, ct, tz, ty);
-            stage_slice<NT>(s, tabs, tz, ty, txs, kk - 1, v);
+            ThetaRow row;
+            if (rowJ) row = rowJ[it];
+            else theta_taps(s, r, rho2, cos((it + 0.5) * (kPI / NS)), row);
+            stage_slice<NT>(s, tabs, row, txs, kk - 1, v);
             if (FIRST) {  // fold the phase-function constants in
                 v[0].x *= s.kR; v[0].y *= s.kR; v[0].z *= s.kR;
                 v[NT - 1].x *= s.kM; v[NT - 1].y *= s.kM; v[NT - 1].z *= s.kM;
@@ -763,28 +781,45 @@ k_inscatterS(const SetDesc *__restrict__ sets, const uint2 *__restrict__ tiles, 
         // the theta-uniform parts of the lookup positions
         for (int itl = threadIdx.x; itl < nth; itl += blockDim.x) {
             const int it = c0 + itl;
-            const double ct = cos((it + 0.5) * (kPI / NS));
-            const double q = s.Rg / r;
-            const double cthetamin = -sqrt(1.0 - q * q);
+            const double sc = s.SW / 1.2;
+            double ct, e1 = 0.0;   // e1: E texels per unit of nu1
+            float dwt;
+            bool ground;
+            float3 tr = make_float3(0.f, 0.f, 0.f);
+            if (rowJ) {
+                const float4 t = s.tground[(size_t)l * NS + it];
+                ct = rowJ[it].ct;
+                e1 = rowJ[it].e1;
+                dwt = rowJ[it].dw;
+                ground = t.w != 0.0f;
+                tr = f3(t);
+            } else {
+                ct = cos((it + 0.5) * (kPI / NS));
+                dwt = (float)((kPI / NS) * (kPI / NS) * sin((it + 0.5) * (kPI / NS)));
+                const double q = s.Rg / r;
+                ground = ct < -sqrt(1.0 - q * q);
+                if (ground) {
+                    const double dg = -r * ct - sqrt(r * r * (ct * ct - 1.0) + s.Rg2);
+                    const double mug = -(r * ct + dg) / s.Rg;
+                    // transmittance(Rg, mug, dg) (common.glsl:272-282); its end point is x itself
+                    const double r1sq = s.Rg2 + dg * dg + 2.0 * s.Rg * mug * dg;
+                    const double r1 = sqrt(r1sq);
+                    const double mu1 = (s.Rg * mug + dg) / r1;
+                    const float h1 = (float)((r1sq - s.Rg2) / (r1 + s.Rg));
+                    tr = s.tground ? ld3(gptr(s.tground) + (size_t)l * NS + it)
+                       : mug > 0.0 ? T_ratio_lin(s, 0.0f, (float)mug, h1, (float)mu1)
+                                   : T_ratio_lin(s, h1, (float)-mu1, 0.0f, (float)-mug);
+                    e1 = dg / s.Rg * sc;
+                }
+            }
             float4 g0 = make_float4(0.f, 0.f, 0.f, 0.f);
             double c1 = 0.0, ce0 = 0.0;
             int jlo = 0, jhi = 0;
-            if (ct < cthetamin) {
-                const double dg = -r * ct - sqrt(r * r * (ct * ct - 1.0) + s.Rg2);
-                const double mug = -(r * ct + dg) / s.Rg;
-                // transmittance(Rg, mug, dg) (common.glsl:272-282); its end point is x itself
-                const double r1sq = s.Rg2 + dg * dg + 2.0 * s.Rg * mug * dg;
-                const double r1 = sqrt(r1sq);
-                const double mu1 = (s.Rg * mug + dg) / r1;
-                const float h1 = (float)((r1sq - s.Rg2) / (r1 + s.Rg));
-                const float3 tr = s.tground ? ld3(gptr(s.tground) + (size_t)l * NS + it)
-                                  : mug > 0.0 ? T_ratio_lin(s, 0.0f, (float)mug, h1, (float)mu1)
-                                              : T_ratio_lin(s, h1, (float)-mu1, 0.0f, (float)-mug);
+            if (ground) {
                 const float gr = (float)(s.alpha / kPI);
                 g0 = make_float4(gr * tr.x, gr * tr.y, gr * tr.z, 1.0f);
                 // E texel coordinate ((r muS + dg nu1)/Rg + 0.2)/1.2 SW - 0.5 as c1 u + ce0
-                const double sc = s.SW / 1.2;
-                const double e1 = dg / s.Rg * sc, e0 = (r * muS / s.Rg + 0.2) * sc - 0.5 + EPAD;
+                const double e0 = (r * muS / s.Rg + 0.2) * sc - 0.5 + EPAD;
                 c1 = e1 / posAd;
                 ce0 = e0 + e1 * (0.5 - posBd) / posAd;   // xg = c1 u + ce0
                 // E cells the lookups of this row can reach: positions [1, NU] up to rounding
@@ -798,8 +833,7 @@ k_inscatterS(const SetDesc *__restrict__ sets, const uint2 *__restrict__ tiles, 
             }
             gdat[3 * itl] = g0;
             // order 2's ground lookup takes xg - 1/2 (its entries' coordinate)
-            gdat[3 * itl + 1] = make_float4((float)c1, (float)(FIRST ? ce0 - 0.5 : ce0), (float)(posAd * muS * ct + posBd - 0.5),
-                                            (float)((kPI / NS) * (kPI / NS) * sin((it + 0.5) * (kPI / NS))));
+            gdat[3 * itl + 1] = make_float4((float)c1, (float)(FIRST ? ce0 - 0.5 : ce0), (float)(posAd * muS * ct + posBd - 0.5), dwt);
             gdat[3 * itl + 2] = make_float4(__int_as_float(jlo), __int_as_float(jhi),
                                             __int_as_float(FIRST ? NP : NP + (jhi - jlo)), 0.f);
         }
@@ -1186,7 +1220,8 @@ __global__ __launch_bounds__(256) void k_irradianceN(const SetDesc *__restrict__
     const double r = s.Rg + h;
     const double muS = -0.2 + (double)i / (s.SW - 1.0) * (1.0 + 0.2);
     const double rho2 = h * (2.0 * s.Rg + h);
-    const double txs = tex4d_umus(s, muS) * s.RMUS - 0.5;
+    const ThetaRow *rowE = s.rowE ? s.rowE + (size_t)j * NTH : nullptr;
+    const double txs = rowE ? s.sunE[i].txs : tex4d_umus(s, muS) * s.RMUS - 0.5;
     const float4 *tabs[2] = {s.dSR4, s.dSM4};
     const float sx = (float)sqrt(fmax(1.0 - muS * muS, 0.0)), sz = (float)muS;
     const float posA = 0.5f * (NU - 1), posB = 0.5f * (NU - 1) + 1.0f;
@@ -1196,12 +1231,11 @@ __global__ __launch_bounds__(256) void k_irradianceN(const SetDesc *__restrict__
         if (c0 > 0) __syncthreads();   // every thread is done with the previous chunk's rows
         for (int e = threadIdx.x; e < nth * NV; e += blockDim.x) {
             const int it = c0 + e / NV, kk = e % NV;
-            const double ct = cos((it + 0.5) * (kPI / NI));
-            const double rmu = r * ct;
-            double tz, ty;
-            tex4d_rmu(s, rho2, rmu, rmu * rmu - rho2, ct, tz, ty);
+            ThetaRow row;
+            if (rowE) row = rowE[it];
+            else theta_taps(s, r, rho2, cos((it + 0.5) * (kPI / NI)), row);
             float4 v[NT];
-            stage_slice<NT>(s, tabs, tz, ty, txs, kk - 1, v);
+            stage_slice<NT>(s, tabs, row, txs, kk - 1, v);
             if (FIRST) {
                 v[0].x *= s.kR; v[0].y *= s.kR; v[0].z *= s.kR;
                 v[NT - 1].x *= s.kM; v[NT - 1].y *= s.kM; v[NT - 1].z *= s.kM;
@@ -1635,23 +1669,20 @@ __global__ __launch_bounds__(256) void k_snview(const SetDesc *__restrict__ sets
 }
 
 // ---------------------------------------------------------------------------
-// Transmittance tables of one precompute (after the T pass, before the passes
-// that use them): every ratio T(x)/T(y) of common.glsl:272-282 the later passes
-// take depends only on the T table and the geometry, not on the order.
-//  k_tview:   T(r, mu, t_i), times the trapezoid weight of sample i, along the view ray of each (layer, mu row) at the
-//             inscatter samples t_i = i limit(r, mu) / nsamp (inscatter1.glsl,
-//             inscatterN.glsl), same tiles as k_inscatter1;
-//  k_tground: T from the ground point seen in direction theta to the layer
-//             radius (inscatterS.glsl:129-138), per (layer, theta row); run on
-//             the dJ tiles, by the workgroup of mu_s column 0 of each layer.
+// Geometry and transmittance tables of one precompute (after the T pass, before the
+// passes that use them): every ratio T(x)/T(y) of common.glsl:272-282 the later passes
+// take, and the table rows of their integrals, depend only on the T table and the
+// geometry, not on the order.  One launch, the theta rows' workgroups first:
+//  theta_items: T from the ground point seen in direction theta to the layer
+//             radius (inscatterS.glsl:129-138) per (layer, theta row), and the rows
+//             and columns of the dJ and dE integrals (ThetaRow, SunColumn);
+//  view_item: T(r, mu, t_i), times the trapezoid weight of sample i, along the view ray
+//             of each (layer, mu row) at the inscatter samples t_i = i limit(r, mu) / nsamp
+//             (inscatter1.glsl, inscatterN.glsl).
 // Both use T_ratio_d (FP64 coordinates; underflow-free with the optical-depth
 // table).
 // ---------------------------------------------------------------------------
-__global__ __launch_bounds__(256) void k_tview(const SetDesc *__restrict__ sets,
-                                               const uint2 *__restrict__ tiles, int nsamp) {
-    const uint2 tl = tiles[blockIdx.x];
-    const SetDesc &s = sets[tl.x];
-    const size_t e = ((size_t)tl.y * kTileY + blockIdx.y) * 256 + threadIdx.x;
+__device__ __forceinline__ void view_item(const SetDesc &s, size_t e, int nsamp) {
     const int line = (int)(e / (nsamp + 1)), i = (int)(e % (nsamp + 1));
     if (line >= s.RR * s.RMU) return;
     const LayerGeom L = s.layers[line / s.RMU];
@@ -1671,18 +1702,19 @@ __global__ __launch_bounds__(256) void k_tview(const SetDesc *__restrict__ sets,
     s.tview[e] = make_float4(t.x * wt, t.y * wt, t.z * wt, (float)(ti / ri));
 }
 
-__global__ __launch_bounds__(256) void k_tground(const SetDesc *__restrict__ sets,
-                                                 const uint2 *__restrict__ tiles, int NS) {
-    const uint2 tl = tiles[blockIdx.x];
-    const SetDesc &s = sets[tl.x];
-    if ((int)tl.y % s.RMUS != 0) return;   // one workgroup per layer
-    const int l = (int)tl.y / s.RMUS;
-    const double r = fmin(fmax(s.layers[l].r, s.Rg), s.Rt);   // inscatterS.glsl:112
-    for (int it = threadIdx.x; it < NS; it += blockDim.x) {
-        const double ct = cos((it + 0.5) * (kPI / NS));
-        const double q = s.Rg / r;
+// Item e of a set's theta tables: ground transmittances of the dJ rows, the dJ rows, the
+// dE rows, the columns, each kind from a multiple of 64 on (a wave has one kind).
+__host__ __device__ __forceinline__ int theta_pad(int n) { return (n + 63) & ~63; }
+__device__ __forceinline__ void theta_items(const SetDesc &s, int e, int NS, int NI) {
+    const int nJ = s.RR * NS, NTH = NI / 2, nE = s.SH * NTH;
+    auto layer_r = [&](int l) { return fmin(fmax(s.layers[l].r, s.Rg), s.Rt); };   // inscatterS.glsl:112
+    if (e < theta_pad(nJ)) {
+        if (e >= nJ) return;
+        const double r = layer_r(e / NS), ct = cos((e % NS + 0.5) * (kPI / NS)), q = s.Rg / r;
         float3 tr = make_float3(0.f, 0.f, 0.f);
-        if (ct < -sqrt(1.0 - q * q)) {
+        double e1 = 0.0;
+        const bool ground = ct < -sqrt(1.0 - q * q);
+        if (ground) {
             const double dg = -r * ct - sqrt(r * r * (ct * ct - 1.0) + s.Rg2);
             const double mug = -(r * ct + dg) / s.Rg;
             const double r1sq = s.Rg2 + dg * dg + 2.0 * s.Rg * mug * dg;
@@ -1690,8 +1722,58 @@ __global__ __launch_bounds__(256) void k_tground(const SetDesc *__restrict__ set
             const double mu1 = (s.Rg * mug + dg) / r1;
             const double h1 = (r1sq - s.Rg2) / (r1 + s.Rg);
             tr = mug > 0.0 ? T_ratio_d(s, 0.0, mug, h1, mu1) : T_ratio_d(s, h1, -mu1, 0.0, -mug);
+            e1 = dg / s.Rg * (s.SW / 1.2);
         }
-        s.tground[(size_t)l * NS + it] = make_float4(tr.x, tr.y, tr.z, 0.f);
+        s.tground[e] = make_float4(tr.x, tr.y, tr.z, ground ? 1.f : 0.f);
+        if (s.rowJ) s.rowJ[e].e1 = e1;
+        return;
+    }
+    e -= theta_pad(nJ);
+    if (!s.rowJ) return;
+    if (e < theta_pad(nJ)) {
+        if (e >= nJ) return;
+        const double r = layer_r(e / NS), th = (e % NS + 0.5) * (kPI / NS), hr = r - s.Rg;
+        ThetaRow row;
+        row.ct = cos(th);
+        theta_taps(s, r, r * r - s.Rg2, row.ct, row);
+        ThetaRow &o = s.rowJ[e];   // all but e1
+        o.ct = row.ct;
+        o.base = row.base; o.dy = row.dy; o.dz = row.dz;
+        o.ay = row.ay; o.az = row.az;
+        o.dw = (float)((kPI / NS) * (kPI / NS) * sin(th));
+        o.eR = (float)exp(-hr / s.HR);
+        o.eM = (float)exp(-hr / s.HM);
+        return;
+    }
+    e -= theta_pad(nJ);
+    if (e < theta_pad(nE)) {
+        if (e >= nE) return;
+        const double h = (double)(e / NTH) / (s.SH - 1.0) * (s.Rt - s.Rg);
+        ThetaRow row = {};
+        row.ct = cos((e % NTH + 0.5) * (kPI / NI));
+        theta_taps(s, s.Rg + h, h * (2.0 * s.Rg + h), row.ct, row);
+        s.rowE[e] = row;
+        return;
+    }
+    e -= theta_pad(nE);
+    if (e >= s.SW + s.RMUS) return;
+    SunColumn c;
+    c.mus = e < s.SW ? -0.2 + (double)e / (s.SW - 1.0) * (1.0 + 0.2) : fmin(fmax(texel_mus(s, e - s.SW), -1.0), 1.0);
+    c.txs = tex4d_umus(s, c.mus) * s.RMUS - 0.5;
+    (e < s.SW ? s.sunE[e] : s.sunJ[e - s.SW]) = c;
+}
+
+// ntheta workgroups of theta items, wpt of them per set, then nview tiles of view items
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void
+k_geometry(const SetDesc *__restrict__ sets, const uint2 *__restrict__ tiles, int ntheta, int wpt, int nview, int nsamp, int NS,
+           int NI) {
+    const int b = (int)blockIdx.x;
+    if (b < ntheta) {
+        theta_items(sets[b / wpt], (b % wpt) * 256 + (int)threadIdx.x, NS, NI);
+    } else {
+        const int v = b - ntheta;
+        const uint2 tl = tiles[v % nview];
+        view_item(sets[tl.x], ((size_t)tl.y * kTileY + v / nview) * 256 + threadIdx.x, nsamp);
     }
 }
 
@@ -1774,14 +1856,15 @@ hipError_t launch_transmittance(const SetDesc *sets, const uint2 *tiles, int nti
     hipLaunchKernelGGL(k_transmittance, dim3(ntiles, kTileY), dim3(256), 0, st, sets, tiles, nsamp);
     return hipGetLastError();
 }
-hipError_t launch_tview(const SetDesc *sets, const uint2 *tiles, int ntiles, int nsamp, hipStream_t st) {
-    if (ntiles <= 0) return hipSuccess;
-    hipLaunchKernelGGL(k_tview, dim3(ntiles, kTileY), dim3(256), 0, st, sets, tiles, nsamp);
-    return hipGetLastError();
+int theta_workgroups(int RR, int RMUS, int SW, int SH, int NS, int NI) {
+    return (2 * theta_pad(RR * NS) + theta_pad(SH * (NI / 2)) + SW + RMUS + 255) / 256;
 }
-hipError_t launch_tground(const SetDesc *sets, const uint2 *tiles, int ntiles, int NS, hipStream_t st) {
-    if (ntiles <= 0) return hipSuccess;
-    hipLaunchKernelGGL(k_tground, dim3(ntiles), dim3(64), 0, st, sets, tiles, NS);
+hipError_t launch_geometry(const SetDesc *sets, int nsets, int wpt, const uint2 *tiles, int nview, int nsamp, int NS, int NI,
+                           hipStream_t st) {
+    if (nview <= 0) return hipSuccess;
+    const int ntheta = nsets * wpt;
+    hipLaunchKernelGGL(k_geometry, dim3(ntheta + nview * kTileY), dim3(256), 0, st, sets, tiles, ntheta, std::max(wpt, 1), nview,
+                       nsamp, NS, NI);
     return hipGetLastError();
 }
 hipError_t launch_irradiance1(const SetDesc *sets, const uint2 *tiles, int ntiles,
