@@ -227,13 +227,15 @@ def main():
     # second kernel: the dSn pass.  Its HBM traffic is a fraction of peak; what
     # it moves is on-chip: per view ray (r layer, mu row) and sample, the staged
     # form blends the 4 dJ rows around the sample (2 layers x 2 mu rows,
-    # RES_NU*RES_MU_S texels of 12 bytes each) into LDS.
+    # RES_NU*RES_MU_S texels of 12 bytes each) into LDS; a row that the sample before
+    # it had too stays in registers, so 2.6 of 4 are loaded per sample at this size.
     tu = eng.tuning()
-    sn_name = "k_inscatterN<%s,false>" % ("true" if tu.get("inscatterN_staged_samples", 0) else "false")
+    sn_texels = -(-p.RES_NU * p.RES_MU_S // 512)    # per thread: rows of more than 512 texels take 2
+    sn_name = "k_inscatterN<%d,false,%d>" % (1 if tu.get("inscatterN_staged_samples", 0) else 0, sn_texels)
     sn_ms = [ms for name, order, ms in times if name == "inscatterN"]
     sn_avg = sum(sn_ms) / len(sn_ms)
     sn_traffic = profiled(TRAFFIC_PROFILE, "traffic", sn_name)
-    row_reads = (p.RES_R * p.RES_MU * (o.inscatter_samples + 1) * 4 * p.RES_NU * p.RES_MU_S * 12)
+    row_reads = int(p.RES_R * p.RES_MU * (o.inscatter_samples + 1) * 2.6 * p.RES_NU * p.RES_MU_S * 12)
     second = {"kernel": sn_name + " (dSn pass, orders 2-%d)" % o.orders,
               "bound": "on-chip: dJ rows gathered per view-ray sample (L2 -> LDS)",
               "avg_launch_ms": round(sn_avg, 4), "launches": len(sn_ms),

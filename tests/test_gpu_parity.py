@@ -625,6 +625,23 @@ def test_reference_configuration_half_storage_against_golden_samples(eng):
             assert steps <= 4.0, (name, steps)
 
 
+@pytest.mark.parametrize("NS,NI", [(5, 6), (4, 2), (16, 32)])
+@pytest.mark.parametrize("lin", [0, 64])
+def test_theta_tables_at_their_edges(eng, NS, NI, lin):
+    """The table of theta rows and sun columns (k_geometry) has its kinds of items padded
+    to waves and one number of workgroups for all sets of a batch: 65, 64 and 2 x NS
+    layer rows, irradiance tables of 2 x 2 and more than a wave of rows, the smallest
+    slices, in one batch; against the oracle at the chain's bar."""
+    o = options(flags=8 | lin, orders=3, spherical_samples=NS, irradiance_samples=NI, inscatter_samples=8,
+                transmittance_samples=60)
+    sets = [small(res=(13, 8, 3, 3), E=(9, 13)), small(res=(64 // NS + 1, 6, 2, 2), E=(2, 2)), small(res=(2, 8, 9, 4), E=(70, 3))]
+    outs = eng.precompute(sets, o)
+    torch.cuda.synchronize()
+    for p, got in zip(sets, outs):
+        for name, x, y in zip("TES", got, O.precompute(p, o)):
+            _assert(name, x.double().cpu().numpy(), y, TOL)
+
+
 # ---------------------------------------------------------------- batching and graphs
 @pytest.mark.parametrize("G,form", [(0, 0), (4, 3)])
 def test_mixed_resolution_batch_equals_single_runs(eng, G, form):
