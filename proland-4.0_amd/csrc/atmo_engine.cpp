@@ -293,6 +293,9 @@ struct DevBuf {
         n = 0;
         hipError_t e = hipMalloc(&p, std::max<size_t>(bytes, 256));
         if (e == hipSuccess) n = bytes;
+        // reported here, and not left pending for the next launch's hipGetLastError (a
+        // later success does not clear it)
+        else (void)hipGetLastError();
         return e;
     }
 };

@@ -70,6 +70,7 @@ struct Buf {
         n = 0;
         hipError_t e = hipMalloc(&p, std::max<size_t>(bytes, 256));
         if (e == hipSuccess) n = bytes;
+        else (void)hipGetLastError();   // not left pending for the next launch
         return e;
     }
     template <class T> T *as() const { return (T *)p; }

@@ -1,0 +1,98 @@
+"""CPU tests of the engine's host code: csrc/atmo_engine.cpp and the launchers of
+csrc/atmo_kernels.hip, compiled for the host only and linked with a host-side HIP
+runtime (native/fake_hip.cpp) that can refuse memory and launches.  Kernels do not run."""
+import ctypes
+import os
+import re
+import shutil
+import subprocess
+
+import pytest
+
+from prolandatmo import lib as L
+from prolandatmo.params import FLAG_NO_AUTOTUNE, AtmoParams, earth, options, with_res
+
+REPO = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+CSRC = os.path.join(REPO, "proland-4.0_amd", "csrc")
+HIPCC = shutil.which("hipcc") or "/opt/rocm/bin/hipcc"
+OK, DEVICE, OOM = 0, 2, 3
+
+
+@pytest.fixture(scope="module")
+def host(tmp_path_factory):
+    d = tmp_path_factory.mktemp("engine_host")
+    host = [HIPCC, "--offload-arch=gfx950", "--offload-host-only", "-O1", "-std=c++17", "-fPIC", "-w", "-x", "hip", "-c"]
+    objs = []
+    for name, src in (("engine", "atmo_engine.cpp"), ("kernels", "atmo_kernels.hip")):
+        objs.append(str(d / (name + ".o")))
+        subprocess.check_call(host + ["-cuid=" + name, os.path.join(CSRC, src), "-o", objs[-1]])
+    native = os.path.join(REPO, "tests", "native")
+    objs.append(str(d / "fake.o"))
+    subprocess.check_call(["g++", "-D__HIP_PLATFORM_AMD__", "-I/opt/rocm/include", "-O1", "-std=c++17", "-fPIC", "-w", "-c",
+                           os.path.join(native, "fake_hip.cpp"), "-o", objs[-1]])
+    so = str(d / "engine_host.so")
+    device_code = set(re.findall(r"__hip_fatbin_\w+", subprocess.check_output(["nm"] + objs, text=True)))
+    # every symbol bound inside the library: the process may hold the real runtime too
+    subprocess.check_call(["g++", "-shared", "-Wl,-Bsymbolic", "-o", so] + objs +
+                          ["-Wl,--defsym=%s=fake_fatbin" % s for s in sorted(device_code)])
+    lib = ctypes.CDLL(so)
+    for name, (res, args) in L.SIGNATURES.items():
+        if hasattr(lib, name):
+            getattr(lib, name).restype, getattr(lib, name).argtypes = res, args
+    lib.fake_memory_limit.argtypes = [ctypes.c_size_t]
+    lib.fake_in_use.restype = ctypes.c_size_t
+    return lib
+
+
+class Engine:
+    """The C ABI's engine on the host runtime; outputs are addresses that nothing reads."""
+
+    def __init__(self, lib):
+        self.lib, self.h = lib, ctypes.c_void_p()
+        lib.fake_reset()
+        assert lib.atmo_engine_create(ctypes.byref(self.h), 0) == OK
+
+    def __enter__(self):
+        return self
+
+    def __exit__(self, *a):
+        self.lib.fake_reset()
+        self.lib.atmo_engine_destroy(self.h)
+
+    def precompute(self, p, o, stream=1):
+        sets = (AtmoParams * 1)(p)
+        out = (L.AtmoTables * 1)(L.AtmoTables(0x1000, 0x2000, 0x3000))
+        return self.lib.atmo_engine_precompute(self.h, sets, 1, ctypes.byref(o), out, ctypes.c_void_p(0x100 * stream))
+
+
+def small(k=0):
+    p = with_res(earth(), 4, 8, 4, 2)
+    p.HR = 8.0 + 0.125 * k
+    return p
+
+
+def plain(orders=4):
+    return options(orders=orders, flags=FLAG_NO_AUTOTUNE)
+
+
+def test_precompute_without_room_for_the_view_samples(host):
+    """A set whose work memory fits only without the table of view-ray samples and the
+    theta rows is computed without them: the refused allocation leaves no error behind."""
+    p, o = small(), plain()
+    with Engine(host) as e:
+        assert e.precompute(p, o) == OK
+        full, launches = host.fake_in_use(), host.fake_launch_count()
+    with Engine(host) as e:
+        host.fake_memory_limit(full - 1024)
+        assert e.precompute(p, o) == OK, host.atmo_last_error()
+        assert host.fake_in_use() < full - 1024
+        assert host.fake_launch_count() == launches - 1   # all but the view samples' kernel
+        assert host.fake_pending() == 0
+
+
+def test_precompute_after_one_that_did_not_fit(host):
+    with Engine(host) as e:
+        host.fake_memory_limit(1 << 16)
+        assert e.precompute(small(), plain()) == OOM
+        host.fake_memory_limit(1 << 40)
+        assert e.precompute(small(1), plain()) == OK, host.atmo_last_error()
