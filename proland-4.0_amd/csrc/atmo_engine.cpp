@@ -421,8 +421,9 @@ struct Plan {
     int snXcd = 1;     // k_inscatterN XCD-banded tile order
     int snForm = 1;    // k_inscatterN: 0 direct gathers, 1 LDS-staged rows
     bool tuned = false;
-    int runs = 0;                  // run_plan calls
-    hipEvent_t done = nullptr;     // behind the launches of the first run, while runs == 1
+    bool ran = false;              // run_plan has been called
+    hipEvent_t done = nullptr;
+    bool done_behind = false;      // `done` is behind everything that the plan has launched
     std::vector<std::vector<char>> staged;   // host sides of the uploads in flight on xs
     // Asynchronous upload; complete once xs has been waited for (uploaded()).
     template <class T>
@@ -1142,8 +1143,9 @@ size_t plan_bytes(const std::vector<atmo_params> &ps, const atmo_options &o, int
 // leaves Plan::done behind; the graph is captured on the second.
 atmo_status run_plan(atmo_engine *e, Plan &pl, const atmo_options &o, hipStream_t hs) {
     atmo_status st;
-    const bool first = pl.runs == 0;
-    pl.runs = std::min(pl.runs, 2) + 1;
+    const bool first = !pl.ran;
+    pl.ran = true;
+    pl.done_behind = false;
     if (o.flags & ATMO_FLAG_TIME_PASSES) {
         PassTimer tm;
         tm.on = true;
@@ -1158,8 +1160,14 @@ atmo_status run_plan(atmo_engine *e, Plan &pl, const atmo_options &o, hipStream_
     } else if (first || (o.flags & ATMO_FLAG_NO_GRAPH)) {
         if ((st = launch_all(pl, hs)) != ATMO_OK) return st;
         if (first) {
-            if (!pl.done) HIPCHK(hipEventCreateWithFlags(&pl.done, hipEventDisableTiming));
-            HIPCHK(hipEventRecord(pl.done, hs));
+            // (an event recorded into a caller's capture could not be waited for outside it)
+            hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+            if (hs) HIPCHK(hipStreamIsCapturing(hs, &cap));
+            if (cap == hipStreamCaptureStatusNone) {
+                if (!pl.done) HIPCHK(hipEventCreateWithFlags(&pl.done, hipEventDisableTiming));
+                HIPCHK(hipEventRecord(pl.done, hs));
+                pl.done_behind = true;
+            }
         }
     } else {
         hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
@@ -1198,7 +1206,7 @@ atmo_status run_plan(atmo_engine *e, Plan &pl, const atmo_options &o, hipStream_
 
 // Replaces the engine's plan.  A plan that has run once, eagerly, may still be at work
 // (a caller that changes its parameters on every call): the new one is built while it
-// is, takes over its work arena (ordered by its event) and the small buffers of the
+// is (Plan::done_behind), takes over its work arena (ordered by its event) and the small buffers of the
 // plan before it (waited for), so that the device does not idle while the host builds:
 // two 32x128x32x8 sets, other ones in every pass, 2.93 -> 2.38 ms (of it 2.25 of kernels).
 // Any other plan, or an arena that is too small or more than twice too large, is
@@ -1212,7 +1220,7 @@ atmo_status change_plan(atmo_engine *e, const atmo_params *sets, int nsets, cons
     for (int i = 0; i < nsets; ++i) total += work_bytes(sets[i], o, true);
     Plan *old = e->plan.get();
     std::unique_ptr<Plan> into;
-    if (old && old->runs == 1 && old->done && total <= old->arena.n && old->arena.n / 2 <= total) {
+    if (old && old->done_behind && total <= old->arena.n && old->arena.n / 2 <= total) {
         into.reset(new Plan);
         if (e->prev) {
             HIPCHK(hipEventSynchronize(e->prev->done));
@@ -1461,6 +1469,7 @@ atmo_status atmo_engine_precompute(atmo_engine *e, const atmo_params *sets, int 
     }
     if ((st = run_plan(e, pl, o, hs)) != ATMO_OK) return st;
     if (tune_after) {
+        pl.done_behind = false;
         if ((st = autotune(pl, hs, tu)) != ATMO_OK) return st;
         {
             std::lock_guard<std::mutex> lk(tuning_mutex());
@@ -1473,7 +1482,10 @@ atmo_status atmo_engine_precompute(atmo_engine *e, const atmo_params *sets, int 
         if ((st = run_plan(e, pl, o, hs)) != ATMO_OK) return st;
     }
     if (o.flags & ATMO_FLAG_CHECK_NUMERICS)
-        if ((st = check_numerics(pl, hs)) != ATMO_OK) return st;
+        if ((st = check_numerics(pl, hs)) != ATMO_OK) {
+            pl.done_behind = false;   // its kernel may still be at work
+            return st;
+        }
     g_err.clear();
     return ATMO_OK;
 }

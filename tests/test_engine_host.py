@@ -96,3 +96,30 @@ def test_precompute_after_one_that_did_not_fit(host):
         assert e.precompute(small(), plain()) == OOM
         host.fake_memory_limit(1 << 40)
         assert e.precompute(small(1), plain()) == OK, host.atmo_last_error()
+
+
+def test_work_memory_of_a_run_that_failed_is_not_handed_over(host):
+    """A plan whose launches fail part way has no event behind the ones that went out:
+    the next plan, on another stream, waits for the device instead of for an event of
+    the plan two before."""
+    with Engine(host) as e:
+        for k in range(2):
+            assert e.precompute(small(k), plain()) == OK
+        host.fake_fail_launch(5)
+        assert e.precompute(small(2), plain()) == DEVICE
+        assert e.precompute(small(3), plain(), stream=2) == OK, host.atmo_last_error()
+        assert e.precompute(small(4), plain(), stream=2) == OK
+        assert host.fake_stale_waits() == 0
+
+
+@pytest.mark.parametrize("after", [1, 2, 3])
+def test_work_memory_is_handed_over_behind_the_last_run(host, after):
+    """Plans that run once on alternating streams, then one that runs `after` times."""
+    with Engine(host) as e:
+        for k in range(4):
+            assert e.precompute(small(k), plain(), stream=1 + k % 2) == OK
+        for _ in range(after):
+            assert e.precompute(small(4), plain(), stream=1) == OK
+        assert e.precompute(small(5), plain(), stream=1) == OK
+        assert host.fake_stale_waits() == 0
+        assert host.fake_pending() == 0
