@@ -1703,10 +1703,11 @@ __device__ __forceinline__ void view_item(const SetDesc &s, size_t e, int nsamp)
 }
 
 // Item e of a set's theta tables: ground transmittances of the dJ rows, the dJ rows, the
-// dE rows, the columns, each kind from a multiple of 64 on (a wave has one kind).
-__host__ __device__ __forceinline__ int theta_pad(int n) { return (n + 63) & ~63; }
-__device__ __forceinline__ void theta_items(const SetDesc &s, int e, int NS, int NI) {
-    const int nJ = s.RR * NS, NTH = NI / 2, nE = s.SH * NTH;
+// dE rows, the columns, each kind from a multiple of 64 on (a wave has one kind).  A kind has
+// at most 2^30 items (2^23 layers or irradiance rows of 128), all of them less than 2^32.
+__host__ __device__ __forceinline__ unsigned theta_pad(unsigned n) { return (n + 63u) & ~63u; }
+__device__ __forceinline__ void theta_items(const SetDesc &s, unsigned e, int NS, int NI) {
+    const unsigned nJ = s.RR * NS, NTH = NI / 2, nE = s.SH * NTH;
     auto layer_r = [&](int l) { return fmin(fmax(s.layers[l].r, s.Rg), s.Rt); };   // inscatterS.glsl:112
     if (e < theta_pad(nJ)) {
         if (e >= nJ) return;
@@ -1756,20 +1757,22 @@ __device__ __forceinline__ void theta_items(const SetDesc &s, int e, int NS, int
         return;
     }
     e -= theta_pad(nE);
-    if (e >= s.SW + s.RMUS) return;
+    const unsigned SW = s.SW;
+    if (e >= SW + s.RMUS) return;
     SunColumn c;
-    c.mus = e < s.SW ? -0.2 + (double)e / (s.SW - 1.0) * (1.0 + 0.2) : fmin(fmax(texel_mus(s, e - s.SW), -1.0), 1.0);
+    c.mus = e < SW ? -0.2 + (double)e / (s.SW - 1.0) * (1.0 + 0.2) : fmin(fmax(texel_mus(s, (int)(e - SW)), -1.0), 1.0);
     c.txs = tex4d_umus(s, c.mus) * s.RMUS - 0.5;
-    (e < s.SW ? s.sunE[e] : s.sunJ[e - s.SW]) = c;
+    (e < SW ? s.sunE[e] : s.sunJ[e - SW]) = c;
 }
 
-// ntheta workgroups of theta items, wpt of them per set, then nview tiles of view items
+// ntheta workgroups of theta items, wpt of them per set from set0 on, then nview tiles of
+// view items
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void
-k_geometry(const SetDesc *__restrict__ sets, const uint2 *__restrict__ tiles, int ntheta, int wpt, int nview, int nsamp, int NS,
-           int NI) {
+k_geometry(const SetDesc *__restrict__ sets, int set0, const uint2 *__restrict__ tiles, int ntheta, int wpt, int nview, int nsamp,
+           int NS, int NI) {
     const int b = (int)blockIdx.x;
     if (b < ntheta) {
-        theta_items(sets[b / wpt], (b % wpt) * 256 + (int)threadIdx.x, NS, NI);
+        theta_items(sets[set0 + b / wpt], (unsigned)(b % wpt) * 256u + threadIdx.x, NS, NI);
     } else {
         const int v = b - ntheta;
         const uint2 tl = tiles[v % nview];
@@ -1857,15 +1860,26 @@ hipError_t launch_transmittance(const SetDesc *sets, const uint2 *tiles, int nti
     return hipGetLastError();
 }
 int theta_workgroups(int RR, int RMUS, int SW, int SH, int NS, int NI) {
-    return (2 * theta_pad(RR * NS) + theta_pad(SH * (NI / 2)) + SW + RMUS + 255) / 256;
+    const long long items = 2LL * theta_pad((unsigned)RR * NS) + theta_pad((unsigned)SH * (NI / 2)) + SW + RMUS;
+    return (int)((items + 255) / 256);
 }
 hipError_t launch_geometry(const SetDesc *sets, int nsets, int wpt, const uint2 *tiles, int nview, int nsamp, int NS, int NI,
                            hipStream_t st) {
     if (nview <= 0) return hipSuccess;
-    const int ntheta = nsets * wpt;
-    hipLaunchKernelGGL(k_geometry, dim3(ntheta + nview * kTileY), dim3(256), 0, st, sets, tiles, ntheta, std::max(wpt, 1), nview,
-                       nsamp, NS, NI);
-    return hipGetLastError();
+    // a launch has less than 2^32 threads: what is beyond takes further ones
+    constexpr int kMost = (1 << 24) - 1;
+    const int each = wpt > 0 ? std::max(1, kMost / wpt) : nsets;   // sets of a launch
+    for (int s0 = 0, v0 = 0; s0 < nsets || v0 < nview;) {
+        const int ns = std::min(nsets - s0, each), ntheta = ns * wpt;
+        const int nv = std::min(nview - v0, (kMost - ntheta) / kTileY);
+        hipLaunchKernelGGL(k_geometry, dim3(ntheta + nv * kTileY), dim3(256), 0, st, sets, s0, tiles + v0, ntheta, std::max(wpt, 1),
+                           nv, nsamp, NS, NI);
+        const hipError_t e = hipGetLastError();
+        if (e != hipSuccess) return e;
+        s0 += ns;
+        v0 += nv;
+    }
+    return hipSuccess;
 }
 hipError_t launch_irradiance1(const SetDesc *sets, const uint2 *tiles, int ntiles,
                               hipStream_t st) {

@@ -23,10 +23,12 @@ def host(tmp_path_factory):
     d = tmp_path_factory.mktemp("engine_host")
     host = [HIPCC, "--offload-arch=gfx950", "--offload-host-only", "-O1", "-std=c++17", "-fPIC", "-w", "-x", "hip", "-c"]
     objs = []
-    for name, src in (("engine", "atmo_engine.cpp"), ("kernels", "atmo_kernels.hip")):
-        objs.append(str(d / (name + ".o")))
-        subprocess.check_call(host + ["-cuid=" + name, os.path.join(CSRC, src), "-o", objs[-1]])
     native = os.path.join(REPO, "tests", "native")
+    for src in (os.path.join(CSRC, "atmo_engine.cpp"), os.path.join(CSRC, "atmo_kernels.hip"),
+                os.path.join(native, "host_calls.cpp")):
+        name = os.path.basename(src).split(".")[0]
+        objs.append(str(d / (name + ".o")))
+        subprocess.check_call(host + ["-cuid=" + name, src, "-o", objs[-1]])
     objs.append(str(d / "fake.o"))
     subprocess.check_call(["g++", "-D__HIP_PLATFORM_AMD__", "-I/opt/rocm/include", "-O1", "-std=c++17", "-fPIC", "-w", "-c",
                            os.path.join(native, "fake_hip.cpp"), "-o", objs[-1]])
@@ -123,3 +125,38 @@ def test_work_memory_is_handed_over_behind_the_last_run(host, after):
         assert e.precompute(small(5), plain(), stream=1) == OK
         assert host.fake_stale_waits() == 0
         assert host.fake_pending() == 0
+
+
+def launches(lib):
+    """(grid, block, dynamic LDS) of every launch so far."""
+    out = []
+    for i in range(lib.fake_launch_count()):
+        grid, block, lds = (ctypes.c_uint * 3)(), ctypes.c_uint(), ctypes.c_size_t()
+        lib.fake_launch(i, grid, ctypes.byref(block), ctypes.byref(lds))
+        out.append((tuple(grid), block.value, lds.value))
+    return out
+
+
+@pytest.mark.parametrize("RR,RMUS,SW,SH,NS,NI", [
+    (32, 32, 64, 16, 16, 32), (2, 2, 2, 2, 1, 2), (64, 64, 64, 16, 32, 32),
+    # the most layers (a table of 2^27 texels) and rows that are accepted, with the most directions
+    (1 << 23, 2, 64, 16, 128, 32), (1 << 23, 2, 2, 1 << 23, 128, 256)])
+def test_theta_table_workgroups(host, RR, RMUS, SW, SH, NS, NI):
+    """Items of the theta tables: ground transmittances and dJ rows, dE rows, columns, the
+    first three each padded to a wave."""
+    pad = lambda n: (n + 63) // 64 * 64
+    items = 2 * pad(RR * NS) + pad(SH * (NI // 2)) + SW + RMUS
+    assert host.call_theta_workgroups(RR, RMUS, SW, SH, NS, NI) == (items + 255) // 256
+
+
+@pytest.mark.parametrize("nsets,wpt,nview", [
+    (1, 11, 51), (3, 0, 7), (1, 1 << 23, 1 << 21), (2, 12_600_000, 3), (1, 2, 5_000_000), (40_000, 1000, 1), (3, 0, 3_000_000)])
+def test_geometry_launches_stay_below_2_to_32_threads(host, nsets, wpt, nview):
+    host.fake_reset()
+    assert host.call_launch_geometry(nsets, wpt, nview) == 0
+    total = 0
+    for grid, block, _ in launches(host):
+        assert block == 256 and grid[1] == grid[2] == 1
+        assert grid[0] * block < 1 << 32
+        total += grid[0]
+    assert total == nsets * wpt + 16 * nview
