@@ -1894,7 +1894,9 @@ hipError_t launch_irradiance1(const SetDesc *sets, const uint2 *tiles, int ntile
 // 21x90x27x5 (135) 58 / 54 / 48 / 85 (spills), 64x256x64x16 (1024, 512 columns)
 // - / 1434 / 1932 / 1143.  So: four columns per thread only where no spill
 // comes with them (three texels).  More columns than that cost more than the gathers
-// they save, and rows of at most 64 texels gather (k_inscatter1's slots).
+// they save, and rows of at most 64 texels gather (k_inscatter1's slots).  The most LDS is
+// that of 3 texels and 4 columns with 384 threads, for 961 to 1024 texels and T of 1536
+// columns: 60 KB dynamic and 4 KB static, of the 160 KB a workgroup can have.
 S1Shape s1_shape(int W4, int TW, bool linT) {
     const int ax = linT ? kSunLin : TW > kXkMax ? kSunWide : TW < kXkMin ? kSunFew : kSunTab;
     S1Shape best = {ax, 0, 0, 256};

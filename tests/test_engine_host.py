@@ -160,3 +160,21 @@ def test_geometry_launches_stay_below_2_to_32_threads(host, nsets, wpt, nview):
         assert grid[0] * block < 1 << 32
         total += grid[0]
     assert total == nsets * wpt + 16 * nview
+
+
+@pytest.mark.parametrize("linear", [0, 1])
+def test_inscatter1_shapes_cover_the_row_and_fit_the_lds(host, linear):
+    """Every row length and T widths from the least to past the staged columns: a staged
+    launch covers the row's texels and T's columns, and takes at most 64 KB of dynamic LDS."""
+    largest = 0
+    for W4 in range(4, 1025):
+        for TW in (2, 63, 64, 128, 256, 257, 512, 1000, 1024, 1025, 1403, 1404, 1536, 1537, 2048, 2049, 4096):
+            shape = (ctypes.c_int * 3)()
+            host.fake_reset()
+            assert host.call_inscatter1(W4, TW, linear, shape) == 0
+            (grid, block, lds), = launches(host)
+            texels, columns, threads = shape
+            assert block == threads <= 512 and lds <= 64 * 1024
+            assert texels == 0 or (texels * threads >= W4 and columns * threads >= TW)
+            largest = max(largest, lds)
+    assert largest == (32 * (4 * 384 + 1) + (0 if linear else 8 * 1536))

@@ -909,6 +909,21 @@ def test_inscatter1_workgroup_shapes(eng, res, tw, samples, lin):
     _assert("S", a[2].double().cpu().numpy(), S, TOL)
 
 
+@pytest.mark.parametrize("lin", [0, FLAG_LINEAR_TRANSMITTANCE])
+@pytest.mark.parametrize("res,tw", [((2, 16, 64, 16), 1403), ((2, 16, 64, 16), 1404), ((2, 16, 64, 16), 1536),
+                                    ((2, 16, 64, 16), 1537), ((2, 16, 62, 16), 1200), ((2, 16, 64, 15), 1536)])
+def test_inscatter1_largest_staging(eng, res, tw, lin):
+    """The largest staging of the single-scattering rows (3 texels and 4 columns per
+    thread, 384 threads: rows of 961 to 1024 texels with 1025 to 1536 columns) and the
+    shapes beside it, within the bar of the whole-chain tests."""
+    p = small(res=res, T=(tw, 12))
+    kw = dict(orders=1, inscatter_samples=12, transmittance_samples=100, flags=8 | lin)
+    S4 = eng.precompute(p, options(**kw))[0][2]
+    torch.cuda.synchronize()
+    T, E, S = O.precompute(p, options(**kw))
+    _assert("S", S4.double().cpu().numpy(), S, TOL)
+
+
 @pytest.mark.parametrize("ci", range(len(CASES)))
 @pytest.mark.parametrize("form", [2, 3])
 def test_pass_inscatterN_staged_form(eng, ci, form):
