@@ -74,8 +74,9 @@ __device__ __forceinline__ float3 T_at(const CDesc &d, double r, double mu) {
     return rgb_bilinear(d.T, d.TW, d.TH, uMu * d.TW - 0.5f, uR * d.TH - 0.5f);
 }
 
-// 1/x in FP64 from the hardware estimate and Newton steps, a few ulp (as sqrt64): what
-// follows rounds to a texel coordinate
+// 1/x in FP64 from the hardware estimate (4.5e-8) and Newton steps: 1.11e-16 relative over
+// 1e-6 .. 3e7, as a division.  NaN at 0 and infinity: a point without a direction, which
+// is NaN in any case (0 / 0), or at the planet's centre, likewise.
 __device__ __forceinline__ double rcp64(double x) {
     double y = __builtin_amdgcn_rcp(x);
     y = fma(y, fma(-x, y, 1.0), y);
@@ -83,11 +84,12 @@ __device__ __forceinline__ double rcp64(double x) {
 }
 
 // texture4D's mu axis (atmosphereShader.glsl:175-199, INSCATTER_NON_LINEAR) as a texel
-// coordinate; the ground branch in the cancellation-free form -rho / (sqrt(delta) - r mu)
+// coordinate; the ground branch in the cancellation-free form -rho / (sqrt(delta) - r mu).
+// (A root's argument is cut at 1e-280, whose root is 0 to a coordinate.)
 __device__ __forceinline__ double mu_coord(const CDesc &d, double rmu, double rho, double rho2, double invrH) {
     const double delta = rmu * rmu - rho2, hr = 0.5 * d.RMU - 1.0;
-    if (rmu < 0.0 && delta > 0.0) return hr - hr * (rho * rcp64(sqrt64(delta) - rmu));
-    return fma((sqrt64(fmax(delta + d.H2, 0.0)) - rmu) * invrH, hr, 0.5 * d.RMU);
+    if (rmu < 0.0 && delta > 0.0) return hr - hr * (rho * rcp64(sqrt64_pos(delta) - rmu));
+    return fma((sqrt64_pos(fmax(delta + d.H2, 1e-280)) - rmu) * invrH, hr, 0.5 * d.RMU);
 }
 // Its mu_s axis as a texel coordinate inside a slice.  atan x = atan x0 + atan((x - x0) /
 // (1 + x x0)) from the camera's x0: the sun's elevation differs little over the rays of a
@@ -121,7 +123,7 @@ __device__ __forceinline__ float4 lerp4(float4 u, float4 v, float w) {
 
 // texture4D: the two trilinear fetches share all but the slice
 __device__ __forceinline__ float4 texture4D(const CDesc &d, double r, double mu, double muS, double nu) {
-    const double rho2 = r * r - d.Rg * d.Rg, rho = sqrt64(fmax(rho2, 0.0));
+    const double rho2 = r * r - d.Rg * d.Rg, rho = sqrt64_pos(fmax(rho2, 1e-280));
     int j0, j1, k0, k1;
     float b, g, w;
     gl_axis_d(mu_coord(d, r * mu, rho, rho2, rcp64(rho + d.H)), d.RMU, j0, j1, b);
@@ -299,7 +301,7 @@ k_in_scattering(CDesc d, const float4 *__restrict__ pts, int n, float4 *__restri
     double cam[3] = {d.cam[0], d.cam[1], d.cam[2]};
     double pt[3] = {p4.x, p4.y, p4.z};
     double v[3] = {pt[0] - cam[0], pt[1] - cam[1], pt[2] - cam[2]};
-    double dist = sqrt64(dot3(v, v));
+    double dist = sqrt64_pos(dot3(v, v));   // NaN for a point at the camera or at infinity, as v is then
     const double idist = rcp64(dist);
     for (int c = 0; c < 3; ++c) v[c] *= idist;
     double r, rMu, mu;
@@ -368,7 +370,7 @@ k_in_scattering(CDesc d, const float4 *__restrict__ pts, int n, float4 *__restri
 #pragma unroll 1
         for (int h = 0; h < (hor ? 2 : 1); ++h) {
             if (hor) {
-                r1 = sqrt64(r * r + dist * dist + 2.0 * r * dist * m);
+                r1 = sqrt64_pos(r * r + dist * dist + 2.0 * r * dist * m);
                 mu1 = (r * m + dist) * rcp64(r1);
             }
             const float4 s0 = INSIDE ? view_S(d, t, r * m, ne, nw) : texture4D(d, r, m, muS, nu);

@@ -94,7 +94,7 @@ __global__ __launch_bounds__(256) void k_transmittance(const SetDesc *__restrict
     const bool below = mu < -sqrt(1.0 - q * q);   // the ground is in the way: no integral
     for (int k = below ? nsamp + 1 : lane; k <= nsamp; k += 16) {
         const double x = k * dx;
-        const double h = sqrt64(fma(x, x + rmu2, r2)) - s.Rg;   // >= 0: the ray ends at the ground
+        const double h = sqrt64_pos(fma(x, x + rmu2, r2)) - s.Rg;   // >= 0: the ray ends at the ground
         const double w = (k == 0 || k == nsamp) ? 0.5 : 1.0;
         sR = fma(w, exp2_64(h * eR), sR);
         sM = fma(w, exp2_64(h * eM), sM);

@@ -265,3 +265,22 @@ def test_rgba16f_uploads_through_the_descriptors_render_like_the_oracle(eng, tmp
     osun, osky = O.sun_sky_irradiance(p, T64, E64, rmus.astype(np.float64))
     _assert("16F sun", sun[:, :3].double().cpu().numpy(), osun, 1e-5)
     _assert("16F skyE", sky[:, :3].double().cpu().numpy(), osky, 1e-5)
+
+
+def test_in_scattering_at_points_without_a_direction(eng):
+    """A point at the camera has no direction (0 / 0): NaN, as the shader's normalize
+    gives; so do infinite and NaN points.  The planet's centre sees no light from there
+    (extinction 0), and the points beside them are those of a call without them."""
+    p = small()
+    T, E, S = eng.precompute(p, options(flags=FLAG_NO_AUTOTUNE))[0]
+    for cam in cameras(p)[:2]:
+        cam = cam.astype(np.float32).astype(np.float64)   # a point can be at it
+        v = C.view(cam, SUNS[0])
+        near = (cam + panorama(4, 4) * 3.0).astype(np.float32)
+        odd = np.array([cam, [np.inf, 0, 0], [0, 0, np.nan], [0, 0, 0]], dtype=np.float32)
+        rad, ext = C.in_scattering(p, T, S, v, np.concatenate([near[:9], odd, near[9:]]))
+        rad0, ext0 = C.in_scattering(p, T, S, v, near)
+        keep = torch.tensor(list(range(9)) + list(range(13, 20)), device="cuda")
+        assert torch.equal(rad[keep], rad0) and torch.equal(ext[keep], ext0)
+        assert torch.isnan(rad[9:12, :3]).all()
+        assert (ext[12, :3] == 0).all() and torch.isfinite(rad[12]).all()
