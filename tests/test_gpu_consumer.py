@@ -284,3 +284,30 @@ def test_in_scattering_at_points_without_a_direction(eng):
         assert torch.equal(rad[keep], rad0) and torch.equal(ext[keep], ext0)
         assert torch.isnan(rad[9:12, :3]).all()
         assert (ext[12, :3] == 0).all() and torch.isfinite(rad[12]).all()
+
+
+def _rays(p, n, seed):
+    """n directions, and n points around the whole planet: far from the camera the sun's
+    elevation at a point has any value."""
+    g = np.random.default_rng(seed)
+    d = g.normal(size=(n, 3))
+    d /= np.linalg.norm(d, axis=1, keepdims=True)
+    r = float(p.Rg) + g.uniform(0.01, 0.99, (n, 1)) * float(p.Rt - p.Rg)
+    return d.astype(np.float32), (r * d).astype(np.float32)
+
+
+@pytest.mark.parametrize("pi", range(len(ATMOS)))
+def test_a_rays_result_does_not_depend_on_the_rays_beside_it(eng, pi):
+    """The points of a call in the order of their sun elevation, then shuffled so that
+    near and far ones share a wave: the same bits."""
+    p = ATMOS[pi]
+    T, E, S = eng.precompute(p, options(flags=FLAG_NO_AUTOTUNE))[0]
+    dirs, pts = _rays(p, 1 << 13, pi)
+    for cam in cameras(p):
+        for sun in SUNS:
+            v = C.view(cam, sun)
+            for f, x in ((C.sky_radiance, dirs), (C.in_scattering, pts)):
+                x = x[np.argsort(x @ sun / np.linalg.norm(x, axis=1))]
+                perm = np.random.default_rng(7).permutation(len(x))
+                for a, b in zip(f(p, T, S, v, x), f(p, T, S, v, x[perm])):
+                    assert torch.equal(a[torch.from_numpy(perm).cuda()], b), f.__name__
