@@ -276,9 +276,11 @@ __global__ __launch_bounds__(512) void k_sky_radiance_inside(CDesc d, const floa
 // inScattering, atmosphereShader.glsl:425-533 (HORIZON_HACK on).  INSIDE: the camera is
 // inside the atmosphere and there are no light shafts (din = sw = 0): its side of the
 // difference and of the extinction comes from the staged view tables.
-// 1280 x 720 points on the 32x128x32x8 tables: 70 -> 40 us.
+// 1280 x 720 points on the 32x128x32x8 tables: 70 -> 35 us.  The other form takes the registers
+// that it needs (183; held to 128 for four waves it spilled): 65536 points from inside 12.5 -> 8.4
+// us, 921600 with light shafts 72 -> 49.
 template <bool INSIDE>
-__global__ __launch_bounds__(INSIDE ? 512 : 256) __attribute__((amdgpu_waves_per_eu(4))) void
+__global__ __launch_bounds__(INSIDE ? 512 : 256) __attribute__((amdgpu_waves_per_eu(INSIDE ? 4 : 2))) void
 k_in_scattering(CDesc d, const float4 *__restrict__ pts, int n, float4 *__restrict__ rad, float4 *__restrict__ ext) {
     extern __shared__ float4 clds[];
     ViewTables t;
