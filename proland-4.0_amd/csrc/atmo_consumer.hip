@@ -129,10 +129,12 @@ __device__ __forceinline__ float4 texture4D(const CDesc &d, double r, double mu,
     return lerp4(lerp4(row(k0, j0), row(k0, j1), b), lerp4(row(k1, j0), row(k1, j1), b), g);
 }
 
-// The tables as a camera inside the atmosphere sees them, staged per workgroup:
-// r and mu_s are the same for every ray, so S blends to [RMU][RNU + 3] (slices -1 to
-// RNU + 1, each column clamped as the fetch clamps it) and T to one row of columns.
-// A lookup then reads 4 and 2 LDS entries instead of 16 texels and 4.
+// The tables as a camera inside the atmosphere sees them: r and mu_s are the same for
+// every ray, so S blends to [RMU][RNU + 3] (slices -1 to RNU + 1, each column clamped as the
+// fetch clamps it) and T to one row of columns.  STAGED: once per workgroup in LDS, where a
+// lookup reads 4 and 2 entries instead of 16 texels and 4; otherwise a lookup blends the
+// entries it needs itself, with the same bits.
+template <bool STAGED>
 struct ViewTables {
     const float4 *S, *T;
     int stride;   // RNU + 3
@@ -140,45 +142,66 @@ struct ViewTables {
 __host__ __device__ __forceinline__ size_t view_entries(const CDesc &d) {
     return (size_t)(d.RMU + 1) * (d.RNU + 3) + d.TW + 1;
 }
-__device__ __forceinline__ ViewTables stage_view(const CDesc &d, float4 *lds) {
+typedef __attribute__((address_space(1))) const char gchar;
+// (a layer of S, at most 2^27 texels of 16 bytes, and the rows of T: scalar bases and 32-bit
+// byte offsets)
+__device__ __forceinline__ float4 view_entry_S(const CDesc &d, int j, int slice) {   // mu row j
+    const size_t layer = (size_t)d.RMU * d.W4 * 16;
+    const gchar *t0 = (const gchar *)d.S + d.k0 * layer, *t1 = (const gchar *)d.S + d.k1 * layer;
+    const int i = slice * d.RMUS + d.i0, last = d.W4 - 1;
+    const unsigned x0 = (unsigned)(j * d.W4 + min(max(i, 0), last)) * 16u, x1 = (unsigned)(j * d.W4 + min(max(i + 1, 0), last)) * 16u;
+    auto at = [](const gchar *t, unsigned x) {
+        const gfloat *q = (const gfloat *)(t + x);
+        return make_float4(q[0], q[1], q[2], q[3]);
+    };
+    return lerp4(lerp4(at(t0, x0), at(t0, x1), d.ia), lerp4(at(t1, x0), at(t1, x1), d.ia), d.kg);
+}
+__device__ __forceinline__ float3 view_entry_T(const CDesc &d, int x) {
+    const gchar *t = (const gchar *)d.T;
+    const unsigned o = (unsigned)min(x, d.TW - 1) * 12u;
+    const gfloat *p = (const gfloat *)(t + (size_t)d.tj0 * d.TW * 12 + o), *q = (const gfloat *)(t + (size_t)d.tj1 * d.TW * 12 + o);
+    return lerp3(make_float3(p[0], p[1], p[2]), make_float3(q[0], q[1], q[2]), d.tb);
+}
+template <bool STAGED>
+__device__ __forceinline__ ViewTables<STAGED> stage_view(const CDesc &d, float4 *lds) {
+    if (!STAGED) return {nullptr, nullptr, 0};
     const int stride = d.RNU + 3, nS = d.RMU * stride;
     float4 *T = lds + (d.RMU + 1) * stride;
-    const gfloat *t = (const gfloat *)d.S;
-    for (int e = threadIdx.x; e < nS + stride; e += blockDim.x) {
-        if (e >= nS) {   // below the last row, where the fraction is 0
-            lds[e] = make_float4(0.f, 0.f, 0.f, 0.f);
-            continue;
-        }
-        const int j = e / stride, i = (e % stride - 1) * d.RMUS + d.i0, last = d.W4 - 1;
-        const int x0 = min(max(i, 0), last), x1 = min(max(i + 1, 0), last);
-        auto at = [&](int k, int x) {
-            const gfloat *q = t + (((size_t)k * d.RMU + j) * d.W4 + x) * 4;
-            return make_float4(q[0], q[1], q[2], q[3]);
-        };
-        lds[e] = lerp4(lerp4(at(d.k0, x0), at(d.k0, x1), d.ia), lerp4(at(d.k1, x0), at(d.k1, x1), d.ia), d.kg);
-    }
-    const gfloat *u = (const gfloat *)d.T;
+    for (int e = threadIdx.x; e < nS + stride; e += blockDim.x)
+        // below the last row, where the fraction is 0: nothing
+        lds[e] = e < nS ? view_entry_S(d, e / stride, e % stride - 1) : make_float4(0.f, 0.f, 0.f, 0.f);
     for (int x = threadIdx.x; x <= d.TW; x += blockDim.x) {
-        const gfloat *p = u + ((size_t)d.tj0 * d.TW + min(x, d.TW - 1)) * 3, *q = u + ((size_t)d.tj1 * d.TW + min(x, d.TW - 1)) * 3;
-        const float3 v = lerp3(make_float3(p[0], p[1], p[2]), make_float3(q[0], q[1], q[2]), d.tb);
+        const float3 v = view_entry_T(d, x);
         T[x] = make_float4(v.x, v.y, v.z, 0.f);
     }
     __syncthreads();
     return {lds, T, stride};
 }
 // texture4D at the camera's r and sun
-__device__ __forceinline__ float4 view_S(const CDesc &d, const ViewTables &v, double rmu, int e, float w) {
+template <bool STAGED>
+__device__ __forceinline__ float4 view_S(const CDesc &d, const ViewTables<STAGED> &v, double rmu, int e, float w) {
     const double y = fmin(fmax(mu_coord(d, rmu, d.rho, d.rho2, d.invrH), 0.0), d.RMU - 1.0), fy = floor(y);
     const float b = (float)(y - fy);
-    const float4 *p = v.S + (int)fy * v.stride + e + 1, *q = p + v.stride;
-    return lerp4(lerp4(p[0], p[1], w), lerp4(q[0], q[1], w), b);
+    if constexpr (STAGED) {
+        const float4 *p = v.S + (int)fy * v.stride + e + 1, *q = p + v.stride;
+        return lerp4(lerp4(p[0], p[1], w), lerp4(q[0], q[1], w), b);
+    } else {
+        const int j0 = (int)fy, j1 = min(j0 + 1, d.RMU - 1);
+        return lerp4(lerp4(view_entry_S(d, j0, e), view_entry_S(d, j0, e + 1), w),
+                     lerp4(view_entry_S(d, j1, e), view_entry_S(d, j1, e + 1), w), b);
+    }
 }
 // T at the camera's r
-__device__ __forceinline__ float3 view_T(const CDesc &d, const ViewTables &v, double mu) {
+template <bool STAGED>
+__device__ __forceinline__ float3 view_T(const CDesc &d, const ViewTables<STAGED> &v, double mu) {
     const float uMu = atanf(((float)mu + 0.15f) * d.f_tMu) * (1.0f / 1.5f);
     const float x = __builtin_amdgcn_fmed3f(uMu * d.TW - 0.5f, 0.0f, (float)(d.TW - 1)), f = floorf(x);
-    const float4 *p = v.T + (int)f;
-    return lerp3(f3(p[0]), f3(p[1]), x - f);
+    if constexpr (STAGED) {
+        const float4 *p = v.T + (int)f;
+        return lerp3(f3(p[0]), f3(p[1]), x - f);
+    } else {
+        return lerp3(view_entry_T(d, (int)f), view_entry_T(d, (int)f + 1), x - f);
+    }
 }
 
 __host__ __device__ __forceinline__ double dot3(const double *a, const double *b) {
@@ -252,12 +275,13 @@ __global__ __launch_bounds__(256) void k_sky_radiance(CDesc d, const float4 *__r
 }
 
 // skyRadiance from inside the atmosphere without light shafts: no ray enters from
-// outside (din = 0).  Workgroups stage the view's tables once and walk the rays.
-// 1920 x 1080 rays on the 32x128x32x8 tables: 50 -> 23 us.
-__global__ __launch_bounds__(512) void k_sky_radiance_inside(CDesc d, const float4 *__restrict__ dirs, int n,
+// outside (din = 0).  STAGED: workgroups stage the view's tables once and walk the rays.
+// 1920 x 1080 rays on the 32x128x32x8 tables: 45 -> 22 us.
+template <bool STAGED>
+__global__ __launch_bounds__(STAGED ? 512 : 256) void k_sky_radiance_inside(CDesc d, const float4 *__restrict__ dirs, int n,
                                                              float4 *__restrict__ rad, float4 *__restrict__ ext) {
     extern __shared__ float4 clds[];
-    const ViewTables t = stage_view(d, clds);
+    const ViewTables<STAGED> t = stage_view<STAGED>(d, clds);
     for (long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (long long)gridDim.x * blockDim.x) {
         const float4 v4 = dirs[i];
         const double v[3] = {v4.x, v4.y, v4.z};
@@ -275,16 +299,15 @@ __global__ __launch_bounds__(512) void k_sky_radiance_inside(CDesc d, const floa
 
 // inScattering, atmosphereShader.glsl:425-533 (HORIZON_HACK on).  INSIDE: the camera is
 // inside the atmosphere and there are no light shafts (din = sw = 0): its side of the
-// difference and of the extinction comes from the staged view tables.
-// 1280 x 720 points on the 32x128x32x8 tables: 70 -> 35 us.  The other form takes the registers
-// that it needs (183; held to 128 for four waves it spilled): 65536 points from inside 12.5 -> 8.4
-// us, 921600 with light shafts 72 -> 49.
-template <bool INSIDE>
-__global__ __launch_bounds__(INSIDE ? 512 : 256) __attribute__((amdgpu_waves_per_eu(INSIDE ? 4 : 2))) void
+// difference and of the extinction comes from the view's tables.
+// 1280 x 720 points on the 32x128x32x8 tables, staged: 70 -> 35 us.  The other forms take the
+// registers that they need (202; held to 128 for four waves they spill): 65536 points from inside
+// 12.5 -> 7.5 us, 921600 with light shafts 72 -> 49.
+template <bool INSIDE, bool STAGED>
+__global__ __launch_bounds__(STAGED ? 512 : 256) __attribute__((amdgpu_waves_per_eu(STAGED ? 4 : 2))) void
 k_in_scattering(CDesc d, const float4 *__restrict__ pts, int n, float4 *__restrict__ rad, float4 *__restrict__ ext) {
     extern __shared__ float4 clds[];
-    ViewTables t;
-    if (INSIDE) t = stage_view(d, clds);
+    const ViewTables<STAGED> t = stage_view<STAGED>(d, clds);
     for (long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (long long)gridDim.x * blockDim.x) {
     const float4 p4 = pts[i];
     double cam[3] = {d.cam[0], d.cam[1], d.cam[2]};
@@ -498,20 +521,27 @@ void view_desc(CDesc &d, bool flat) {
     axis(std::sqrt(std::fmax(r - d.Rg, 0.0) / (d.Rt - d.Rg)) * d.TH - 0.5, d.TH, d.tj0, d.tj1, d.tb);
 }
 
-// Staged view tables from 2^17 rays on: below, both forms take less than the call itself
-// (14 us; 131072 points 14.3 staged, 16.0 before; 262144 20 against 25), and a workgroup
-// would stage about 20 KB for fewer than one ray per thread.  At most 64 KB, two
+// Staged view tables pay from some rays per staged entry on (1676 entries for 32x128x32x8 with
+// 256 T columns, 3316 for 32x160x32x16): every workgroup stages them all.  GPU time of a
+// frame's rays in us, each lookup blending its own / staged:
+//   sky         131072 rays  4.4 / 6.7 and 4.5 / 10.2;  262144  6.4 / 7.9 and 6.8 / 11.3;
+//               921600  16.1 / 15.1 and 16.0 / 19.1;  2073600  29.1 / 23.2 and 29.1 / 26.8
+//   scattering  262144 points  15.7 / 22.6 and 15.6 / 30.1;  921600  42.4 / 41.6 and 42.7 / 51.4;
+//               2073600  85.5 / 73.3 and 85.5 / 84.6
+// Scattered directions, whose own lookups share no cache lines, cross earlier: 262144 rays 11.6 /
+// 8.2 and 12.0 / 11.6; 921600 points 57.9 / 52.1 and 63.7 / 63.3.  At most 64 KB, two
 // workgroups per CU.
-constexpr int kInsideMin = 1 << 17;
+constexpr int kSkyPerEntry = 128, kAerialPerEntry = 512;
 constexpr size_t kInsideLds = 64 * 1024;
 // Workgroups of 512 threads: one per CU for the sky (2073600 rays with 256 / 512 / 1024:
 // 23.1 / 25.2 / 30.4 us), two for the scattering, whose own lookups wait more
 // (921600 points: 43.9 / 39.4 / 45.7).
 constexpr int kSkyGroups = 256, kAerialGroups = 512;
-bool use_inside(const CDesc &d, int n) {
-    return d.inside && n >= kInsideMin && view_entries(d) * sizeof(float4) <= kInsideLds;
+bool use_staged(const CDesc &d, int n, int per_entry) {
+    const size_t entries = view_entries(d);
+    return d.inside && entries * sizeof(float4) <= kInsideLds && (size_t)n >= per_entry * entries;
 }
-int inside_groups(int n, int most) { return std::min((int)(((long long)n + 511) / 512), most); }
+int staged_groups(int n, int most) { return std::min((int)(((long long)n + 511) / 512), most); }
 
 }  // namespace
 }  // namespace atmo
@@ -534,10 +564,13 @@ atmo_status atmo_sky_radiance(const atmo_params *p, const float *T, const float 
     d.T = T;
     d.S = S;
     atmo::view_desc(d, false);
-    if (atmo::use_inside(d, n))
-        hipLaunchKernelGGL(atmo::k_sky_radiance_inside, dim3(atmo::inside_groups(n, atmo::kSkyGroups)), dim3(512),
+    if (atmo::use_staged(d, n, atmo::kSkyPerEntry))
+        hipLaunchKernelGGL(atmo::k_sky_radiance_inside<true>, dim3(atmo::staged_groups(n, atmo::kSkyGroups)), dim3(512),
                            atmo::view_entries(d) * sizeof(float4), (hipStream_t)stream, d, (const float4 *)dirs, n,
                            (float4 *)radiance, (float4 *)extinction);
+    else if (d.inside)
+        hipLaunchKernelGGL(atmo::k_sky_radiance_inside<false>, dim3((n + 255) / 256), dim3(256), 0, (hipStream_t)stream, d,
+                           (const float4 *)dirs, n, (float4 *)radiance, (float4 *)extinction);
     else
         hipLaunchKernelGGL(atmo::k_sky_radiance, dim3((n + 255) / 256), dim3(256), 0, (hipStream_t)stream, d,
                            (const float4 *)dirs, n, (float4 *)radiance, (float4 *)extinction);
@@ -560,12 +593,15 @@ atmo_status atmo_in_scattering(const atmo_params *p, const float *T, const float
     d.T = T;
     d.S = S;
     atmo::view_desc(d, true);
-    if (atmo::use_inside(d, n))
-        hipLaunchKernelGGL(atmo::k_in_scattering<true>, dim3(atmo::inside_groups(n, atmo::kAerialGroups)), dim3(512),
+    if (atmo::use_staged(d, n, atmo::kAerialPerEntry))
+        hipLaunchKernelGGL((atmo::k_in_scattering<true, true>), dim3(atmo::staged_groups(n, atmo::kAerialGroups)), dim3(512),
                            atmo::view_entries(d) * sizeof(float4), (hipStream_t)stream, d, (const float4 *)points, n,
                            (float4 *)radiance, (float4 *)extinction);
+    else if (d.inside)
+        hipLaunchKernelGGL((atmo::k_in_scattering<true, false>), dim3((n + 255) / 256), dim3(256), 0, (hipStream_t)stream, d,
+                           (const float4 *)points, n, (float4 *)radiance, (float4 *)extinction);
     else
-        hipLaunchKernelGGL(atmo::k_in_scattering<false>, dim3((n + 255) / 256), dim3(256), 0, (hipStream_t)stream, d,
+        hipLaunchKernelGGL((atmo::k_in_scattering<false, false>), dim3((n + 255) / 256), dim3(256), 0, (hipStream_t)stream, d,
                            (const float4 *)points, n, (float4 *)radiance, (float4 *)extinction);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return atmo::cfail(ATMO_ERR_DEVICE, "k_in_scattering: %s", hipGetErrorString(e));

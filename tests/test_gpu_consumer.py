@@ -311,3 +311,21 @@ def test_a_rays_result_does_not_depend_on_the_rays_beside_it(eng, pi):
                 perm = np.random.default_rng(7).permutation(len(x))
                 for a, b in zip(f(p, T, S, v, x), f(p, T, S, v, x[perm])):
                     assert torch.equal(a[torch.from_numpy(perm).cuda()], b), f.__name__
+
+
+@pytest.mark.parametrize("res", [(8, 32, 8, 4), (4, 130, 8, 32)])
+def test_a_rays_result_does_not_depend_on_the_size_of_its_call(eng, res):
+    """2^18 + 1 rays in one call (from inside, with view tables in LDS where they fit 64 KB,
+    which those of 130 mu rows and 32 nu slices do not) and in tiles of 1 to 65536 (without,
+    and the sky's with from 37888 rays on): the same bits."""
+    p = small(res=res)
+    T, E, S = eng.precompute(p, options(orders=2, flags=FLAG_NO_AUTOTUNE))[0]
+    dirs, pts = _rays(p, (1 << 18) + 1, 5)
+    cuts = [0, 1, 2, 67, 1091, 9283, 74819, 140355, 200000, len(dirs)]
+    for ci, cam in enumerate(cameras(p)):
+        v = C.view(cam, SUNS[ci % 2])
+        for f, x in ((C.sky_radiance, dirs), (C.in_scattering, pts)):
+            whole = f(p, T, S, v, x)
+            tiles = [f(p, T, S, v, x[i:j]) for i, j in zip(cuts, cuts[1:])]
+            for k in (0, 1):
+                assert torch.equal(whole[k], torch.cat([t[k] for t in tiles])), (f.__name__, ci, k)
