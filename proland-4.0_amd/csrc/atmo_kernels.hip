@@ -11,47 +11,49 @@
 
 namespace atmo {
 
-// 2^y for y <= 1000, at least 2^-1000, 1.4e-14 relative: a polynomial in the fraction
-// (degree 9, fitted to the relative error on |f| <= 1/2), the integer part added to the
-// exponent.
+// 2^y for y <= 1000, at least 2^-1000 (also for NaN), 1.4e-16 relative: a polynomial in the
+// fraction (degree 11, interpolated in Chebyshev points of |f| <= 1/2), the integer part
+// added to the exponent.
 constexpr double kLog2e = 1.4426950408889634;
 __device__ __forceinline__ double exp2_64(double y) {
     constexpr double kRound64 = 6755399441055744.0;   // 1.5 2^52
     y = fmax(y, -1000.0);
     const double t = y + kRound64, f = y - (t - kRound64);
-    double p = fma(f, 1.0150099678576792e-07, 1.3259402170656473e-06);
-    p = fma(f, p, 1.5252986067042296e-05);
-    p = fma(f, p, 0.00015403434961948063);
-    p = fma(f, p, 0.001333355761545632);
-    p = fma(f, p, 0.009618129192050495);
-    p = fma(f, p, 0.055504108668700244);
-    p = fma(f, p, 0.24022650695649567);
-    p = fma(f, p, 0.6931471805598719);
-    p = fma(f, p, 1.0000000000000133);
+    double p = fma(f, 4.4554725442721574e-10, 7.0742005955524935e-09);
+    p = fma(f, p, 1.0178059245425577e-07);
+    p = fma(f, p, 1.3215432498125634e-06);
+    p = fma(f, p, 1.5252733836823374e-05);
+    p = fma(f, p, 0.00015403530463804289);
+    p = fma(f, p, 0.0013333558146410734);
+    p = fma(f, p, 0.009618129107587189);
+    p = fma(f, p, 0.05550410866482161);
+    p = fma(f, p, 0.2402265069591016);
+    p = fma(f, p, 0.6931471805599453);
+    p = fma(f, p, 1.0);
     return __hiloint2double(__double2hiint(p) + (__double2loint(t) << 20), __double2loint(p));
 }
 
-// tan x for x in [0, 1.5], 4e-15 relative: from the Taylor series of sine and cosine at x / 2
-// (terms below 1e-18 left out).  A tenth of the library's code, which reduces any argument.
+// tan x for x in [0, 1.5], 5.5e-16 relative (x = 1.5 m itself is rounded, which moves tan x by
+// up to 2.3e-15): from the Taylor series of sine and cosine at half of x, or of pi/2 - x
+// from 0.8 on (terms below 1e-17 left out).  A tenth of the library's code, which reduces
+// any argument.
 __device__ __forceinline__ double tan_col(double x) {
-    const double y = 0.5 * x, z = y * y;
-    double s = fma(z, 2.8114572543455206e-15, -7.647163731819816e-13);
-    s = fma(z, s, 1.6059043836821613e-10);
-    s = fma(z, s, -2.505210838544172e-08);
+    const bool co = x > 0.8;
+    const double y = 0.5 * (co ? (1.5707963267948966 - x) + 6.123233995736766e-17 : x), z = y * y;
+    double s = fma(z, 1.6059043836821613e-10, -2.505210838544172e-08);
     s = fma(z, s, 2.7557319223985893e-06);
     s = fma(z, s, -0.0001984126984126984);
     s = fma(z, s, 0.008333333333333333);
     s = fma(z, s, -0.16666666666666666);
     s = fma(y * z, s, y);
-    double c = fma(z, 4.779477332387385e-14, -1.1470745597729725e-11);
-    c = fma(z, c, 2.08767569878681e-09);
-    c = fma(z, c, -2.755731922398589e-07);
+    double c = fma(z, 2.08767569878681e-09, -2.755731922398589e-07);
     c = fma(z, c, 2.48015873015873e-05);
     c = fma(z, c, -0.001388888888888889);
     c = fma(z, c, 0.041666666666666664);
     c = fma(z, c, -0.5);
     c = fma(z, c, 1.0);
-    return 2.0 * s * c / fma(-s, s, c * c);
+    const double n = 2.0 * s * c, d = fma(-s, s, c * c);
+    return co ? d / n : n / d;
 }
 
 // ---------------------------------------------------------------------------
