@@ -110,16 +110,16 @@ __global__ __launch_bounds__(256) void k_transmittance(const SetDesc *__restrict
         // sun_centres: tan(1.5 m), its leading part in row 0 and the rest in row 1
         double c = j < 2 ? tm : 0.0;
         const float ck = j == 0 ? (float)c : j == 1 ? (float)(c - (double)(float)c) : 0.0f;
-        double dR = below ? 1e9 : sR * dx;
-        double dM = below ? 1e9 : sM * dx;
-        double tau[3];
+        // no number where the ray's length is none (the sums above are finite in any case)
+        double dR = below ? 1e9 : fma(sR, dx, dx - dx);
+        double dM = below ? 1e9 : fma(sM, dx, dx - dx);
+        double tau[3], T[3];
 #pragma unroll
-        for (int k = 0; k < 3; ++k) tau[k] = (double)s.bR[k] * dR + (double)s.bME[k] * dM;
-        float4 o;
-        o.x = (float)exp2_64(tau[0] * -kLog2e);
-        o.y = (float)exp2_64(tau[1] * -kLog2e);
-        o.z = (float)exp2_64(tau[2] * -kLog2e);
-        o.w = 0.0f;
+        for (int k = 0; k < 3; ++k) {
+            tau[k] = (double)s.bR[k] * dR + (double)s.bME[k] * dM;
+            T[k] = tau[k] == tau[k] ? exp2_64(tau[k] * -kLog2e) : tau[k];
+        }
+        float4 o = make_float4((float)T[0], (float)T[1], (float)T[2], 0.0f);
         o = q16(o, s.hs);
         s.T4[t] = o;
         if (s.tau4)

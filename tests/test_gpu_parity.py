@@ -8,6 +8,8 @@ where the pass has no amplifying step.
 """
 import os
 
+import math
+
 import numpy as np
 import pytest
 
@@ -76,6 +78,23 @@ def test_pass_transmittance(eng, ci):
     T4 = torch.zeros((p.TRANSMITTANCE_H, p.TRANSMITTANCE_W, 4), device="cuda")
     eng.pass_transmittance(p, o, T4)
     _assert("T", rgb(T4), O.transmittance(p, o), 1e-5)
+
+
+def test_pass_transmittance_without_an_end_of_the_ray(eng):
+    """RL = infinity: a ray that does not meet the ground has no length, and its
+    transmittance is no number (the numeric check finds it); towards the ground it is 0."""
+    p = CASES[0].copy()
+    p.RL = math.inf
+    T4 = torch.zeros((p.TRANSMITTANCE_H, p.TRANSMITTANCE_W, 4), device="cuda")
+    eng.pass_transmittance(p, options(), T4)
+    m = (np.arange(p.TRANSMITTANCE_W) + 0.5) / p.TRANSMITTANCE_W
+    t = (np.arange(p.TRANSMITTANCE_H) + 0.5) / p.TRANSMITTANCE_H
+    mu = -0.15 + np.tan(1.5 * m) / np.tan(1.5) * 1.15
+    r = p.Rg + t * t * (p.Rt - p.Rg)
+    below = mu[None, :] < -np.sqrt(1 - (p.Rg / r[:, None]) ** 2)
+    T = rgb(T4)
+    assert below.any() and not below.all()
+    assert np.isnan(T[~below]).all() and (T[below] == 0).all()
 
 
 @pytest.mark.parametrize("ci", range(len(CASES)))
