@@ -35,7 +35,7 @@ struct LayerGeom {
 // parameterisation: mu_s and, in txb, mu_s + 0.2.
 struct ColGeom {
     float mus, ck, lo, kb, kb2, txb;
-    float hi, lo64;   // mu_s in two parts, for FP64 uses
+    double mus64;     // mu_s
 };
 
 // A view-ray sample of the dSn pass (k_snview): what does not involve the sun.
@@ -82,7 +82,7 @@ struct SetDesc {
     int n4;                         // RR * RMU * W4
     // tables (device pointers)
     float4 *T4, *dE4, *E4, *dSR4, *dSM4, *dJ4, *S4;
-    float4 *tau4;                   // optical depth -ln T of the T texels (rgb), or null
+    float4 *tau4;                   // optical depth -ln T of the T texels (rgb; w: sun_centres), or null
     // transmittances along the view ray of each (layer, mu row) at the inscatter
     // samples (trapezoid weights folded in), [RR][RMU][nsamp + 1] (w: the sample's t / r_i), and from the ground point to each layer
     // radius per theta row of the spherical integral, [RR][NS]; null: computed

@@ -179,11 +179,10 @@ ColGeom col_geom(const atmo_params &p, const atmo_options &o, int m) {
     const double k = (double)(float)std::tan(1.26 * 1.1), f = m / (p.RES_MU_S - 1.0);
     const double muS = lin ? -0.2 + f * 1.2 : std::tan((2.0 * f - 1.0 + 0.26) * 1.1) / std::tan(1.26 * 1.1);
     const double mub = std::max(muS, -0.1975);
-    const float hi = (float)muS, lo = (float)(muS - (double)hi);
-    if (lin) return {(float)muS, 0.f, 0.f, 0.f, 0.f, (float)(muS + 0.2), hi, lo};
+    if (lin) return {(float)muS, 0.f, 0.f, 0.f, 0.f, (float)(muS + 0.2), muS};
     return {(float)(k * muS), (float)(k * (muS - mub)), (float)(k * (-0.1975 - mub)), (float)(k * mub),
             (float)(1.0 + k * mub * (k * mub)),
-            (float)((std::atan(mub * std::tan(1.26 * 1.1)) / 1.1 + (1.0 - 0.26)) * 0.5 * (p.RES_MU_S - 1.0)), hi, lo};
+            (float)((std::atan(mub * std::tan(1.26 * 1.1)) / 1.1 + (1.0 - 0.26)) * 0.5 * (p.RES_MU_S - 1.0)), muS};
 }
 
 void fill_desc(SetDesc &s, const atmo_params &p) {

@@ -107,9 +107,8 @@ __global__ __launch_bounds__(256) void k_transmittance(const SetDesc *__restrict
         sM += __shfl_xor(sM, off, 16);
     }
     if (lane == 0 && valid) {
-        // sun_centres: tan(1.5 m), its leading part in row 0 and the rest in row 1
-        double c = j < 2 ? tm : 0.0;
-        const float ck = j == 0 ? (float)c : j == 1 ? (float)(c - (double)(float)c) : 0.0f;
+        // sun_centres: the bits of tan(1.5 m), the upper half in row 0 and the lower in row 1
+        const float ck = __int_as_float(j == 0 ? __double2hiint(tm) : j == 1 ? __double2loint(tm) : 0);
         // no number where the ray's length is none (the sums above are finite in any case)
         double dR = below ? 1e9 : fma(sR, dx, dx - dx);
         double dM = below ? 1e9 : fma(sM, dx, dx - dx);
@@ -297,16 +296,16 @@ __device__ __forceinline__ void sun_column(const SunAxis &x, const SunCell &c, f
     }
 }
 // Centres of the T table's columns: from the spare component of the first two rows of
-// optical depths (k_transmittance), high and low part, where there are any.
+// optical depths (k_transmittance), upper and lower half of their bits, where there are any.
 __device__ __forceinline__ void sun_centres(const SetDesc &s, double *xk) {
     for (int k = threadIdx.x; k < s.TW; k += blockDim.x)
-        xk[k] = s.tau4 ? (double)s.tau4[k].w + (double)s.tau4[s.TW + k].w : tan(1.5 * (k + 0.5) / s.TW);
+        xk[k] = s.tau4 ? __hiloint2double(__float_as_int(s.tau4[k].w), __float_as_int(s.tau4[s.TW + k].w)) : tan(1.5 * (k + 0.5) / s.TW);
 }
 // nu and r mu_s of the texel in column x
 __device__ __forceinline__ void s1_texel(const SetDesc &s, int x, double r, double &nu, double &muSr) {
     const ColGeom c = s.cols[x % s.RMUS];
     nu = -1.0 + (double)(x / s.RMUS) / (s.RNU - 1.0) * 2.0;
-    muSr = ((double)c.hi + (double)c.lo64) * r;
+    muSr = c.mus64 * r;
 }
 // The terms of sample i of the row (l, y); BY_PARITY: row weights for k_inscatter1_rows.
 // Stores the row's sample distance in dx.
