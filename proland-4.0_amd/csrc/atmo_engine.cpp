@@ -185,6 +185,29 @@ ColGeom col_geom(const atmo_params &p, const atmo_options &o, int m) {
             (float)((std::atan(mub * std::tan(1.26 * 1.1)) / 1.1 + (1.0 - 0.26)) * 0.5 * (p.RES_MU_S - 1.0)), muS};
 }
 
+size_t align256(size_t b) { return (b + 255) & ~(size_t)255; }
+
+// Layers, then the mu_s columns, of every set, for one upload; byte offsets of each set's.
+std::vector<char> pack_geom(const atmo_params *sets, int nsets, const atmo_options &o, std::vector<size_t> &loff,
+                            std::vector<size_t> &coff) {
+    std::vector<LayerGeom> layers;
+    std::vector<ColGeom> cols;
+    loff.clear();
+    coff.clear();
+    for (int i = 0; i < nsets; ++i) {
+        loff.push_back(layers.size() * sizeof(LayerGeom));
+        coff.push_back(cols.size() * sizeof(ColGeom));
+        for (int l = 0; l < sets[i].RES_R; ++l) layers.push_back(layer_geom(sets[i], l));
+        for (int m = 0; m < sets[i].RES_MU_S; ++m) cols.push_back(col_geom(sets[i], o, m));
+    }
+    const size_t cols_off = align256(layers.size() * sizeof(LayerGeom));
+    std::vector<char> h(cols_off + cols.size() * sizeof(ColGeom));
+    memcpy(h.data(), layers.data(), layers.size() * sizeof(LayerGeom));
+    memcpy(h.data() + cols_off, cols.data(), cols.size() * sizeof(ColGeom));
+    for (size_t &c : coff) c += cols_off;
+    return h;
+}
+
 void fill_desc(SetDesc &s, const atmo_params &p) {
     memset(&s, 0, sizeof s);
     s.Rg = p.Rg; s.Rt = p.Rt; s.RL = p.RL;
@@ -214,8 +237,6 @@ void fill_desc(SetDesc &s, const atmo_params &p) {
     s.W4 = s.RMUS * s.RNU;
     s.n4 = s.RR * s.RMU * s.W4;
 }
-
-size_t align256(size_t b) { return (b + 255) & ~(size_t)255; }
 
 struct SetSizes {
     size_t nT, nE, n4;
@@ -1036,20 +1057,8 @@ atmo_status build_plan(hipStream_t xs, const atmo_params *sets, int nsets, const
         total += work_bytes(sets[i], o, view);
     }
     HIPCHK(R.get(pl->arena, total));
-    // layers, then the mu_s columns of every set
-    std::vector<LayerGeom> layers;
-    std::vector<ColGeom> cols;
-    std::vector<size_t> loff(nsets), coff(nsets);
-    for (int i = 0; i < nsets; ++i) {
-        loff[i] = layers.size();
-        coff[i] = cols.size();
-        for (int l = 0; l < sets[i].RES_R; ++l) layers.push_back(layer_geom(sets[i], l));
-        for (int m = 0; m < sets[i].RES_MU_S; ++m) cols.push_back(col_geom(sets[i], o, m));
-    }
-    const size_t cols_off = align256(layers.size() * sizeof(LayerGeom));
-    std::vector<char> geom(cols_off + cols.size() * sizeof(ColGeom));
-    memcpy(geom.data(), layers.data(), layers.size() * sizeof(LayerGeom));
-    memcpy(geom.data() + cols_off, cols.data(), cols.size() * sizeof(ColGeom));
+    std::vector<size_t> loff, coff;
+    const std::vector<char> geom = pack_geom(sets, nsets, o, loff, coff);
     HIPCHK(R.get(pl->dlayers, geom.size()));
     HIPCHK(pl->upload(pl->dlayers, geom));
     // descriptors (output pointers are filled in per call)
@@ -1082,8 +1091,8 @@ atmo_status build_plan(hipStream_t xs, const atmo_params *sets, int nsets, const
         }
         s.dJb = 12;  // the ray gathers of dSn read 12 bytes per texel
         set_table_flags(s, o);
-        s.layers = (const LayerGeom *)pl->dlayers.p + loff[i];
-        s.cols = (const ColGeom *)((const char *)pl->dlayers.p + cols_off) + coff[i];
+        s.layers = (const LayerGeom *)((const char *)pl->dlayers.p + loff[i]);
+        s.cols = (const ColGeom *)((const char *)pl->dlayers.p + coff[i]);
     }
     HIPCHK(R.get(pl->dsets, nsets * sizeof(SetDesc)));
     // tiles
@@ -1595,16 +1604,12 @@ static atmo_status pass_setup(atmo_engine *e, const atmo_params *p, const atmo_o
     HIPCHK(hipSetDevice(e->device));
     fill_desc(s, *p);
     set_table_flags(s, oo);
-    std::vector<LayerGeom> layers;
-    for (int l = 0; l < p->RES_R; ++l) layers.push_back(layer_geom(*p, l));
-    std::vector<ColGeom> cols;
-    for (int m = 0; m < p->RES_MU_S; ++m) cols.push_back(col_geom(*p, oo, m));
-    const size_t cols_off = align256(layers.size() * sizeof(LayerGeom));
-    HIPCHK(e->pass_layers.ensure(cols_off + cols.size() * sizeof(ColGeom)));
-    HIPCHK(h2d(e->pass_layers.p, layers.data(), layers.size() * sizeof(LayerGeom), e->cap));
-    s.layers = (const LayerGeom *)e->pass_layers.p;
-    s.cols = (const ColGeom *)((char *)e->pass_layers.p + cols_off);
-    HIPCHK(h2d((char *)e->pass_layers.p + cols_off, cols.data(), cols.size() * sizeof(ColGeom), e->cap));
+    std::vector<size_t> loff, coff;
+    const std::vector<char> geom = pack_geom(p, 1, oo, loff, coff);
+    HIPCHK(e->pass_layers.ensure(geom.size()));
+    HIPCHK(h2d(e->pass_layers.p, geom.data(), geom.size(), e->cap));
+    s.layers = (const LayerGeom *)((const char *)e->pass_layers.p + loff[0]);
+    s.cols = (const ColGeom *)((const char *)e->pass_layers.p + coff[0]);
     return ATMO_OK;
 }
 
