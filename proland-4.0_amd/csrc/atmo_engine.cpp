@@ -640,11 +640,11 @@ void build_sn_tiles(const std::vector<atmo_params> &ps, int snXcd, std::vector<u
     }
 }
 
-// Tile tables of every pass for a batch.  The spherical-integral passes list
+// Tile tables of every pass (only: of that one) for a batch.  The spherical-integral passes list
 // the most expensive tiles first so mixed-resolution batches drain evenly.
 void build_tiles(const std::vector<atmo_params> &ps, const atmo_options &o,
                  std::vector<uint2> &tiles, int off[P_COUNT], int cnt[P_COUNT], int snXcd = 1,
-                 Segs *out = nullptr) {
+                 Segs *out = nullptr, int only = -1) {
     tiles.clear();
     Segs local;
     Segs &sg = out ? *out : local;
@@ -652,6 +652,8 @@ void build_tiles(const std::vector<atmo_params> &ps, const atmo_options &o,
     const int n = (int)ps.size();
     for (int pass = 0; pass < P_COUNT; ++pass) {
         off[pass] = (int)tiles.size();
+        cnt[pass] = 0;
+        if (only >= 0 && pass != only) continue;
         if (pass == P_SN) {
             if (o.orders >= 2) build_sn_tiles(ps, snXcd, tiles, sg.n);
             cnt[pass] = (int)tiles.size() - off[pass];
@@ -678,6 +680,7 @@ void build_tiles(const std::vector<atmo_params> &ps, const atmo_options &o,
             continue;
         }
         std::vector<std::pair<double, uint2>> v;
+        std::vector<int> split(n, 1);   // dj_split of the sets
         for (int i = 0; i < n; ++i) {
             const atmo_params &p = ps[i];
             SetSizes z = sizes(p);
@@ -690,8 +693,9 @@ void build_tiles(const std::vector<atmo_params> &ps, const atmo_options &o,
                 // grouped by the per-set G (descending), most expensive first inside a group
                 nt = (long long)p.RES_R * p.RES_MU_S;
                 cost = jg_for_set(p) * 1e12 + (double)p.RES_MU * p.RES_NU;
-                if (dj_split(p, o) > 1)   // behind the others, the sets of one split together
-                    cost = -((dj_split(p, o) * 1e4 + p.RES_MU) * 1e4 + p.RES_NU);
+                if (o.orders >= 2) split[i] = dj_split(p, o);
+                if (split[i] > 1)   // behind the others, the sets of one split together
+                    cost = -((split[i] * 1e4 + p.RES_MU) * 1e4 + p.RES_NU);
                 break;
             case P_EN: nt = (long long)z.nE; cost = (double)p.RES_NU; break;
             case P_VIEW:
@@ -715,7 +719,7 @@ void build_tiles(const std::vector<atmo_params> &ps, const atmo_options &o,
                     sg.j.back().cnt += 1;
                     continue;
                 }
-                JSeg g{jg_for_set(p), (int)i, 0, dj_split(p, o)};
+                JSeg g{jg_for_set(p), (int)i, 0, split[v[i].second.x]};
                 if (g.DS > 1) {
                     g.RMU = p.RES_MU;
                     g.NU = p.RES_NU;
@@ -1623,9 +1627,9 @@ static atmo_status pass_run(atmo_engine *e, const atmo_params *p, const atmo_opt
     int off[P_COUNT], cnt[P_COUNT];
     std::vector<atmo_params> ps(1, *p);
     atmo_options ot = o;
-    ot.orders = std::max(ot.orders, 2);  // every pass gets its tiles
+    ot.orders = std::max(ot.orders, 2);  // any pass gets its tiles
     Segs segs;
-    build_tiles(ps, ot, tiles, off, cnt, 1, &segs);
+    build_tiles(ps, ot, tiles, off, cnt, 1, &segs, pass);
     HIPCHK(e->pass_tiles.ensure(tiles.size() * sizeof(uint2)));
     HIPCHK(h2d(e->pass_tiles.p, tiles.data(), tiles.size() * sizeof(uint2), e->cap));
     size_t oJT, oJW, oE;
