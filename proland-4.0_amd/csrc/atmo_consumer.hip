@@ -309,95 +309,95 @@ k_in_scattering(CDesc d, const float4 *__restrict__ pts, int n, float4 *__restri
     extern __shared__ float4 clds[];
     const ViewTables<STAGED> t = stage_view<STAGED>(d, clds);
     for (long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (long long)gridDim.x * blockDim.x) {
-    const float4 p4 = pts[i];
-    double cam[3] = {d.cam[0], d.cam[1], d.cam[2]};
-    double pt[3] = {p4.x, p4.y, p4.z};
-    double v[3] = {pt[0] - cam[0], pt[1] - cam[1], pt[2] - cam[2]};
-    double dist = sqrt64_pos(dot3(v, v));   // NaN for a point at the camera or at infinity, as v is then
-    const double idist = rcp64(dist);
-    for (int c = 0; c < 3; ++c) v[c] *= idist;
-    double r, rMu, mu;
-    const double shift = d.cm[2] - cam[2];   // flat-terrain coordinates (Rg) or 0
-    cam[2] = d.cm[2];
-    pt[2] += shift;
-    rMu = dot3(cam, v);
-    if (INSIDE) {
-        r = d.r;
-        mu = rMu * d.invr;
-    } else {
-        r = sqrt(dot3(cam, cam));
-        mu = rMu / r;
-        const double sw = fmin(fmax(d.shaft, 0.0), dist);
-        for (int c = 0; c < 3; ++c) pt[c] -= v[c] * sw;
-        const double q = rMu * rMu - r * r + d.Rt * d.Rt;
-        const double din = q >= 0.0 ? fmax(-rMu - sqrt(q), 0.0) : 0.0;
-        if (din > 0.0 && din < dist) {
-            for (int c = 0; c < 3; ++c) cam[c] += din * v[c];
-            rMu += din;
-            mu = rMu / d.Rt;
-            r = d.Rt;
-            dist -= din;
-        }
-    }
-    float4 out = make_float4(0.f, 0.f, 0.f, 0.f), ex = make_float4(1.f, 1.f, 1.f, 0.f);
-    if (INSIDE || r <= d.Rt) {
-        const double nu = dot3(v, d.sun);
-        const double muS = INSIDE ? d.muS : dot3(cam, d.sun) / r;
-        if (INSIDE) {   // r is that of :472 already
-            for (int c = 0; c < 3; ++c) pt[c] *= d.near_f;
-        } else if (r < d.near) {
-            const double f = d.near / r;
-            r *= f;
-            for (int c = 0; c < 3; ++c) pt[c] *= f;
-        }
-        double r1 = sqrt64(dot3(pt, pt)), ir1 = rcp64(r1);
-        double mu1 = dot3(pt, v) * ir1;
-        const double muS1 = dot3(pt, d.sun) * ir1;
-        float3 e;
-        if (INSIDE) {   // T_ratio with the camera's end from its row
-            const bool up = mu > 0.0;
-            const float3 x = view_T(d, t, up ? mu : -mu), y = T_at(d, r1, up ? mu1 : -mu1);
-            e = up ? make_float3(x.x / y.x, x.y / y.y, x.z / y.z) : make_float3(y.x / x.x, y.y / x.y, y.z / x.z);
-            e = make_float3(fminf(e.x, 1.f), fminf(e.y, 1.f), fminf(e.z, 1.f));
-        } else {
-            e = T_ratio(d, r, mu, r1, mu1, mu > 0.0);
-        }
-        ex = make_float4(e.x, e.y, e.z, 0.f);
-        float nw;
-        const int ne = nu_coord(d, nu, nw);
-        const double EPS = 0.004;
-        double lim;
+        const float4 p4 = pts[i];
+        double cam[3] = {d.cam[0], d.cam[1], d.cam[2]};
+        double pt[3] = {p4.x, p4.y, p4.z};
+        double v[3] = {pt[0] - cam[0], pt[1] - cam[1], pt[2] - cam[2]};
+        double dist = sqrt64_pos(dot3(v, v));   // NaN for a point at the camera or at infinity, as v is then
+        const double idist = rcp64(dist);
+        for (int c = 0; c < 3; ++c) v[c] *= idist;
+        double r, rMu, mu;
+        const double shift = d.cm[2] - cam[2];   // flat-terrain coordinates (Rg) or 0
+        cam[2] = d.cm[2];
+        pt[2] += shift;
+        rMu = dot3(cam, v);
         if (INSIDE) {
-            lim = d.lim;
+            r = d.r;
+            mu = rMu * d.invr;
         } else {
-            const double qg = d.Rg / r;
-            lim = -sqrt(1.0 - qg * qg);
-        }
-        // next to the horizon: between the two sides of it (one loop body: the lookups
-        // of both sides at once would take 250 registers)
-        const bool hor = fabs(mu - lim) < EPS;
-        const float wh = hor ? (float)(((mu - lim) + EPS) / (2.0 * EPS)) : 0.f;
-        double m = hor ? lim - EPS : mu;
-        float4 is = make_float4(0.f, 0.f, 0.f, 0.f);
-#pragma unroll 1
-        for (int h = 0; h < (hor ? 2 : 1); ++h) {
-            if (hor) {
-                r1 = sqrt64_pos(r * r + dist * dist + 2.0 * r * dist * m);
-                mu1 = (r * m + dist) * rcp64(r1);
+            r = sqrt(dot3(cam, cam));
+            mu = rMu / r;
+            const double sw = fmin(fmax(d.shaft, 0.0), dist);
+            for (int c = 0; c < 3; ++c) pt[c] -= v[c] * sw;
+            const double q = rMu * rMu - r * r + d.Rt * d.Rt;
+            const double din = q >= 0.0 ? fmax(-rMu - sqrt(q), 0.0) : 0.0;
+            if (din > 0.0 && din < dist) {
+                for (int c = 0; c < 3; ++c) cam[c] += din * v[c];
+                rMu += din;
+                mu = rMu / d.Rt;
+                r = d.Rt;
+                dist -= din;
             }
-            const float4 s0 = INSIDE ? view_S(d, t, r * m, ne, nw) : texture4D(d, r, m, muS, nu);
-            const float4 s1 = texture4D(d, r1, mu1, muS1, nu);
-            const float4 x = make_float4(fmaxf(s0.x - s1.x * e.x, 0.f), fmaxf(s0.y - s1.y * e.y, 0.f),
-                                         fmaxf(s0.z - s1.z * e.z, 0.f), fmaxf(s0.w - s1.w * e.x, 0.f));
-            is = h == 0 ? x : lerp4(is, x, wh);
-            m = lim + EPS;
         }
-        const float f = fminf(fmaxf((float)muS / 0.02f, 0.f), 1.f);  // smoothstep(0, 0.02, muS)
-        is.w *= f * f * (3.f - 2.f * f);
-        out = combine(d, is, nu);
-    }
-    rad[i] = out;
-    if (ext) ext[i] = ex;
+        float4 out = make_float4(0.f, 0.f, 0.f, 0.f), ex = make_float4(1.f, 1.f, 1.f, 0.f);
+        if (INSIDE || r <= d.Rt) {
+            const double nu = dot3(v, d.sun);
+            const double muS = INSIDE ? d.muS : dot3(cam, d.sun) / r;
+            if (INSIDE) {   // r is that of :472 already
+                for (int c = 0; c < 3; ++c) pt[c] *= d.near_f;
+            } else if (r < d.near) {
+                const double f = d.near / r;
+                r *= f;
+                for (int c = 0; c < 3; ++c) pt[c] *= f;
+            }
+            double r1 = sqrt64(dot3(pt, pt)), ir1 = rcp64(r1);
+            double mu1 = dot3(pt, v) * ir1;
+            const double muS1 = dot3(pt, d.sun) * ir1;
+            float3 e;
+            if (INSIDE) {   // T_ratio with the camera's end from its row
+                const bool up = mu > 0.0;
+                const float3 x = view_T(d, t, up ? mu : -mu), y = T_at(d, r1, up ? mu1 : -mu1);
+                e = up ? make_float3(x.x / y.x, x.y / y.y, x.z / y.z) : make_float3(y.x / x.x, y.y / x.y, y.z / x.z);
+                e = make_float3(fminf(e.x, 1.f), fminf(e.y, 1.f), fminf(e.z, 1.f));
+            } else {
+                e = T_ratio(d, r, mu, r1, mu1, mu > 0.0);
+            }
+            ex = make_float4(e.x, e.y, e.z, 0.f);
+            float nw;
+            const int ne = nu_coord(d, nu, nw);
+            const double EPS = 0.004;
+            double lim;
+            if (INSIDE) {
+                lim = d.lim;
+            } else {
+                const double qg = d.Rg / r;
+                lim = -sqrt(1.0 - qg * qg);
+            }
+            // next to the horizon: between the two sides of it (one loop body: the lookups
+            // of both sides at once would take 250 registers)
+            const bool hor = fabs(mu - lim) < EPS;
+            const float wh = hor ? (float)(((mu - lim) + EPS) / (2.0 * EPS)) : 0.f;
+            double m = hor ? lim - EPS : mu;
+            float4 is = make_float4(0.f, 0.f, 0.f, 0.f);
+#pragma unroll 1
+            for (int h = 0; h < (hor ? 2 : 1); ++h) {
+                if (hor) {
+                    r1 = sqrt64_pos(r * r + dist * dist + 2.0 * r * dist * m);
+                    mu1 = (r * m + dist) * rcp64(r1);
+                }
+                const float4 s0 = INSIDE ? view_S(d, t, r * m, ne, nw) : texture4D(d, r, m, muS, nu);
+                const float4 s1 = texture4D(d, r1, mu1, muS1, nu);
+                const float4 x = make_float4(fmaxf(s0.x - s1.x * e.x, 0.f), fmaxf(s0.y - s1.y * e.y, 0.f),
+                                             fmaxf(s0.z - s1.z * e.z, 0.f), fmaxf(s0.w - s1.w * e.x, 0.f));
+                is = h == 0 ? x : lerp4(is, x, wh);
+                m = lim + EPS;
+            }
+            const float f = fminf(fmaxf((float)muS / 0.02f, 0.f), 1.f);  // smoothstep(0, 0.02, muS)
+            is.w *= f * f * (3.f - 2.f * f);
+            out = combine(d, is, nu);
+        }
+        rad[i] = out;
+        if (ext) ext[i] = ex;
     }
 }
 

@@ -70,8 +70,7 @@ struct SetDesc {
     double tMu;          // tan(1.5) / 1.15  (getTransmittanceUV, FP64 lookups)
     float bR[3], bMS[3], bME[3];
     // FP32 constants
-    float f_Rg, f_dRt, f_inv_dRt;   // Rg, Rt - Rg, 1/(Rt - Rg)
-    float f_H, f_invH;
+    float f_Rg, f_inv_dRt;          // Rg, 1/(Rt - Rg)
     float f_tMu;                    // tan(1.5) / 1.15  (getTransmittanceUV)
     float f_tMuS;                   // tan(1.26 * 1.1)  (texture4D uMuS)
     float kR;                       // 3 / (16 pi)
@@ -84,9 +83,10 @@ struct SetDesc {
     float4 *T4, *dE4, *E4, *dSR4, *dSM4, *dJ4, *S4;
     float4 *tau4;                   // optical depth -ln T of the T texels (rgb; w: sun_centres), or null
     // transmittances along the view ray of each (layer, mu row) at the inscatter
-    // samples (trapezoid weights folded in), [RR][RMU][nsamp + 1] (w: the sample's t / r_i), and from the ground point to each layer
-    // radius per theta row of the spherical integral, [RR][NS]; null: computed
-    // inline from T (pass-level entry points)
+    // samples, trapezoid weights folded in (w: the sample's t / r_i), [RR][RMU][nsamp + 1];
+    // and from the ground point to each layer radius per theta row of the spherical
+    // integral (w: 1 for a ground row), [RR][NS]; null: computed inline from T
+    // (pass-level entry points)
     float4 *tview, *tground;
     SnView *view;                   // [RR][RMU][nsamp + 1]; null: computed in k_inscatterN
     // [RR][NS] and [SH][NI/2]; [RMUS] and [SW]; null: computed in the dJ and dE kernels
@@ -204,24 +204,14 @@ __device__ __forceinline__ float3 bilinear(const float4 *__restrict__ tab, int W
 __device__ __forceinline__ float T_ur(const SetDesc &s, float h) {
     return s.linT ? fmaxf(h, 0.0f) * s.f_inv_dRt : sqrtf(fmaxf(h, 0.0f) * s.f_inv_dRt);
 }
-template <bool LIN>   // the parameterisation fixed at compile time (inner loops)
-__device__ __forceinline__ float T_umu_t(const SetDesc &s, float mu) {
-    return LIN ? (mu + 0.15f) * (1.0f / 1.15f) : atanf((mu + 0.15f) * s.f_tMu) * (1.0f / 1.5f);
-}
 __device__ __forceinline__ float T_umu(const SetDesc &s, float mu) {
-    return s.linT ? T_umu_t<true>(s, mu) : T_umu_t<false>(s, mu);
+    return s.linT ? (mu + 0.15f) * (1.0f / 1.15f) : atanf((mu + 0.15f) * s.f_tMu) * (1.0f / 1.5f);
 }
 
-// The same T coordinates in FP64 (the sun's lookups of the single-scattering
-// pass: next to the horizon T is steep, and an FP32 coordinate's ~3e-8 moves a
-// grazing sun's T by ~1e-4).
+// uR in FP64 (the sun's lookups of the single-scattering pass)
 __device__ __forceinline__ double T_ur_d(const SetDesc &s, double h) {
     const double hc = fmax(h, 0.0), dRt = s.Rt - s.Rg;
     return s.linT ? hc / dRt : sqrt(hc / dRt);
-}
-template <bool LIN>
-__device__ __forceinline__ double T_umu_d(const SetDesc &s, double mu) {
-    return LIN ? (mu + 0.15) / 1.15 : atan((mu + 0.15) * s.tMu) / 1.5;
 }
 
 // common.glsl:223-226: T(r, mu), bilinear.
@@ -310,16 +300,6 @@ __device__ __forceinline__ float3 T_ratio_d(const SetDesc &s, double hx, double 
         }
     }
     return make_float3(r[0], r[1], r[2]);
-}
-
-// Phase functions, common.glsl:290-297.
-__device__ __forceinline__ float phaseR(const SetDesc &s, float mu) {
-    return s.kR * fmaf(mu, mu, 1.0f);
-}
-__device__ __forceinline__ float phaseM(const SetDesc &s, float mu) {
-    float x = fmaf(s.m2g, mu, s.g2p1);
-    float y = rsqrtf(x);
-    return s.kM * fmaf(mu, mu, 1.0f) * (y * y * y);
 }
 
 // sqrt in FP64 from the hardware estimate (5.3e-8) and Newton steps: 1.11e-16 relative over
@@ -419,14 +399,6 @@ __device__ __forceinline__ double tex4d_umus(const SetDesc &s, double muS) {
     return 0.5 / s.RMUS +
            (atan(fmax(muS, -0.1975) * tan(1.26 * 1.1)) / 1.1 + (1.0 - 0.26)) * 0.5 *
                (1.0 - 1.0 / s.RMUS);
-}
-
-// FP32 uMuS texel offset inside a slice: uMuS * RMUS - 0.5.
-template <bool LIN>   // the parameterisation fixed at compile time (inner loops)
-__device__ __forceinline__ float tex4d_txs_f(const SetDesc &s, float muS) {
-    if (LIN) return fmaxf(muS + 0.2f, 0.0f) * (1.0f / 1.2f) * (float)(s.RMUS - 1);
-    float a = atanf(fmaxf(muS, -0.1975f) * s.f_tMuS) * (1.0f / 1.1f) + 0.74f;
-    return a * 0.5f * (float)(s.RMUS - 1);
 }
 
 }  // namespace atmo

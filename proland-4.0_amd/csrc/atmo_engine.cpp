@@ -219,10 +219,7 @@ void fill_desc(SetDesc &s, const atmo_params &p) {
     s.bMS[0] = p.betaMSca.x; s.bMS[1] = p.betaMSca.y; s.bMS[2] = p.betaMSca.z;
     s.bME[0] = p.betaMEx.x; s.bME[1] = p.betaMEx.y; s.bME[2] = p.betaMEx.z;
     s.f_Rg = (float)s.Rg;
-    s.f_dRt = (float)(s.Rt - s.Rg);
     s.f_inv_dRt = (float)(1.0 / (s.Rt - s.Rg));
-    s.f_H = (float)s.H;
-    s.f_invH = (float)(1.0 / s.H);
     s.tMu = std::tan(1.5) / 1.15;
     s.f_tMu = (float)s.tMu;
     s.f_tMuS = (float)std::tan(1.26 * 1.1);

@@ -55,7 +55,6 @@ hipError_t launch_irradiance1(const SetDesc *sets, const uint2 *tiles, int ntile
 int theta_workgroups(int RR, int RMUS, int SW, int SH, int NS, int NI);
 hipError_t launch_geometry(const SetDesc *sets, int nsets, int wpt, const uint2 *tiles, int nview, int nsamp, int NS, int NI,
                            hipStream_t st);
-// linT / lin4: the sets' parameterisation flags (one per batch), compiled in
 // G: texels per thread (2, 3, 4 or 8); CH: theta rows per staging round; RNU:
 // the largest RES_NU of the launch's sets; DS: slots of the workgroup's threads the
 // theta rows are dealt to (1: none; more: all rows staged at once)
@@ -66,7 +65,8 @@ hipError_t launch_irradianceN(const SetDesc *sets, const uint2 *tiles, int ntile
                               const void *dirs, bool first, size_t lds, hipStream_t st);
 // The dSn pass, one mu row (tile) per workgroup.  form: 0 direct gathers, 1
 // LDS-staged rows (both read SetDesc::view and tview), 2 LDS-staged rows without
-// SetDesc::view.  W4max: the most texels of a row of the launch's sets.
+// SetDesc::view.  W4max: the most texels of a row of the launch's sets.  lin4: their
+// parameterisation (one per batch), compiled in.
 struct SnShape {
     int texels, threads;   // per thread (1 .. 3), per workgroup (a multiple of 64 up to 512)
 };
@@ -76,8 +76,8 @@ SnShape sn_shape(int W4);   // W4 <= 1024
 constexpr int kXkMax = 2048;   // T columns whose centres are staged for the sun lookups
 struct S1Shape {
     int axis;      // how the mu axis of the sun's T lookup is found
-    int texels;    // per thread, 1 to 3 with LDS-staged T rows, 0: gathers
-    int columns;   // T columns staged per thread (1, 2)
+    int texels;    // per thread, 1 to 4 with LDS-staged T rows, 0: gathers
+    int columns;   // T columns staged per thread (1, 2 or 4)
     int threads;   // per workgroup
 };
 S1Shape s1_shape(int W4, int TW, bool linT);

@@ -3,10 +3,13 @@
 // MLP 14 -> 256 -> 256 -> 256 -> 4 (kNL = 3 hidden layers), act() on the hidden
 // layers.  Layers are numbered as for four hidden layers: the output layer is
 // "layer 5" and the last hidden layer's activations "H4" whatever kNL is.  The
-// kNG = kNL - 1 256x256 layers (96 % of the FLOPs) run on the BF16 matrix cores
-// (v_mfma_f32_32x32x16_bf16, FP32 accumulation) in one LDS-tiled GEMM kernel
-// with transposable operands and fused epilogues; the thin first and last
-// layers, the loss, the reductions and Adam are FP32 vector code.
+// kNG = kNL - 1 256x256 layers hold 96 % of the FLOPs.
+//   inference (k_mlp_infer): all layers of a set's texels in one kernel, FP16 on the
+//     matrix cores with FP32 accumulation;
+//   training (k_train_rows, k_train_dw, k_train_reduce): forward and backward of a
+//     batch, bf16 hidden products, everything else FP32;
+//   predict: a kernel per layer (k_layer1_fwd, k_gemm_act, k_layer5), bf16 hidden
+//     products.
 #include "surrogate_kernels.h"
 
 #include <algorithm>
