@@ -180,16 +180,18 @@ ATMO_API atmo_status atmo_engine_pass_times(atmo_engine *e, atmo_pass_time *out,
  * the G whose workgroup-occupancy cost ceil(RES_MU * ceil(RES_NU / G) / 256) * G
  * is lowest, reported as 0) and the k_inscatterN forms (direct gathers /
  * LDS-staged blended rows) give bit-identical tables: tuning changes the time
- * only.  Times in ms: inscatterS_ms[i] for
- * 2 / 3 / 4 / 8 / per-set texels per thread (one order-2 + (orders-2) later
- * launches), inscatterN_ms[9f + x] for form f (0 direct, 1 staged), tile
+ * only.  Order 2's k_inscatterS and the later orders' are chosen apart, each by
+ * its own time.  Times in ms: inscatterS_ms[i] for
+ * 2 / 3 / 4 / 8 / per-set texels per thread (the sum of one order-2 and (orders-2)
+ * later launches), inscatterN_ms[9f + x] for form f (0 direct, 1 staged), tile
  * order x (0 mu rows, 1 XCD-banded mu rows, 2 XCD-banded view lines sorted by
  * impact parameter); -1 = not timed (the other entries of inscatterN_ms, the
  * direct form where the table of view-ray samples did not fit, the per-set
  * k_inscatterS choice when every set makes the same one). */
 typedef struct atmo_tuning {
     int tuned;
-    int inscatterS_texels_per_thread;  /* 2, 3, 4, 8; 0: per set */
+    int inscatterS_texels_per_thread;  /* 2, 3, 4, 8; 0: per set; of the orders >= 3 (of order 2
+                                          where the plan ends with it) */
     int inscatterN_rows_per_workgroup;  /* 1 */
     int inscatterN_xcd_order;      /* 0, 1 or 2 (see inscatterN_ms) */
     float inscatterS_ms[5];

@@ -1383,7 +1383,7 @@ atmo_status atmo_engine_tuning(atmo_engine *e, atmo_tuning *out) {
     if (!e || !out) return fail(ATMO_ERR_INVALID_ARGUMENT, "bad arguments");
     memset(out, 0, sizeof *out);
     out->tuned = !e->last_key.empty();
-    out->inscatterS_texels_per_thread = e->last_tuning.jG;
+    out->inscatterS_texels_per_thread = e->plan && e->plan->opts.orders == 2 ? e->last_tuning.jG1 : e->last_tuning.jG;
     out->inscatterN_rows_per_workgroup = 1;
     out->inscatterN_xcd_order = e->last_tuning.snXcd;
     for (int i = 0; i < 5; ++i) out->inscatterS_ms[i] = e->last_tuning.msJ[i];
