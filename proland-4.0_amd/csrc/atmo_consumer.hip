@@ -534,8 +534,8 @@ void view_desc(CDesc &d, bool flat) {
 constexpr int kSkyPerEntry = 128, kAerialPerEntry = 512;
 constexpr size_t kInsideLds = 64 * 1024;
 // Workgroups of 512 threads: one per CU for the sky (2073600 rays with 256 / 512 / 1024:
-// 23.1 / 25.2 / 30.4 us), two for the scattering, whose own lookups wait more
-// (921600 points: 43.9 / 39.4 / 45.7).
+// 22.2 / 23.8 / 28.0 us), two for the scattering, whose own lookups wait more
+// (921600 points: 40.6 / 34.8 / 39.5).
 constexpr int kSkyGroups = 256, kAerialGroups = 512;
 bool use_staged(const CDesc &d, int n, int per_entry) {
     const size_t entries = view_entries(d);

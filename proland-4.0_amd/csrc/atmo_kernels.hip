@@ -60,11 +60,11 @@ __device__ __forceinline__ double tan_col(double x) {
 // Pass T — transmittance.glsl:78-98.  FP64 trapezoid of exp(-h/H) for both
 // scale heights at once; 16 lanes share one texel's samples.
 // tile = 16 consecutive texels.  Bound by FP64 issue: the library's exp and square
-// root take about 95 instructions a sample, exp2_64 and sqrt64 50, and the tables are
+// root take about 95 instructions a sample, exp2_64 and sqrt64_pos 54, and the tables are
 // FP32 (256x64 texels, 500 samples: 28 -> 21 us); nearly half of the texels of the
 // tangent parameterisation look at the ground and need no samples, and straight code
-// without the library's argument reductions is fetched in time (-> 19.4; 24 sets 515 ->
-// 290 us).  A single set is left with its latency: 4 waves per SIMD, half of them idle.
+// without the library's argument reductions is fetched in time (-> 20; 24 sets 515 ->
+// 310 us).  A single set is left with its latency: 4 waves per SIMD, half of them idle.
 // ---------------------------------------------------------------------------
 __global__ __launch_bounds__(256) void k_transmittance(const SetDesc *__restrict__ sets,
                                                        const uint2 *__restrict__ tiles,
