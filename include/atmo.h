@@ -156,7 +156,9 @@ typedef struct atmo_tables {
 /* Batched precompute of nsets independent parameter sets (each with its own
  * table resolutions) into caller-allocated device tables out[0..nsets).
  * Work tables are allocated (and kept) by the engine.  Replaces running the
- * reference's preprocess once per set. */
+ * reference's preprocess once per set.  On a stream in capture: with the sets, options
+ * and outputs of the engine's last call only; the captured graph uses the engine's work
+ * tables, until the engine's next call with others. */
 ATMO_API atmo_status atmo_engine_precompute(atmo_engine *e, const atmo_params *sets, int nsets,
                                             const atmo_options *opts, const atmo_tables *out,
                                             void *stream);

@@ -1155,6 +1155,12 @@ atmo_status run_plan(atmo_engine *e, Plan &pl, const atmo_options &o, hipStream_
     const bool first = !pl.ran;
     pl.ran = true;
     pl.done_behind = false;
+    // Into a caller's capture the kernels are launched one by one: a graph launched there is not
+    // captured (the caller's graph stays empty), and an event recorded there could not be
+    // waited for outside it
+    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+    if (hs) HIPCHK(hipStreamIsCapturing(hs, &cap));
+    const bool capturing = cap != hipStreamCaptureStatusNone;
     if (o.flags & ATMO_FLAG_TIME_PASSES) {
         PassTimer tm;
         tm.on = true;
@@ -1166,23 +1172,16 @@ atmo_status run_plan(atmo_engine *e, Plan &pl, const atmo_options &o, hipStream_
             HIPCHK(hipEventElapsedTime(&ms, r.a, r.b));
             e->times.push_back({r.pass, r.order, ms});
         }
-    } else if (first || (o.flags & ATMO_FLAG_NO_GRAPH)) {
+    } else if (first || capturing || (o.flags & ATMO_FLAG_NO_GRAPH)) {
         if ((st = launch_all(pl, hs)) != ATMO_OK) return st;
-        if (first) {
-            // (an event recorded into a caller's capture could not be waited for outside it)
-            hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
-            if (hs) HIPCHK(hipStreamIsCapturing(hs, &cap));
-            if (cap == hipStreamCaptureStatusNone) {
-                if (!pl.done) HIPCHK(hipEventCreateWithFlags(&pl.done, hipEventDisableTiming));
-                HIPCHK(hipEventRecord(pl.done, hs));
-                pl.done_behind = true;
-            }
+        if (first && !capturing) {
+            if (!pl.done) HIPCHK(hipEventCreateWithFlags(&pl.done, hipEventDisableTiming));
+            HIPCHK(hipEventRecord(pl.done, hs));
+            pl.done_behind = true;
         }
     } else {
-        hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
-        if (!pl.gexec && hs) HIPCHK(hipStreamIsCapturing(hs, &cap));
-        bool eager = cap != hipStreamCaptureStatusNone;   // no capture inside the caller's
-        if (!pl.gexec && !eager) {
+        bool eager = false;
+        if (!pl.gexec) {
             HIPCHK(hipStreamBeginCapture(e->cap, hipStreamCaptureModeThreadLocal));
             atmo_status cs = launch_all(pl, e->cap);
             hipGraph_t g = nullptr;

@@ -1041,3 +1041,32 @@ def test_precision_study_configuration(eng):
     err = np.abs(flat - g["S_val"]) / den
     print("S samples max %s mean %.3e" % (np.array2string(err.max(axis=0), precision=3), err.mean()), flush=True)
     assert err.max() <= TOL
+
+
+@pytest.mark.parametrize("flags", [0, FLAG_NO_AUTOTUNE])
+@pytest.mark.parametrize("before", [1, 2, 3])
+def test_precompute_in_a_callers_capture(before, flags):
+    """A call with the sets and outputs of the one before it, captured after 1 to 3 calls
+    (the engine has no graph of its own yet, or has one): every replay gives the eager
+    call's tables, with eager calls between the replays."""
+    p, o = small(res=(6, 16, 6, 4)), options(flags=flags)
+    e = L.Engine(0)
+    st = torch.cuda.Stream()
+    outs = [L.alloc_outputs(p)]
+    for _ in range(before):
+        e.precompute([p], o, outs=outs, stream=st)
+    st.synchronize()
+    ref = [t.clone() for t in outs[0]]
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g, stream=st):
+        e.precompute([p], o, outs=outs, stream=st)
+    for _ in range(3):
+        for run in (g.replay, lambda: e.precompute([p], o, outs=outs, stream=st)):
+            for t in outs[0]:
+                t.fill_(-1.0)
+            torch.cuda.synchronize()
+            run()
+            torch.cuda.synchronize()
+            for a, b in zip(outs[0], ref):
+                assert torch.equal(a, b)
+    e.close()
